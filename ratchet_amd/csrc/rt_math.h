@@ -9,11 +9,26 @@
 typedef _Float16 half_t;
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
+// n / d for operands and a quotient far from overflow and from the subnormals: the reciprocal, the quotient, one
+// correction by the exact remainder.  Four instructions where the general division takes ten, which also refine the
+// reciprocal, scale the operands and put the special cases right.  This is not correctly rounded for every pair of
+// operands: rt_tanhf's two divisions see only the pairs that its 2^32 arguments lead to, and on this chip all of its
+// results (and GELU's) equal those with the general division.
+__device__ __forceinline__ float rt_div_mid(float n, float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float q = n * r;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), r, q);
+}
+
 #define RT_FN __device__ inline
 #define RT_TABLE __device__ static const
+#define RT_DIV(n, d) rt_div_mid(n, d)
+#define RT_MED3(v, lo, hi) __builtin_amdgcn_fmed3f(v, lo, hi)
 #include "rt_libm.h"
 #undef RT_FN
 #undef RT_TABLE
+#undef RT_DIV
+#undef RT_MED3
 
 // ---- 16-bit helpers -------------------------------------------------------------------------------------
 __device__ __forceinline__ float h2f(half_t h) { return (float)h; }

@@ -413,3 +413,20 @@ def test_empty_tensors_are_no_ops(dev):
     ]
     assert calls == [0] * len(calls), calls
     assert same_bits(y.to_numpy(), keep)
+
+
+# ---------------------------------------------------------------- f32 tanh / gelu where the tanh changes its course
+@pytest.mark.parametrize("op", ["tanh", "gelu"])
+def test_tanh_and_gelu_bits_over_the_float_range(dev, oracle, op):
+    """Every 1021st bit pattern, and each boundary of the algorithm (|x| = 1 and 22, the whole multiples of ln2 / 2 that
+    its reduction subtracts and the half ones at which it goes to the next, the subnormals, infinity, NaN) with its
+    neighbours: the same bits as the C library's."""
+    marks = [1.0, 22.0, 2.0 ** -126, 2.0 ** -149, 2.0 ** -26, 2.0 ** -55] + [k * np.log(2) / 4 for k in range(1, 130)]
+    near = np.array(marks, np.float32).view(np.uint32)[:, None].astype(np.int64) + np.arange(-3, 4)
+    bits = np.concatenate([np.arange(0, 2 ** 32, 1021, dtype=np.int64), near.ravel(), near.ravel() + 2 ** 31, [0x7f800000, 0xff800000, 0x7fc00000, 0x80000000]])
+    bits = bits[(bits >= 0) & (bits < 2 ** 32)]
+    x = bits.astype(np.uint32).view(np.float32)
+    got, want = dev.unary(op, dev.upload(x)).to_numpy(), oracle.unary(op, x)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32))
