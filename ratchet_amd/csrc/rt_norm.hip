@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__
 // there once at the start, and after the statistics the block reads LDS, normalises and streams the result out,
 // instead of fetching x a second time through a loop of dependent load / store pairs.
 constexpr int NP_BLOCK = 320;
-constexpr uint32_t NP_KEEP_MAX_COLS = 4096;
+constexpr uint32_t NP_KEEP_MAX_COLS = 3072;
 constexpr size_t NP_KEEP_BYTES_PER_TILE = 256 * 16 + 2 * 32 * 16;   // the block's x vectors, one scale and one bias vector per column group
 typedef _Float16 np_h8 __attribute__((ext_vector_type(8)));
 // run += the 32 f16 values packed in four vectors, left to right: each add is 1.0 * widen(f16) + run in one instruction
@@ -668,6 +668,259 @@ __global__ void __launch_bounds__(NP_BLOCK) norm_pipe16_kernel(const T* __restri
                 st_stream(reinterpret_cast<v4u*>(yrow) + c, out.u);
             }
         }
+    }
+}
+
+// The same walk for rows of 8 to NF_MAX_COLS columns as a stream: persistent blocks that take groups of 8 rows in turn.
+// The loader threads keep a group's rows in registers (NT vectors a thread) from the load to the store, and in step t of
+// a group, while wave 0 walks tile t, they normalise and store tile t of the group before and load the tile PF steps
+// ahead, across the groups: x is read once, and reads, walk and writes go on side by side instead of in phases that all
+// blocks of the chip pass at the same time.
+// What bounds it: with one group per block the walk (about 2.3 ns a column, whatever is left of the chip); with several,
+// memory, and in bf16 the vector instructions of the output (58 us for the [16384,3072] LayerNorm whose bytes take 38 at
+// the rate of a large copy; f16 43).  A walker occupies its SIMD's vector unit fully with 8 rows as with 30, which is why a block carries
+// up to 30 rows and a CU one block: with blocks of 8 rows, two to a CU, the same LayerNorm took 54 us in f16.
+// Rows of any length from 8 columns and on any element boundary: no access leaves the row; the last vector of a row is
+// its last eight elements, for the walk shifted so that none of them counts twice, and written with the same values as
+// the one before it where they overlap.
+// A row's vector is 16 bytes at `base + offset` through a buffer descriptor of the group's rows; where there is nothing to
+// load or to store (columns past the end, rows past the end, the group before the first) the offset lies outside of it and
+// the access is dropped, which keeps the step free of branches around memory instructions: the compiler then counts
+// exactly how many may stay in flight at each wait.
+// f rounded to bf16 and widened again, in one instruction: converted into the high half of a word whose low half is bf16(0) = 0
+__device__ __forceinline__ float np_round_bf16(float f) {
+    uint32_t r;
+    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(f));
+    return u2f(r);
+}
+// norm_one, with a bias, on the eight elements of a vector.  bf16 goes in f32 form from step to step, two instructions each (through
+// Ar<bf16_t> the roundings and widenings take four), and is packed once at the end.
+template <typename T, int KIND> __device__ __forceinline__ v4u norm_vec16(const v4u& x, const RowStats<T>& st, const v4u& scale, const v4u& bias) {
+    v4u out;
+    if constexpr (std::is_same<T, bf16_t>::value) {
+        const float mu = Ar<T>::widen(st.mu), rs = Ar<T>::widen(st.r);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            float v[2] = {u2f(x[w] << 16), u2f(x[w] & 0xffff0000u)};
+            const float s[2] = {u2f(scale[w] << 16), u2f(scale[w] & 0xffff0000u)}, b[2] = {u2f(bias[w] << 16), u2f(bias[w] & 0xffff0000u)};
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (KIND == NORM_LAYER) v[h] = np_round_bf16(v[h] - mu);
+                v[h] = np_round_bf16(v[h] * rs) * s[h];
+                if (KIND == NORM_LAYER) v[h] = np_round_bf16(v[h]) + b[h];
+            }
+            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(out[w]) : "v"(v[0]), "v"(v[1]));
+        }
+    } else {
+        np_h8 v = __builtin_bit_cast(np_h8, x);
+        if (KIND == NORM_LAYER) v = v - st.mu;
+        v = v * st.r * __builtin_bit_cast(np_h8, scale);
+        if (KIND == NORM_LAYER) v = v + __builtin_bit_cast(np_h8, bias);
+        out = __builtin_bit_cast(v4u, v);
+    }
+    return out;
+}
+constexpr uint32_t NF_MAX_COLS = 5120;                       // 20 vectors a thread
+// run += the sixteen f32 values of four vectors, left to right (as one asm statement: with ordinary adds the compiler reads
+// a whole tile ahead, into 256 registers)
+__device__ __forceinline__ void np_add_f32x16(float& run, const v4u& a, const v4u& b, const v4u& c, const v4u& d) {
+#define NP_ADD(N) "v_add_f32 %0, %0, %" #N "\n"
+    asm(NP_ADD(1) NP_ADD(2) NP_ADD(3) NP_ADD(4) NP_ADD(5) NP_ADD(6) NP_ADD(7) NP_ADD(8) NP_ADD(9) NP_ADD(10) NP_ADD(11) NP_ADD(12) NP_ADD(13)
+        NP_ADD(14) NP_ADD(15) NP_ADD(16)
+        : "+v"(run)
+        : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]),
+          "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]));
+#undef NP_ADD
+}
+template <typename T, int KIND, int NT, int RB>
+__global__ void __launch_bounds__(64 + RB * 32) norm_flow16_kernel(const T* x, const T* __restrict__ scale, const T* __restrict__ bias, T* y,
+                                                               uint64_t rows, uint32_t cols, uint32_t groups, uint32_t R, float eps) {
+    constexpr int TC = 256, PAD = 4, PAD16 = 8;
+    constexpr int PF = 2;                                      // tiles loaded ahead; a group's step t uses slot t % PF
+    constexpr int NSUM = (KIND == NORM_LAYER) ? 2 : 1;
+    constexpr bool H16 = std::is_same<T, half_t>::value;                         // 16-bit tiles and the fma_mix chain
+    constexpr int PITCH = H16 ? (TC + PAD16) * 2 / 16 : (TC + PAD) * 4 / 16;     // of a tile row, in 16-byte vectors
+    constexpr int NW = H16 ? 4 : 8;                                              // vectors that hold 32 values
+    static_assert(NT % 2 == 0 && NT % PF == 0, "the two tile buffers and the load slots are those of the same step in every group");
+    __shared__ v4u tile[2][NSUM][RB][PITCH];                                     // [.][0] = squares, [.][1] = values
+    __shared__ float sums[2][NSUM][RB];                                          // of the block's even and odd groups
+    extern __shared__ __attribute__((aligned(16))) v4u nf_affine[];              // [ntiles * 32] scale, the same of bias
+    const uint32_t ntiles = (cols + TC - 1) / TC, nvec = (cols + 7) / 8;         // ntiles <= NT; steps beyond it are empty
+    const uint32_t n_mine = (groups - blockIdx.x + gridDim.x - 1) / gridDim.x;   // groups of this block: blockIdx.x, + gridDim.x, ...
+
+    // Barriers: one per step (tile t is in LDS; wave 0 passes the one of step t + 1 when it has read all of tile t) and one
+    // at the end (the last group's sums are published).
+    if (threadIdx.x < 64) {
+        // ---------------------------------------------------------------- wave 0: the sequential sums
+        __builtin_amdgcn_s_setprio(3);
+        const uint32_t wrow = threadIdx.x % RB, wsum = (threadIdx.x / RB) % NSUM;   // lanes beyond NSUM * RB shadow and never publish
+        for (uint32_t it = 0; it < n_mine; it++) {
+            float run = 0.0f;
+            __syncthreads();                                                    // tile 0 is in LDS
+            v4u cur[NW], nxt[NW];
+#pragma unroll
+            for (int k = 0; k < NW; k++) cur[k] = nxt[k] = tile[0][wsum][wrow][k];
+            for (uint32_t t = 0; t < ntiles; t++) {
+                const v4u* here = tile[t & 1][wsum][wrow];
+                const v4u* next = tile[(t + 1) & 1][wsum][wrow];
+#pragma unroll
+                for (int c = 0; c < TC / 32; c++) {
+                    if (c + 1 < TC / 32) {
+#pragma unroll
+                        for (int k = 0; k < NW; k++) nxt[k] = here[(c + 1) * NW + k];
+                    } else if (t + 1 < ntiles) {
+                        // taken before the tile's last 32 adds, whose operands are in registers: the chain does not wait
+                        // for LDS at the next tile's start
+                        __syncthreads();                                        // tile t + 1 is in LDS
+#pragma unroll
+                        for (int k = 0; k < NW; k++) nxt[k] = next[k];
+                    }
+                    if constexpr (H16) {
+                        np_add_f16x32(run, cur[0], cur[1], cur[2], cur[3]);
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < NW; k += 4) np_add_f32x16(run, cur[k], cur[k + 1], cur[k + 2], cur[k + 3]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < NW; k++) cur[k] = nxt[k];
+                }
+            }
+            if (threadIdx.x < NSUM * RB) sums[it & 1][wsum][wrow] = run;
+            for (uint32_t t = ntiles; t < (uint32_t)NT; t++) __syncthreads();   // the empty steps
+        }
+        __syncthreads();                                                        // the last group's sums are published
+        return;
+    }
+
+    // -------------------------------------------------------------------- waves 1..4: load, square, normalise, store
+    const uint32_t lt = threadIdx.x - 64;
+    const uint32_t r = lt >> 5, cv = lt & 31;                                   // row, vector within the tile
+    const uint32_t row_bytes = cols * 2;
+    constexpr uint32_t OOB = 0x80000000u;
+    const uint32_t last = ntiles - 1;
+    // This thread's vector of a tile: where it starts in its row, in bytes from the tile's first column.  In a row's last
+    // tile the last vector starts eight elements before the row's end, and there is none behind it.
+    const uint32_t tail_col = last * TC + cv * 8;
+    const uint32_t off_main = cv * 16;
+    const uint32_t off_tail = tail_col >= cols ? OOB : ((tail_col + 8 > cols ? cols - 8 : tail_col) - last * TC) * 2;
+    const uint32_t drop = tail_col < cols && tail_col + 8 > cols ? tail_col + 8 - cols : 0u;    // its elements that the vector before holds too
+    // of tile t: its first column is added last (it may take an `off_tail` from before the tile back into the row)
+    auto pick = [&](uint32_t t, uint32_t row, uint32_t row_tail) -> uint32_t {
+        uint32_t l = last;
+        asm volatile("" : "+s"(l));                                             // compared afresh: kept in registers, the masks of all steps would spill
+        return (t < l ? row : t == l ? row_tail : OOB) + t * (TC * 2);
+    };
+    struct Group {                                                              // the same for the whole block but for `row`
+        const T* x;                                                             // 16-byte boundary at or before the first row
+        T* y;
+        uint32_t bytes_x, bytes_y;                                              // from there to the last row's end
+        uint32_t row_x, row_y, tail_x, tail_y;                                  // this thread's vector in tile 0 and in the last one (less its columns), or OOB
+    };
+    auto group_of = [&](uint32_t it) -> Group {
+        Group g;
+        const uint64_t row0 = ((uint64_t)blockIdx.x + (uint64_t)it * gridDim.x) * R;
+        const bool ok = it < n_mine;
+        const uint32_t nrows = !ok ? 0u : rows - row0 < (uint64_t)R ? (uint32_t)(rows - row0) : R;
+        const T* gx = x + (ok ? row0 : 0) * cols;
+        T* gy = y + (ok ? row0 : 0) * cols;
+        const uint32_t sx = (uint32_t)((uintptr_t)gx & 15u), sy = (uint32_t)((uintptr_t)gy & 15u);
+        g.x = reinterpret_cast<const T*>(reinterpret_cast<const char*>(gx) - sx);
+        g.y = reinterpret_cast<T*>(reinterpret_cast<char*>(gy) - sy);
+        g.bytes_x = sx + nrows * row_bytes;
+        g.bytes_y = sy + nrows * row_bytes;
+        const bool have = r < nrows, have_tail = have && off_tail != OOB;
+        g.row_x = have ? sx + r * row_bytes + off_main : OOB;
+        g.row_y = have ? sy + r * row_bytes + off_main : OOB;
+        g.tail_x = have_tail ? sx + r * row_bytes + off_tail : OOB;
+        g.tail_y = have_tail ? sy + r * row_bytes + off_tail : OOB;
+        return g;
+    };
+    auto load = [&](const Group& g, uint32_t t) -> v4u {
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(g.x), 0, g.bytes_x, 0x00020000);
+        return __builtin_amdgcn_raw_buffer_load_b128(rx, pick(t, g.row_x, g.tail_x), 0, 2);            // 2: non-temporal
+    };
+    Group cur = group_of(0), nxt = group_of(1), prev = group_of(n_mine);        // prev: no rows, its stores are dropped
+    v4u pre[PF], held[NT];
+#pragma unroll
+    for (int k = 0; k < PF; k++) pre[k] = load(cur, k);
+    for (uint32_t c = lt; c < nvec; c += RB * 32) {
+        const uint32_t at = c * 8 + 8 > cols ? cols - 8 : c * 8;
+        v4u v;
+        __builtin_memcpy(&v, scale + at, 16);
+        nf_affine[c] = v;
+        if (KIND == NORM_LAYER) {                                               // without a bias -0, which changes no value that it is added to
+            v = v4u{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+            if (bias) __builtin_memcpy(&v, bias + at, 16);
+            nf_affine[ntiles * (TC / 8) + c] = v;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++) held[t] = v4u{0u, 0u, 0u, 0u};
+    RowStats<T> st;
+    st.mu = st.r = Ar<T>::conv(0.0f);
+    auto put = [&](int t) {                                                     // tile t of the group before
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(prev.y, 0, prev.bytes_y, 0x00020000);
+        uint32_t l = last, c = cv;                                              // opaque: else all of scale and bias is kept in registers across the groups
+        asm volatile("" : "+s"(l), "+v"(c));
+        c += ((uint32_t)t < l ? (uint32_t)t : l) * (TC / 8);
+        const v4u sc = nf_affine[c], bi = KIND == NORM_LAYER ? nf_affine[ntiles * (TC / 8) + c] : v4u{0u, 0u, 0u, 0u};
+        const v4u out = norm_vec16<T, KIND>(held[t], st, sc, bi);
+        __builtin_amdgcn_raw_buffer_store_b128(out, ry, pick(t, prev.row_y, prev.tail_y), 0, 2);
+    };
+    for (uint32_t it = 0; it < n_mine; it++) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const v4u mine = pre[t % PF];                                       // zeros past the row's end: +0.0 terms leave the running sums
+            uint32_t l = last;
+            asm volatile("" : "+s"(l));
+            if ((uint32_t)t <= l) {
+                v4u xv = mine;
+                if ((uint32_t)t == l) {                                         // only the elements that the vector before does not hold
+                    if (drop & 1) xv = v4u{(xv[0] >> 16) | (xv[1] << 16), (xv[1] >> 16) | (xv[2] << 16), (xv[2] >> 16) | (xv[3] << 16), xv[3] >> 16};
+                    if (drop & 2) xv = v4u{xv[1], xv[2], xv[3], 0u};
+                    if (drop & 4) xv = v4u{xv[2], xv[3], 0u, 0u};
+                }
+                if constexpr (H16) {
+                    const np_h8 h = __builtin_bit_cast(np_h8, xv);
+                    tile[t & 1][0][r][cv] = __builtin_bit_cast(v4u, h * h);     // T(x*x): eight f16 products, each rounded once
+                    if (KIND == NORM_LAYER) tile[t & 1][NSUM - 1][r][cv] = xv;
+                } else {
+                    v4u sq[2], wide[2];
+#pragma unroll
+                    for (int w = 0; w < 4; w++) {
+                        const float lo = u2f(xv[w] << 16), hi = u2f(xv[w] & 0xffff0000u);
+                        wide[w / 2][w % 2 * 2] = f2u(lo);
+                        wide[w / 2][w % 2 * 2 + 1] = f2u(hi);
+                        sq[w / 2][w % 2 * 2] = f2u(np_round_bf16(lo * lo));
+                        sq[w / 2][w % 2 * 2 + 1] = f2u(np_round_bf16(hi * hi));
+                    }
+                    tile[t & 1][0][r][cv * 2] = sq[0];
+                    tile[t & 1][0][r][cv * 2 + 1] = sq[1];
+                    if (KIND == NORM_LAYER) {
+                        tile[t & 1][NSUM - 1][r][cv * 2] = wide[0];
+                        tile[t & 1][NSUM - 1][r][cv * 2 + 1] = wide[1];
+                    }
+                }
+            }
+            pre[t % PF] = t + PF < NT ? load(cur, t + PF) : load(nxt, t + PF - NT);
+            __syncthreads();                                                    // tile t is in LDS; with t = 0 the sums of the group before
+            if (t == 0)
+                st = finish_stats<T, KIND>(KIND == NORM_LAYER ? sums[(it & 1) ^ 1][NSUM - 1][r] : 0.0f, sums[(it & 1) ^ 1][0][r], cols, eps);
+            put(t);
+#pragma unroll
+            for (int w = 0; w < 4; w++) asm volatile("v_mov_b32 %0, %1" : "+v"(held[t][w]) : "v"(mine[w]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        prev = cur;
+        cur = nxt;
+        nxt = group_of(it + 2);
+    }
+    __syncthreads();                                                            // the last group's sums are published
+    st = finish_stats<T, KIND>(KIND == NORM_LAYER ? sums[(n_mine & 1) ^ 1][NSUM - 1][r] : 0.0f, sums[(n_mine & 1) ^ 1][0][r], cols, eps);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        put(t);
+        if (t % 3 == 2) __builtin_amdgcn_sched_barrier(0);                      // not all of scale and bias at once
     }
 }
 
@@ -1352,6 +1605,29 @@ int launch_norm16_rb(rt_device* dev, const void* x, const void* scale, const voi
     return RT_OK;
 }
 
+template <typename T, int KIND, int RB>
+int launch_norm16_flow(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
+    // one block per CU; the groups as even as they can be over the fewest rounds
+    const uint64_t cus = (uint64_t)dev->num_cus, rounds = (rows + cus * RB - 1) / (cus * RB);
+    const uint32_t R = (uint32_t)((rows + cus * rounds - 1) / (cus * rounds));
+    const uint64_t groups = (rows + R - 1) / R;
+    RT_REQUIRE(groups <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");
+    const uint32_t nt = (cols + 255) / 256;
+    const size_t affine_bytes = (size_t)nt * 512 * (KIND == NORM_LAYER ? 2 : 1);
+#define RT_FLOW(NT)                                                                                                                  \
+    hipLaunchKernelGGL((norm_flow16_kernel<T, KIND, NT, RB>), dim3((unsigned)(groups < cus ? groups : cus)), dim3(64 + RB * 32),     \
+                       affine_bytes, dev->stream, (const T*)x, (const T*)scale, (const T*)bias, (T*)y, rows, cols, (uint32_t)groups, R, eps)
+    if (nt <= 2) RT_FLOW(2);
+    else if (nt <= 4) RT_FLOW(4);
+    else if (nt <= 8) RT_FLOW(8);
+    else if (nt <= 12) RT_FLOW(12);
+    else if (nt <= 16) RT_FLOW(16);
+    else RT_FLOW(20);
+#undef RT_FLOW
+    RT_CHECK_LAUNCH("norm_flow16_kernel");
+    return RT_OK;
+}
+
 // the row walk is latency bound, so prefer many small row groups until the chip is covered a few times over
 template <typename T, int KIND>
 int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
@@ -1364,6 +1640,27 @@ int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* 
     // where rows come in several rounds ([8192,3072] 25.5 against 22.1 us, [65536,512] 43 against 25).
     if (vec_ok && KIND == NORM_RMS && cols >= 256 && cols <= 4096 && rows <= 16ull * (uint64_t)dev->num_cus)
         return launch_rms16_par<T>(dev, x, scale, y, rows, cols, eps);
+    // The streaming kernel: rows that are not whole aligned vectors always (against norm_seq16_kernel: [1001,1001] 23.5 ->
+    // 6.8 us, [8000,1001] 35.8 -> 12, RMSNorm [16000,3001] bf16 127 -> 50).  Rows of whole vectors where they are many or long:
+    // there the kernel below reads x twice and puts a walker for every 8 rows on the SIMDs (LayerNorm [16384,3072] f16
+    // 52 -> 43 us, bf16 74 -> 58, RMSNorm bf16 55 -> 46; [32768,4096] f16 123 -> 100, RMSNorm bf16 135 -> 105).  In between
+    // that one's several blocks per CU win: [8192,2560] f16 19 against 23 us, [4096,1024] 6.9 against 7.5, and so they
+    // do for short rows ([16384,384] f16 9.8 against 10.8).  bf16 LayerNorm, whose walker needs the f32 tiles of both
+    // sums, gains earlier: [8192,1024] 16.6 -> 14.6 us, [2048,2560] 16.4 -> 14.9.
+    const uint64_t cus = (uint64_t)dev->num_cus;
+    const bool many = rows > 40 * cus;
+    bool flow = cols >= 8 && cols <= NF_MAX_COLS;
+    if (flow && vec_ok) {
+        const bool bf16_layer = std::is_same<T, bf16_t>::value && KIND == NORM_LAYER;
+        flow = cols > NP_KEEP_MAX_COLS || (many && cols > 512) || (bf16_layer && (rows > 24 * cus || (rows <= 8 * cus && cols > 512)));
+    }
+    if (flow) {
+        // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; with fewer rows than that gives
+        // every CU, fewer, so that all of them have some
+        if (many) return launch_norm16_flow<T, KIND, 30>(dev, x, scale, bias, y, rows, cols, eps);
+        if (rows > 8 * cus) return launch_norm16_flow<T, KIND, 16>(dev, x, scale, bias, y, rows, cols, eps);
+        return launch_norm16_flow<T, KIND, 8>(dev, x, scale, bias, y, rows, cols, eps);
+    }
     if (vec_ok) {
         const uint64_t blocks = (rows + 7) / 8;
         RT_REQUIRE(blocks <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");

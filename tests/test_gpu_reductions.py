@@ -500,6 +500,42 @@ def test_norms_16_bit_both_output_passes(dev, oracle, rows, cols, kind):
         assert np.array_equal(np.asarray(got).view(np.uint16), np.asarray(want).view(np.uint16)), (name, rows, cols, kind)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 8), (7, 9), (9, 255), (2049, 257), (300, 1001), (33, 2047), (2100, 3071), (8, 4097), (300, 5113), (300, 5120), (6200, 520),   # one group a block
+                                       (10300, 13), (10300, 520), (11000, 777), (16000, 1041), (31000, 264)])                                                         # several, the last ones short
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_streaming_kernel(dev, oracle, rows, cols, kind):
+    """Rows that are not whole vectors, long rows and many rows stream through persistent blocks: the oracle's bits, for
+    tensors that start 2, 6 and 14 bytes past a 16-byte boundary as well (x and y not alike) and for y == x, and not a
+    byte written outside of y."""
+    rng = np.random.default_rng(316)
+    bf = kind == "bf16"
+    conv = (lambda a: _bf16(oracle, a)) if bf else (lambda a: np.asarray(a, np.float32).astype(np.float16))
+    x = conv(rng.standard_normal((rows, cols)) * 1.5 + 0.25)
+    w, b = conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols))
+    dw, db = dev.upload(w, bf16=bf), dev.upload(b, bf16=bf)
+    want = {"layer": oracle.layer_norm(x, w, b, 1e-5, bf16=bf, intended=True), "plain": oracle.layer_norm(x, w, None, 1e-5, bf16=bf, intended=True),
+            "rms": oracle.rms_norm(x, w, 1e-5, bf16=bf, intended=True)}
+
+    def run(name, src, dst):
+        if name == "rms":
+            dev.rms_norm(src, dw, 1e-5, out=dst)
+        else:
+            dev.layer_norm(src, dw, db if name == "layer" else None, 1e-5, out=dst)
+
+    for xo, yo in ((0, 0), (1, 0), (3, 7)):
+        flat = np.zeros(rows * cols + 16, x.dtype)
+        flat[xo:xo + rows * cols] = x.ravel()
+        src = dev.upload(flat, bf16=bf)
+        for name in want:
+            dst = dev.upload(np.full(rows * cols + 16, 7, x.dtype), bf16=bf)
+            run(name, src.view(xo, (rows, cols)), dst.view(yo, (rows, cols)))
+            got = dst.to_numpy()
+            assert np.array_equal(got[yo:yo + rows * cols].view(np.uint16), np.asarray(want[name]).view(np.uint16).ravel()), (name, xo, yo)
+            assert (got[:yo] == 7).all() and (got[yo + rows * cols:] == 7).all(), (name, xo, yo)
+        run("layer", src.view(xo, (rows, cols)), src.view(xo, (rows, cols)))
+        assert np.array_equal(src.to_numpy()[xo:xo + rows * cols].view(np.uint16), np.asarray(want["layer"]).view(np.uint16).ravel()), ("in place", xo)
+
+
 @pytest.mark.parametrize("cols", [256, 512, 1000, 1536, 2560, 3072, 4096])
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_rms_norm_16_bit_row_sums_replayed_in_parallel(dev, oracle, cols, kind):
