@@ -42,7 +42,7 @@ struct rt_device {
     unsigned np_attr_set;   // 16-bit norm instantiations (LDS-resident rows) whose dynamic-LDS limit has been raised on this device
     uint64_t sp_attr_set;   // streaming softmax instantiations whose dynamic-LDS limit has been raised on this device
     uint64_t sp_ragged_attr_set;   // the same for the ragged-row variants
-    uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads
+    uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads (bits 0..15) and for those of f16 rows of 4097 to 8192 columns
     unsigned ry_attr_set;          // the same for the one-wave-per-row softmax (rt_softmax_replay.hip)
     uint16_t rp_resident[2][9];    // wave-per-row RMSNorm: blocks of an instantiation ([f16, bf16][vectors per lane]) that one CU holds; 0 = not asked yet
     // row sums of one launch of the streaming softmax's ragged-row variant (RT_SM_ROW_SUMS 16-bit values, allocated with the device)

@@ -170,7 +170,11 @@ template <> struct SpType<bf16_t> {
 // finished by softmax16_edges_kernel from x, the table and that sum.  An aligned vector that holds one byte of the tensor
 // lies in a mapped page, so the loads are safe at the tensor's ends too.  A row's span can be one vector longer than
 // NSTEP steps hold (2047 columns starting 14 bytes into a vector): wave 0 reads that vector itself and adds it last.
-template <typename T, int NSTEP, bool FULL, int MASK, bool RAGGED = false>
+//
+// LONG (rows of SP_TC * SP_MAX_STEPS up to twice that many columns): a group has 15 rows and a step 1024 columns.  The two
+// vectors a loader thread handles in a step lie 512 columns apart in ONE row instead of in two rows, and the walker walks
+// 1024 columns between barriers, so that the registers hold rows twice as long and x is read and y written once.
+template <typename T, int NSTEP, bool FULL, int MASK, bool RAGGED = false, bool LONG = false>
 __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16_t* __restrict__ table, const T* x, const T* mask, T* y,
                                                                     uint64_t rows, uint32_t cols, SpSched sch, uint16_t* row_sums,
                                                                     const uint32_t* __restrict__ tiles) {
@@ -186,10 +190,14 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     // mask), so one mask vector serves both and the register of the second holds the mask of the step after next
     constexpr bool PAIR = MASK == 2;
     static_assert(!RAGGED || (PARK && !FULL), "the ragged variant parks in registers and has no full-step shortcut");
+    static_assert(!LONG || (PARK && !RAGGED && !PAIR), "the long variant parks in registers, on rows of whole vectors");
+    constexpr int STEP_COLS = LONG ? 2 * SP_TC : SP_TC;      // columns of a row per step
+    constexpr int GROUP_ROWS = LONG ? SP_HALF : SP_ROWS;     // rows of a group
+    static_assert(GROUP_ROWS * (STEP_COLS + SP_PAD) * sizeof(uint16_t) <= SP_TILE_BYTES, "the tile of a step fits its place in LDS");
     static_assert(!PAIR || (PARK && !RAGGED && NSTEP % 2 == 0), "the paired variant parks in registers and alternates two mask slots");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint16_t* lut = reinterpret_cast<uint16_t*>(smem);
-    uint16_t (*tile)[SP_TC + SP_PAD] = reinterpret_cast<uint16_t (*)[SP_TC + SP_PAD]>(smem + SP_LUT_BYTES);
+    uint16_t (*tile)[STEP_COLS + SP_PAD] = reinterpret_cast<uint16_t (*)[STEP_COLS + SP_PAD]>(smem + SP_LUT_BYTES);
     uint16_t (*sums)[32] = reinterpret_cast<uint16_t (*)[32]>(smem + SP_LUT_BYTES + SP_TILE_BYTES);
 
     // table -> LDS
@@ -209,7 +217,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         // ------------------------------------------------------------------ wave 0: the walk, nothing else
         __builtin_amdgcn_s_setprio(3);
         const uint32_t lane = threadIdx.x;
-        const uint32_t wr = lane < SP_ROWS ? lane : 0;       // lanes 30..63 shadow row 0 and never publish
+        const uint32_t wr = lane < GROUP_ROWS ? lane : 0;    // lanes past the group's rows shadow row 0; their sums are never read
         const v4u* trow = reinterpret_cast<const v4u*>(tile[wr]);
         typename ST::Run run = ST::zero();
         uint32_t gpar = 0;
@@ -255,9 +263,9 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 // 16 values per chunk; the LDS reads of the next chunk are in flight during the 16 dependent adds
                 v4u c0 = trow[0], c1 = trow[1];
 #pragma unroll
-                for (int c = 0; c < SP_TC / 16; c++) {
+                for (int c = 0; c < STEP_COLS / 16; c++) {
                     v4u n0 = c0, n1 = c1;
-                    if (c + 1 < SP_TC / 16) {
+                    if (c + 1 < STEP_COLS / 16) {
                         n0 = trow[(c + 1) * 2];
                         n1 = trow[(c + 1) * 2 + 1];
                     }
@@ -334,14 +342,14 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             sp_item(sch, blockIdx.x, G, it, rep, pg);
 #pragma unroll
             for (int h = 0; h < NCROW; h++) {
-                const uint32_t r = PAIR ? rr : rr + h * SP_HALF;
+                const uint32_t r = PAIR || LONG ? rr : rr + h * SP_HALF;
                 const uint32_t prow = pg * sch.R + r;
                 const bool ok = it < n_items && r < sch.R && prow < sch.P && sch.tile_stride != 0;
                 uint32_t q, mrow;
                 fd_divmod((PAIR ? rep * 2 : rep) * sch.P + prow, sch.pm_div, q, mrow);
                 const uint32_t base = __builtin_amdgcn_readfirstlane(ok ? (uint32_t)RT_SM_TILES_HEAD + mrow * sch.tile_stride : 0u);
 #pragma unroll
-                for (int t = 0; t < NCLS; t++) cw[h][t] = __builtin_amdgcn_readfirstlane(tiles[base + t]);
+                for (int t = 0; t < NCLS; t++) cw[h][t] = __builtin_amdgcn_readfirstlane(tiles[base + (LONG ? 2 * t + h : t)]);
             }
         }
     };
@@ -350,7 +358,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         sp_item(sch, blockIdx.x, G, it, rep, pg);
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const uint32_t r = PAIR ? rr : rr + h * SP_HALF;
+            const uint32_t r = PAIR || LONG ? rr : rr + h * SP_HALF;
             const uint32_t prow = pg * sch.R + r;            // row inside the period
             const uint32_t per = PAIR ? rep * 2 + h : rep;
             const bool ok = it < n_items && r < sch.R && prow < sch.P && per < sch.reps;
@@ -366,7 +374,8 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 }
                 continue;
             }
-            xo[h] = __builtin_amdgcn_readfirstlane(ok ? row * row_bytes : OOB);
+            // (LONG: h = 1 is the second half of each of the row's steps)
+            xo[h] = __builtin_amdgcn_readfirstlane(ok ? row * row_bytes + (LONG ? h * SP_TC * 2 : 0) : OOB);
             if (MASK) {
                 uint32_t q, mrow;
                 fd_divmod(row, sch.pm_div, q, mrow);
@@ -377,10 +386,10 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         }
     };
     const uint32_t cbyte = ccol * 2;
-    auto past_end = [&](uint32_t t) -> bool { return !(PARK && FULL) && t * SP_TC + ccol >= cols; };
-    auto step_off = [&](uint32_t row_off, uint32_t t) -> uint32_t {   // per-lane offset of this thread's vector in step t of a row
-        if (past_end(t)) return OOB;
-        return row_off + t * (SP_TC * 2) + cbyte;
+    auto past_end = [&](uint32_t t, int h) -> bool { return !(PARK && FULL) && t * STEP_COLS + (LONG ? h * SP_TC : 0) + ccol >= cols; };
+    auto step_off = [&](uint32_t row_off, uint32_t t, int h) -> uint32_t {   // per-lane offset of this thread's vector h in step t of a row
+        if (past_end(t, h)) return OOB;
+        return row_off + t * (STEP_COLS * 2) + cbyte;
     };
     // RAGGED: the same in span coordinates.  The vector at span byte p holds row bytes [sh, sh + row_bytes) ∩ [p, p + 16).
     auto span_load_off = [&](uint32_t row_off, uint32_t sh, uint32_t t) -> uint32_t {
@@ -391,8 +400,10 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         const uint32_t p = t * (SP_TC * 2) + cbyte;
         return (p >= sh && p + 16 <= sh + row_bytes) ? row_off + p : OOB;
     };
-    auto ld_off = [&](uint32_t row_off, uint32_t sh, uint32_t t) -> uint32_t { return RAGGED ? span_load_off(row_off, sh, t) : step_off(row_off, t); };
-    auto st_off = [&](uint32_t row_off, uint32_t sh, uint32_t t) -> uint32_t { return RAGGED ? span_store_off(row_off, sh, t) : step_off(row_off, t); };
+    auto ld_off = [&](uint32_t row_off, uint32_t sh, uint32_t t, int h) -> uint32_t { return RAGGED ? span_load_off(row_off, sh, t) : step_off(row_off, t, h); };
+    auto st_off = [&](uint32_t row_off, uint32_t sh, uint32_t t, int h) -> uint32_t { return RAGGED ? span_store_off(row_off, sh, t) : step_off(row_off, t, h); };
+    // this thread's vector h of the step in the tile
+    auto in_tile = [&](int h) -> v4u* { return reinterpret_cast<v4u*>(LONG ? &tile[rr][ccol + h * SP_TC] : &tile[rr + h * SP_HALF][ccol]); };
     // RAGGED with MASK: the sixteen mask bytes for the vector at span byte p start at mask byte mq + p, which is only
     // element aligned: they straddle the aligned mask vectors at (mq & ~15) + p and 16 bytes on, (mq & 15) bytes into the
     // first.  A lane loads the first; the second is its right neighbour's first (one wave shift), except for lane 63,
@@ -477,7 +488,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     auto read_prev_sum = [&](uint32_t par) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const uint32_t sb = __builtin_amdgcn_readfirstlane((uint32_t)sums[par][rr + h * SP_HALF]);
+            const uint32_t sb = __builtin_amdgcn_readfirstlane((uint32_t)sums[par][LONG ? rr : rr + h * SP_HALF]);
             const float s = ST::widen_bits(sb);
             s_prev[h] = s;
             // normal, finite, not tiny: the reciprocal-plus-correction quotient is exact there
@@ -490,7 +501,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     // A wave whose 512 values of this step are all -inf (the part of a row that a causal mask covers) takes exp(-inf) for
     // all of them without the eight table reads per lane; the test is wave-wide, so the branch is a scalar one.
     const uint32_t exp_ninf = __builtin_amdgcn_readfirstlane((uint32_t)lut[ST::NEG_INF_PAIR & 0xffffu] * 0x10001u);
-    auto exp_in_place = [&](v4u& in, const v4u& m, uint32_t t, uint32_t sh) {
+    auto exp_in_place = [&](v4u& in, const v4u& m, uint32_t t, uint32_t sh, int h) {
         if (MASK) in = ST::add_vec(in, m);                   // scores + mask in the 16-bit type, as the separate add would round it
         const bool mine = ((in[0] ^ ST::NEG_INF_PAIR) | (in[1] ^ ST::NEG_INF_PAIR) | (in[2] ^ ST::NEG_INF_PAIR) | (in[3] ^ ST::NEG_INF_PAIR)) == 0;
         if (__builtin_amdgcn_ballot_w64(!mine) == 0) {
@@ -499,7 +510,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
             for (int w = 0; w < 4; w++) in[w] = sp_exp_pair(lut, in[w]);
         }
-        if (RAGGED ? t * (SP_TC * 2) + cbyte >= sh + row_bytes : past_end(t)) in = v4u{0, 0, 0, 0};
+        if (RAGGED ? t * (SP_TC * 2) + cbyte >= sh + row_bytes : past_end(t, h)) in = v4u{0, 0, 0, 0};
     };
     // RAGGED: the neighbours' elements in a row's first and last vector are zeroed in the tile, after the vector has been
     // written there (on the LDS copy, so that the data registers of the main path stay untouched: masking them in a branch
@@ -551,15 +562,15 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
         for (int k = 0; k < PF; k++) {
 #pragma unroll
-            for (int h = 0; h < 2; h++) pre[k][h] = load_x(ld_off(cur[h], pcur[h], k));
+            for (int h = 0; h < 2; h++) pre[k][h] = load_x(ld_off(cur[h], pcur[h], k, h));
 #pragma unroll
             for (int h = 0; h < 2; h++) store_y(v4u{0, 0, 0, 0}, OOB);
         }
         if (MASK && !RAGGED) {                               // PAIR: the mask of steps 0 and 1 (NSTEP is even, so 1 exists)
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                mpre[h] = PAIR ? load_m_tile(step_off(cur[0] - pcur[0], h), ccur[0][TILES ? h : 0])
-                               : load_m_tile(step_off(cur[h] - pcur[h], 0), ccur[PAIR ? 0 : h][0]);
+                mpre[h] = PAIR ? load_m_tile(step_off(cur[0] - pcur[0], h, 0), ccur[0][TILES ? h : 0])
+                               : load_m_tile(step_off(cur[h] - pcur[h], 0, h), ccur[PAIR ? 0 : h][0]);
         }
         if (MASK && RAGGED) {
 #pragma unroll
@@ -579,10 +590,10 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                                  : PAIR           ? tile_value(mpre[t % 2], ccur[0][TILES ? t : 0])
                                  : TILES          ? tile_value(mpre[h], ccur[PAIR ? 0 : h][TILES ? t : 0])
                                                   : mpre[h],
-                                 t, pcur[h]);
+                                 t, pcur[h], h);
                 __syncthreads();                             // A: wave 0 has left the previous tile
-                *reinterpret_cast<v4u*>(&tile[rr][ccol]) = pre[t % PF][0];
-                *reinterpret_cast<v4u*>(&tile[rr + SP_HALF][ccol]) = pre[t % PF][1];
+                *in_tile(0) = pre[t % PF][0];
+                *in_tile(1) = pre[t % PF][1];
                 if (RAGGED) {
                     zero_outside(t, pcur[0], rr);
                     zero_outside(t, pcur[1], rr + SP_HALF);
@@ -593,12 +604,12 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 if (MASK && !RAGGED && !PAIR) {
 #pragma unroll
                     for (int h = 0; h < 2; h++)
-                        mpre[h] = (t + 1 < NSTEP) ? load_m_tile(step_off(cur[h] - pcur[h], t + 1), ccur[PAIR ? 0 : h][TILES && t + 1 < NSTEP ? t + 1 : 0])
-                                                  : load_m_tile(step_off(nxt[h] - pnxt[h], 0), cnxt[PAIR ? 0 : h][0]);
+                        mpre[h] = (t + 1 < NSTEP) ? load_m_tile(step_off(cur[h] - pcur[h], t + 1, h), ccur[PAIR ? 0 : h][TILES && t + 1 < NSTEP ? t + 1 : 0])
+                                                  : load_m_tile(step_off(nxt[h] - pnxt[h], 0, h), cnxt[PAIR ? 0 : h][0]);
                 }
                 if (PAIR)                                    // this step's slot is free: the mask of two steps ahead
-                    mpre[t % 2] = (t + 2 < NSTEP) ? load_m_tile(step_off(cur[0] - pcur[0], t + 2), ccur[0][PAIR && t + 2 < NSTEP ? t + 2 : 0])
-                                                  : load_m_tile(step_off(nxt[0] - pnxt[0], t + 2 - NSTEP), cnxt[0][PAIR && t + 2 >= NSTEP ? t + 2 - NSTEP : 0]);
+                    mpre[t % 2] = (t + 2 < NSTEP) ? load_m_tile(step_off(cur[0] - pcur[0], t + 2, 0), ccur[0][PAIR && t + 2 < NSTEP ? t + 2 : 0])
+                                                  : load_m_tile(step_off(nxt[0] - pnxt[0], t + 2 - NSTEP, 0), cnxt[0][PAIR && t + 2 >= NSTEP ? t + 2 - NSTEP : 0]);
                 if (MASK && RAGGED) {
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
@@ -608,14 +619,14 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 }
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    pre[t % PF][h] = (t + PF < NSTEP) ? load_x(ld_off(cur[h], pcur[h], t + PF)) : load_x(ld_off(nxt[h], pnxt[h], t + PF - NSTEP));
+                    pre[t % PF][h] = (t + PF < NSTEP) ? load_x(ld_off(cur[h], pcur[h], t + PF, h)) : load_x(ld_off(nxt[h], pnxt[h], t + PF - NSTEP, h));
                 __syncthreads();                             // B: parked for the walk
                 if (t == 0) read_prev_sum(gpar ^ 1);         // published by wave 0 before it reached barrier A
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t));   // first group: prev is OOB, the store is dropped
+                    store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t, h));   // first group: prev is OOB, the store is dropped
                     // this group's values come back from the tile, which stays intact until the next barrier A
-                    e[t][h] = *reinterpret_cast<const v4u*>(&tile[rr + h * SP_HALF][ccol]);
+                    e[t][h] = *in_tile(h);
                 }
             }
 #pragma unroll
@@ -643,7 +654,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
         for (int t = 0; t < NSTEP; t++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t));
+            for (int h = 0; h < 2; h++) store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t, h));
     } else {
         // One flat loop over the steps of all groups, two steps per trip (nsteps is even; a step past the row end moves
         // nothing).  Per step and row: exp values to the tile and to y, x of two steps ahead, the previous group's exp
@@ -656,10 +667,10 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             for (int h = 0; h < 2; h++) store_park(v4u{0, 0, 0, 0}, OOB);
             if (MASK) {
 #pragma unroll
-                for (int h = 0; h < 2; h++) mpre[h] = load_m(step_off(cur[h] - pcur[h], 0));
+                for (int h = 0; h < 2; h++) mpre[h] = load_m(step_off(cur[h] - pcur[h], 0, h));
             }
 #pragma unroll
-            for (int h = 0; h < 2; h++) pre[k][h] = load_x(step_off(cur[h], k));
+            for (int h = 0; h < 2; h++) pre[k][h] = load_x(step_off(cur[h], k, h));
 #pragma unroll
             for (int h = 0; h < 2; h++) store_y(v4u{0, 0, 0, 0}, OOB);
 #pragma unroll
@@ -672,27 +683,27 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             for (int k = 0; k < 2; k++) {
                 const uint32_t t = t0 + k;
 #pragma unroll
-                for (int h = 0; h < 2; h++) exp_in_place(pre[k][h], mpre[h], t, 0);
+                for (int h = 0; h < 2; h++) exp_in_place(pre[k][h], mpre[h], t, 0, h);
                 __syncthreads();                             // A
                 *reinterpret_cast<v4u*>(&tile[rr][ccol]) = pre[k][0];
                 *reinterpret_cast<v4u*>(&tile[rr + SP_HALF][ccol]) = pre[k][1];
 #pragma unroll
-                for (int h = 0; h < 2; h++) store_park(pre[k][h], step_off(cur[h], t));      // parked in y (kept in cache: read back soon)
+                for (int h = 0; h < 2; h++) store_park(pre[k][h], step_off(cur[h], t, h));      // parked in y (kept in cache: read back soon)
                 const bool wrap = t + 2 >= nsteps;           // two steps ahead is in the block's next group
                 const uint32_t ta = wrap ? t + 2 - nsteps : t + 2;
                 if (MASK) {
                     const bool w1 = t + 1 >= nsteps;
 #pragma unroll
-                    for (int h = 0; h < 2; h++) mpre[h] = load_m(step_off(w1 ? nxt[h] - pnxt[h] : cur[h] - pcur[h], w1 ? 0 : t + 1));
+                    for (int h = 0; h < 2; h++) mpre[h] = load_m(step_off(w1 ? nxt[h] - pnxt[h] : cur[h] - pcur[h], w1 ? 0 : t + 1, h));
                 }
 #pragma unroll
-                for (int h = 0; h < 2; h++) pre[k][h] = load_x(step_off(wrap ? nxt[h] : cur[h], ta));
+                for (int h = 0; h < 2; h++) pre[k][h] = load_x(step_off(wrap ? nxt[h] : cur[h], ta, h));
                 __syncthreads();                             // B
                 if (t == 0) read_prev_sum(gpar ^ 1);
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    store_y(quotients(qpre[k][h], h), step_off(prev[h], t));
-                    qpre[k][h] = load_y(step_off(wrap ? cur[h] : prev[h], ta));
+                    store_y(quotients(qpre[k][h], h), step_off(prev[h], t, h));
+                    qpre[k][h] = load_y(step_off(wrap ? cur[h] : prev[h], ta, h));
                 }
             }
             t0 += 2;
@@ -719,8 +730,8 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             for (int k = 0; k < 2; k++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    store_y(quotients(qpre[k][h], h), step_off(prev[h], t + k));
-                    qpre[k][h] = load_y(step_off(prev[h], t + k + 2 < nsteps ? t + k + 2 : 0xffffu));
+                    store_y(quotients(qpre[k][h], h), step_off(prev[h], t + k, h));
+                    qpre[k][h] = load_y(step_off(prev[h], t + k + 2 < nsteps ? t + k + 2 : 0xffffu, h));
                 }
         }
     }
@@ -825,6 +836,17 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     if (rc) return rc;
     const uint32_t nt = (cols + SP_TC - 1) / SP_TC;
     if (ragged && nt > SP_MAX_STEPS) return RT_OK;           // (a ragged row's one vector past its last step is the walker's)
+    // f16 rows of 4097 to 8192 columns stay in registers, 15 to a group (the LONG variant): two passes over memory instead of
+    // four, and the walk, on half as many rows at a time, is what bounds it (1.9 us per 512 columns with its barriers; five
+    // rounds of 13 rows on [1,8,2048,8192]).  Parked in y / in registers, with a causal mask: [1,8,2048,8192] 207 / 155 us,
+    // [1,8,2048,6144] 144 / 119, [1,8,2048,4608] 117 / 101, [1,32,1000,7000] 313 / 282, [1,16,1000,5000] 115 / 108, [1,8,100,8192] 49 / 35;
+    // [1,8,512,8192], whose 4096 rows are one round of 16-row groups and two of 15, 64 us either way.  The bf16 walk takes
+    // 5 ns an element and half as many rows at a time cost more than the two passes on most shapes
+    // ([1,8,2048,8192] 243 / 264 us, [1,32,1000,7000] with a mask 432 / 530): bf16 parks in y.
+    constexpr bool LONG_ROWS = std::is_same<T, half_t>::value;
+    const bool longer = LONG_ROWS && !ragged && nt > SP_MAX_STEPS && nt <= 2 * SP_MAX_STEPS;
+    const uint32_t long_steps = nt <= 10 ? 5 : nt <= 12 ? 6 : 8;       // of 1024 columns
+    const bool long_full = longer && cols == long_steps * 2 * SP_TC;
     const bool full = !ragged && cols % SP_TC == 0 && nt != 7 && nt <= 8;
 #define RT_SP(NS, F, M)                                                                                                              \
     do {                                                                                                                             \
@@ -854,6 +876,24 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         else if (nt <= 4) RT_SP_PAIR(4, F);                 \
         else if (nt <= 6) RT_SP_PAIR(6, F);                 \
         else RT_SP_PAIR(8, F);                              \
+    } while (0)
+#define RT_SP_LONG(NS, F, M)                                                                                                         \
+    do {                                                                                                                             \
+        const uint32_t bit = 1u << (16 + (NS == 5 ? 0 : NS == 6 ? 4 : 8) + (F ? 2 : 0) + (M ? 1 : 0));                               \
+        if (!(dev->sp_pair_attr_set & bit)) {                                                                                        \
+            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, M, false, true>),             \
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
+            dev->sp_pair_attr_set |= bit;                                                                                            \
+        }                                                                                                                            \
+        hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, M, false, true>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES,         \
+                           dev->stream, table, xc, (const T*)mask, yc, n, cols, sch, (uint16_t*)nullptr,                             \
+                           (const uint32_t*)dev->sm_mask_tiles);                                                                     \
+    } while (0)
+#define RT_SP_LONG_NS(F, M)                                 \
+    do {                                                    \
+        if (long_steps == 5) RT_SP_LONG(5, F, M);           \
+        else if (long_steps == 6) RT_SP_LONG(6, F, M);      \
+        else RT_SP_LONG(8, F, M);                           \
     } while (0)
 #define RT_SP_RAGGED(NS, M)                                                                                                          \
     do {                                                                                                                             \
@@ -900,7 +940,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // one mask row for two heads: rows of an even number of steps under a mask that repeats every P rows
         const bool pair = mask && !ragged && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
         sch.item_reps = pair ? (sch.reps + 1) / 2 : sch.reps;
-        const uint32_t rmax = pair ? SP_HALF : SP_ROWS, rmul = pair ? 2 : 1;
+        const uint32_t rmax = pair || longer ? SP_HALF : SP_ROWS, rmul = pair ? 2 : 1;
         // rows per group: every block runs ceil(groups / grid) rounds of 8-or-fewer steps whatever the group holds, so
         // 4370 groups of 30 rows on 256 CUs cost 18 rounds where 17.07 are needed; 27-row groups make 19 full rounds.
         // A step takes the longer of the walk (1.5 us whatever the group holds) and the group's memory time (2 KiB per
@@ -934,7 +974,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
                 };
                 uint32_t pick = sch.R, pick_x = xcds_of(sch.R);
                 uint64_t pick_cost = best;
-                for (uint32_t R = SP_ROWS; R >= 1; R--) {
+                for (uint32_t R = rmax; R >= 1; R--) {
                     const uint64_t cost = cost_of(R);
                     if (cost * 20 > best * 21) continue;
                     const uint32_t xc = xcds_of(R);
@@ -964,8 +1004,8 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // costs that one 3 us, 6.8e12 and 7.0e12 leave 5 us of its dependence on where the buffers lie).
         if (blocks == dev->num_cus && !ragged && (!mask || pair)) {
             const double rate = RT_PACE_BYTES_PER_S;
-            const double group_bytes = (double)sch.R * rmul * cols * 2 * (nt > SP_MAX_STEPS ? 4 : 2);     // in and out (long rows: parked and read back)
-            const double steps = nt > SP_MAX_STEPS ? sch.nsteps : nt == 7 ? 8 : nt;          // the steps the kernel variant takes per group
+            const double group_bytes = (double)sch.R * rmul * cols * 2 * (nt > SP_MAX_STEPS && !longer ? 4 : 2);     // in and out (long rows: parked and read back)
+            const double steps = longer ? long_steps : nt > SP_MAX_STEPS ? sch.nsteps : nt == 7 ? 8 : nt;          // the steps the kernel variant takes per group
             sch.pace = (uint32_t)(group_bytes / steps * blocks / rate * dev->wall_clock_hz + 0.5);
             if (dev->debug_softmax_pace) sch.pace = dev->debug_softmax_pace;
             sch.phase_fx = sch.pace > 0xffffu ? 0 : (sch.pace << 16) / blocks;
@@ -975,7 +1015,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // nothing that could be measured ([1,32,2048,2048] and [1,32,2560,2560]: 111 and 188 us either way), and the
         // pass over the mask is a launch of 3 us ([8,32,512,512] 71 -> 68 us, a decode step's [1,32,1,4096] 29 -> 26 us).
         sch.tile_stride = 0;
-        if (mask && !ragged && nt <= SP_MAX_STEPS && (uint64_t)sch.PM * nt <= RT_SM_MASK_TILES && rt_aligned(mask, 16) &&
+        if (mask && !ragged && (nt <= SP_MAX_STEPS || longer) && (uint64_t)sch.PM * nt + (longer ? 3 : 0) <= RT_SM_MASK_TILES && rt_aligned(mask, 16) &&
             (uint64_t)sch.PM * cols * sizeof(T) >= (16ull << 20)) {
             const uint32_t ntiles = sch.PM * nt;
             const uint32_t per_block = (BLOCK / 64) * MT_PER_WAVE;
@@ -994,7 +1034,17 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
             RT_CHECK_LAUNCH("softmax16_edges_kernel");
             continue;
         }
-        if (nt > SP_MAX_STEPS) {                         // long rows: exp values parked in y
+        if (longer) {
+            if constexpr (LONG_ROWS) {
+                if (mask) {
+                    if (long_full) RT_SP_LONG_NS(true, 1);
+                    else RT_SP_LONG_NS(false, 1);
+                } else {
+                    if (long_full) RT_SP_LONG_NS(true, 0);
+                    else RT_SP_LONG_NS(false, 0);
+                }
+            }
+        } else if (nt > SP_MAX_STEPS) {                  // longer rows: exp values parked in y
             if (mask) RT_SP(0, false, true);
             else RT_SP(0, false, false);
         } else if (pair) {
@@ -1012,6 +1062,8 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
 #undef RT_SP_NS
 #undef RT_SP_PAIR_NS
 #undef RT_SP_PAIR
+#undef RT_SP_LONG_NS
+#undef RT_SP_LONG
 #undef RT_SP_RAGGED_NS
 #undef RT_SP_RAGGED
 #undef RT_SP

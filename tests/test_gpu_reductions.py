@@ -258,7 +258,7 @@ def test_softmax_bf16_streaming_kernel(dev, oracle, shape):
 @pytest.mark.parametrize("shape,kind", [((1, 70, 8192), "f16"), ((2, 33, 4104), "f16"), ((1, 3, 51200), "f16"), ((1, 100, 6008), "f16"),
                                         ((1, 40, 8192), "bf16"), ((1, 5, 20000), "bf16")])
 def test_softmax_16_bit_long_rows(dev, oracle, shape, kind):
-    """rows of more than 4096 columns: the exp values are parked in y and read back once the row sum is known; also in place"""
+    """rows of more than 4096 columns (few f16 rows of up to 8192: one wave a row; the others park the exp values in y and read them back once the row sum is known); also in place"""
     rng = np.random.default_rng(306)
     n = shape[-1]
     xf = (rng.standard_normal(shape) * 2).astype(np.float32)
@@ -282,6 +282,45 @@ def test_softmax_16_bit_long_rows(dev, oracle, shape, kind):
         dev.softmax(dx, out=dx)
         got = dx.to_numpy()
         assert not ((got != want) & ~(isnan(got) & isnan(want))).any(), shape
+
+
+@pytest.mark.parametrize("rows,cols", [(530, 4104), (1100, 5112), (1040, 5120), (1100, 5128), (4000, 6144), (530, 6152), (544, 7680), (1100, 8184), (4100, 8192)])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, kind):
+    """fifteen rows a block in registers, a thread's two vectors 512 columns apart in one row: the oracle's bits where a row
+    ends in the first and in the second half of a step, with one group a block and several, in place, without a mask, under
+    a mask of two periods large enough for the table of tile classes (uniform and mixed tiles) and under a single mask row"""
+    rng = np.random.default_rng(317)
+    bf = kind == "bf16"
+    conv = (lambda a: _bf16(oracle, a)) if bf else (lambda a: np.asarray(a, np.float32).astype(np.float16))
+    xf = rng.standard_normal((rows, cols)).astype(np.float32)
+    _special_rows(xf, cols)
+    x = conv(xf)
+    period = rows // 2
+    mf = np.where(np.arange(cols)[None, :] > np.arange(period)[:, None] * (cols // period), -np.inf, 0.0).astype(np.float32)
+    mf[:, 512:1024] = -0.5
+    masks = {"none": None, "half": conv(mf), "row": conv(mf[period // 2:period // 2 + 1])}
+
+    def check(got, want, what):
+        g, w = np.asarray(got).view(np.uint16), np.asarray(want).view(np.uint16)
+        top = 0x7f80 if bf else 0x7c00
+        bad = (g != w) & ~(((g & 0x7fff) > top) & ((w & 0x7fff) > top))
+        assert not bad.any(), (what, rows, cols, kind, int(bad.sum()), np.argwhere(bad)[:4])
+
+    for name, mask in masks.items():
+        dx = dev.upload(x.reshape(1, 2, period, cols), bf16=bf)
+        if mask is None:
+            want = oracle.softmax(x, bf16=bf)
+            got = dev.softmax(dx).to_numpy()
+            dev.softmax(dx, out=dx)
+        else:
+            dm = dev.upload(mask, bf16=bf)
+            spread = np.ascontiguousarray(np.broadcast_to(mask, (2, period, cols)).reshape(rows, cols))
+            want = oracle.softmax(oracle.binary("add", x, spread, bf16=bf), bf16=bf)
+            got = dev.softmax_masked(dx, dm).to_numpy()
+            dev.softmax_masked(dx, dm, out=dx)
+        check(got.reshape(rows, cols), want, name)
+        check(dx.to_numpy().reshape(rows, cols), want, name + " in place")
 
 
 @pytest.mark.parametrize("shape,kind", [((2, 4, 333, 1001), "f16"), ((1, 3, 100, 199), "f16"), ((70, 4095), "f16"), ((7, 4097), "f16"), ((50, 2047), "f16"), ((90, 511), "f16"), ((40, 2305), "f16"), ((45, 1535), "f16"), ((33, 3071), "f16"), ((33, 513), "f16"),
