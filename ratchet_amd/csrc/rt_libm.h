@@ -2,12 +2,12 @@
 // against the C library there (tests/device_math_check.cpp does, with g++): the includer defines
 //   RT_FN     the function qualifiers (`__device__ inline` in the kernels, `static inline` on the host)
 //   RT_TABLE  the qualifiers of a constant table (`__device__ static const` / `static const`)
-//   RT_DIV, RT_MED3  optionally, rt_tanhf's division (operands and quotient far from the ends of the float range) and the
-//             middle one of (v, lo, hi); the plain C++ expressions otherwise
+//   RT_DIV, RT_MED3  optionally, rt_tanhf's division and the middle one of (v, lo, hi); the plain C++ expressions otherwise
+//             (rt_math.h takes a shorter division; device_math_check.cpp says which results could hang on that)
 //
 // The libm routines of the unary ops are restated operation by operation so that their float32 results equal, bit for
 // bit, what the x86-64 glibc 2.35 `tanhf`, `expf`, `logf`, `sinf` and `cosf` return (checked on the CPU over all 2^32
-// inputs with this same code compiled by g++).  ratchet's CPU executor calls exactly those through Rust's f32::tanh /
+// inputs with this code compiled by g++, tanhf's with the kernels' division too).  ratchet's CPU executor calls exactly those through Rust's f32::tanh /
 // f32::exp / f32::ln / f32::sin / f32::cos (crates/ratchet-core/src/cpu/unary.rs:46-65, cpu/softmax.rs:30, cpu/rope.rs), and GELU's `1 + tanh(..)` cancellation turns a
 // 1-ulp tanh difference into hundreds of ulps, so "close" is not good enough there.
 //   tanhf/expm1f: the classic fdlibm float algorithms (float arithmetic only).

@@ -9,11 +9,14 @@
 typedef _Float16 half_t;
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
-// n / d for operands and a quotient far from overflow and from the subnormals: the reciprocal, the quotient, one
-// correction by the exact remainder.  Four instructions where the general division takes ten, which also refine the
-// reciprocal, scale the operands and put the special cases right.  This is not correctly rounded for every pair of
-// operands: rt_tanhf's two divisions see only the pairs that its 2^32 arguments lead to, and on this chip all of its
-// results (and GELU's) equal those with the general division.
+// n / d in rt_tanhf: the reciprocal, the quotient, one correction by the exact remainder.  Four instructions where the
+// general division takes ten, which also refine the reciprocal, scale the operands and put the special cases right.
+// This is not correctly rounded for every pair of operands, but rt_tanhf's two divisions see only the pairs that its 2^32
+// arguments lead to: d is in [1, 2^64], so the reciprocal is a normal float, and a quotient in the subnormal range or zero
+// comes with d = 2 and an n that is twice a float (-em1 for |x| below 2^-25), so it is exact.
+// With v_rcp_f32 anywhere within its one ulp all results equal the C library's but for 113 arguments of either sign, whose
+// second quotient hangs on the reciprocal's last bit: tests/device_math_check.cpp finds them on the CPU, and
+// test_tanh_where_the_division_hangs_on_the_reciprocal holds this chip's results on them to the C library's.
 __device__ __forceinline__ float rt_div_mid(float n, float d) {
     const float r = __builtin_amdgcn_rcpf(d);
     const float q = n * r;

@@ -1,15 +1,41 @@
-// Host check of the kernels' libm-level routines: ratchet_amd/csrc/rt_libm.h compiled as plain C++ (the very text the
-// kernels compile for the GPU) against this machine's C library, which is what the reference's f32::tanh / f32::exp / f32::ln / f32::sin / f32::cos
-// resolve to (crates/ratchet-core/src/cpu/unary.rs:46-65, cpu/softmax.rs:30).  Bit equality is required (any NaN equals
-// any NaN).  Inputs: every `stride`-th float bit pattern over the whole 2^32 range (stride 1 = exhaustive), every value
-// that a 16-bit input can widen to, and the breakpoints of the algorithms.  Build: g++ -O2 -ffp-contract=off.
+// Host check of the kernels' libm-level routines: ratchet_amd/csrc/rt_libm.h compiled as plain C++ against this machine's
+// C library, which is what the reference's f32::tanh / f32::exp / f32::ln / f32::sin / f32::cos resolve to
+// (crates/ratchet-core/src/cpu/unary.rs:46-65, cpu/softmax.rs:30).  Bit equality is required (any NaN equals any NaN).
+// Inputs: every `stride`-th float bit pattern over the whole 2^32 range (stride 1 = exhaustive), every value that a 16-bit
+// input can widen to, and the breakpoints of the algorithms.  Build: g++ -O2 -ffp-contract=off.
 // Usage: device_math_check [stride]   -> prints "tanhf <n> expm1f <n> expf <n> logf <n> sinf <n> cosf <n> f2bf <n> checked <m>", exit code 0 iff all n are 0.
+//
+// The kernels compile the same text but for two expressions of rt_tanhf that rt_math.h replaces: the median of three by the
+// instruction for it, which gives the same values, and the division by rt_div_mid, which is not correctly rounded for all
+// operands and whose result may hang on the last bit of the GPU's reciprocal instruction.  What that can change is found
+// here: the short division with each reciprocal correctly rounded, an ulp lower and an ulp higher (the instruction is
+// within one), in all combinations.  With correctly rounded reciprocals every result is the C library's; with the others
+// 113 positive inputs (and their negatives) differ, which tests/golden/tanh_division_inputs.txt lists and
+// test_tanh_where_the_division_hangs_on_the_reciprocal puts to the GPU.  All other inputs give the C library's result
+// whichever of the three the instruction returns.
+// Usage: device_math_check division FILE [stride]   -> every `stride`-th positive float: prints the sensitive inputs that
+//   FILE does not list, then "sensitive <n> unlisted <n> listed <n> insensitive <n> wrong <n> checked <m>" (insensitive: of the
+//   listed; wrong: with correctly rounded reciprocals); exit code 0 iff unlisted, insensitive and wrong are 0.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <set>
 
+// 0: the plain division; 1: rt_div_mid of rt_math.h, its reciprocals off by off[0] and off[1] ulps
+static int division = 0, off[2], nth;
+static inline float divide(float n, float d) {
+    if (division == 0) return n / d;
+    float r = 1.0f / d;
+    uint32_t bits;
+    memcpy(&bits, &r, 4);
+    bits += (uint32_t)off[nth++ & 1];
+    memcpy(&r, &bits, 4);
+    const float q = n * r;
+    return fmaf(fmaf(-d, q, n), r, q);
+}
+#define RT_DIV(n, d) divide(n, d)
 #define RT_FN static inline
 #define RT_TABLE static const
 #include "rt_libm.h"
@@ -40,7 +66,46 @@ struct Counts {
     }
 };
 
+static int check_division(const char* file, unsigned long long stride) {
+    std::set<uint32_t> listed;
+    FILE* f = fopen(file, "r");
+    if (!f) return 2;
+    char word[256];
+    while (fscanf(f, "%255s", word) == 1) {
+        if (word[0] == '#') {
+            if (!fgets(word, sizeof word, f)) break;                             // a comment's rest
+            continue;
+        }
+        listed.insert((uint32_t)strtoul(word, nullptr, 16));
+    }
+    fclose(f);
+    unsigned long long sensitive = 0, unlisted = 0, insensitive = 0, wrong = 0, checked = 0;
+    division = 1;
+    auto is_sensitive = [&](uint32_t bits) {
+        const float x = u2f(bits), want = tanhf(x);
+        bool any = false;
+        for (int k = 0; k < 9; k++) {
+            off[0] = k / 3 - 1, off[1] = k % 3 - 1, nth = 0;
+            const bool differs = !same(rt_tanhf(x), want);
+            any |= differs;
+            if (k == 4 && differs) wrong++;
+        }
+        checked++;
+        return any;
+    };
+    for (unsigned long long u = 0; u <= 0x7f800000u; u += stride)
+        if (is_sensitive((uint32_t)u)) {
+            sensitive++;
+            if (!listed.count((uint32_t)u)) unlisted++, printf("%08x\n", (uint32_t)u);
+        }
+    for (uint32_t u : listed) insensitive += !is_sensitive(u);
+    printf("sensitive %llu unlisted %llu listed %llu insensitive %llu wrong %llu checked %llu\n", sensitive, unlisted, (unsigned long long)listed.size(),
+           insensitive, wrong, checked);
+    return (unlisted | insensitive | wrong) ? 1 : 0;
+}
+
 int main(int argc, char** argv) {
+    if (argc > 2 && !strcmp(argv[1], "division")) return check_division(argv[2], argc > 3 ? strtoull(argv[3], nullptr, 10) : 1021);
     const unsigned long long stride = argc > 1 ? strtoull(argv[1], nullptr, 10) : 1021;
     Counts c;
     for (unsigned long long u = 0; u < (1ull << 32); u += stride) c.one((uint32_t)u);

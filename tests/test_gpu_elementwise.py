@@ -5,6 +5,8 @@ Bars (same seeded inputs on both sides):
   f32 transcendental unaries .... <= 2 ulp (tanh, gelu, exp, silu, sigmoid are expected to be bit-exact)
   f16 unaries ................... <= 1e-3 with the reference's all_close rule; checked exhaustively over all 65536 inputs
 """
+import os
+
 import numpy as np
 import pytest
 
@@ -430,3 +432,24 @@ def test_tanh_and_gelu_bits_over_the_float_range(dev, oracle, op):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32))
+
+
+def test_tanh_where_the_division_hangs_on_the_reciprocal(dev, oracle):
+    """The inputs whose tanh changes if the GPU's reciprocal instruction is an ulp off (device_math_check finds them; every
+    other one gives the C library's bits whatever that bit is), with both signs and their neighbours: the same bits as the
+    C library's.  f32 GELU on inputs whose tanh argument is one of them as well."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden", "tanh_division_inputs.txt")
+    with open(path) as f:
+        listed = np.array([int(w, 16) for line in f if not line.startswith("#") for w in line.split()], np.int64)
+    assert len(listed) == 113
+    pos = (listed[:, None] + np.arange(-2, 3)).ravel()
+    x = np.concatenate([pos, pos + 2 ** 31]).astype(np.uint32).view(np.float32)
+    assert np.array_equal(dev.unary("tanh", dev.upload(x)).to_numpy().view(np.uint32), oracle.unary("tanh", x).view(np.uint32))
+    # GELU's tanh argument is about 0.79788456 x (1 + 0.044715 x^2): the x that reaches a listed one by fixed-point steps in f64, and the floats around it
+    t = listed.astype(np.uint32).view(np.float32).astype(np.float64)
+    g = t.copy()
+    for _ in range(60):
+        g = t / (0.7978845608028654 * (1 + 0.044715 * g * g))
+    gb = (g.astype(np.float32).view(np.uint32).astype(np.int64)[:, None] + np.arange(-3, 4)).ravel()
+    x = np.concatenate([gb, gb + 2 ** 31]).astype(np.uint32).view(np.float32)
+    assert np.array_equal(dev.unary("gelu", dev.upload(x)).to_numpy().view(np.uint32), oracle.unary("gelu", x).view(np.uint32))
