@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__
 // there once at the start, and after the statistics the block reads LDS, normalises and streams the result out,
 // instead of fetching x a second time through a loop of dependent load / store pairs.
 constexpr int NP_BLOCK = 320;
-constexpr uint32_t NP_KEEP_MAX_COLS = 3072;
+constexpr uint32_t NP_KEEP_MAX_COLS = 4096;
 constexpr size_t NP_KEEP_BYTES_PER_TILE = 256 * 16 + 2 * 32 * 16;   // the block's x vectors, one scale and one bias vector per column group
 typedef _Float16 np_h8 __attribute__((ext_vector_type(8)));
 // run += the 32 f16 values packed in four vectors, left to right: each add is 1.0 * widen(f16) + run in one instruction
@@ -1605,6 +1605,55 @@ int launch_norm16_rb(rt_device* dev, const void* x, const void* scale, const voi
     return RT_OK;
 }
 
+// the steps that norm_flow16_kernel takes per group for rows of `nt` tiles
+inline uint32_t nf_steps(uint32_t nt) { return nt <= 2 ? 2 : nt <= 4 ? 4 : nt <= 8 ? 8 : nt <= 12 ? 12 : nt <= 16 ? 16 : 20; }
+
+// Where norm_flow16_kernel takes a launch.  Both sides were timed on 1 to 1 million rows, inputs and outputs moving through
+// 580 MB; the figures are us, the other kernel / this one.
+// Rows that are not whole aligned vectors: against norm_seq16_kernel, which reads element by element but starts a row with
+// little to do.  This kernel walks whole 256-column tiles, two at least, so rows of up to 128 columns gain only in large
+// numbers, and those of more than 64 also where the launch is a single round of walks (LayerNorm f16: [256,257] 9.0 / 5.5,
+// [10240,257] 14.7 / 8.5, [10240,31] 5.6 / 7.5, [50000,31] 30 / 16; bf16 [10240,13] 5.9 / 10.1, RMSNorm bf16 [65536,13] 15.7 / 21.9).
+inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
+    if (rows < 16 && cols <= 160) return false;
+    if (cols > 128) return true;
+    if (cols > 64) return rows <= 16 * cus || rows >= (!bf16 ? 60 : layer ? 100 : 64) * cus || (!bf16 && !layer && cols > 96);
+    if (layer) return rows >= (bf16 ? 129 : 120) * cus;
+    if (!bf16) return rows >= (cols > 40 ? 60 : 120) * cus && cols >= 12;
+    return (cols >= 40 && rows >= 120 * cus) || (cols >= 24 && rows > 256 * cus);
+}
+// Rows of whole aligned vectors: against norm_pipe16_kernel, whose blocks of 8 rows share the CUs and overlap one another,
+// while rows fit the chip in a few rounds, and which needs no empty steps.  Many rows come to memory, which that one
+// reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51, RMSNorm bf16 [12288,3072] 47 / 34).  Up to 40
+// rows a CU, f16 and RMSNorm gain on rows of more than 3072 columns that fill the steps (RMSNorm f16 [7000,4096] 27.8 / 23.5,
+// against [5000,3328] 17.6 / 18.9), RMSNorm in bf16 more widely ([2048,4104] 25.6 / 20).  bf16 LayerNorm, whose walker
+// needs the f32 tiles of both sums, gains in a single round of 8 rows a block ([2048,2560] 16.3 / 14.6, not three tiles in
+// four steps or five in eight: [2048,1280] 9.7 / 10.2) and once its blocks of 8 rows no longer keep their rows in LDS
+// ([7000,2560] 35 / 25.6; [5000,2560] 21.3 / 25.8), except for short rows and for 9000 to 10000 rows in steps a quarter empty
+// ([9000,1280] 22.7 / 26.1, [9000,1792] 29.4 / 27.9).
+inline bool nf_takes_aligned(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
+    const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);
+    if (bf16 && layer) {
+        if (rows <= 8 * cus) return cols > 768 && nt != 5;
+        if (rows <= 16 * cus) return cols > 3328;
+        if (rows <= 24 * cus || cols <= 128) return false;
+        if (cols <= 256) return rows > 48 * cus;
+        if (rows <= 32 * cus || rows > 42 * cus) return true;
+        return nt * 5 >= steps * 4;
+    }
+    // (bf16: not the row counts around 64 a CU, three rounds of 22 rows here and whole rounds there, in steps a quarter empty:
+    // RMSNorm [16384,1280] 23.8 / 25.9)
+    if (rows > 40 * cus) return cols > 512 && !(bf16 && nt * 5 < steps * 4 && rows > 60 * cus && rows <= 66 * cus);
+    if (cols <= 3072) return false;
+    if (bf16) {
+        if (rows <= 16 * cus) return true;
+        if (rows <= 24 * cus) return cols > 3584;
+        return rows <= 32 * cus || nt == steps;
+    }
+    if (nt == steps) return layer || rows > 8 * cus;
+    return layer && rows >= 64 && rows <= 16 * cus && cols > 3328;
+}
+
 template <typename T, int KIND, int RB>
 int launch_norm16_flow(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
     // one block per CU; the groups as even as they can be over the fewest rounds
@@ -1614,14 +1663,15 @@ int launch_norm16_flow(rt_device* dev, const void* x, const void* scale, const v
     RT_REQUIRE(groups <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");
     const uint32_t nt = (cols + 255) / 256;
     const size_t affine_bytes = (size_t)nt * 512 * (KIND == NORM_LAYER ? 2 : 1);
+    const uint32_t steps = nf_steps(nt);
 #define RT_FLOW(NT)                                                                                                                  \
     hipLaunchKernelGGL((norm_flow16_kernel<T, KIND, NT, RB>), dim3((unsigned)(groups < cus ? groups : cus)), dim3(64 + RB * 32),     \
                        affine_bytes, dev->stream, (const T*)x, (const T*)scale, (const T*)bias, (T*)y, rows, cols, (uint32_t)groups, R, eps)
-    if (nt <= 2) RT_FLOW(2);
-    else if (nt <= 4) RT_FLOW(4);
-    else if (nt <= 8) RT_FLOW(8);
-    else if (nt <= 12) RT_FLOW(12);
-    else if (nt <= 16) RT_FLOW(16);
+    if (steps == 2) RT_FLOW(2);
+    else if (steps == 4) RT_FLOW(4);
+    else if (steps == 8) RT_FLOW(8);
+    else if (steps == 12) RT_FLOW(12);
+    else if (steps == 16) RT_FLOW(16);
     else RT_FLOW(20);
 #undef RT_FLOW
     RT_CHECK_LAUNCH("norm_flow16_kernel");
@@ -1640,26 +1690,17 @@ int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* 
     // where rows come in several rounds ([8192,3072] 25.5 against 22.1 us, [65536,512] 43 against 25).
     if (vec_ok && KIND == NORM_RMS && cols >= 256 && cols <= 4096 && rows <= 16ull * (uint64_t)dev->num_cus)
         return launch_rms16_par<T>(dev, x, scale, y, rows, cols, eps);
-    // The streaming kernel: rows that are not whole aligned vectors always (against norm_seq16_kernel: [1001,1001] 23.5 ->
-    // 6.8 us, [8000,1001] 35.8 -> 12, RMSNorm [16000,3001] bf16 127 -> 50).  Rows of whole vectors where they are many or long:
-    // there the kernel below reads x twice and puts a walker for every 8 rows on the SIMDs (LayerNorm [16384,3072] f16
-    // 52 -> 43 us, bf16 74 -> 58, RMSNorm bf16 55 -> 46; [32768,4096] f16 123 -> 100, RMSNorm bf16 135 -> 105).  In between
-    // that one's several blocks per CU win: [8192,2560] f16 19 against 23 us, [4096,1024] 6.9 against 7.5, and so they
-    // do for short rows ([16384,384] f16 9.8 against 10.8).  bf16 LayerNorm, whose walker needs the f32 tiles of both
-    // sums, gains earlier: [8192,1024] 16.6 -> 14.6 us, [2048,2560] 16.4 -> 14.9.
     const uint64_t cus = (uint64_t)dev->num_cus;
-    const bool many = rows > 40 * cus;
-    bool flow = cols >= 8 && cols <= NF_MAX_COLS;
-    if (flow && vec_ok) {
-        const bool bf16_layer = std::is_same<T, bf16_t>::value && KIND == NORM_LAYER;
-        flow = cols > NP_KEEP_MAX_COLS || (many && cols > 512) || (bf16_layer && (rows > 24 * cus || (rows <= 8 * cus && cols > 512)));
-    }
-    if (flow) {
-        // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; with fewer rows than that gives
-        // every CU, fewer, so that all of them have some
-        if (many) return launch_norm16_flow<T, KIND, 30>(dev, x, scale, bias, y, rows, cols, eps);
-        if (rows > 8 * cus) return launch_norm16_flow<T, KIND, 16>(dev, x, scale, bias, y, rows, cols, eps);
-        return launch_norm16_flow<T, KIND, 8>(dev, x, scale, bias, y, rows, cols, eps);
+    constexpr bool BF16 = std::is_same<T, bf16_t>::value, LAYER = KIND == NORM_LAYER;
+    if (cols >= 8 && cols <= NF_MAX_COLS &&
+        (vec_ok ? nf_takes_aligned(BF16, LAYER, rows, cols, cus) : nf_takes_ragged(BF16, LAYER, rows, cols, cus))) {
+        // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; fewer where that takes no more
+        // rounds (a walk costs the same for any number of rows: RMSNorm f16 [5000,4096] 27 us in two rounds of 16, 21 in one of
+        // 30).  LayerNorm rows of 20 steps: three rounds of 16 rather than two of 30, which spill ([10240,5113] f16 56 / 62)
+        if (rows <= 8 * cus) return launch_norm16_flow<T, KIND, 8>(dev, x, scale, bias, y, rows, cols, eps);
+        if (rows <= 16 * cus || (rows > 30 * cus && rows <= (LAYER && cols > 4096 ? 40 : 32) * cus))
+            return launch_norm16_flow<T, KIND, 16>(dev, x, scale, bias, y, rows, cols, eps);
+        return launch_norm16_flow<T, KIND, 30>(dev, x, scale, bias, y, rows, cols, eps);
     }
     if (vec_ok) {
         const uint64_t blocks = (rows + 7) / 8;

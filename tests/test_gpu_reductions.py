@@ -521,8 +521,9 @@ def test_norms_f16(dev, oracle, shape):
     assert mismatch_count(got, want) == 0, mismatch_count(got, want)
 
 
-@pytest.mark.parametrize("rows,cols,kind", [(13, 2560, "f16"), (2048, 4096, "f16"), (2051, 3072, "bf16"), (5, 8, "bf16"), (300, 264, "f16"),   # all blocks resident: output pass from LDS
-                                            (40000, 256, "f16"), (9000, 1536, "bf16"), (64, 4104, "f16")])                              # more blocks than fit, rows too long: x re-read
+@pytest.mark.parametrize("rows,cols,kind", [(13, 2560, "f16"), (512, 3072, "f16"), (2051, 3072, "bf16"), (1000, 3712, "f16"), (5, 8, "bf16"), (300, 264, "f16"),   # all blocks resident: output pass from LDS
+                                            (40000, 256, "f16"), (8195, 2560, "f16"), (9000, 1536, "bf16"), (5003, 4096, "bf16"), (4101, 4608, "f16"),               # more blocks than fit, rows too long: x re-read
+                                            (2048, 4096, "f16"), (64, 4104, "f16")])                                                                                   # LayerNorm streams through persistent blocks
 def test_norms_16_bit_both_output_passes(dev, oracle, rows, cols, kind):
     """the 16-bit reference norms keep the raw rows, scale and bias in LDS for the output pass when every block of the
     launch is resident at once, and re-read x otherwise: same bits either way, with and without bias, ragged last block"""
@@ -539,8 +540,9 @@ def test_norms_16_bit_both_output_passes(dev, oracle, rows, cols, kind):
         assert np.array_equal(np.asarray(got).view(np.uint16), np.asarray(want).view(np.uint16)), (name, rows, cols, kind)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 8), (7, 9), (9, 255), (2049, 257), (300, 1001), (33, 2047), (2100, 3071), (8, 4097), (300, 5113), (300, 5120), (6200, 520),   # one group a block
-                                       (10300, 13), (10300, 520), (11000, 777), (16000, 1041), (31000, 264)])                                                         # several, the last ones short
+@pytest.mark.parametrize("rows,cols", [(9, 255), (2049, 257), (300, 1001), (33, 2047), (2100, 3071), (8, 4097), (300, 5113), (300, 5120),   # one group a block
+                                       (10300, 520), (11000, 777), (16000, 1041), (31000, 264),                                          # several, the last ones short
+                                       (1, 8), (7, 9), (6200, 520), (10300, 13)])                                                        # other kernels, for some or all of the tensors
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_norms_16_bit_streaming_kernel(dev, oracle, rows, cols, kind):
     """Rows that are not whole vectors, long rows and many rows stream through persistent blocks: the oracle's bits, for
@@ -573,6 +575,87 @@ def test_norms_16_bit_streaming_kernel(dev, oracle, rows, cols, kind):
             assert (got[:yo] == 7).all() and (got[yo + rows * cols:] == 7).all(), (name, xo, yo)
         run("layer", src.view(xo, (rows, cols)), src.view(xo, (rows, cols)))
         assert np.array_equal(src.to_numpy()[xo:xo + rows * cols].view(np.uint16), np.asarray(want["layer"]).view(np.uint16).ravel()), ("in place", xo)
+
+
+def _norms_16_bit(dev, oracle, x, w, b, bf, xo, yo):
+    """LayerNorm and RMSNorm of x, `xo` and `yo` elements into their buffers: the oracle's bits (any NaN for a NaN), nothing
+    written outside of y"""
+    rows, cols = x.shape
+    flat = np.zeros(rows * cols + 16, x.dtype)
+    flat[xo:xo + rows * cols] = x.ravel()
+    src, dw, db = dev.upload(flat, bf16=bf).view(xo, (rows, cols)), dev.upload(w, bf16=bf), dev.upload(b, bf16=bf)
+    top = 0x7f80 if bf else 0x7c00
+    for name, want in (("layer", oracle.layer_norm(x, w, b, 1e-5, bf16=bf, intended=True)), ("rms", oracle.rms_norm(x, w, 1e-5, bf16=bf, intended=True))):
+        dst = dev.upload(np.full(rows * cols + 16, 7, x.dtype), bf16=bf)
+        if name == "rms":
+            dev.rms_norm(src, dw, 1e-5, out=dst.view(yo, (rows, cols)))
+        else:
+            dev.layer_norm(src, dw, db, 1e-5, out=dst.view(yo, (rows, cols)))
+        got = dst.to_numpy()
+        assert (got[:yo] == 7).all() and (got[yo + rows * cols:] == 7).all(), (name, xo, yo)
+        g, e = got[yo:yo + rows * cols].view(np.uint16), np.asarray(want).view(np.uint16).ravel()
+        bad = (g != e) & ~(((g & 0x7fff) > top) & ((e & 0x7fff) > top))
+        assert not bad.any(), (name, rows, cols, bf, int(bad.sum()), np.flatnonzero(bad)[:8])
+
+
+def _conv16(oracle, kind):
+    def conv(a):
+        with np.errstate(over="ignore"):
+            return _bf16(oracle, a) if kind == "bf16" else np.asarray(a, np.float32).astype(np.float16)
+
+    return conv
+
+
+@pytest.mark.parametrize("rows,cols,off", [(2100, 3841, 1), (2100, 4096, 0), (2100, 5113, 3),                                              # 16 rows a block, 16 and 20 steps
+                                           (4200, 3071, 1), (4200, 4095, 5), (4200, 5113, 1),                                              # 30 rows a block, one group
+                                           (8200, 2305, 1), (8200, 3072, 0), (8200, 4095, 1), (8200, 5113, 1), (9000, 4609, 1),                            # and two
+                                           (15400, 2049, 1), (15400, 3072, 0), (10300, 4096, 0), (10300, 5120, 0)])                        # and three, the last one short
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_streaming_kernel_long_rows(dev, oracle, rows, cols, off, kind):
+    """the streaming kernel's larger instantiations, on rows of whole vectors and on others"""
+    rng = np.random.default_rng(318)
+    conv = _conv16(oracle, kind)
+    x = conv(rng.standard_normal((rows, cols), np.float32) * np.float32(1.5) + np.float32(0.25))
+    _norms_16_bit(dev, oracle, x, conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), kind == "bf16", off, off and 7 - off)
+
+
+@pytest.mark.parametrize("rows,cols,off", [(300, 1001, 1), (2100, 2560, 1), (4200, 777, 3), (10300, 1024, 0), (300, 5120, 0)])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_streaming_kernel_special_values(dev, oracle, rows, cols, off, kind):
+    """rows with infinities, NaN, subnormals, zeros and values whose squares overflow or vanish, at both ends of a row and
+    across it, and such values among scale and bias"""
+    rng = np.random.default_rng(319)
+    conv = _conv16(oracle, kind)
+    big, tiny, sub = (2e38, 1e-25, 3e-39) if kind == "bf16" else (6e4, 2e-4, 3e-6)
+    xf = rng.standard_normal((rows, cols)).astype(np.float32)
+    special = np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, big, -big, tiny, -tiny, sub, -sub], np.float32)
+    scales = np.where(np.isfinite(special) & (special != 0), np.minimum(np.abs(special), 1e38), 1.0).astype(np.float32)
+    for i, v in enumerate(special):
+        xf[i, 0] = xf[20 + i, -1] = xf[40 + i, cols // 2] = v
+        xf[60 + i, :] = v                                                    # a row of nothing else
+        xf[80 + i] *= scales[i] / 5
+        xf[100 + i, ::7] = v
+    xf[120, :-1] = 0.0
+    xf[rows - 1, 3] = np.inf
+    wf, bf = (1 + 0.02 * rng.standard_normal(cols)).astype(np.float32), (0.02 * rng.standard_normal(cols)).astype(np.float32)
+    wf[5:5 + len(special)], bf[30:30 + len(special)] = special, special
+    wf[-1], bf[-2] = sub, np.nan
+    _norms_16_bit(dev, oracle, conv(xf), conv(wf), conv(bf), kind == "bf16", off, off)
+
+
+@pytest.mark.parametrize("rows,cols,off", [(15, 160, 1), (16, 160, 1), (15, 161, 1), (4096, 100, 1), (4097, 100, 1), (15359, 65, 1), (15360, 65, 1), (16384, 97, 1), (25600, 97, 1),   # ragged
+                                           (15360, 41, 1), (30720, 9, 1), (30720, 12, 1), (30720, 40, 1), (33024, 13, 1), (65537, 24, 1), (300, 5121, 1), (300, 7, 1),
+                                           (2048, 776, 0), (2048, 1280, 0), (2048, 3336, 0), (2049, 3336, 0), (2049, 4104, 0), (4096, 3592, 0), (4097, 3592, 0), (6144, 520, 0), (6145, 520, 0),
+                                           (6145, 256, 0), (12289, 256, 0), (7681, 3848, 0), (8192, 1280, 0), (8193, 1280, 0), (8193, 1800, 0), (8193, 3848, 0), (10241, 512, 0), (10241, 520, 0),
+                                           (10753, 1280, 0), (63, 3336, 0), (64, 3336, 0), (2048, 5120, 0), (2049, 5120, 0), (15361, 1280, 0), (16897, 1280, 0), (300, 5128, 0)])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_both_sides_of_the_kernel_choice(dev, oracle, rows, cols, off, kind):
+    """the same bits on either side of the lines at which another kernel, or another number of rows a block, takes over
+    (on 256 CUs)"""
+    rng = np.random.default_rng(320)
+    conv = _conv16(oracle, kind)
+    x = conv(rng.standard_normal((rows, cols), np.float32) * np.float32(1.5) + np.float32(0.25))
+    _norms_16_bit(dev, oracle, x, conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), kind == "bf16", off, off)
 
 
 @pytest.mark.parametrize("cols", [256, 512, 1000, 1536, 2560, 3072, 4096])
