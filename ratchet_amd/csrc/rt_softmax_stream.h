@@ -836,17 +836,8 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     if (rc) return rc;
     const uint32_t nt = (cols + SP_TC - 1) / SP_TC;
     if (ragged && nt > SP_MAX_STEPS) return RT_OK;           // (a ragged row's one vector past its last step is the walker's)
-    // f16 rows of 4097 to 8192 columns stay in registers, 15 to a group (the LONG variant): two passes over memory instead of
-    // four, and the walk, on half as many rows at a time, is what bounds it (1.9 us per 512 columns with its barriers; five
-    // rounds of 13 rows on [1,8,2048,8192]).  Parked in y / in registers, with a causal mask: [1,8,2048,8192] 207 / 155 us,
-    // [1,8,2048,6144] 144 / 119, [1,8,2048,4608] 117 / 101, [1,32,1000,7000] 313 / 282, [1,16,1000,5000] 115 / 108, [1,8,100,8192] 49 / 35;
-    // [1,8,512,8192], whose 4096 rows are one round of 16-row groups and two of 15, 64 us either way.  The bf16 walk takes
-    // 5 ns an element and half as many rows at a time cost more than the two passes on most shapes
-    // ([1,8,2048,8192] 243 / 264 us, [1,32,1000,7000] with a mask 432 / 530): bf16 parks in y.
     constexpr bool LONG_ROWS = std::is_same<T, half_t>::value;
-    const bool longer = LONG_ROWS && !ragged && nt > SP_MAX_STEPS && nt <= 2 * SP_MAX_STEPS;
     const uint32_t long_steps = nt <= 10 ? 5 : nt <= 12 ? 6 : 8;       // of 1024 columns
-    const bool long_full = longer && cols == long_steps * 2 * SP_TC;
     const bool full = !ragged && cols % SP_TC == 0 && nt != 7 && nt <= 8;
 #define RT_SP(NS, F, M)                                                                                                              \
     do {                                                                                                                             \
@@ -940,7 +931,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // one mask row for two heads: rows of an even number of steps under a mask that repeats every P rows
         const bool pair = mask && !ragged && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
         sch.item_reps = pair ? (sch.reps + 1) / 2 : sch.reps;
-        const uint32_t rmax = pair || longer ? SP_HALF : SP_ROWS, rmul = pair ? 2 : 1;
+        const uint32_t rmul = pair ? 2 : 1;
         // rows per group: every block runs ceil(groups / grid) rounds of 8-or-fewer steps whatever the group holds, so
         // 4370 groups of 30 rows on 256 CUs cost 18 rounds where 17.07 are needed; 27-row groups make 19 full rounds.
         // A step takes the longer of the walk (1.5 us whatever the group holds) and the group's memory time (2 KiB per
@@ -952,19 +943,19 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // of which pulls the mask rows into its own L2.  Among the sizes within 5 % of the cheapest, the one that keeps a
         // mask group on the fewest XCDs is taken ([1,16,4096,4096] with a causal mask: 27 rows, 152 groups a period, 211 us;
         // the cheapest size by the count alone, 26 rows and 158 groups, 224 us; 114 against 121 us on [1,32,2048,2048]).
-        {
-            auto cost_of = [&](uint32_t R) -> uint64_t {
-                const uint64_t groups = (uint64_t)((sch.P + R - 1) / R) * sch.item_reps;
-                const uint64_t rounds = (groups + dev->num_cus - 1) / dev->num_cus;
-                return rounds * (R * rmul + 1 > 18 ? R * rmul + 1 : 18);
-            };
+        auto rounds_of = [&](uint32_t R) -> uint64_t {
+            const uint64_t groups = (uint64_t)((sch.P + R - 1) / R) * sch.item_reps;
+            return (groups + dev->num_cus - 1) / dev->num_cus;
+        };
+        auto rows_per_group = [&](uint32_t rmax) -> uint32_t {
+            auto cost_of = [&](uint32_t R) -> uint64_t { return rounds_of(R) * (R * rmul + 1 > 18 ? R * rmul + 1 : 18); };
             uint64_t best = ~0ull;
-            sch.R = rmax;
+            uint32_t pick = rmax;
             for (uint32_t R = rmax; R >= 1; R--) {
                 const uint64_t cost = cost_of(R);
                 if (cost <= best) {
                     best = cost;
-                    sch.R = R;
+                    pick = R;
                 }
             }
             if (mask && sch.reps > 1 && !pair) {
@@ -972,7 +963,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
                     const uint32_t g = ((sch.P + R - 1) / R) % 8;
                     return g == 0 ? 1 : (g % 4 == 0) ? 2 : (g % 2 == 0) ? 4 : 8;
                 };
-                uint32_t pick = sch.R, pick_x = xcds_of(sch.R);
+                uint32_t pick_x = xcds_of(pick);
                 uint64_t pick_cost = best;
                 for (uint32_t R = rmax; R >= 1; R--) {
                     const uint64_t cost = cost_of(R);
@@ -984,9 +975,31 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
                         pick_cost = cost;
                     }
                 }
-                sch.R = pick;
             }
+            return pick;
+        };
+        sch.R = rows_per_group(pair ? SP_HALF : SP_ROWS);
+        // f16 rows of 4097 to 8192 columns: in registers, 15 to a group (the LONG variant), or 30 to a group and parked in y?
+        // In registers x is read and y written once, and the walk is the bound: 1.87 us per 512 columns with its barriers, on
+        // half as many rows at a time and in steps of 1024 columns, of which 5, 6 or 8 are taken.  Parked, a round takes the
+        // longer of its steps and its four passes over memory (3/8 ns per column of a group's rows), and the last one's
+        // quotients follow.  So the registers win where the rows come to memory ([1,8,2048,8192] with a causal mask 200 us
+        // parked / 156 in registers, [1,8,2048,4608] 116 / 101) and where all rows are one round either way ([1,8,100,8192]
+        // 49 / 35), and lose where they take one round more or walk far past the row's end ([4096,4104] 39.5 / 44.7,
+        // [4096,6152] 54 / 67, [5000,6656] 57 / 67, [8000,6152] 87 / 96).  Over 800 sizes with inputs and outputs moving
+        // through 580 MB the pick costs 0.2 % on average against the better one of the two, and 8 % at most.
+        // The bf16 walk takes 5 ns an element; in registers it was slower without a mask and on short periods ([1,8,2048,8192]
+        // 243 parked / 264, rows of 1000-row periods with a mask 432 / 530) and faster with a mask of whole rounds
+        // ([1,8,2048,8192] 344 / 293): bf16 parks in y.
+        bool longer = false;
+        if (LONG_ROWS && !ragged && nt > SP_MAX_STEPS && nt <= 2 * SP_MAX_STEPS) {
+            const uint32_t R = rows_per_group(SP_HALF);
+            const uint64_t in_registers = rounds_of(R) * long_steps * 3740;                                  // ns
+            const uint64_t memory = (uint64_t)sch.R * cols * 3 / 8, walk = (uint64_t)sch.nsteps * 2000;
+            longer = in_registers <= rounds_of(sch.R) * (memory > walk ? memory : walk) + (uint64_t)sch.nsteps * 400;
+            if (longer) sch.R = R;
         }
+        const bool long_full = longer && cols == long_steps * 2 * SP_TC;
         sch.GP = (sch.P + sch.R - 1) / sch.R;
         sch.pace = sch.phase_fx = 0;                         // set below, once the grid is known
         sch.gp_div = make_fastdiv(sch.GP);

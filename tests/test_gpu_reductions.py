@@ -323,6 +323,12 @@ def test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, ki
         check(dx.to_numpy().reshape(rows, cols), want, name + " in place")
 
 
+@pytest.mark.parametrize("rows,cols", [(4096, 4104), (4700, 8192), (6000, 5000), (6144, 6144), (7000, 6152), (8200, 4104)])
+def test_softmax_f16_rows_of_4097_to_8192_columns_in_several_rounds(dev, oracle, rows, cols):
+    """more rows than one round of fifteen a block: in registers or parked in y, whichever takes less time, the oracle's bits"""
+    test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, "f16")
+
+
 @pytest.mark.parametrize("shape,kind", [((2, 4, 333, 1001), "f16"), ((1, 3, 100, 199), "f16"), ((70, 4095), "f16"), ((7, 4097), "f16"), ((50, 2047), "f16"), ((90, 511), "f16"), ((40, 2305), "f16"), ((45, 1535), "f16"), ((33, 3071), "f16"), ((33, 513), "f16"),
                                         ((1000, 193), "f16"), ((61, 2561), "f16"), ((2, 2, 77, 1001), "bf16"), ((40, 3001), "bf16"), ((31, 1535), "bf16"), ((900, 250), "bf16")])
 def test_softmax_16_bit_ragged_rows_stream(dev, oracle, shape, kind):
