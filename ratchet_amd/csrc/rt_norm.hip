@@ -329,18 +329,16 @@ __global__ void __launch_bounds__(BLOCK) norm_via32_generic_kernel(const T* __re
 
 // ------------------------------------------------------------------------------------------------------------------
 // 16-bit LayerNorm / RMSNorm with the reference's sequential f32 accumulation.
-// A block owns RB consecutive rows.  Pass A: per column tile, all threads load 16-byte vectors, widen x and T(x*x) to
-// f32 and park them in LDS; lanes [0, RB) then add the squares of "their" row left to right, lanes [RB, 2RB) the values
+// A block owns RB consecutive rows.  Pass A: per column tile, all threads load elements, widen x and T(x*x) to f32 and park
+// them in LDS; lanes [0, RB) then add the squares of "their" row left to right, lanes [RB, 2RB) the values
 // (LayerNorm only).  Pass B re-reads x (from cache: the block touched it moments ago), normalises and stores.
 // ------------------------------------------------------------------------------------------------------------------
-template <typename T, int RB, int KIND, bool VEC>
+template <typename T, int RB, int KIND>
 __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__ x, const T* __restrict__ scale,
                                                            const T* __restrict__ bias, T* __restrict__ y, uint64_t rows, uint32_t cols,
                                                            float eps) {
     constexpr int TC = 128;
     constexpr int PAD = 4;
-    constexpr int VE = VEC ? 8 : 1;
-    constexpr int TV = TC / VE;
     constexpr int NSUM = (KIND == NORM_LAYER) ? 2 : 1;
     __shared__ __attribute__((aligned(16))) float tile[NSUM][RB][TC + PAD];      // [0] = squares, [1] = values
     __shared__ float sums[NSUM][RB];
@@ -353,32 +351,12 @@ __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__
 
     for (uint32_t c0 = 0; c0 < cols; c0 += TC) {
         const uint32_t ncol = (cols - c0 < (uint32_t)TC) ? cols - c0 : (uint32_t)TC;
-        for (uint32_t idx = threadIdx.x; idx < (uint32_t)RB * TV; idx += BLOCK) {
-            const uint32_t r = idx / TV, col = (idx % TV) * VE;
+        for (uint32_t idx = threadIdx.x; idx < (uint32_t)RB * TC; idx += BLOCK) {
+            const uint32_t r = idx / TC, col = idx % TC;
             if (r < nrows && col < ncol) {
-                const T* src = x + (row0 + r) * cols + c0 + col;
-                if (VEC) {
-                    Vec16<T> in;
-                    in.u = *reinterpret_cast<const v4u*>(src);
-                    float sq[8], xv[8];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        sq[q] = Ar<T>::widen(Ar<T>::mul(in.e[q], in.e[q]));
-                        xv[q] = Ar<T>::widen(in.e[q]);
-                    }
-                    float4* d0 = reinterpret_cast<float4*>(&tile[0][r][col]);
-                    d0[0] = make_float4(sq[0], sq[1], sq[2], sq[3]);
-                    d0[1] = make_float4(sq[4], sq[5], sq[6], sq[7]);
-                    if (KIND == NORM_LAYER) {
-                        float4* d1 = reinterpret_cast<float4*>(&tile[NSUM - 1][r][col]);
-                        d1[0] = make_float4(xv[0], xv[1], xv[2], xv[3]);
-                        d1[1] = make_float4(xv[4], xv[5], xv[6], xv[7]);
-                    }
-                } else {
-                    const T e = *src;
-                    tile[0][r][col] = Ar<T>::widen(Ar<T>::mul(e, e));
-                    if (KIND == NORM_LAYER) tile[NSUM - 1][r][col] = Ar<T>::widen(e);
-                }
+                const T e = x[(row0 + r) * cols + c0 + col];
+                tile[0][r][col] = Ar<T>::widen(Ar<T>::mul(e, e));
+                if (KIND == NORM_LAYER) tile[NSUM - 1][r][col] = Ar<T>::widen(e);
             }
         }
         __syncthreads();
@@ -406,26 +384,15 @@ __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__
     }
     __syncthreads();
 
-    const uint32_t cvec = cols / VE;
     for (uint32_t r = 0; r < nrows; r++) {
         RowStats<T> st;
         st.mu = s_mu[r];
         st.r = s_r[r];
         const T* src = x + (row0 + r) * cols;
         T* dst = y + (row0 + r) * cols;
-        for (uint32_t cv = threadIdx.x; cv < cvec; cv += BLOCK) {
-            if (VEC) {
-                Vec16<T> in, sc, bi, out;
-                in.u = reinterpret_cast<const v4u*>(src)[cv];
-                sc.u = reinterpret_cast<const v4u*>(scale)[cv];
-                if (KIND == NORM_LAYER && bias) bi.u = reinterpret_cast<const v4u*>(bias)[cv];
-#pragma unroll
-                for (int q = 0; q < 8; q++) out.e[q] = norm_one<T, KIND>(in.e[q], st, sc.e[q], bi.e[q], bias != nullptr);
-                st_stream(reinterpret_cast<v4u*>(dst) + cv, out.u);
-            } else {
-                const T b = (KIND == NORM_LAYER && bias) ? bias[cv] : Ar<T>::conv(0.0f);
-                dst[cv] = norm_one<T, KIND>(src[cv], st, scale[cv], b, bias != nullptr);
-            }
+        for (uint32_t c = threadIdx.x; c < cols; c += BLOCK) {
+            const T b = (KIND == NORM_LAYER && bias) ? bias[c] : Ar<T>::conv(0.0f);
+            dst[c] = norm_one<T, KIND>(src[c], st, scale[c], b, bias != nullptr);
         }
     }
 }
@@ -1593,14 +1560,8 @@ template <typename T, int KIND, int RB>
 int launch_norm16_rb(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
     const uint64_t blocks = (rows + RB - 1) / RB;
     RT_REQUIRE(blocks <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");
-    const bool vec_ok = (cols % 8 == 0) && rt_aligned(x, 16) && rt_aligned(y, 16) && rt_aligned(scale, 16) && (!bias || rt_aligned(bias, 16));
-    if (vec_ok) {
-        hipLaunchKernelGGL((norm_seq16_kernel<T, RB, KIND, true>), dim3((unsigned)blocks), dim3(BLOCK), 0, dev->stream, (const T*)x,
-                           (const T*)scale, (const T*)bias, (T*)y, rows, cols, eps);
-    } else {
-        hipLaunchKernelGGL((norm_seq16_kernel<T, RB, KIND, false>), dim3((unsigned)blocks), dim3(BLOCK), 0, dev->stream, (const T*)x,
-                           (const T*)scale, (const T*)bias, (T*)y, rows, cols, eps);
-    }
+    hipLaunchKernelGGL((norm_seq16_kernel<T, RB, KIND>), dim3((unsigned)blocks), dim3(BLOCK), 0, dev->stream, (const T*)x,
+                       (const T*)scale, (const T*)bias, (T*)y, rows, cols, eps);
     RT_CHECK_LAUNCH("norm_seq16_kernel");
     return RT_OK;
 }
