@@ -302,9 +302,11 @@ int rt_pool_trim(rt_device* dev) {
 // The reference's pool ages its unused buffers by passes (gpu/pools/dynamic_resource_pool.rs:140-190, called at the top of
 // every resolve: tensor.rs:800, gpu/device.rs:275-277): a buffer released during pass p can be reclaimed during pass
 // p + 1 and is destroyed at the start of pass p + 2 if nobody did.  The same here: a block parked before the previous
-// call of this function, and still parked, goes back to the driver.  A program that repeats its passes reuses every
-// block each time and never gets here with anything to free, so the steady state stays free of hipFree (and of the wait
-// for the stream that has to precede it); one whose sizes drift no longer grows the parked set without bound.  While a
+// call of this function, and still parked, goes back to the driver.  A program that repeats one pass reuses every block
+// each time and never gets here with anything to free, so its steady state stays free of hipFree (and of the wait for the
+// stream that has to precede it); one whose sizes drift no longer grows the parked set without bound.  A step of several
+// passes of its own sizes (a token that resolves four graphs one after the other) does pay: what a pass of one step
+// released is two passes old when the next step's second pass begins, is freed there and allocated again.  While a
 // device is capturing nothing is freed: the blocks wait for the first pass that begins outside a capture.
 int rt_pool_begin_pass(rt_device* dev) {
     int rc = rt_enter(dev);

@@ -638,22 +638,6 @@ __global__ void __launch_bounds__(NP_BLOCK) norm_pipe16_kernel(const T* __restri
     }
 }
 
-// The same walk for rows of 8 to NF_MAX_COLS columns as a stream: persistent blocks that take groups of 8 rows in turn.
-// The loader threads keep a group's rows in registers (NT vectors a thread) from the load to the store, and in step t of
-// a group, while wave 0 walks tile t, they normalise and store tile t of the group before and load the tile PF steps
-// ahead, across the groups: x is read once, and reads, walk and writes go on side by side instead of in phases that all
-// blocks of the chip pass at the same time.
-// What bounds it: with one group per block the walk (about 2.3 ns a column, whatever is left of the chip); with several,
-// memory, and in bf16 the vector instructions of the output (58 us for the [16384,3072] LayerNorm whose bytes take 38 at
-// the rate of a large copy; f16 43).  A walker occupies its SIMD's vector unit fully with 8 rows as with 30, which is why a block carries
-// up to 30 rows and a CU one block: with blocks of 8 rows, two to a CU, the same LayerNorm took 54 us in f16.
-// Rows of any length from 8 columns and on any element boundary: no access leaves the row; the last vector of a row is
-// its last eight elements, for the walk shifted so that none of them counts twice, and written with the same values as
-// the one before it where they overlap.
-// A row's vector is 16 bytes at `base + offset` through a buffer descriptor of the group's rows; where there is nothing to
-// load or to store (columns past the end, rows past the end, the group before the first) the offset lies outside of it and
-// the access is dropped, which keeps the step free of branches around memory instructions: the compiler then counts
-// exactly how many may stay in flight at each wait.
 // f rounded to bf16 and widened again, in one instruction: converted into the high half of a word whose low half is bf16(0) = 0
 __device__ __forceinline__ float np_round_bf16(float f) {
     uint32_t r;
@@ -687,7 +671,6 @@ template <typename T, int KIND> __device__ __forceinline__ v4u norm_vec16(const 
     }
     return out;
 }
-constexpr uint32_t NF_MAX_COLS = 5120;                       // 20 vectors a thread
 // run += the sixteen f32 values of four vectors, left to right (as one asm statement: with ordinary adds the compiler reads
 // a whole tile ahead, into 256 registers)
 __device__ __forceinline__ void np_add_f32x16(float& run, const v4u& a, const v4u& b, const v4u& c, const v4u& d) {
@@ -699,6 +682,26 @@ __device__ __forceinline__ void np_add_f32x16(float& run, const v4u& a, const v4
           "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]));
 #undef NP_ADD
 }
+// The same walk for rows of 8 to NF_MAX_COLS columns as a stream: persistent blocks, one to a CU, that take groups of up to
+// RB rows (8, 16 or 30) in turn.  The RB / 2 loader waves keep a group's rows in registers (NT vectors a thread) from the
+// load to the store, and in step t of a group, while wave 0 walks tile t, they normalise and store tile t of the group
+// before and load the tile PF steps ahead, across the groups: x is read once, and reads, walk and writes go on side by
+// side instead of in phases that all blocks of the chip pass at the same time.
+// What bounds it: with one group per block the walk (about 2.3 ns a column, whatever is left of the chip); with several,
+// memory, and in bf16 the vector instructions of the output (58 us for the [16384,3072] LayerNorm whose bytes take 38 at
+// the rate of a large copy; f16 43).  A walker occupies its SIMD's vector unit fully with 8 rows as with 30, which is why a
+// block carries up to 30 rows and a CU one block: with blocks of 8 rows, two to a CU, the same LayerNorm took 54 us in f16.
+// A group takes NT steps whatever its rows hold (2, 4, 8, 12, 16 and 20 exist): 1032 columns are five tiles in eight steps.
+// The LayerNorm variants of 20 steps and 30 rows hold more than their 128 registers: f16 spills 15 of them (52 bytes of
+// scratch a lane), bf16 5 (20 bytes); no other one does.
+// Rows of any length from 8 columns and on any element boundary: no access leaves the row; the last vector of a row is
+// its last eight elements, for the walk shifted so that none of them counts twice, and written with the same values as
+// the one before it where they overlap.
+// A row's vector is 16 bytes at `base + offset` through a buffer descriptor of the group's rows; where there is nothing to
+// load or to store (columns past the end, rows past the end, the group before the first) the offset lies outside of it and
+// the access is dropped, which keeps the step free of branches around memory instructions: the compiler then counts
+// exactly how many may stay in flight at each wait.
+constexpr uint32_t NF_MAX_COLS = 5120;                       // 20 vectors a thread
 template <typename T, int KIND, int NT, int RB>
 __global__ void __launch_bounds__(64 + RB * 32) norm_flow16_kernel(const T* x, const T* __restrict__ scale, const T* __restrict__ bias, T* y,
                                                                uint64_t rows, uint32_t cols, uint32_t groups, uint32_t R, float eps) {
@@ -759,7 +762,7 @@ __global__ void __launch_bounds__(64 + RB * 32) norm_flow16_kernel(const T* x, c
         return;
     }
 
-    // -------------------------------------------------------------------- waves 1..4: load, square, normalise, store
+    // -------------------------------------------------------------------- the other waves: load, square, normalise, store
     const uint32_t lt = threadIdx.x - 64;
     const uint32_t r = lt >> 5, cv = lt & 31;                                   // row, vector within the tile
     const uint32_t row_bytes = cols * 2;

@@ -158,7 +158,7 @@ template <> struct SpType<bf16_t> {
     static constexpr bool CHUNK_ASM = true;                                       // the walker adds sixteen values per asm statement (add_chunk)
 };
 
-// NSTEP > 0: rows of up to NSTEP * 512 columns, exp values parked in registers.  NSTEP == 0: longer rows; the exp values
+// NSTEP > 0: rows of up to NSTEP * 512 columns (LONG: 1024), exp values parked in registers.  NSTEP == 0: longer rows; the exp values
 // are parked in y instead and read back (by the thread that wrote them) when the row sum is known: 4 bytes of traffic per
 // element and byte of the type instead of 2, any row length.
 //
@@ -174,6 +174,8 @@ template <> struct SpType<bf16_t> {
 // LONG (rows of SP_TC * SP_MAX_STEPS up to twice that many columns): a group has 15 rows and a step 1024 columns.  The two
 // vectors a loader thread handles in a step lie 512 columns apart in ONE row instead of in two rows, and the walker walks
 // 1024 columns between barriers, so that the registers hold rows twice as long and x is read and y written once.
+// NSTEP is 5, 6 or 8: rows of 4097 to 4608 columns walk 5120, those of 6145 to 7168 walk 8192.  The masked variants of 5 and
+// 8 steps spill 4 to 8 of their 128 vector registers (20 bytes of scratch a lane).
 template <typename T, int NSTEP, bool FULL, int MASK, bool RAGGED = false, bool LONG = false>
 __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16_t* __restrict__ table, const T* x, const T* mask, T* y,
                                                                     uint64_t rows, uint32_t cols, SpSched sch, uint16_t* row_sums,

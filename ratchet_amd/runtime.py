@@ -158,6 +158,10 @@ class Event:
 
 
 class Device:
+    """One GPU: its storage pool, and the ops, which are enqueued on a stream of the device's own and return at once.  No other
+    stream is ordered with that one, torch's current stream included: who fills a buffer or reads a result through torch (or
+    lets such a buffer go back to the pool) waits for that stream first, and calls sync() before the other side reads."""
+
     def __init__(self, ordinal=0):
         self.lib = _lib.load()
         self.handle = None
