@@ -24,16 +24,19 @@ constexpr int BLOCK = 256;
 //        (162 400 of the CU's 163 840 bytes), so exp is one ds_read_u16 per element with the bit pattern as the index:
 //        no range clamping, no NaN special case.
 //   sum: per 512-column step the exp values also go to an LDS tile; lanes 0..29 of wave 0 each walk one row of the
-//        tile left to right with dependent v_add_f16 (3 ns each on this chip with the LDS reads the wave issues in
-//        between, 1.5 us per step; bf16: v_add_f32 and v_cvt_pk_bf16_f32 into the high half of a word, two dependent
-//        instructions and one that moves the operand into place, 5 ns).  The tile is single
+//        tile left to right with dependent v_add_f16 (a one-wave probe: 4.2 cycles each, the issue rate; bf16: v_add_f32 and
+//        v_cvt_pk_bf16_f32 into the high half of a word, two dependent instructions, and one that moves the operand into
+//        place, 12.1 cycles).  64 values are added while the LDS reads of the next 64 are in flight; left to the compiler the
+//        reads stood four adds before their use and every 32 adds waited for LDS ([1,8,2048,8192] f16, which the walk
+//        bounds: 156 -> 132 us).  The tile is single
 //        buffered with two barriers per step: the loaders look up step t+1 into registers and divide / store the
 //        previous group's step t while wave 0 walks step t, and only the short LDS write of the tile sits between the
-//        barriers with wave 0 idle.  A step is 30 KiB in and 30 KiB out of HBM per CU, about 2 us at a CU's share of
-//        8 TB/s, so the walk stays hidden; wave 0 is kept free of any other work and raises its issue priority.
-//   divide: the outputs of group g are produced while group g+1 streams in: y = e / sum with the quotient computed as
-//        q0 = e * (1/sum) plus one fma correction, which is the correctly rounded f16 quotient for normal finite sums
-//        (checked against IEEE division over operand pairs on the GPU); other sums, and bf16, take the IEEE path.
+//        barriers, during which wave 0 adds half of the 64 values that it holds.  A step is 30 KiB in and 30 KiB out of HBM
+//        per CU, about 2 us at a CU's share of 8 TB/s, so the f16 walk stays hidden; wave 0 is kept free of any other work
+//        and raises its issue priority.
+//   divide: the outputs of group g are produced while group g+1 streams in: y = e / sum from the reciprocal of the sum where
+//        that rounds as the division does (SpType::short_quotients: two instructions a value in f16, two and a half in bf16,
+//        against fourteen of the IEEE division, which took bf16 [1,32,4096,4096] from 550 to 700 us); other sums divide.
 //   mask: with MASK, a second operand (one [P, cols] block shared by every period of P rows, e.g. an [S, T] attention
 //        mask under B * H heads) is added to x in the 16-bit type as the vectors arrive: scores.add(mask).softmax() without the sum
 //        ever reaching memory, bit-identical to the two separate ops.
@@ -54,10 +57,18 @@ typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// exp of two packed f16 bit patterns: two lookups in the full 65536-entry table (NaN, inf and the saturated ends included)
-__device__ __forceinline__ uint32_t sp_exp_pair(const uint16_t* lut, uint32_t p) {
-    return (uint32_t)lut[p & 0xffffu] | ((uint32_t)lut[p >> 16] << 16);
+// exp of a 16-bit pattern, the low or the high half of a word: one lookup in the full 65536-entry table (NaN, inf and the saturated
+// ends included), which lies at the start of LDS: the address is one shift of the selected half (as C the compiler spends two
+// instructions on it)
+__device__ __forceinline__ uint32_t sp_exp_lo(uint32_t p) {
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(p) : "v"(1u), "v"(p));
+    return *(const __attribute__((address_space(3))) uint16_t*)p;
 }
+__device__ __forceinline__ uint32_t sp_exp_hi(uint32_t p) {
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(p) : "v"(1u), "v"(p));
+    return *(const __attribute__((address_space(3))) uint16_t*)p;
+}
+__device__ __forceinline__ uint32_t sp_exp_pair(uint32_t p) { return sp_exp_lo(p) | sp_exp_hi(p) << 16; }
 
 // Which 30-row groups a block works on.  Rows come in `reps` periods of P rows (P = all rows when nothing repeats; P = the
 // rows one mask covers when a mask is added, e.g. S rows per head for an [S, T] mask under B * H heads); a period holds
@@ -106,7 +117,21 @@ template <> struct SpType<half_t> {
     static __device__ __forceinline__ v4u add_vec(const v4u& a, const v4u& b) {    // eight f16 sums, rounded as the separate add does
         return __builtin_bit_cast(v4u, __builtin_bit_cast(h16x8, a) + __builtin_bit_cast(h16x8, b));
     }
-    static constexpr bool SHORT_DIVISION = true;
+    // e / s for both halves of a word, s in [SHORT_MIN, SHORT_MAX]: e * rinv + e * rlow, where rinv + rlow is 1 / s to 48 bits, so
+    // the f32 quotient is off by one rounding.  Two 11-bit significands never divide to the middle between two f16 values and stay
+    // 2^-23 away from it, so f16 of that quotient is f16 of e / s (all pairs compared on the CPU; subnormal results too: their
+    // middles are exact f32 values).
+    static constexpr bool SHORT_TWO = true;
+    static constexpr float SHORT_MIN = 6.103515625e-05f, SHORT_MAX = 65504.0f;
+    static __device__ __forceinline__ uint32_t short_quotients(uint32_t e, float rinv, float rlow) {
+        const h16x2 v = __builtin_bit_cast(h16x2, e);
+        float q0 = __builtin_fmaf((float)v[0], rinv, __builtin_fmaf((float)v[0], rlow, 0.0f));
+        float q1 = __builtin_fmaf((float)v[1], rinv, __builtin_fmaf((float)v[1], rlow, 0.0f));
+        // keep the f32 quotient and its conversion apart: fused into v_fma_mixlo_f16 the pair rounds
+        // subnormal f16 results differently from fma-then-convert
+        asm volatile("" : "+v"(q0), "+v"(q1));
+        return round_pair(q0, q1);
+    }
     static constexpr bool CHUNK_ASM = false;                                      // the walker adds pair by pair
     static constexpr uint32_t NEG_INF_PAIR = 0xfc00fc00u;                         // two -inf
 };
@@ -154,7 +179,14 @@ template <> struct SpType<bf16_t> {
         return r;
     }
     static constexpr uint32_t NEG_INF_PAIR = 0xff80ff80u;
-    static constexpr bool SHORT_DIVISION = false;                                 // the quotient's range is f32's: always the IEEE division
+    // e / s for both halves of a word, s in [SHORT_MIN, SHORT_MAX]: e * (1 / s) is within 2^-23 of the quotient, and the quotient
+    // of two 8-bit significands is no closer than 2^-17 to the middle between two bf16 values (and never on it), or, where the
+    // result is subnormal, an exact f32 value when it is on the middle (all pairs compared on the CPU)
+    static constexpr bool SHORT_TWO = false;
+    static constexpr float SHORT_MIN = 0x1p-100f, SHORT_MAX = 0x1p100f;
+    static __device__ __forceinline__ uint32_t short_quotients(uint32_t e, float rinv, float) {
+        return cvt_pk(u2f(e << 16) * rinv, u2f(e & 0xffff0000u) * rinv);
+    }
     static constexpr bool CHUNK_ASM = true;                                       // the walker adds sixteen values per asm statement (add_chunk)
 };
 
@@ -223,6 +255,19 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         const v4u* trow = reinterpret_cast<const v4u*>(tile[wr]);
         typename ST::Run run = ST::zero();
         uint32_t gpar = 0;
+        constexpr int WALK_VECS = 8;
+        v4u held[WALK_VECS];
+        auto add_values = [&](const v4u (&v)[WALK_VECS], int from, int to) {     // onto `run`, left to right
+            if constexpr (ST::CHUNK_ASM) {
+#pragma unroll
+                for (int k = from; k < to; k += 2) ST::add_chunk(run, v[k], v[k + 1]);
+            } else {
+#pragma unroll
+                for (int k = from; k < to; k++)
+#pragma unroll
+                    for (int w = 0; w < 4; w++) ST::add_pair(run, v[k][w]);
+            }
+        };
         // the blocks take their steps out of phase with each other: block b starts b / grid of a step late
         uint32_t t_step = 0, t_last = 0, t_avg = sch.pace, t_slow = sch.pace + sch.pace / 5;
         if constexpr (PACED) {
@@ -257,38 +302,38 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                     }
                 }
             }
+            uint32_t steps = nsteps;
+            if constexpr (NSTEP == 1) asm volatile("" : "+s"(steps));    // kept a loop: as straight-line code it took 150 registers too many
 #pragma unroll 1
-            for (uint32_t t = 0; t < nsteps; t++) {
+            for (uint32_t t = 0; t < steps; t++) {
                 if (PACED && sch.pace) rt_pace_step(t_step, t_last, t_avg, sch.pace, t_slow);   // the walker is the block's clock
-                __syncthreads();                             // A
+                __syncthreads();                             // A: the loaders may overwrite the tile, its last values are in `held`
+                if (t > 0) add_values(held, 0, WALK_VECS / 2);
                 __syncthreads();                             // B: tile t is in LDS
-                // 16 values per chunk; the LDS reads of the next chunk are in flight during the 16 dependent adds
-                v4u c0 = trow[0], c1 = trow[1];
+                v4u ahead[WALK_VECS];
 #pragma unroll
-                for (int c = 0; c < STEP_COLS / 16; c++) {
-                    v4u n0 = c0, n1 = c1;
-                    if (c + 1 < STEP_COLS / 16) {
-                        n0 = trow[(c + 1) * 2];
-                        n1 = trow[(c + 1) * 2 + 1];
-                    }
-                    if constexpr (ST::CHUNK_ASM) {
-                        ST::add_chunk(run, c0, c1);
-                    } else {
+                for (int k = 0; k < WALK_VECS; k++) ahead[k] = trow[k];
+                __builtin_amdgcn_sched_barrier(0);           // here and below: left alone, the scheduler moves the reads down to their use
+                if (t > 0) add_values(held, WALK_VECS / 2, WALK_VECS);
 #pragma unroll
-                        for (int w = 0; w < 4; w++) ST::add_pair(run, c0[w]);
+                for (int c = 0; c < STEP_COLS / 8 / WALK_VECS; c++) {
 #pragma unroll
-                        for (int w = 0; w < 4; w++) ST::add_pair(run, c1[w]);
-                    }
-                    c0 = n0;
-                    c1 = n1;
+                    for (int k = 0; k < WALK_VECS; k++) held[k] = ahead[k];
+                    if (c + 1 == STEP_COLS / 8 / WALK_VECS) break;
+#pragma unroll
+                    for (int k = 0; k < WALK_VECS; k++) ahead[k] = trow[(c + 1) * WALK_VECS + k];
+                    __builtin_amdgcn_sched_barrier(0);
+                    add_values(held, 0, WALK_VECS);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
+            add_values(held, 0, WALK_VECS);
             if (RAGGED && tail_end) {
                 if (MASK) tailv = ST::add_vec(tailv, tailm);
 #pragma unroll
                 for (int w = 0; w < 4; w++) {                // elements past the row's end count as +0
                     const uint32_t keep = ((uint32_t)(4 * w) < tail_end ? 0xffffu : 0u) | ((uint32_t)(4 * w + 2) < tail_end ? 0xffff0000u : 0u);
-                    ST::add_pair(run, sp_exp_pair(lut, tailv[w]) & keep);
+                    ST::add_pair(run, sp_exp_pair(tailv[w]) & keep);
                 }
             }
             if (lane < SP_ROWS) sums[gpar][lane] = ST::run_bits(run);
@@ -459,29 +504,16 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     auto store_park = [&](const v4u& v, uint32_t off) { __builtin_amdgcn_raw_buffer_store_b128(v, ry, off, 0, 0); };   // read back soon
 
     // sum of the previous group's rows, reciprocal, and whether the short division applies: wave-uniform as well
-    float s_prev[2] = {1.0f, 1.0f}, rinv_prev[2] = {1.0f, 1.0f};
+    float s_prev[2] = {1.0f, 1.0f}, rinv_prev[2] = {1.0f, 1.0f}, rlow_prev[2] = {0.0f, 0.0f};
     bool fast_prev[2] = {true, true};
 
     auto quotients = [&](const v4u& ev, int h) -> v4u {      // e / sum of the previous group
         v4u out;
-        const float s = s_prev[h], rinv = rinv_prev[h];
-        if (ST::SHORT_DIVISION && fast_prev[h]) {
+        if (fast_prev[h]) {
 #pragma unroll
-            for (int w = 0; w < 4; w++) {
-                // v_fma_mix_f32 reads the f16 halves of ev[w] directly: a = e * r (+0), rem = e - s * a; no separate conversions
-                float a0, a1, m0, m1;
-                asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(a0) : "v"(ev[w]), "s"(rinv));
-                asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(a1) : "v"(ev[w]), "s"(rinv));
-                asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel_hi:[0,0,1]" : "=v"(m0) : "s"(s), "v"(a0), "v"(ev[w]));
-                asm("v_fma_mix_f32 %0, -%1, %2, %3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(m1) : "s"(s), "v"(a1), "v"(ev[w]));
-                float q0 = __builtin_fmaf(m0, rinv, a0);
-                float q1 = __builtin_fmaf(m1, rinv, a1);
-                // keep the f32 quotient and its conversion apart: fused into v_fma_mixlo_f16 the pair rounds
-                // subnormal f16 results differently from fma-then-convert
-                asm volatile("" : "+v"(q0), "+v"(q1));
-                out[w] = ST::round_pair(q0, q1);
-            }
+            for (int w = 0; w < 4; w++) out[w] = ST::short_quotients(ev[w], rinv_prev[h], rlow_prev[h]);
         } else {
+            const float s = s_prev[h];
 #pragma unroll
             for (int w = 0; w < 4; w++) out[w] = ST::round_pair(ST::widen_bits(ev[w] & 0xffffu) / s, ST::widen_bits(ev[w] >> 16) / s);
         }
@@ -493,26 +525,43 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             const uint32_t sb = __builtin_amdgcn_readfirstlane((uint32_t)sums[par][LONG ? rr : rr + h * SP_HALF]);
             const float s = ST::widen_bits(sb);
             s_prev[h] = s;
-            // normal, finite, not tiny: the reciprocal-plus-correction quotient is exact there
-            fast_prev[h] = (s >= 6.103515625e-05f) && (s < __builtin_huge_valf());
-            rinv_prev[h] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, fast_prev[h] ? 1.0f / s : 0.0f)));
+            fast_prev[h] = s >= ST::SHORT_MIN && s <= ST::SHORT_MAX;
+            const float rinv = fast_prev[h] ? 1.0f / s : 0.0f;
+            rinv_prev[h] = u2f(__builtin_amdgcn_readfirstlane(f2u(rinv)));
+            if (ST::SHORT_TWO) rlow_prev[h] = u2f(__builtin_amdgcn_readfirstlane(f2u(__builtin_fmaf(-s, rinv, 1.0f) * rinv)));
         }
     };
     // exp of the vector that arrived, in place (zeros past the row end: adding +0 is a no-op; rows past the tensor's end
     // read zeros and their sums are never used)
-    // A wave whose 512 values of this step are all -inf (the part of a row that a causal mask covers) takes exp(-inf) for
+    // A wave whose values of this step are all -inf (the part of a row that a causal mask covers) takes exp(-inf) for
     // all of them without the eight table reads per lane; the test is wave-wide, so the branch is a scalar one.
     const uint32_t exp_ninf = __builtin_amdgcn_readfirstlane((uint32_t)lut[ST::NEG_INF_PAIR & 0xffffu] * 0x10001u);
-    auto exp_in_place = [&](v4u& in, const v4u& m, uint32_t t, uint32_t sh, int h) {
-        if (MASK) in = ST::add_vec(in, m);                   // scores + mask in the 16-bit type, as the separate add would round it
-        const bool mine = ((in[0] ^ ST::NEG_INF_PAIR) | (in[1] ^ ST::NEG_INF_PAIR) | (in[2] ^ ST::NEG_INF_PAIR) | (in[3] ^ ST::NEG_INF_PAIR)) == 0;
-        if (__builtin_amdgcn_ballot_w64(!mine) == 0) {
-            in = v4u{exp_ninf, exp_ninf, exp_ninf, exp_ninf};
-        } else {
-#pragma unroll
-            for (int w = 0; w < 4; w++) in[w] = sp_exp_pair(lut, in[w]);
+    auto exp_in_place = [&](v4u (&in)[2], const v4u& m0, const v4u& m1, uint32_t t, const uint32_t (&sh)[2]) {
+        if (MASK) {                                          // scores + mask in the 16-bit type, as the separate add would round it
+            in[0] = ST::add_vec(in[0], m0);
+            in[1] = ST::add_vec(in[1], m1);
         }
-        if (RAGGED ? t * (SP_TC * 2) + cbyte >= sh + row_bytes : past_end(t, h)) in = v4u{0, 0, 0, 0};
+        bool mine = true;                                    // both vectors at once, so that their table reads are in flight together
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int w = 0; w < 4; w++) mine &= in[h][w] == ST::NEG_INF_PAIR;
+        if (__builtin_amdgcn_ballot_w64(!mine) == 0) {
+            in[0] = in[1] = v4u{exp_ninf, exp_ninf, exp_ninf, exp_ninf};
+        } else {
+            uint32_t lo[8], hi[8];
+#pragma unroll
+            for (int w = 0; w < 8; w++) {
+                lo[w] = sp_exp_lo(in[w / 4][w % 4]);
+                hi[w] = sp_exp_hi(in[w / 4][w % 4]);
+            }
+            __builtin_amdgcn_sched_barrier(0);               // all sixteen reads are issued before the first is waited for
+#pragma unroll
+            for (int w = 0; w < 8; w++) in[w / 4][w % 4] = lo[w] | hi[w] << 16;
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            if (RAGGED ? t * (SP_TC * 2) + cbyte >= sh[h] + row_bytes : past_end(t, h)) in[h] = v4u{0, 0, 0, 0};
     };
     // RAGGED: the neighbours' elements in a row's first and last vector are zeroed in the tile, after the vector has been
     // written there (on the LDS copy, so that the data registers of the main path stay untouched: masking them in a branch
@@ -585,14 +634,14 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         for (uint32_t it = 0; it < n_items; it++) {
 #pragma unroll
             for (int t = 0; t < NSTEP; t++) {
+                v4u m[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    exp_in_place(pre[t % PF][h],
-                                 (MASK && RAGGED) ? mask_funnel(mpre[h], mhi[h], mcur[h])
-                                 : PAIR           ? tile_value(mpre[t % 2], ccur[0][TILES ? t : 0])
-                                 : TILES          ? tile_value(mpre[h], ccur[PAIR ? 0 : h][TILES ? t : 0])
-                                                  : mpre[h],
-                                 t, pcur[h], h);
+                    m[h] = (MASK && RAGGED) ? mask_funnel(mpre[h], mhi[h], mcur[h])
+                           : PAIR           ? tile_value(mpre[t % 2], ccur[0][TILES ? t : 0])
+                           : TILES          ? tile_value(mpre[h], ccur[PAIR ? 0 : h][TILES ? t : 0])
+                                            : mpre[h];
+                exp_in_place(pre[t % PF], m[0], m[1], t, pcur);
                 __syncthreads();                             // A: wave 0 has left the previous tile
                 *in_tile(0) = pre[t % PF][0];
                 *in_tile(1) = pre[t % PF][1];
@@ -684,8 +733,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const uint32_t t = t0 + k;
-#pragma unroll
-                for (int h = 0; h < 2; h++) exp_in_place(pre[k][h], mpre[h], t, 0, h);
+                exp_in_place(pre[k], mpre[0], mpre[1], t, pcur);
                 __syncthreads();                             // A
                 *reinterpret_cast<v4u*>(&tile[rr][ccol]) = pre[k][0];
                 *reinterpret_cast<v4u*>(&tile[rr + SP_HALF][ccol]) = pre[k][1];

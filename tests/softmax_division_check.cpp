@@ -1,0 +1,52 @@
+// Host check of the streaming softmax's short divisions (SpType<T>::short_quotients in ratchet_amd/csrc/rt_softmax_stream.h):
+// for every exp value e >= 0 and every `stride`-th row sum s inside the range where the kernel takes them, the short form
+// must round to the bits of the correctly rounded f32 quotient rounded to the 16-bit type, which is what the reference's
+// half types compute.  Build: g++ -O2 -ffp-contract=off -mfma.   Usage: softmax_division_check STRIDE
+// prints "f16 <n> bf16 <n> checked <m>" (n: pairs that differ), exit code 0 iff both are 0.
+#include <cmath>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+static float u2f(uint32_t u) { float f; memcpy(&f, &u, 4); return f; }
+static uint32_t f2u(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
+static uint16_t to_bf16(float f) {                            // finite, nearest even
+    const uint32_t u = f2u(f);
+    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+}
+static float from_f16(uint16_t h) {                           // h >= 0, finite
+    return (h & 0x7c00) ? u2f(((uint32_t)h << 13) + 0x38000000u) : (float)h * 0x1p-24f;
+}
+static uint16_t to_f16(float f) {                             // 0 <= f, nearest even
+    if (f >= 65520.0f) return 0x7c00;
+    if (f < 0x1p-14f) return (uint16_t)(f2u(f + 0.5f) - 0x3f000000u);      // one f32 step of [0.5, 1) is 2^-24, a subnormal f16 step
+    const uint32_t u = f2u(f);
+    return (uint16_t)((u + 0xfffu + ((u >> 13) & 1u) - 0x38000000u) >> 13);
+}
+
+int main(int argc, char** argv) {
+    const unsigned stride = argc > 1 ? (unsigned)strtoul(argv[1], nullptr, 10) : 1;
+    unsigned long long bad16 = 0, badbf = 0, checked = 0;
+    for (uint32_t sb = 0x0400; sb < 0x7c00; sb += stride) {   // 2^-14 .. 65504
+        const float s = from_f16((uint16_t)sb), rinv = 1.0f / s, rlow = fmaf(-s, rinv, 1.0f) * rinv;
+        for (uint32_t eb = 0; eb < 0x7c00; eb++) {
+            const float e = from_f16((uint16_t)eb);
+            bad16 += to_f16(fmaf(e, rinv, fmaf(e, rlow, 0.0f))) != to_f16(e / s);
+            checked++;
+        }
+    }
+    for (uint32_t sb = 0x0080; sb < 0x7f80; sb += stride) {
+        const float s = u2f(sb << 16);
+        if (s < 0x1p-100f || s > 0x1p100f) continue;
+        const float rinv = 1.0f / s;
+        for (uint32_t eb = 0; eb < 0x7f80; eb++) {
+            const float e = u2f(eb << 16), q = e / s;
+            if (std::isinf(q)) break;                         // a sum is never below its terms
+            badbf += to_bf16(e * rinv) != to_bf16(q);
+            checked++;
+        }
+    }
+    printf("f16 %llu bf16 %llu checked %llu\n", bad16, badbf, checked);
+    return bad16 || badbf;
+}

@@ -1,0 +1,45 @@
+"""GPU parity of the streaming 16-bit softmax at the places where its parts can go wrong: the range in which row sums take the
+short division, and the edges of the walker's 64-value chunks and 512-column steps.  Bit-exact against the CPU oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    from ratchet_amd import Device
+
+    d = Device(0)
+    yield d
+    d.close()
+
+
+def _to(oracle, a, bf):
+    a = np.asarray(a, np.float32)
+    return oracle.cast(a, np.uint16, dst_bf16=True) if bf else a.astype(np.float16)
+
+
+def _same(got, want, bf):
+    g, w = got.view(np.uint16), want.view(np.uint16)
+    lim = 0x7f80 if bf else 0x7c00
+    return bool((((g == w) | (((g & 0x7fff) > lim) & ((w & 0x7fff) > lim)))).all())
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("cols", [8, 64, 72, 504, 512, 520, 1024, 1096, 2176, 4096])
+def test_row_sums_on_both_sides_of_the_short_division(dev, oracle, cols, kind):
+    """rows shifted so that their sums run from subnormal (f16) or below 2^-100 (bf16), through the range of the short
+    division, to infinity; with results that are subnormal themselves"""
+    bf = kind == "bf16"
+    rng = np.random.default_rng(cols)
+    top = 88.0 if bf else 11.0
+    low = -92.0 if bf else -17.0
+    rows = 256
+    x = rng.standard_normal((1, rows, cols)).astype(np.float32)
+    x[0] += np.linspace(low, top - np.log(cols), rows)[:, None].astype(np.float32)
+    x[0, ::7] = np.where(rng.random((len(x[0, ::7]), cols)) < 0.9, x[0, ::7] - (40.0 if bf else 8.0), x[0, ::7])
+    x[0, 3], x[0, 5], x[0, 9, : cols // 2] = top + 3, -np.inf, -np.inf
+    xb = _to(oracle, x, bf)
+    want = oracle.softmax(xb, bf16=bf)
+    assert _same(dev.softmax(dev.upload(xb, bf16=bf)).to_numpy(), want, bf)
