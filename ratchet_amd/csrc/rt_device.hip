@@ -152,22 +152,21 @@ int rt_device_create(int ordinal, rt_device** out) {
         delete dev;
         return rt_fail_hip(e, "hipMalloc(scratch)");
     }
-    e = hipMalloc((void**)&dev->sm_row_sums, RT_SM_ROW_SUMS * sizeof(uint16_t) + (RT_SM_TILES_HEAD + RT_SM_MASK_TILES) * sizeof(uint32_t));
+    e = hipMalloc((void**)&dev->sm_mask_tiles, (RT_SM_TILES_HEAD + RT_SM_MASK_TILES) * sizeof(uint32_t));
     if (e == hipSuccess) {
-        dev->sm_mask_tiles = reinterpret_cast<uint32_t*>(dev->sm_row_sums + RT_SM_ROW_SUMS);
         e = hipMemset(dev->sm_mask_tiles, 0xff, RT_SM_TILES_HEAD * sizeof(uint32_t));
-        if (e != hipSuccess) (void)hipFree(dev->sm_row_sums);
+        if (e != hipSuccess) (void)hipFree(dev->sm_mask_tiles);
     }
     if (e != hipSuccess) {
         (void)hipFree(dev->gn_scratch);
         (void)hipStreamDestroy(dev->stream);
         delete dev->pool;
         delete dev;
-        return rt_fail_hip(e, "hipMalloc(row sums)");
+        return rt_fail_hip(e, "hipMalloc(mask tiles)");
     }
     int rc = rt_norm_device_init(dev);
     if (rc) {
-        (void)hipFree(dev->sm_row_sums);
+        (void)hipFree(dev->sm_mask_tiles);
         (void)hipFree(dev->gn_scratch);
         (void)hipStreamDestroy(dev->stream);
         delete dev->pool;
@@ -190,7 +189,7 @@ int rt_device_destroy(rt_device* dev) {
             if (dev->unary_lut_via32[t][i]) (void)hipFree(dev->unary_lut_via32[t][i]);
         }
     if (dev->gn_scratch) (void)hipFree(dev->gn_scratch);
-    if (dev->sm_row_sums) (void)hipFree(dev->sm_row_sums);
+    if (dev->sm_mask_tiles) (void)hipFree(dev->sm_mask_tiles);
     // buffers the caller never returned are released with the device, like the parked ones
     for (auto& kv : dev->pool->parked) (void)hipFree(kv.second.ptr);
     for (auto& kv : dev->pool->live) (void)hipFree(kv.first);

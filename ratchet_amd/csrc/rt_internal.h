@@ -9,7 +9,6 @@
 #include "../../include/ratchet_hip.h"
 #include "../../include/ratchet_hip_debug.h"
 
-constexpr size_t RT_SM_ROW_SUMS = 1u << 19;
 constexpr size_t RT_SM_MASK_TILES = 1u << 18;   // 512-column tiles of a mask that the streaming softmax can classify per launch
 constexpr size_t RT_SM_TILES_HEAD = 16;         // entries in front of them that always read "load this tile"
 // An operand that repeats over the leading dims of the output (an [S, T] mask under B * H heads) is re-read once per
@@ -45,9 +44,7 @@ struct rt_device {
     uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads (bits 0..15) and for those of f16 rows of 4097 to 8192 columns
     unsigned ry_attr_set;          // the same for the one-wave-per-row softmax (rt_softmax_replay.hip)
     uint16_t rp_resident[2][9];    // wave-per-row RMSNorm: blocks of an instantiation ([f16, bf16][vectors per lane]) that one CU holds; 0 = not asked yet
-    // row sums of one launch of the streaming softmax's ragged-row variant (RT_SM_ROW_SUMS 16-bit values, allocated with the device)
-    uint16_t* sm_row_sums;
-    // one word per 512-column tile of the mask of a masked streaming softmax (behind the row sums, in the same allocation): the
+    // one word per 512-column tile of the mask of a masked streaming softmax (allocated with the device): the
     // tile's value twice when all its elements are equal, 0xffffffff when the tile has to be loaded; the first RT_SM_TILES_HEAD
     // words always hold 0xffffffff
     uint32_t* sm_mask_tiles;

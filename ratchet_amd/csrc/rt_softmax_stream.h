@@ -1,5 +1,4 @@
-// The streaming 16-bit softmax (f16 / bf16 reference arithmetic in one pass over HBM), its launcher and the second launch
-// of its ragged-row variant.  Included by one translation unit per element type (rt_softmax_stream_f16.hip,
+// The streaming 16-bit softmax (f16 / bf16 reference arithmetic in one pass over HBM) and its launcher.  Included by one translation unit per element type (rt_softmax_stream_f16.hip,
 // rt_softmax_stream_bf16.hip): the kernel has some sixty instantiations per type, and the two compile side by side.
 #ifndef RT_SOFTMAX_STREAM_H
 #define RT_SOFTMAX_STREAM_H
@@ -194,14 +193,11 @@ template <> struct SpType<bf16_t> {
 // are parked in y instead and read back (by the thread that wrote them) when the row sum is known: 4 bytes of traffic per
 // element and byte of the type instead of 2, any row length.
 //
-// RAGGED (rows that are not whole aligned vectors, e.g. 1001 columns; x and y 16-byte aligned, no mask, parked variant):
-// every row is handled over the span of aligned 16-byte vectors that covers it.  Row r starts `sh` = (r * cols * 2) % 16
-// bytes into its first vector; span elements outside the row belong to the neighbouring rows: they are zeroed after the
-// table lookup (adding +0 leaves the running sum as it is), and a vector that is not entirely inside its row is not
-// stored.  Wave 0 also writes each row's sum to `row_sums`; the elements of those ragged vectors (at most 14 per row) are
-// finished by softmax16_edges_kernel from x, the table and that sum.  An aligned vector that holds one byte of the tensor
-// lies in a mapped page, so the loads are safe at the tensor's ends too.  A row's span can be one vector longer than
-// NSTEP steps hold (2047 columns starting 14 bytes into a vector): wave 0 reads that vector itself and adds it last.
+// RAGGED (rows that are not whole 16-byte vectors, e.g. 1001 columns; parked in registers): the vectors of a row start at its
+// first element, whatever its alignment, and the last one is the row's last eight elements: it overlaps the vector before
+// it, counts for the walk without the elements that both hold, and is stored with the same values.  No access leaves the row.
+// (Before, the rows ran over the aligned vectors that cover them, with the mask shifted into place between lanes and the
+// vectors shared by two rows left to a second launch: [1,32,1001,1001] f16 masked 48 us, now 39.)
 //
 // LONG (rows of SP_TC * SP_MAX_STEPS up to twice that many columns): a group has 15 rows and a step 1024 columns.  The two
 // vectors a loader thread handles in a step lie 512 columns apart in ONE row instead of in two rows, and the walker walks
@@ -210,8 +206,7 @@ template <> struct SpType<bf16_t> {
 // 8 steps spill 4 to 8 of their 128 vector registers (20 bytes of scratch a lane).
 template <typename T, int NSTEP, bool FULL, int MASK, bool RAGGED = false, bool LONG = false>
 __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16_t* __restrict__ table, const T* x, const T* mask, T* y,
-                                                                    uint64_t rows, uint32_t cols, SpSched sch, uint16_t* row_sums,
-                                                                    const uint32_t* __restrict__ tiles) {
+                                                                    uint64_t rows, uint32_t cols, SpSched sch, const uint32_t* __restrict__ tiles) {
     typedef SpType<T> ST;
     constexpr bool PARK = NSTEP > 0;
     // The plain variant and the paired masked one hold their steps to a pace (see launch_stream16).  The paired one does
@@ -228,7 +223,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     constexpr int STEP_COLS = LONG ? 2 * SP_TC : SP_TC;      // columns of a row per step
     constexpr int GROUP_ROWS = LONG ? SP_HALF : SP_ROWS;     // rows of a group
     static_assert(GROUP_ROWS * (STEP_COLS + SP_PAD) * sizeof(uint16_t) <= SP_TILE_BYTES, "the tile of a step fits its place in LDS");
-    static_assert(!PAIR || (PARK && !RAGGED && NSTEP % 2 == 0), "the paired variant parks in registers and alternates two mask slots");
+    static_assert(!PAIR || (PARK && NSTEP % 2 == 0), "the paired variant parks in registers and alternates two mask slots");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint16_t* lut = reinterpret_cast<uint16_t*>(smem);
     uint16_t (*tile)[STEP_COLS + SP_PAD] = reinterpret_cast<uint16_t (*)[STEP_COLS + SP_PAD]>(smem + SP_LUT_BYTES);
@@ -276,32 +271,6 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             t_last -= sch.pace;
         }
         for (uint32_t it = 0; it < n_items; it++) {
-            // RAGGED: a row that starts sh bytes into its first vector can reach up to 14 bytes past its last step.  That
-            // one vector is fetched here, at the start of the group, and added after the group's last step.
-            uint32_t my_row = 0, tail_end = 0;               // tail_end: bytes of the row inside the extra vector, 0 = none
-            bool my_ok = false;
-            v4u tailv = {0, 0, 0, 0}, tailm = {0, 0, 0, 0};
-            if (RAGGED) {
-                uint32_t rep, pg;
-                sp_item(sch, blockIdx.x, gridDim.x, it, rep, pg);
-                const uint32_t prow = pg * sch.R + lane;
-                my_ok = lane < sch.R && prow < sch.P;
-                my_row = rep * sch.P + prow;
-                const uint32_t off = my_row * (cols * 2);
-                const uint32_t end = (off & 15u) + cols * 2; // one past the row's last byte, in span coordinates
-                if (my_ok && end > nsteps * (SP_TC * 2)) {
-                    tail_end = end - nsteps * (SP_TC * 2);
-                    tailv = *reinterpret_cast<const v4u*>(reinterpret_cast<const char*>(x) + (off & ~15u) + nsteps * (SP_TC * 2));
-                    if (MASK) {                              // its mask elements, one by one (the mask row has its own alignment)
-                        uint32_t q, mrow;
-                        fd_divmod(my_row, sch.pm_div, q, mrow);
-                        const uint16_t* mp = reinterpret_cast<const uint16_t*>(mask) + (uint64_t)mrow * cols + (nsteps * (SP_TC * 2) - (off & 15u)) / 2;
-#pragma unroll
-                        for (int e = 0; e < 7; e++)
-                            if ((uint32_t)(2 * e) < tail_end) tailm[e >> 1] |= (uint32_t)mp[e] << (16 * (e & 1));
-                    }
-                }
-            }
             uint32_t steps = nsteps;
             if constexpr (NSTEP == 1) asm volatile("" : "+s"(steps));    // kept a loop: as straight-line code it took 150 registers too many
 #pragma unroll 1
@@ -328,16 +297,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 }
             }
             add_values(held, 0, WALK_VECS);
-            if (RAGGED && tail_end) {
-                if (MASK) tailv = ST::add_vec(tailv, tailm);
-#pragma unroll
-                for (int w = 0; w < 4; w++) {                // elements past the row's end count as +0
-                    const uint32_t keep = ((uint32_t)(4 * w) < tail_end ? 0xffffu : 0u) | ((uint32_t)(4 * w + 2) < tail_end ? 0xffff0000u : 0u);
-                    ST::add_pair(run, sp_exp_pair(tailv[w]) & keep);
-                }
-            }
             if (lane < SP_ROWS) sums[gpar][lane] = ST::run_bits(run);
-            if (RAGGED && my_ok) row_sums[my_row] = ST::run_bits(run);
             run = ST::zero();
             gpar ^= 1;
         }
@@ -355,13 +315,11 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     const uint32_t rr = __builtin_amdgcn_readfirstlane(lt >> 6);   // rows rr and rr + 15 of the group: the same for the whole wave
     const uint32_t ccol = (lt & 63) * 8;                     // column of this thread's vectors inside a step
     const uint32_t row_bytes = cols * 2;
-    // the launcher keeps this below 2^31; the ragged variant's last vector may reach past the tensor's last element
-    const uint32_t nbytes = RAGGED ? (uint32_t)((rows * row_bytes + 15) & ~15ull) : (uint32_t)(rows * row_bytes);
+    const uint32_t nbytes = (uint32_t)(rows * row_bytes);    // the launcher keeps this below 2^31
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(x), 0, nbytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, 0, nbytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rm =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(MASK ? mask : x), 0,
-                                          MASK ? (RAGGED ? (sch.PM * row_bytes + 15) & ~15u : sch.PM * row_bytes) : nbytes, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(MASK ? mask : x), 0, MASK ? sch.PM * row_bytes : nbytes, 0x00020000);
     constexpr uint32_t OOB = 0x80000000u;                    // >= nbytes, and stays so after adding a column offset
     const uint32_t G = gridDim.x;
 
@@ -369,9 +327,6 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     // needed for data): byte offset of rows rr / rr + 15 of item `it` in x / y, or OOB, and the difference between that
     // and the row's offset in the mask (for a row that does not exist the mask offset is arbitrary, which is harmless:
     // the load is range checked, and what is computed from it is never stored).
-    // (RAGGED: xo is the offset of the row's first span vector and mdiff carries sh, the row's start inside that vector)
-    // (RAGGED with MASK: mq is the mask byte that lines up with the row's span origin, mask row offset minus sh; it is only
-    // element aligned, and negative for the mask's first row when sh > 0)
     // With a mask, register-parked rows of whole vectors: the classes of the NSTEP tiles of each of the wave's mask rows
     // (one row when paired), in scalar registers (see mask_tiles_kernel)
     constexpr bool TILES = MASK && PARK && !RAGGED;
@@ -400,7 +355,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             }
         }
     };
-    auto item_off = [&](uint32_t it, uint32_t (&xo)[2], uint32_t (&mdiff)[2], uint32_t (&mq)[2]) {
+    auto item_off = [&](uint32_t it, uint32_t (&xo)[2], uint32_t (&mdiff)[2]) {
         uint32_t rep, pg;
         sp_item(sch, blockIdx.x, G, it, rep, pg);
 #pragma unroll
@@ -410,17 +365,6 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             const uint32_t per = PAIR ? rep * 2 + h : rep;
             const bool ok = it < n_items && r < sch.R && prow < sch.P && per < sch.reps;
             const uint32_t row = per * sch.P + prow;
-            mq[h] = 0;
-            if (RAGGED) {
-                xo[h] = __builtin_amdgcn_readfirstlane(ok ? (row * row_bytes) & ~15u : OOB);
-                mdiff[h] = __builtin_amdgcn_readfirstlane((row * row_bytes) & 15u);
-                if (MASK) {
-                    uint32_t q, mrow;
-                    fd_divmod(row, sch.pm_div, q, mrow);
-                    mq[h] = __builtin_amdgcn_readfirstlane(mrow * row_bytes - ((row * row_bytes) & 15u));
-                }
-                continue;
-            }
             // (LONG: h = 1 is the second half of each of the row's steps)
             xo[h] = __builtin_amdgcn_readfirstlane(ok ? row * row_bytes + (LONG ? h * SP_TC * 2 : 0) : OOB);
             if (MASK) {
@@ -436,55 +380,25 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     auto past_end = [&](uint32_t t, int h) -> bool { return !(PARK && FULL) && t * STEP_COLS + (LONG ? h * SP_TC : 0) + ccol >= cols; };
     auto step_off = [&](uint32_t row_off, uint32_t t, int h) -> uint32_t {   // per-lane offset of this thread's vector h in step t of a row
         if (past_end(t, h)) return OOB;
+        if (RAGGED) {                                        // the row's last vector starts eight elements before its end
+            const uint32_t at = t * (STEP_COLS * 2) + cbyte;
+            return row_off + (at < row_bytes - 16 ? at : row_bytes - 16);
+        }
         return row_off + t * (STEP_COLS * 2) + cbyte;
     };
-    // RAGGED: the same in span coordinates.  The vector at span byte p holds row bytes [sh, sh + row_bytes) ∩ [p, p + 16).
-    auto span_load_off = [&](uint32_t row_off, uint32_t sh, uint32_t t) -> uint32_t {
-        const uint32_t p = t * (SP_TC * 2) + cbyte;
-        return p >= sh + row_bytes ? OOB : row_off + p;
+    // RAGGED: the elements of a row's last vector that the one before it holds too, of this thread's vector (0 for all others)
+    const uint32_t last_step = RAGGED ? (cols - 1) / STEP_COLS : 0;
+    const uint32_t tail_drop = RAGGED && last_step * STEP_COLS + ccol < cols && last_step * STEP_COLS + ccol + 8 > cols ? last_step * STEP_COLS + ccol + 8 - cols : 0;
+    auto for_walk = [&](v4u v, uint32_t t) -> v4u {          // without them, zeros (which the sum does not notice) behind
+        if (t == last_step) {
+            if (tail_drop & 1) v = v4u{(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), v[3] >> 16};
+            if (tail_drop & 2) v = v4u{v[1], v[2], v[3], 0u};
+            if (tail_drop & 4) v = v4u{v[2], v[3], 0u, 0u};
+        }
+        return v;
     };
-    auto span_store_off = [&](uint32_t row_off, uint32_t sh, uint32_t t) -> uint32_t {     // only vectors entirely inside the row
-        const uint32_t p = t * (SP_TC * 2) + cbyte;
-        return (p >= sh && p + 16 <= sh + row_bytes) ? row_off + p : OOB;
-    };
-    auto ld_off = [&](uint32_t row_off, uint32_t sh, uint32_t t, int h) -> uint32_t { return RAGGED ? span_load_off(row_off, sh, t) : step_off(row_off, t, h); };
-    auto st_off = [&](uint32_t row_off, uint32_t sh, uint32_t t, int h) -> uint32_t { return RAGGED ? span_store_off(row_off, sh, t) : step_off(row_off, t, h); };
     // this thread's vector h of the step in the tile
     auto in_tile = [&](int h) -> v4u* { return reinterpret_cast<v4u*>(LONG ? &tile[rr][ccol + h * SP_TC] : &tile[rr + h * SP_HALF][ccol]); };
-    // RAGGED with MASK: the sixteen mask bytes for the vector at span byte p start at mask byte mq + p, which is only
-    // element aligned: they straddle the aligned mask vectors at (mq & ~15) + p and 16 bytes on, (mq & 15) bytes into the
-    // first.  A lane loads the first; the second is its right neighbour's first (one wave shift), except for lane 63,
-    // which loads its own.  An offset before the mask's start wraps to a huge one and is dropped like any other.
-    auto mask_lo_off = [&](uint32_t mq, uint32_t sh, uint32_t t) -> uint32_t {
-        const uint32_t p = t * (SP_TC * 2) + cbyte;
-        return p >= sh + row_bytes + 16 ? OOB : (mq & ~15u) + p;      // also the lane after the row's last vector: it feeds its left neighbour
-    };
-    auto mask_hi_off = [&](uint32_t mq, uint32_t sh, uint32_t t) -> uint32_t {
-        const uint32_t p = t * (SP_TC * 2) + cbyte;
-        return (cbyte != 63 * 16 || p >= sh + row_bytes) ? OOB : (mq & ~15u) + p + 16;
-    };
-    auto mask_funnel = [&](const v4u& lo, const v4u& hi_own, uint32_t mq) -> v4u {
-        const uint32_t d = mq & 15u;                         // the same for the whole wave: branches, not selects
-        uint32_t cat[8];
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            cat[w] = lo[w];
-            // lane i takes lane i + 1's value; lane 63 keeps the vector it loaded itself
-            cat[w + 4] = (uint32_t)__builtin_amdgcn_update_dpp((int)hi_own[w], (int)lo[w], 0x130, 0xf, 0xf, false);
-        }
-        v4u out;
-        switch (d >> 2) {
-#define RT_PICK(O)                                                                                                              \
-    _Pragma("unroll") for (int w = 0; w < 4; w++)                                                                              \
-        out[w] = (d & 2) ? __builtin_amdgcn_alignbyte(cat[w + O + 1 < 8 ? w + O + 1 : 7], cat[w + O], 2) : cat[w + O];
-            case 0: RT_PICK(0) break;
-            case 1: RT_PICK(1) break;
-            case 2: RT_PICK(2) break;
-            default: RT_PICK(3) break;
-#undef RT_PICK
-        }
-        return out;
-    };
     auto load_x = [&](uint32_t off) -> v4u { return __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 2); };   // 2: non-temporal
     auto load_m = [&](uint32_t off) -> v4u { return __builtin_amdgcn_raw_buffer_load_b128(rm, off, 0, 0); };   // re-read by other heads
     // A mask tile whose elements are all equal is not loaded (the offset goes outside the buffer, which costs no memory
@@ -492,10 +406,12 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     // class word
     constexpr uint32_t TILE_MIXED = 0xffffffffu;
     auto load_m_tile = [&](uint32_t off, uint32_t cw) -> v4u {
+        if (!TILES) return load_m(off);
         const uint32_t skip = __builtin_amdgcn_readfirstlane(cw != TILE_MIXED ? OOB : 0u);
         return load_m(off | skip);
     };
     auto tile_value = [&](const v4u& loaded, uint32_t cw) -> v4u {
+        if (!TILES) return loaded;
         const uint32_t fill = __builtin_amdgcn_readfirstlane(cw != TILE_MIXED ? cw : 0u);
         return v4u{loaded[0] | fill, loaded[1] | fill, loaded[2] | fill, loaded[3] | fill};
     };
@@ -536,7 +452,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
     // A wave whose values of this step are all -inf (the part of a row that a causal mask covers) takes exp(-inf) for
     // all of them without the eight table reads per lane; the test is wave-wide, so the branch is a scalar one.
     const uint32_t exp_ninf = __builtin_amdgcn_readfirstlane((uint32_t)lut[ST::NEG_INF_PAIR & 0xffffu] * 0x10001u);
-    auto exp_in_place = [&](v4u (&in)[2], const v4u& m0, const v4u& m1, uint32_t t, const uint32_t (&sh)[2]) {
+    auto exp_in_place = [&](v4u (&in)[2], const v4u& m0, const v4u& m1, uint32_t t) {
         if (MASK) {                                          // scores + mask in the 16-bit type, as the separate add would round it
             in[0] = ST::add_vec(in[0], m0);
             in[1] = ST::add_vec(in[1], m1);
@@ -561,39 +477,12 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         }
 #pragma unroll
         for (int h = 0; h < 2; h++)
-            if (RAGGED ? t * (SP_TC * 2) + cbyte >= sh[h] + row_bytes : past_end(t, h)) in[h] = v4u{0, 0, 0, 0};
+            if (past_end(t, h)) in[h] = v4u{0, 0, 0, 0};
     };
-    // RAGGED: the neighbours' elements in a row's first and last vector are zeroed in the tile, after the vector has been
-    // written there (on the LDS copy, so that the data registers of the main path stay untouched: masking them in a branch
-    // cost 50 vector registers).  Which step and lane hold those two vectors is the same for the whole wave (sh lives in a
-    // scalar register), so every test below is a scalar branch except the one that picks the lane, and the zeros go out
-    // as at most three aligned writes of 8, 4 and 2 bytes.
-    auto zero_outside = [&](uint32_t t, uint32_t sh, uint32_t trow_idx) {
-        unsigned char* trb = reinterpret_cast<unsigned char*>(&tile[trow_idx][0]);
-        if (t == 0 && sh != 0 && cbyte == 0) {               // bytes [0, sh) of the span belong to the row before
-            if (sh & 8) *reinterpret_cast<uint64_t*>(trb) = 0;
-            if (sh & 4) *reinterpret_cast<uint32_t*>(trb + (sh & 8)) = 0;
-            if (sh & 2) *reinterpret_cast<uint16_t*>(trb + (sh & 12)) = 0;
-        }
-        const uint32_t end = sh + row_bytes, pe = end & ~15u;        // the vector at span byte pe holds the row's end
-        if ((end & 15u) != 0 && t == pe / (SP_TC * 2) && cbyte == (pe & (SP_TC * 2 - 1))) {
-            uint32_t at = (pe & (SP_TC * 2 - 1)) + (end & 15u);      // bytes [at, next vector) belong to the row after
-            if (at & 2) {
-                *reinterpret_cast<uint16_t*>(trb + at) = 0;
-                at += 2;
-            }
-            if (at & 4) {
-                *reinterpret_cast<uint32_t*>(trb + at) = 0;
-                at += 4;
-            }
-            if (at & 8) *reinterpret_cast<uint64_t*>(trb + at) = 0;
-        }
-    };
-
-    uint32_t cur[2], nxt[2], prev[2] = {OOB, OOB}, pcur[2], pnxt[2], pprev[2] = {0, 0}, mcur[2], mnxt[2];
-    uint32_t ccur[NCROW][NCLS], cnxt[NCROW][NCLS];
-    item_off(0, cur, pcur, mcur);
-    item_off(1, nxt, pnxt, mnxt);
+    uint32_t cur[2], nxt[2], prev[2] = {OOB, OOB}, pcur[2], pnxt[2];
+    uint32_t ccur[NCROW][NCLS] = {}, cnxt[NCROW][NCLS] = {};
+    item_off(0, cur, pcur);
+    item_off(1, nxt, pnxt);
     item_tiles(0, ccur);
     item_tiles(1, cnxt);
     uint32_t gpar = 0;
@@ -605,7 +494,6 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
         static_assert(NSTEP % PF == 0 && PF <= 5, "prefetch slots must tile the steps of a row");
         v4u e[NSTEP][2];                                     // exp values of the group in flight, 8 halves per vector
         v4u pre[PF][2], mpre[2];                             // x: PF steps in flight; mask: one (L2 hits: a short distance is enough)
-        v4u mhi[2];                                          // RAGGED: lane 63's second mask vector
 #pragma unroll
         for (int t = 0; t < NSTEP; t++) e[t][0] = e[t][1] = v4u{0, 0, 0, 0};
         // The pending memory operations at the top of the group loop are the same on entry as after a group (two loads, two
@@ -613,72 +501,60 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
         for (int k = 0; k < PF; k++) {
 #pragma unroll
-            for (int h = 0; h < 2; h++) pre[k][h] = load_x(ld_off(cur[h], pcur[h], k, h));
+            for (int h = 0; h < 2; h++) pre[k][h] = load_x(step_off(cur[h], k, h));
 #pragma unroll
             for (int h = 0; h < 2; h++) store_y(v4u{0, 0, 0, 0}, OOB);
         }
-        if (MASK && !RAGGED) {                               // PAIR: the mask of steps 0 and 1 (NSTEP is even, so 1 exists)
+        if (MASK) {                                          // PAIR: the mask of steps 0 and 1 (NSTEP is even, so 1 exists)
 #pragma unroll
             for (int h = 0; h < 2; h++)
                 mpre[h] = PAIR ? load_m_tile(step_off(cur[0] - pcur[0], h, 0), ccur[0][TILES ? h : 0])
                                : load_m_tile(step_off(cur[h] - pcur[h], 0, h), ccur[PAIR ? 0 : h][0]);
         }
-        if (MASK && RAGGED) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                mpre[h] = load_m(mask_lo_off(mcur[h], pcur[h], 0));
-                mhi[h] = load_m(mask_hi_off(mcur[h], pcur[h], 0));
-            }
-        }
-
         for (uint32_t it = 0; it < n_items; it++) {
 #pragma unroll
             for (int t = 0; t < NSTEP; t++) {
                 v4u m[2];
 #pragma unroll
                 for (int h = 0; h < 2; h++)
-                    m[h] = (MASK && RAGGED) ? mask_funnel(mpre[h], mhi[h], mcur[h])
-                           : PAIR           ? tile_value(mpre[t % 2], ccur[0][TILES ? t : 0])
-                           : TILES          ? tile_value(mpre[h], ccur[PAIR ? 0 : h][TILES ? t : 0])
-                                            : mpre[h];
-                exp_in_place(pre[t % PF], m[0], m[1], t, pcur);
+                    m[h] = PAIR    ? tile_value(mpre[t % 2], ccur[0][TILES ? t : 0])
+                           : TILES ? tile_value(mpre[h], ccur[PAIR ? 0 : h][TILES ? t : 0])
+                                   : mpre[h];
+                exp_in_place(pre[t % PF], m[0], m[1], t);
                 __syncthreads();                             // A: wave 0 has left the previous tile
-                *in_tile(0) = pre[t % PF][0];
-                *in_tile(1) = pre[t % PF][1];
-                if (RAGGED) {
-                    zero_outside(t, pcur[0], rr);
-                    zero_outside(t, pcur[1], rr + SP_HALF);
-                }
+                // RAGGED: the steps that can be a row's last, where the tile gets the last vector without its first elements
+                constexpr int LAST_FROM = NSTEP == 8 ? 6 : NSTEP - 1;
+                const bool tail = RAGGED && t >= LAST_FROM;
+                *in_tile(0) = tail ? for_walk(pre[t % PF][0], t) : pre[t % PF][0];
+                *in_tile(1) = tail ? for_walk(pre[t % PF][1], t) : pre[t % PF][1];
                 // the registers are free again: next loads, PF steps ahead, possibly in the block's next group
                 // (loads return in order: the mask of the next step goes first, so that waiting for it does not wait for x
                 // of the step after)
-                if (MASK && !RAGGED && !PAIR) {
+                if (MASK && !PAIR) {
 #pragma unroll
                     for (int h = 0; h < 2; h++)
                         mpre[h] = (t + 1 < NSTEP) ? load_m_tile(step_off(cur[h] - pcur[h], t + 1, h), ccur[PAIR ? 0 : h][TILES && t + 1 < NSTEP ? t + 1 : 0])
                                                   : load_m_tile(step_off(nxt[h] - pnxt[h], 0, h), cnxt[PAIR ? 0 : h][0]);
                 }
                 if (PAIR)                                    // this step's slot is free: the mask of two steps ahead
-                    mpre[t % 2] = (t + 2 < NSTEP) ? load_m_tile(step_off(cur[0] - pcur[0], t + 2, 0), ccur[0][PAIR && t + 2 < NSTEP ? t + 2 : 0])
-                                                  : load_m_tile(step_off(nxt[0] - pnxt[0], t + 2 - NSTEP, 0), cnxt[0][PAIR && t + 2 >= NSTEP ? t + 2 - NSTEP : 0]);
-                if (MASK && RAGGED) {
+                    mpre[t % 2] = (t + 2 < NSTEP) ? load_m_tile(step_off(cur[0] - pcur[0], t + 2, 0), ccur[0][TILES && t + 2 < NSTEP ? t + 2 : 0])
+                                                  : load_m_tile(step_off(nxt[0] - pnxt[0], t + 2 - NSTEP, 0), cnxt[0][TILES && t + 2 >= NSTEP ? t + 2 - NSTEP : 0]);
+                auto load_ahead = [&]() {
 #pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        mpre[h] = (t + 1 < NSTEP) ? load_m(mask_lo_off(mcur[h], pcur[h], t + 1)) : load_m(mask_lo_off(mnxt[h], pnxt[h], 0));
-                        mhi[h] = (t + 1 < NSTEP) ? load_m(mask_hi_off(mcur[h], pcur[h], t + 1)) : load_m(mask_hi_off(mnxt[h], pnxt[h], 0));
-                    }
-                }
-#pragma unroll
-                for (int h = 0; h < 2; h++)
-                    pre[t % PF][h] = (t + PF < NSTEP) ? load_x(ld_off(cur[h], pcur[h], t + PF, h)) : load_x(ld_off(nxt[h], pnxt[h], t + PF - NSTEP, h));
+                    for (int h = 0; h < 2; h++)
+                        pre[t % PF][h] = (t + PF < NSTEP) ? load_x(step_off(cur[h], t + PF, h)) : load_x(step_off(nxt[h], t + PF - NSTEP, h));
+                };
+                if (!tail) load_ahead();
                 __syncthreads();                             // B: parked for the walk
                 if (t == 0) read_prev_sum(gpar ^ 1);         // published by wave 0 before it reached barrier A
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t, h));   // first group: prev is OOB, the store is dropped
-                    // this group's values come back from the tile, which stays intact until the next barrier A
-                    e[t][h] = *in_tile(h);
+                    store_y(quotients(e[t][h], h), step_off(prev[h], t, h));   // first group: prev is OOB, the store is dropped
+                    // this group's values come back from the tile, which stays intact until the next barrier A; those of a
+                    // step whose tile is not all of them are still here, and the next loads wait for that
+                    e[t][h] = tail ? pre[t % PF][h] : *in_tile(h);
                 }
+                if (tail) load_ahead();
             }
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -686,12 +562,8 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 cur[h] = nxt[h];
             }
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                pprev[h] = pcur[h];
-                pcur[h] = pnxt[h];
-                mcur[h] = mnxt[h];
-            }
-            item_off(it + 2, nxt, pnxt, mnxt);
+            for (int h = 0; h < 2; h++) pcur[h] = pnxt[h];
+            item_off(it + 2, nxt, pnxt);
 #pragma unroll
             for (int h = 0; h < NCROW; h++)
 #pragma unroll
@@ -705,7 +577,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
         for (int t = 0; t < NSTEP; t++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) store_y(quotients(e[t][h], h), st_off(prev[h], pprev[h], t, h));
+            for (int h = 0; h < 2; h++) store_y(quotients(e[t][h], h), step_off(prev[h], t, h));
     } else {
         // One flat loop over the steps of all groups, two steps per trip (nsteps is even; a step past the row end moves
         // nothing).  Per step and row: exp values to the tile and to y, x of two steps ahead, the previous group's exp
@@ -733,7 +605,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
 #pragma unroll
             for (int k = 0; k < 2; k++) {
                 const uint32_t t = t0 + k;
-                exp_in_place(pre[k], mpre[0], mpre[1], t, pcur);
+                exp_in_place(pre[k], mpre[0], mpre[1], t);
                 __syncthreads();                             // A
                 *reinterpret_cast<v4u*>(&tile[rr][ccol]) = pre[k][0];
                 *reinterpret_cast<v4u*>(&tile[rr + SP_HALF][ccol]) = pre[k][1];
@@ -766,7 +638,7 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 }
                 pcur[0] = pnxt[0];
                 pcur[1] = pnxt[1];
-                item_off(trip / (nsteps / 2) + 2, nxt, pnxt, mnxt);
+                item_off(trip / (nsteps / 2) + 2, nxt, pnxt);
                 gpar ^= 1;
             }
         }
@@ -785,35 +657,6 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
                 }
         }
     }
-}
-
-// The ragged-row variant's second launch: the elements of a row's first and last span vectors when those vectors are
-// shared with a neighbouring row (at most 7 + 7 per row), from x (plus the mask), the exp table and the row sum the streaming kernel
-// left in row_sums.  Sixteen threads per row: 0..7 the elements of the first span vector, 8..15 those of the last.
-// The quotient is the IEEE division the streaming kernel's short division reproduces.
-template <typename T>
-__global__ void __launch_bounds__(BLOCK) softmax16_edges_kernel(const uint16_t* __restrict__ table, const T* x, const T* __restrict__ mask,
-                                                                uint32_t mask_rows, T* y, const uint16_t* __restrict__ row_sums,
-                                                                uint64_t rows, uint32_t cols) {
-    const uint64_t gid = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const uint64_t row = gid >> 4;
-    if (row >= rows) return;
-    const uint32_t j = (uint32_t)gid & 7u;
-    const bool tail = (gid & 8u) != 0;
-    const uint64_t first = row * cols;
-    const uint32_t shift = (uint32_t)(first & 7);
-    const uint32_t last_vec = (shift + cols - 1) >> 3;       // index of the row's last span vector
-    const bool first_whole = shift == 0 && cols >= 8;
-    const bool last_whole = ((shift + cols) & 7) == 0 && (last_vec > 0 || shift == 0);
-    if (tail ? (last_vec == 0 || last_whole) : first_whole) return;
-    const uint32_t e = (tail ? last_vec * 8 : 0) + j;        // element of the span
-    if (e < shift || e - shift >= cols) return;
-    const uint64_t at = first + (e - shift);
-    T xv = x[at];
-    if (mask) xv = Ar<T>::add(xv, mask[(row % mask_rows) * cols + (e - shift)]);     // row r takes mask row r % mask_rows
-    const uint16_t xb = __builtin_bit_cast(uint16_t, xv);
-    const T ev = __builtin_bit_cast(T, table[xb]);
-    y[at] = Ar<T>::div(ev, __builtin_bit_cast(T, row_sums[row]));
 }
 
 // The class of every 512-column tile of a mask, for the masked variants of the streaming kernel that park in registers:
@@ -859,9 +702,9 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     constexpr int TI = sizeof(typename SpType<T>::Run) == 4 ? 1 : 0;         // table and attribute index: 0 f16, 1 bf16
     const uint64_t row_bytes = (uint64_t)cols * 2;
     if (!mask) period = rows;
-    const bool ragged = cols % 8 != 0;                       // rows over their covering aligned vectors, finished by the edges kernel
+    const bool ragged = cols % 8 != 0;                       // rows from their first element on, the last vector over the one before it
     // with a mask: in one launch only, and a mask on a 16-byte boundary
-    if (ragged && mask && (!rt_aligned(mask, 16) || rows * row_bytes > 0x7fffffe0ull || rows > RT_SM_ROW_SUMS)) return RT_OK;
+    if (ragged && mask && (!rt_aligned(mask, 16) || rows * row_bytes > 0x7fffffe0ull)) return RT_OK;
     // the kernel addresses a launch with 32-bit byte offsets below 2^31: larger tensors go in chunks of whole periods
     // (whole 30-row groups when nothing repeats)
     uint64_t chunk_rows;
@@ -869,9 +712,8 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         if (period * row_bytes > 0x7fffffffull) return RT_OK;
         chunk_rows = (0x7fffffffull / (period * row_bytes)) * period;
     } else if (ragged) {
-        // a chunk's row sums must fit the device's buffer, and every chunk must start on a 16-byte boundary (8 rows do)
-        uint64_t max_rows = 0x7fffffe0ull / row_bytes;
-        if (max_rows > RT_SM_ROW_SUMS) max_rows = RT_SM_ROW_SUMS;
+        // every chunk must start on a 16-byte boundary (8 rows do)
+        const uint64_t max_rows = 0x7fffffe0ull / row_bytes;
         chunk_rows = rows <= max_rows ? rows : max_rows / 120 * 120;
         if (chunk_rows == 0) return RT_OK;
     } else {
@@ -885,7 +727,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     int rc = rt_unary_table(dev, TI, RT_EXP, &table);
     if (rc) return rc;
     const uint32_t nt = (cols + SP_TC - 1) / SP_TC;
-    if (ragged && nt > SP_MAX_STEPS) return RT_OK;           // (a ragged row's one vector past its last step is the walker's)
+    if (ragged && nt > SP_MAX_STEPS) return RT_OK;
     constexpr bool LONG_ROWS = std::is_same<T, half_t>::value;
     const uint32_t long_steps = nt <= 10 ? 5 : nt <= 12 ? 6 : 8;       // of 1024 columns
     const bool full = !ragged && cols % SP_TC == 0 && nt != 7 && nt <= 8;
@@ -898,7 +740,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
             dev->sp_attr_set |= bit;                                                                                                 \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, M>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES, dev->stream, table,  \
-                           xc, (const T*)mask, yc, n, cols, sch, (uint16_t*)nullptr, (const uint32_t*)dev->sm_mask_tiles);          \
+                           xc, (const T*)mask, yc, n, cols, sch, (const uint32_t*)dev->sm_mask_tiles);          \
     } while (0)
 #define RT_SP_PAIR(NS, F)                                                                                                            \
     do {                                                                                                                             \
@@ -909,7 +751,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
             dev->sp_pair_attr_set |= bit;                                                                                            \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, 2>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES, dev->stream, table,  \
-                           xc, (const T*)mask, yc, n, cols, sch, (uint16_t*)nullptr, (const uint32_t*)dev->sm_mask_tiles);          \
+                           xc, (const T*)mask, yc, n, cols, sch, (const uint32_t*)dev->sm_mask_tiles);          \
     } while (0)
 #define RT_SP_PAIR_NS(F)                                    \
     do {                                                    \
@@ -927,7 +769,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
             dev->sp_pair_attr_set |= bit;                                                                                            \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, M, false, true>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES,         \
-                           dev->stream, table, xc, (const T*)mask, yc, n, cols, sch, (uint16_t*)nullptr,                             \
+                           dev->stream, table, xc, (const T*)mask, yc, n, cols, sch, \
                            (const uint32_t*)dev->sm_mask_tiles);                                                                     \
     } while (0)
 #define RT_SP_LONG_NS(F, M)                                 \
@@ -938,14 +780,14 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     } while (0)
 #define RT_SP_RAGGED(NS, M)                                                                                                          \
     do {                                                                                                                             \
-        const uint64_t bit = 1ull << ((M ? 16 : 0) + TI * 8 + (NS == 1 ? 0 : NS == 2 ? 1 : NS == 4 ? 2 : NS == 6 ? 4 : NS == 3 ? 5 : NS == 5 ? 6 : 3)); \
+        const uint64_t bit = 1ull << (M * 16 + TI * 8 + (NS == 8 ? 7 : NS));                                                         \
         if (!(dev->sp_ragged_attr_set & bit)) {                                                                                      \
             RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, false, M, true>),                \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
-            dev->sp_ragged_attr_set |= bit;                                                                                              \
+            dev->sp_ragged_attr_set |= bit;                                                                                          \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, false, M, true>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES,            \
-                           dev->stream, table, xc, (const T*)mask, yc, n, cols, sch, dev->sm_row_sums, (const uint32_t*)nullptr);                              \
+                           dev->stream, table, xc, (const T*)mask, yc, n, cols, sch, (const uint32_t*)nullptr);                      \
     } while (0)
 #define RT_SP_RAGGED_NS(M)                                  \
     do {                                                    \
@@ -979,7 +821,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         sch.reps = (uint32_t)(n / sch.P);
         sch.nsteps = (nt + 1) & ~1u;
         // one mask row for two heads: rows of an even number of steps under a mask that repeats every P rows
-        const bool pair = mask && !ragged && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
+        const bool pair = mask && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
         sch.item_reps = pair ? (sch.reps + 1) / 2 : sch.reps;
         const uint32_t rmul = pair ? 2 : 1;
         // rows per group: every block runs ceil(groups / grid) rounds of 8-or-fewer steps whatever the group holds, so
@@ -1088,13 +930,17 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
             sch.tile_stride = nt;
         }
         if (ragged) {
-            if (mask) RT_SP_RAGGED_NS(true);
-            else RT_SP_RAGGED_NS(false);
+            if (pair) {
+                if (nt <= 2) RT_SP_RAGGED(2, 2);
+                else if (nt <= 4) RT_SP_RAGGED(4, 2);
+                else if (nt <= 6) RT_SP_RAGGED(6, 2);
+                else RT_SP_RAGGED(8, 2);
+            } else if (mask) {
+                RT_SP_RAGGED_NS(1);
+            } else {
+                RT_SP_RAGGED_NS(0);
+            }
             RT_CHECK_LAUNCH("softmax16_stream_kernel");
-            const uint64_t eblocks = (n * 16 + BLOCK - 1) / BLOCK;
-            hipLaunchKernelGGL((softmax16_edges_kernel<T>), dim3((unsigned)eblocks), dim3(BLOCK), 0, dev->stream, table, xc, (const T*)mask,
-                               sch.PM, yc, (const uint16_t*)dev->sm_row_sums, n, cols);
-            RT_CHECK_LAUNCH("softmax16_edges_kernel");
             continue;
         }
         if (longer) {

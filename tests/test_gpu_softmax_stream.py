@@ -43,3 +43,22 @@ def test_row_sums_on_both_sides_of_the_short_division(dev, oracle, cols, kind):
     xb = _to(oracle, x, bf)
     want = oracle.softmax(xb, bf16=bf)
     assert _same(dev.softmax(dev.upload(xb, bf16=bf)).to_numpy(), want, bf)
+
+
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+@pytest.mark.parametrize("cols", [193, 505, 513, 1001, 1023, 1535, 1537, 2047, 2561, 3073, 3583, 3585, 4095])
+def test_ragged_rows_under_a_mask_shared_by_heads(dev, oracle, cols, kind):
+    """rows that are not whole vectors, whose last vector overlaps the one before it, under an [S, T] mask of three heads: the
+    variant that takes a mask row for two heads (an even number of 512-column steps), with a head left over, and the other one"""
+    bf = kind == "bf16"
+    rng = np.random.default_rng(cols)
+    x = _to(oracle, 2 * rng.standard_normal((1, 3, 250, cols)), bf)
+    m = np.triu(np.full((250, cols), -np.inf, np.float32), k=1 + max(cols - 250, 0))
+    m[100:140] = rng.standard_normal((40, cols))
+    m = _to(oracle, m, bf)
+    full = np.ascontiguousarray(np.broadcast_to(m, x.shape))
+    want = oracle.softmax(oracle.binary("add", x, full, bf16=bf), bf16=bf)
+    dx, dm = dev.upload(x, bf16=bf), dev.upload(m, bf16=bf)
+    assert _same(dev.softmax_masked(dx, dm).to_numpy(), want, bf)
+    dev.softmax_masked(dx, dm, out=dx)
+    assert _same(dx.to_numpy(), want, bf)
