@@ -37,7 +37,6 @@ struct rt_device {
     uint16_t* unary_lut_via32[2][RT_UNARY_COUNT];
     int lut_attr_set;
     int gated_attr_set[2];
-    unsigned gn_lds_attr_set;
     unsigned np_attr_set;   // 16-bit norm instantiations (LDS-resident rows) whose dynamic-LDS limit has been raised on this device
     uint64_t sp_attr_set;   // streaming softmax instantiations whose dynamic-LDS limit has been raised on this device
     uint64_t sp_ragged_attr_set;   // the same for the ragged-row variants

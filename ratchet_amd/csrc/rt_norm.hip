@@ -901,6 +901,19 @@ __global__ void __launch_bounds__(64 + RB * 32) norm_flow16_kernel(const T* x, c
 // apply kernel: same grid; every block combines the group's partials (Chan et al.), then normalises its slice:
 //               y = (x - mean) * rstd * w[c] + b[c], f32 arithmetic, rounded to T once.
 // ------------------------------------------------------------------------------------------------------------------
+// The f32 arithmetic of GroupNorm on an element as it was loaded: the widening of an f16 operand is part of the fused
+// multiply-add (v_fma_mix_f32), so an f16 element costs one instruction for the mean, two for the variance and three for the output
+// where widening, adding, multiplying and rounding one by one cost 2, 4 and 6.  1 * e + acc rounds as e + acc does; the squares and
+// the last multiplication are rounded once less than as separate operations.
+template <typename T> __device__ __forceinline__ float gn_plus(T e, float acc) {
+    if constexpr (std::is_same<T, half_t>::value) return __builtin_fmaf((float)e, 1.0f, acc);
+    else return Ar<T>::widen(e) + acc;
+}
+template <typename T> __device__ __forceinline__ float gn_dev2(T e, float mean, float acc) {
+    const float d = gn_plus<T>(e, -mean);
+    return __builtin_fmaf(d, d, acc);
+}
+
 // VE = elements per access: 16 / sizeof(T) on the vector path (slices, groups and base pointers are multiples of it), 1 otherwise
 template <typename T, int VE>
 __global__ void __launch_bounds__(BLOCK) gn_stats_kernel(const T* __restrict__ x, float* __restrict__ part, uint32_t glen,
@@ -918,9 +931,9 @@ __global__ void __launch_bounds__(BLOCK) gn_stats_kernel(const T* __restrict__ x
             Vec16<T> v;
             v.u = *reinterpret_cast<const v4u*>(xs + i);
 #pragma unroll
-            for (int q = 0; q < VE; q++) acc += Ar<T>::widen(v.e[q]);
+            for (int q = 0; q < VE; q++) acc = gn_plus<T>(v.e[q], acc);
         } else {
-            acc += Ar<T>::widen(xs[i]);
+            acc = gn_plus<T>(xs[i], acc);
         }
     }
     acc = wave_sum(acc);
@@ -939,13 +952,9 @@ __global__ void __launch_bounds__(BLOCK) gn_stats_kernel(const T* __restrict__ x
             Vec16<T> v;
             v.u = *reinterpret_cast<const v4u*>(xs + i);
 #pragma unroll
-            for (int q = 0; q < VE; q++) {
-                const float d = Ar<T>::widen(v.e[q]) - mean;
-                m2 += d * d;
-            }
+            for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v.e[q], mean, m2);
         } else {
-            const float d = Ar<T>::widen(xs[i]) - mean;
-            m2 += d * d;
+            m2 = gn_dev2<T>(xs[i], mean, m2);
         }
     }
     m2 = wave_sum(m2);
@@ -986,7 +995,7 @@ __global__ void __launch_bounds__(BLOCK) gn_stats_reg_kernel(const T* __restrict
 #pragma unroll
     for (int k = 0; k < NV; k++) {
 #pragma unroll
-        for (int q = 0; q < VE; q++) acc += Ar<T>::widen(v[k].e[q]);             // vectors past the slice hold zeros
+        for (int q = 0; q < VE; q++) acc = gn_plus<T>(v[k].e[q], acc);             // vectors past the slice hold zeros
     }
     acc = wave_sum(acc);
     if (lane == 0) red[wave] = acc;
@@ -1000,10 +1009,7 @@ __global__ void __launch_bounds__(BLOCK) gn_stats_reg_kernel(const T* __restrict
     for (int k = 0; k < NV; k++) {
         if (threadIdx.x + k * BLOCK < nvec) {
 #pragma unroll
-            for (int q = 0; q < VE; q++) {
-                const float d = Ar<T>::widen(v[k].e[q]) - mean;
-                m2 += d * d;
-            }
+            for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
         }
     }
     m2 = wave_sum(m2);
@@ -1021,8 +1027,8 @@ __global__ void __launch_bounds__(BLOCK) gn_stats_reg_kernel(const T* __restrict
 }
 
 // y = (x - mean) * rstd * w[c] + b[c] for the VE elements of one vector that starts at element e0 of its group, whose first
-// channel is cbase.  With L a multiple of VE the vector lies in one channel; otherwise the channel is stepped element by
-// element (a vector of [.., 1500] f16 rows crosses into the next channel, with L < VE into several).
+// channel is cbase.  With L a multiple of VE the vector lies in one channel; a vector of longer rows lies in at most two (both
+// are read ahead and chosen element by element), and where L < VE the channel is stepped.
 template <typename T>
 __device__ __forceinline__ v4u gn_affine_vec(const Vec16<T>& v, uint32_t e0, uint32_t cbase, FastDiv L, const T* __restrict__ scale,
                                              const T* __restrict__ bias, float mean, float rstd) {
@@ -1034,18 +1040,22 @@ __device__ __forceinline__ v4u gn_affine_vec(const Vec16<T>& v, uint32_t e0, uin
         const float w = scale ? Ar<T>::widen(scale[c]) : 1.0f;
         const float b = bias ? Ar<T>::widen(bias[c]) : 0.0f;
 #pragma unroll
-        for (int q = 0; q < VE; q++) {
-            const float t = (Ar<T>::widen(v.e[q]) - mean) * rstd;
-            o.e[q] = Ar<T>::conv(t * w + b);
-        }
+        for (int q = 0; q < VE; q++) o.e[q] = Ar<T>::conv(__builtin_fmaf(gn_plus<T>(v.e[q], -mean) * rstd, w, b));
+    } else if (L.d >= VE) {
+        const uint32_t left = L.d - (e0 - ch * L.d);                       // elements of the vector in channel c, if fewer than VE
+        const uint32_t c1 = left < (uint32_t)VE ? c + 1 : c;
+        const float w0 = scale ? Ar<T>::widen(scale[c]) : 1.0f, w1 = scale ? Ar<T>::widen(scale[c1]) : 1.0f;
+        const float b0 = bias ? Ar<T>::widen(bias[c]) : 0.0f, b1 = bias ? Ar<T>::widen(bias[c1]) : 0.0f;
+#pragma unroll
+        for (int q = 0; q < VE; q++)
+            o.e[q] = Ar<T>::conv(__builtin_fmaf(gn_plus<T>(v.e[q], -mean) * rstd, (uint32_t)q < left ? w0 : w1, (uint32_t)q < left ? b0 : b1));
     } else {
         uint32_t r = e0 - ch * L.d;
 #pragma unroll
         for (int q = 0; q < VE; q++) {
             const float w = scale ? Ar<T>::widen(scale[c]) : 1.0f;
             const float b = bias ? Ar<T>::widen(bias[c]) : 0.0f;
-            const float t = (Ar<T>::widen(v.e[q]) - mean) * rstd;
-            o.e[q] = Ar<T>::conv(t * w + b);
+            o.e[q] = Ar<T>::conv(__builtin_fmaf(gn_plus<T>(v.e[q], -mean) * rstd, w, b));
             if (++r == L.d) {
                 r = 0;
                 c++;
@@ -1105,8 +1115,7 @@ __global__ void __launch_bounds__(BLOCK) gn_apply_kernel(const T* __restrict__ x
             const uint32_t c = g * cpg + fd_div(i, L);
             const float w = scale ? Ar<T>::widen(scale[c]) : 1.0f;
             const float b = bias ? Ar<T>::widen(bias[c]) : 0.0f;
-            const float t = (Ar<T>::widen(xs[i]) - meanf) * rstd;
-            ys[i] = Ar<T>::conv(t * w + b);
+            ys[i] = Ar<T>::conv(__builtin_fmaf(gn_plus<T>(xs[i], -meanf) * rstd, w, b));
         }
     }
 }
@@ -1724,123 +1733,100 @@ int norm_entry(rt_device* dev, int kind, int dt, const void* x, const void* scal
     }
 }
 
-// Few, small groups (the latency-bound case: 32 groups of 96 KB in the reference's Whisper-style shape): one launch, one
-// 1024-thread block per (batch, group), the group staged in LDS once, then mean, squared deviations and the output all
-// come from LDS.  Same definitions as the two-kernel path (mean, then the variance about that mean, f32 arithmetic).
-constexpr int GN_LDS_BLOCK = 1024;
-constexpr size_t GN_LDS_MAX_BYTES = 144 * 1024;
-constexpr size_t GN_REG_MAX_BYTES = 16 * 1024 * 16;           // what gn_reg_kernel holds without spilling: 16 vectors in each of 1024 threads
-
-template <typename T>
-__global__ void __launch_bounds__(GN_LDS_BLOCK) gn_lds_kernel(const T* __restrict__ x, const T* __restrict__ scale, const T* __restrict__ bias,
-                                                              T* __restrict__ y, uint32_t glen, uint32_t cpg, uint32_t groups, FastDiv L,
-                                                              float eps) {
-    constexpr int VE = 16 / sizeof(T);
-    extern __shared__ __attribute__((aligned(16))) unsigned char gn_smem[];
-    v4u* stage = reinterpret_cast<v4u*>(gn_smem);
-    const uint32_t grp = blockIdx.x, g = grp % groups;
-    const v4u* xs = reinterpret_cast<const v4u*>(x + (uint64_t)grp * glen);
-    v4u* ys = reinterpret_cast<v4u*>(y + (uint64_t)grp * glen);
-    const uint32_t nvec = glen / VE;
-    float acc = 0.0f;
-    for (uint32_t i0 = threadIdx.x; i0 < nvec; i0 += GN_LDS_BLOCK * 8) {    // eight loads in flight per thread
-        Vec16<T> v[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const uint32_t i = i0 + k * GN_LDS_BLOCK;
-            if (i < nvec) v[k].u = ld_stream(xs + i);
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const uint32_t i = i0 + k * GN_LDS_BLOCK;
-            if (i < nvec) {
-                stage[i] = v[k].u;
-#pragma unroll
-                for (int q = 0; q < VE; q++) acc += Ar<T>::widen(v[k].e[q]);
-            }
-        }
-    }
-    const float mean = row_sum<GN_LDS_BLOCK>(acc) / (float)glen;
-    float m2 = 0.0f;
-    for (uint32_t i = threadIdx.x; i < nvec; i += GN_LDS_BLOCK) {           // a thread re-reads what it wrote itself
-        Vec16<T> v;
-        v.u = stage[i];
-#pragma unroll
-        for (int q = 0; q < VE; q++) {
-            const float d = Ar<T>::widen(v.e[q]) - mean;
-            m2 += d * d;
-        }
-    }
-    const float var = row_sum<GN_LDS_BLOCK>(m2) / (float)glen;
-    const float rstd = 1.0f / __builtin_sqrtf(var + eps);
-    for (uint32_t i = threadIdx.x; i < nvec; i += GN_LDS_BLOCK) {
-        Vec16<T> v;
-        v.u = stage[i];
-        st_stream(ys + i, gn_affine_vec<T>(v, i * VE, g * cpg, L, scale, bias, mean, rstd));
-    }
-}
-
-// The group in the registers of 1024-thread blocks (thread t holds vectors t, t + 1024, ...; NV of them), for groups too
-// large for the LDS of gn_lds_kernel (one block per group) and for small problems of few groups (32 groups of 96 KB on 256
-// CUs): there `slices` blocks per group, all in one launch and without any wait between blocks.  Every block of a group
-// loads the WHOLE group and reduces it to the same mean and variance in the same order, so the blocks of a group agree
-// bit for bit without exchanging anything; each then normalises and stores only its own run of nvec / slices vectors.
-// The repeated reads of a group hit the L2 of the XCD its blocks share (see the block -> (group, slice) map in
-// launch_gn), so HBM still sees the group once.  Same definitions as gn_lds_kernel.
-template <typename T, int NV>
-__global__ void __launch_bounds__(GN_LDS_BLOCK) gn_reg_kernel(const T* __restrict__ x, const T* __restrict__ scale, const T* __restrict__ bias,
-                                                              T* __restrict__ y, uint32_t glen, uint32_t cpg, uint32_t groups, FastDiv L,
-                                                              float eps, uint32_t slices, uint32_t per_xcd) {
+// GroupNorm in one launch: the group in the registers of one block (thread t of BT holds vectors t, t + BT, ...; NV of them), so
+// HBM sees it once; mean, squared deviations and the output are computed from the registers, with the definitions of the two-kernel
+// path (mean, then the variance about that mean, f32 arithmetic).  What bounds it is how much of a CU's loads, reductions and
+// stores run at the same time: WPE is the number of waves per SIMD that the registers leave room for, and with the sizes that
+// launch_gn takes two blocks or more share a CU, one storing while another loads ([16,512,3000] f16, 512 groups of 94 KiB: 22.6 us with the
+// group in LDS, one block to a CU, 20.1 with 1024 threads of 6 vectors, 20.4 with 512 of 12; [128,256,3000] f16 97 -> 61 us = 6.4 TB/s;
+// [64,256,1500] f32 35.3 -> 29.3 us).
+// SPAN: groups that do not start or end on a vector boundary, over the aligned vectors that cover them.  The elements of the
+// neighbouring groups in the first and the last of those stay out of the sums and are not written (such vectors are stored element
+// by element); an aligned vector that holds one byte of the tensor lies in a mapped page.  [16,320,3001] f16 55 -> 15 us against
+// the element-wise launches.
+// Few groups (fewer than half as many as CUs): `slices` blocks per group, all in one launch and without any wait between blocks.  Every
+// block of a group loads the WHOLE group and reduces it to the same mean and variance in the same order, so the blocks of a
+// group agree bit for bit without exchanging anything; each then normalises and stores only its own run of nvec / slices
+// vectors.  The repeated reads of a group hit the L2 of the XCD its blocks share (see launch_gn_reg).
+template <typename T, int NV, int BT, int WPE, bool SPAN>
+__global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x, const T* __restrict__ scale, const T* __restrict__ bias,
+                                                         T* __restrict__ y, uint32_t glen, uint32_t cpg, uint32_t groups, FastDiv L, float eps,
+                                                         uint32_t slices, uint32_t per_xcd) {
     constexpr int VE = 16 / sizeof(T);
     // blocks are handed to the 8 XCDs round robin: pair index p runs over the (group, slice) pairs of one XCD first
     const uint32_t p = per_xcd ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
     const uint32_t grp = p / slices, slice = p - grp * slices, g = grp % groups;
-    const v4u* xs = reinterpret_cast<const v4u*>(x + (uint64_t)grp * glen);
-    v4u* ys = reinterpret_cast<v4u*>(y + (uint64_t)grp * glen);
-    const uint32_t nvec = glen / VE;
+    const uint64_t first = (uint64_t)grp * glen;
+    const uint32_t shift = SPAN ? (uint32_t)(first & (VE - 1)) : 0;
+    const v4u* xs = reinterpret_cast<const v4u*>(x) + first / VE;
+    v4u* ys = reinterpret_cast<v4u*>(y) + first / VE;
+    const uint32_t nvec = SPAN ? (shift + glen + VE - 1) / VE : glen / VE;
+    auto ragged = [&](uint32_t i) -> bool { return SPAN && i < nvec && (i == 0 || i == nvec - 1); };
+    auto inside = [&](uint32_t i, int q) -> bool { return i * VE + (uint32_t)q - shift < glen; };
     Vec16<T> v[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        const uint32_t i = threadIdx.x + k * GN_LDS_BLOCK;
+        const uint32_t i = threadIdx.x + k * BT;
         v[k].u = v4u{0u, 0u, 0u, 0u};
-        if (i < nvec) v[k].u = xs[i];
+        if (i < nvec) v[k].u = slices > 1 ? xs[i] : ld_stream(xs + i);
     }
     float acc = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; k++) {
+        const uint32_t i = threadIdx.x + k * BT;
+        if (ragged(i)) {
 #pragma unroll
-        for (int q = 0; q < VE; q++) acc += Ar<T>::widen(v[k].e[q]);         // vectors past the group hold zeros
+            for (int q = 0; q < VE; q++)
+                if (inside(i, q)) acc = gn_plus<T>(v[k].e[q], acc);
+        } else {
+#pragma unroll
+            for (int q = 0; q < VE; q++) acc = gn_plus<T>(v[k].e[q], acc);       // vectors past the group hold zeros
+        }
     }
-    const float mean = row_sum<GN_LDS_BLOCK>(acc) / (float)glen;
-    // the group stays in registers as it was loaded.  With 16 vectors a thread the widened values of one pass must not be kept
-    // for the next (the compiler otherwise keeps them and spills); with fewer it may keep what fits (32 groups of 93 KiB f16,
-    // 6 vectors a thread: 8.3 us when every pass widens again, 6.3 us when not)
+    const float mean = row_sum<BT>(acc) / (float)glen;
+    // the group stays in registers as it was loaded: the widened values of one pass must not be kept for the next, but with few
+    // blocks of few vectors, which run alone on their CU and where keeping what fits saves instructions (32 groups of 93 KiB f16
+    // 6.0 us, 6.8 when every pass widens again)
+    constexpr bool KEEP = sizeof(T) == 4 || (WPE <= 4 && NV <= 9);
     auto forget = [&]() {
-        if (NV < 16) return;
 #pragma unroll
         for (int k = 0; k < NV; k++) asm volatile("" : "+v"(v[k].u[0]), "+v"(v[k].u[1]), "+v"(v[k].u[2]), "+v"(v[k].u[3]));
     };
-    forget();
+    if (!KEEP) forget();
     float m2 = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        if (threadIdx.x + k * GN_LDS_BLOCK < nvec) {
+        const uint32_t i = threadIdx.x + k * BT;
+        if (ragged(i)) {
 #pragma unroll
-            for (int q = 0; q < VE; q++) {
-                const float d = Ar<T>::widen(v[k].e[q]) - mean;
-                m2 += d * d;
-            }
+            for (int q = 0; q < VE; q++)
+                if (inside(i, q)) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
+        } else if (i < nvec) {
+#pragma unroll
+            for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
         }
     }
-    const float var = row_sum<GN_LDS_BLOCK>(m2) / (float)glen;
-    forget();
+    const float var = row_sum<BT>(m2) / (float)glen;
+    if (!KEEP) forget();
     const float rstd = 1.0f / __builtin_sqrtf(var + eps);
     const uint32_t lo = (uint32_t)(((uint64_t)nvec * slice) / slices), hi = (uint32_t)(((uint64_t)nvec * (slice + 1)) / slices);
 #pragma unroll
     for (int k = 0; k < NV; k++) {
-        const uint32_t i = threadIdx.x + k * GN_LDS_BLOCK;
-        if (i >= lo && i < hi) {
-            st_stream(ys + i, gn_affine_vec<T>(v[k], i * VE, g * cpg, L, scale, bias, mean, rstd));
+        const uint32_t i = threadIdx.x + k * BT;
+        if (i < lo || i >= hi) continue;
+        if (ragged(i)) {
+            T* yg = y + first;
+#pragma unroll
+            for (int q = 0; q < VE; q++) {
+                const uint32_t e = i * VE + (uint32_t)q - shift;
+                if (e < glen) {
+                    const uint32_t c = g * cpg + fd_div(e, L);
+                    const float w = scale ? Ar<T>::widen(scale[c]) : 1.0f, b = bias ? Ar<T>::widen(bias[c]) : 0.0f;
+                    yg[e] = Ar<T>::conv(__builtin_fmaf(gn_plus<T>(v[k].e[q], -mean) * rstd, w, b));
+                }
+            }
+        } else {
+            st_stream(ys + i, gn_affine_vec<T>(v[k], i * VE - shift, g * cpg, L, scale, bias, mean, rstd));
         }
     }
 }
@@ -1881,6 +1867,18 @@ __global__ void __launch_bounds__(BLOCK) gn_combine_kernel(const float* __restri
     }
 }
 
+template <typename T, int NV, int BT, int WPE, bool SPAN>
+int launch_gn_reg(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint32_t bg, uint32_t glen, uint32_t cpg,
+                  uint32_t groups, uint32_t L, float eps, uint32_t slices) {
+    // with a block count that the 8 XCDs share evenly, block b (on XCD b % 8) takes pair (b % 8) * blocks / 8 + b / 8, which
+    // puts the slices of a group on one XCD (all of them when bg is a multiple of 8)
+    const uint32_t blocks = bg * slices, per_xcd = (slices > 1 && blocks % 8 == 0) ? blocks / 8 : 0;
+    hipLaunchKernelGGL((gn_reg_kernel<T, NV, BT, WPE, SPAN>), dim3(blocks), dim3(BT), 0, dev->stream, (const T*)x, (const T*)scale, (const T*)bias,
+                       (T*)y, glen, cpg, groups, make_fastdiv(L), eps, slices, per_xcd);
+    RT_CHECK_LAUNCH("gn_reg_kernel");
+    return RT_OK;
+}
+
 // fixed_scratch == nullptr: partial statistics go to the device's own buffer, grown from the driver when a problem needs
 // more; otherwise to fixed_scratch (GN_STATIC_SCRATCH_BYTES), and a problem that needs more is refused.
 template <typename T>
@@ -1896,66 +1894,8 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
     if (splits > 2048) splits = 2048;
     if (splits < 1) splits = 1;
     constexpr int VEMAX = 16 / sizeof(T);
-    const bool vec = (glen % VEMAX == 0) && rt_aligned(x, 16) && rt_aligned(y, 16);    // every group starts on a vector boundary
-    // Which path, for vector-aligned groups (measured on 256 CUs; the two or three launches below spread any problem over the
-    // whole chip in small blocks, the one-launch kernels read HBM once but run 1024-thread blocks that hold whole groups):
-    //   few groups (at most half as many as CUs) of up to 9 vectors a thread (144 KiB; 12 vectors, 192 KiB, in f32):
-    //        gn_reg_kernel, several blocks per group (32 groups of 93 KiB f16 6.3 us against 6.9 for the launches, 96 groups
-    //        7.5 against 10.2 for gn_lds_kernel, 128 groups of 187 KiB f32 12.0 against 13.0 with one block per group).  16-bit
-    //        groups beyond 9 vectors a thread widen to more registers than a thread has: 64 groups of 160 KiB f16 13.3 us
-    //        against 9.6 for the launches
-    //   up to 144 KiB, more groups than that (and at most eight times as many as CUs): gn_lds_kernel
-    //        (93 KiB f16 x 256 groups 12.1 us against 15.2 for the launches, 64 KiB x 1024 28.4 against 34.4; gn_reg_kernel
-    //        on these is within 8 % either way, except 47 KiB f16 x 2048: 53.6 against 42.3)
-    //   f32 groups of 144 to 192 KiB, at least half as many groups as CUs, and of up to 256 KiB (16 vectors a thread; 20 and
-    //        24 spill), at least as many groups as CUs: gn_reg_kernel, one block per group (187 KiB x 256 groups 20.0 us
-    //        against 25.3 for the launches, 256 KiB x 256 27.3 against 32.9, x 1024 107 against 125; 256 KiB x 128: 16.5
-    //        against 16.4).  In 16 bits the launches are as fast or faster on these (160 KiB x 128 groups 13.3 us against
-    //        16.9, 256 KiB x 512 64.2 against 65.8)
-    //   everything else: the launches below
-    const size_t gbytes = (size_t)glen * sizeof(T);
-    const uint32_t cus = (uint32_t)dev->num_cus;
-    const uint32_t nv_group = (glen / VEMAX + GN_LDS_BLOCK - 1) / GN_LDS_BLOCK;          // vectors a thread of gn_reg_kernel would hold
-    const bool reg_few = 2u * bg <= cus && (nv_group <= 9 || (sizeof(T) == 4 && nv_group <= 12));
-    const bool reg_large = sizeof(T) == 4 && gbytes > GN_LDS_MAX_BYTES && bg <= 8u * cus &&
-                           ((gbytes <= GN_REG_MAX_BYTES * 3 / 4 && 2u * bg >= cus) || (gbytes <= GN_REG_MAX_BYTES && bg >= cus));
-    if (vec && (reg_few || reg_large)) {
-        uint32_t slices = reg_few && bg <= cus ? cus / bg : 1;
-        if (slices > 32) slices = 32;
-        const uint32_t nvec = glen / VEMAX;
-        if (slices > nvec) slices = nvec;
-        const uint32_t blocks = bg * slices;
-        // with a block count that the 8 XCDs share evenly, block b (on XCD b % 8) takes pair (b % 8) * blocks / 8 + b / 8, which
-        // puts the slices of a group on one XCD (all of them when bg is a multiple of 8)
-        const uint32_t per_xcd = (slices > 1 && blocks % 8 == 0) ? blocks / 8 : 0;
-        const uint32_t nv = (nvec + GN_LDS_BLOCK - 1) / GN_LDS_BLOCK;
-        const dim3 grid(blocks), block(GN_LDS_BLOCK);
-#define RT_GN_REG(NVC)                                                                                                                      \
-    hipLaunchKernelGGL((gn_reg_kernel<T, NVC>), grid, block, 0, dev->stream, (const T*)x, (const T*)scale, (const T*)bias, (T*)y, glen, cpg, \
-                       groups, make_fastdiv(L), eps, slices, per_xcd)
-        if (nv <= 1) RT_GN_REG(1);
-        else if (nv <= 2) RT_GN_REG(2);
-        else if (nv <= 4) RT_GN_REG(4);
-        else if (nv <= 6) RT_GN_REG(6);
-        else if (nv <= 9) RT_GN_REG(9);
-        else if (nv <= 12) RT_GN_REG(12);
-        else RT_GN_REG(16);
-#undef RT_GN_REG
-        RT_CHECK_LAUNCH("gn_reg_kernel");
-        return RT_OK;
-    }
-    if (vec && gbytes <= GN_LDS_MAX_BYTES && 8u * bg >= 3u * cus && bg <= 8u * cus) {
-        const int ti = sizeof(T) == 4 ? 0 : (std::is_same<T, half_t>::value ? 1 : 2);
-        if (!(dev->gn_lds_attr_set & (1u << ti))) {
-            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(gn_lds_kernel<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)GN_LDS_MAX_BYTES));
-            dev->gn_lds_attr_set |= 1u << ti;
-        }
-        hipLaunchKernelGGL((gn_lds_kernel<T>), dim3(bg), dim3(GN_LDS_BLOCK), (size_t)glen * sizeof(T), dev->stream, (const T*)x, (const T*)scale,
-                           (const T*)bias, (T*)y, glen, cpg, groups, make_fastdiv(L), eps);
-        RT_CHECK_LAUNCH("gn_lds_kernel");
-        return RT_OK;
-    }
+    const bool aligned = rt_aligned(x, 16) && rt_aligned(y, 16);
+    const bool vec = (glen % VEMAX == 0) && aligned;    // every group starts on a vector boundary
     // slices of at most 32 KiB stay in the registers of their 256-thread block (8 vectors a thread), in the stats launch and
     // in the apply launch: more, smaller slices when the rule above leaves them larger
     constexpr uint32_t GN_SLICE_REG_VEC = 8;
@@ -1971,11 +1911,52 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
     const bool slice_reg = vec && chunk <= slice_reg_elems;
     const uint32_t slice_nv = slice_reg ? (chunk / VEMAX + BLOCK - 1) / BLOCK : 0;
     const size_t need = ((size_t)bg * splits + bg) * 3 * sizeof(float);           // partials, then one combined triple per group
-    if (fixed_scratch) {
+    if (fixed_scratch)                                                              // whichever path the problem then takes
         RT_REQUIRE(need <= GN_STATIC_SCRATCH_BYTES, RT_ERR_SIZE,
                    "rt_group_norm_static: %u (batch, group) pairs in %u slices need %zu bytes of partial statistics, the fixed buffer holds %zu",
                    bg, splits, need, GN_STATIC_SCRATCH_BYTES);
-    } else if (need > dev->gn_scratch_bytes) {
+    // Which path (measured on 256 CUs, us against the launches below or the next kernel that would hold the group):
+    //   at most half as many groups as CUs, up to 144 KiB (192 in f32): 1024 threads, cus / groups blocks per group (32 groups of
+    //        93 KiB f16 5.8, 6.9 by launches; ragged [2,320,3001] f16 7.9 / 10.7).  Larger ones in 16 bits go to the launches (64 groups
+    //        of 160 KiB f16 13.3 / 9.6)
+    //   more groups: one block per group, as many threads as leave two blocks or more to a CU.  Up to 12, 24 and 48 KiB: 256, 512,
+    //        512 threads of at most 3, 3, 6 vectors (8 KiB x 512 groups 5.0, 5.5 - 6.1 with wider blocks; 47 KiB x 2048 33.8, 35.7
+    //        with 1024 threads); up to 96 KiB: 1024 threads of 4 or 6 (94 KiB x 256 groups 9.9, 11.5 with 512 threads of 12); up to
+    //        128 KiB 512 threads of 16, which leave room for a second block where 1024 of 8 spill (125 KiB f32 x 512 21.2 / 26.6); up
+    //        to 192 KiB 1024 threads of 9 or 12, one block to a CU (141 KiB f16 x 512 31.7, 39.4 by launches; 188 KiB f16 x 512 39.5 / 46.8)
+    //   f32 groups of 192 to 256 KiB (16 vectors a thread; 20 and 24 spill), at least as many groups as CUs: 250 KiB x 512 43.6, 61.9
+    //        by launches; 256 KiB x 128: 16.5 / 16.4.  In 16 bits such groups go to the launches (x 512 64.2, 65.8 with 16 vectors)
+    //   everything else: the launches below
+    const uint32_t cus = (uint32_t)dev->num_cus;
+    const uint32_t nvec = vec ? glen / VEMAX : (glen + 2 * VEMAX - 2) / VEMAX;          // the most vectors a group touches
+#define RT_GN_REG(NVC, BTC, WPEC)                                                                                                    \
+    return vec ? launch_gn_reg<T, NVC, BTC, WPEC, false>(dev, x, scale, bias, y, bg, glen, cpg, groups, L, eps, slices)          \
+               : launch_gn_reg<T, NVC, BTC, WPEC, true>(dev, x, scale, bias, y, bg, glen, cpg, groups, L, eps, slices)
+    if (aligned && 2u * bg <= cus && nvec <= (sizeof(T) == 4 ? 12288u : 9216u)) {
+        uint32_t slices = x == y ? 1 : cus / bg;                        // in place, a block must not store what another still loads
+        if (slices > 32) slices = 32;
+        if (slices > nvec) slices = nvec;
+        if (nvec <= 1024) RT_GN_REG(1, 1024, 4);
+        if (nvec <= 2048) RT_GN_REG(2, 1024, 4);
+        if (nvec <= 4096) RT_GN_REG(4, 1024, 4);
+        if (nvec <= 6144) RT_GN_REG(6, 1024, 4);
+        if (nvec <= 9216) RT_GN_REG(9, 1024, 4);
+        RT_GN_REG(12, 1024, 4);
+    }
+    if (aligned && 2u * bg > cus) {
+        const uint32_t slices = 1;
+        if (nvec <= 768) RT_GN_REG(3, 256, 8);
+        if (nvec <= 1536) RT_GN_REG(3, 512, 8);
+        if (nvec <= 3072) RT_GN_REG(6, 512, 8);
+        if (nvec <= 4096) RT_GN_REG(4, 1024, 8);
+        if (nvec <= 6144) RT_GN_REG(6, 1024, 8);
+        if (nvec <= 8192) RT_GN_REG(16, 512, 4);
+        if (nvec <= 9216) RT_GN_REG(9, 1024, 4);
+        if (nvec <= 12288) RT_GN_REG(12, 1024, 4);
+        if (sizeof(T) == 4 && nvec <= 16384 && bg >= cus) RT_GN_REG(16, 1024, 4);
+    }
+#undef RT_GN_REG
+    if (!fixed_scratch && need > dev->gn_scratch_bytes) {
         RT_NO_CAPTURE(dev, "growing the GroupNorm scratch");
         RT_HIP(hipStreamSynchronize(dev->stream));
         RT_HIP(hipFree(dev->gn_scratch));

@@ -795,6 +795,25 @@ def test_group_norm(dev, oracle, B, C, L, G, dtype):
     assert bad == 0, (bad, mx)
 
 
+@pytest.mark.parametrize("glen", [6144, 6152, 12296, 24584, 32776, 49160, 65544, 73736, 98312,     # f16 groups one vector over what each block shape holds
+                                  1, 5, 2049, 24571, 49149, 73723])                               # groups that start and end inside a vector
+@pytest.mark.parametrize("B", [1, 13])                                                           # several blocks per group; one block per group
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_group_norm_at_the_edges_of_the_block_shapes(dev, oracle, glen, B, dtype):
+    """130 groups (10 with B = 1) of one and of two channels around the sizes where a wider block takes over, and ragged ones, which
+    share vectors with their neighbours: nothing of those is summed or written, also in place.  Tolerances of test_group_norm"""
+    rng = np.random.default_rng(glen)
+    tol = 1e-5 if dtype == np.float32 else 1e-3
+    for C, L in ((10, glen), (20, glen // 2)) if glen % 2 == 0 else ((10, glen),):
+        x = randn(rng, (B, C, L), dtype)
+        w, b = randn(rng, C, dtype), randn(rng, C, dtype)
+        want = oracle.group_norm(x, 10, w, b, 1e-5)
+        dx = dev.upload(x)
+        for got in (dev.group_norm(dx, 10, dev.upload(w), dev.upload(b), 1e-5), dev.group_norm(dx, 10, dev.upload(w), dev.upload(b), 1e-5, out=dx)):
+            bad, mx = oracle.count_not_close(got.to_numpy(), want, tol, tol)
+            assert bad == 0, (C, L, bad, mx)
+
+
 def test_group_norm_many_groups_too_large_for_lds(dev, oracle):
     """288 groups of 160 KB in f32 (more pairs than CUs, groups over what the LDS kernel stages): one block per group with the
     group in registers, two rounds of blocks; against the oracle"""
