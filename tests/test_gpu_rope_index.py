@@ -65,6 +65,27 @@ def test_rope_16bit_layouts(dev, oracle, shape, dim, offset):
         assert np.array_equal(inplace.view(np.uint16), got.view(np.uint16))
 
 
+@pytest.mark.parametrize("shape,dim", [((1, 8, 333, 80), 32),         # one row a thread and trip (fewer than two blocks to a CU), a ragged last block of positions
+                                       ((3, 32, 333, 80), 32),        # two rows, the last trip of a block ragged
+                                       ((2, 33, 1100, 128), 128),     # whole 256-byte rows (512 in f32), over 32 MiB in f32: in place through the same kernel
+                                       ((4, 33, 1100, 128), 64),      # ... over 32 MiB in 16 bits, pass-through columns
+                                       ((1, 3, 5, 2112), 2112)])      # wider than a block: the slot kernel
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_rope_trips_and_in_place_by_size(dev, oracle, shape, dim, kind):
+    """every kernel and trip length the dispatch picks by size, out of place and in place, against the oracle bit for bit"""
+    rng = np.random.default_rng(606)
+    xf = rng.standard_normal(shape).astype(np.float32)
+    bf = kind == "bf16"
+    if kind == "f32":
+        x, want = xf, oracle.rope(xf, dim, 10000.0, 11)
+    else:
+        x = oracle.cast(xf, np.uint16, dst_bf16=True) if bf else xf.astype(np.float16)
+        want = oracle.cast(oracle.rope(oracle.cast(x, np.float32, src_bf16=bf), dim, 10000.0, 11), np.uint16 if bf else np.float16, dst_bf16=bf)
+    d = dev.upload(x, bf16=bf)
+    for got in (dev.rope(d, dim, 10000.0, 11), dev.rope(d, dim, 10000.0, 11, out=d)):
+        assert same_bits(got.to_numpy(), np.asarray(want))
+
+
 def test_rope_f32_off_vector_alignment(dev, oracle):
     """an operand 4 bytes off 16-byte alignment takes the scalar kernel: same results as the aligned call"""
     rng = np.random.default_rng(606)
