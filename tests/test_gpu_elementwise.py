@@ -299,6 +299,41 @@ def test_storage_pool_reuses_blocks_in_stream_order(oracle):
         d.close()
 
 
+@pytest.mark.parametrize("n", [1, 3, 127, 128, 129, 1024, 4095, 4096, 4097, 16384])       # 16 KiB = 4096 values is the last size through pinned memory
+def test_downloads_of_either_path_bring_the_bytes_of_the_moment(n):
+    """whole blocks of up to 16 KiB come through the device's pinned buffer, larger ones and windows into a block by the runtime's copy; a later
+    download shows later contents, and two threads on one device get their own bytes"""
+    import threading
+
+    from ratchet_amd import Device
+
+    d = Device(0)
+    try:
+        rng = np.random.default_rng(n)
+        x, y = rng.integers(0, 2**31, n).astype(np.uint32), rng.integers(0, 2**31, n).astype(np.uint32)
+        dx, dy = d.upload(x), d.upload(y)
+        assert np.array_equal(dx.to_numpy(), x) and np.array_equal(dy.to_numpy(), y)
+        assert np.array_equal(dx.view(n // 2, (n - n // 2,)).to_numpy(), x[n // 2:])
+        dx.zero_()
+        assert not dx.to_numpy().any()
+        dx.view(0, (n,)).upload(x)
+        wrong = []
+
+        def fetch(buf, want):
+            for _ in range(50):
+                if not np.array_equal(buf.to_numpy(), want):
+                    wrong.append(want.shape)
+
+        threads = [threading.Thread(target=fetch, args=a) for a in ((dx, x), (dy, y))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong
+    finally:
+        d.close()
+
+
 def test_storage_pool_ages_unused_blocks_by_passes():
     """rt_pool_begin_pass is the reference's begin_pass (gpu/pools/dynamic_resource_pool.rs:140-190): a block freed during
     pass p can be taken again during passes p and p + 1 and goes back to the driver at the start of pass p + 2 if nobody
