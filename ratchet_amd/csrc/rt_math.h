@@ -40,24 +40,46 @@ __device__ __forceinline__ uint16_t h_bits(half_t h) { return __builtin_bit_cast
 __device__ __forceinline__ half_t bits_h(uint16_t u) { return __builtin_bit_cast(half_t, u); }
 
 // ---- wave64 reductions ----------------------------------------------------------------------------------
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// One butterfly step: the value of the lane whose index differs in bit OFF, joined with this lane's by `f` (commutative).  32 and 16 are
+// register swaps of half waves and of rows of 16 lanes, the rest DPP moves inside a row, without the trip through LDS of a
+// shuffle (about 60 cycles a step, six steps a reduction).  8 and 4 rotate a row of 16: the same partner, or after the steps before one that
+// holds the same value, so 4 needs the step of 8 before it (groups of 8 lanes and fewer take the shuffle there).
+template <int OFF, bool ROW, typename F> __device__ __forceinline__ float wave_step(float v, F f) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    if constexpr (OFF == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return f(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    } else if constexpr (OFF == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return f(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+    } else if constexpr (OFF == 4 && !ROW) {
+        return f(v, __shfl_xor(v, 4, 64));
+    } else {
+        constexpr int CTRL = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4E : 0xB1;      // row_ror:8, row_ror:4, quad_perm 2301, 1032
+        const int o = __builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xf, 0xf, false);
+        return f(v, __builtin_bit_cast(float, o));
+    }
+}
+template <int LANES, typename F> __device__ __forceinline__ float lanes_join(float v, F f) {
+    if constexpr (LANES >= 64) v = wave_step<32, true>(v, f);
+    if constexpr (LANES >= 32) v = wave_step<16, true>(v, f);
+    if constexpr (LANES >= 16) v = wave_step<8, true>(v, f);
+    if constexpr (LANES >= 8) v = wave_step<4, (LANES >= 16)>(v, f);
+    if constexpr (LANES >= 4) v = wave_step<2, true>(v, f);
+    if constexpr (LANES >= 2) v = wave_step<1, true>(v, f);
     return v;
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
+struct JoinSum { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+struct JoinMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
+__device__ __forceinline__ float wave_sum(float v) { return lanes_join<64>(v, JoinSum()); }
+__device__ __forceinline__ float wave_max(float v) { return lanes_join<64>(v, JoinMax()); }
 
 // Reduction over the LANES threads that share a row: a group of 2..64 neighbouring lanes of a wave (a butterfly over the
 // group; LANES == 64 is the whole wave), or a whole 256-thread block, whose four wave results meet in LDS and are added
 // in a fixed order.  Every thread of the block must call the block form.
 template <int LANES> __device__ __forceinline__ float row_sum(float v) {
     if constexpr (LANES <= 64) {
-#pragma unroll
-        for (int off = LANES / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        v = lanes_join<LANES>(v, JoinSum());
     } else {
         v = wave_sum(v);
         __shared__ float red[LANES / 64];
@@ -72,8 +94,7 @@ template <int LANES> __device__ __forceinline__ float row_sum(float v) {
 }
 template <int LANES> __device__ __forceinline__ float row_max(float v) {
     if constexpr (LANES <= 64) {
-#pragma unroll
-        for (int off = LANES / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+        v = lanes_join<LANES>(v, JoinMax());
     } else {
         v = wave_max(v);
         __shared__ float red[LANES / 64];
