@@ -1736,14 +1736,26 @@ int norm_entry(rt_device* dev, int kind, int dt, const void* x, const void* scal
     }
 }
 
+// the waves' sums of a block, added in double: at the size of a whole group's sum each of these additions would cost half an ulp of it
+template <int BT> __device__ __forceinline__ double gn_block_sum(float v) {
+    __shared__ float red[BT / WAVE];
+    v = wave_sum(v);
+    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    double t = (double)red[0];
+#pragma unroll
+    for (int w = 1; w < BT / WAVE; w++) t += (double)red[w];
+    return t;
+}
+
 // 1 / sqrt(m2 / n + eps) to about half an ulp in f32 arithmetic: what the quotient and the sum lost to rounding (n is exact: a group
 // in registers has fewer than 2^24 elements) and what the reciprocal root is off by go into one correction.  The launches for larger
-// groups compute this in double; every group held in registers is now at least as close to 64 bits as they are (f32 [8,320,4097]
-// 7.0e-8 without the correction, 5.7e-8 by the launches).  Where the correction means nothing (a variance of 0, inf or NaN) it is left out.
-__device__ __forceinline__ float gn_rstd(float m2, float n, float eps) {
-    const float q = m2 / n, v = q + eps, r = 1.0f / __builtin_sqrtf(v);
+// groups compute this in double; with the double sum above, every group held in registers is at least as close to 64 bits as they are
+// (f32 [8,320,4097] 5.1e-8, 7.0e-8 without the two, 5.7e-8 by the launches; they cost 0.1 us of a small launch and 0.5 of the [16,512,3000]).  Where the correction means nothing (a variance of 0, inf or NaN) it is left out.
+__device__ __forceinline__ float gn_rstd(double m2d, float n, float eps) {
+    const float m2 = (float)m2d, q = m2 / n, v = q + eps, r = 1.0f / __builtin_sqrtf(v);
     const float part = v - q;
-    const float lost = ((q - (v - part)) + (eps - part)) + __builtin_fmaf(-q, n, m2) / n;
+    const float lost = ((q - (v - part)) + (eps - part)) + (__builtin_fmaf(-q, n, m2) + (float)(m2d - (double)m2)) / n;
     const float p = v * r;
     const float e = (__builtin_fmaf(-p, r, 1.0f) - __builtin_fmaf(v, r, -p) * r) - lost * r * r;
     return __builtin_fabsf(e) < 0.5f ? __builtin_fmaf(0.5f * r, e, r) : r;
@@ -1754,7 +1766,7 @@ __device__ __forceinline__ float gn_rstd(float m2, float n, float eps) {
 // path (mean, then the variance about that mean, f32 arithmetic).  What bounds it is how much of a CU's loads, reductions and
 // stores run at the same time: WPE is the number of waves per SIMD that the registers leave room for, and with the sizes that
 // launch_gn takes two blocks or more share a CU, one storing while another loads ([16,512,3000] f16, 512 groups of 94 KiB: 22.6 us with the
-// group in LDS, one block to a CU, 20.1 with 1024 threads of 6 vectors, 20.4 with 512 of 12; [128,256,3000] f16 97 -> 61 us = 6.4 TB/s;
+// group in LDS, one block to a CU, 20.3 with 1024 threads of 6 vectors, 20.4 with 512 of 12; [128,256,3000] f16 97 -> 61 us = 6.4 TB/s;
 // [64,256,1500] f32 35.3 -> 29.3 us).
 // SPAN: groups that do not start or end on a vector boundary, over the aligned vectors that cover them.  The elements of the
 // neighbouring groups in the first and the last of those stay out of the sums and are not written (such vectors are stored element
@@ -1822,7 +1834,7 @@ __global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x
             for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
         }
     }
-    const float rstd = gn_rstd(row_sum<BT>(m2), (float)glen, eps);
+    const float rstd = gn_rstd(gn_block_sum<BT>(m2), (float)glen, eps);
     if (!KEEP) forget();
     const uint32_t lo = (uint32_t)(((uint64_t)nvec * slice) / slices), hi = (uint32_t)(((uint64_t)nvec * (slice + 1)) / slices);
 #pragma unroll
