@@ -72,6 +72,33 @@ template <int LANES, typename F> __device__ __forceinline__ float lanes_join(flo
 struct JoinSum { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 struct JoinMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
 __device__ __forceinline__ float wave_sum(float v) { return lanes_join<64>(v, JoinSum()); }
+// the same butterfly on doubles, whose two halves move side by side
+template <int OFF> __device__ __forceinline__ double wave_step_sum(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    uint32_t a[2], b[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const uint32_t w = (uint32_t)(u >> (32 * k));
+        if constexpr (OFF >= 16) {
+            const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(w, w, false, false) : __builtin_amdgcn_permlane16_swap(w, w, false, false);
+            a[k] = r[0];
+            b[k] = r[1];
+        } else {
+            constexpr int CTRL = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4E : 0xB1;
+            a[k] = w;
+            b[k] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, CTRL, 0xf, 0xf, false);
+        }
+    }
+    return __builtin_bit_cast(double, (uint64_t)a[1] << 32 | a[0]) + __builtin_bit_cast(double, (uint64_t)b[1] << 32 | b[0]);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v = wave_step_sum<32>(v);
+    v = wave_step_sum<16>(v);
+    v = wave_step_sum<8>(v);
+    v = wave_step_sum<4>(v);
+    v = wave_step_sum<2>(v);
+    return wave_step_sum<1>(v);
+}
 __device__ __forceinline__ float wave_max(float v) { return lanes_join<64>(v, JoinMax()); }
 
 // Reduction over the LANES threads that share a row: a group of 2..64 neighbouring lanes of a wave (a butterfly over the

@@ -1736,16 +1736,18 @@ int norm_entry(rt_device* dev, int kind, int dt, const void* x, const void* scal
     }
 }
 
-// the waves' sums of a block, added in double: at the size of a whole group's sum each of these additions would cost half an ulp of it
-template <int BT> __device__ __forceinline__ double gn_block_sum(float v) {
-    __shared__ float red[BT / WAVE];
-    v = wave_sum(v);
-    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = v;
+// the threads' sums of a block, added in double: at the size of a whole group's sum each of these additions would cost half an ulp of it.
+// `red` is the call's own: a second call may write while a wave still reads for the first
+template <int BT> __device__ __forceinline__ double gn_block_sum(float v, double (&red)[BT / WAVE]) {
+    const double sum = wave_sum((double)v);
+    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = sum;
     __syncthreads();
-    double t = (double)red[0];
-#pragma unroll
-    for (int w = 1; w < BT / WAVE; w++) t += (double)red[w];
-    return t;
+    constexpr int N = BT / WAVE;                             // 4, 8 or 16 sums, repeated over the lanes: the same butterfly in every wave
+    double t = red[threadIdx.x & (N - 1)];
+    if constexpr (N == 16) t = wave_step_sum<8>(t);
+    if constexpr (N >= 8) t = wave_step_sum<4>(t);
+    t = wave_step_sum<2>(t);
+    return wave_step_sum<1>(t);
 }
 
 // 1 / sqrt(m2 / n + eps) to about half an ulp in f32 arithmetic: what the quotient and the sum lost to rounding (n is exact: a group
@@ -1778,9 +1780,9 @@ __device__ __forceinline__ float gn_rstd(double m2d, float n, float eps) {
 // vectors.  The repeated reads of a group hit the L2 of the XCD its blocks share (see launch_gn_reg).
 template <typename T, int NV, int BT, int WPE, bool SPAN>
 __global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x, const T* __restrict__ scale, const T* __restrict__ bias,
-                                                         T* __restrict__ y, uint32_t glen, uint32_t cpg, uint32_t groups, FastDiv L, float eps,
-                                                         uint32_t slices, uint32_t per_xcd) {
-    constexpr int VE = 16 / sizeof(T);
+                                                         T* __restrict__ y, uint32_t glen, double inv_n, uint32_t cpg, uint32_t groups, FastDiv L,
+                                                         float eps, uint32_t slices, uint32_t per_xcd) {
+    constexpr int VE = 16 / sizeof(T);                       // inv_n: 1 / glen
     // blocks are handed to the 8 XCDs round robin: pair index p runs over the (group, slice) pairs of one XCD first
     const uint32_t p = per_xcd ? (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
     const uint32_t grp = p / slices, slice = p - grp * slices, g = grp % groups;
@@ -1811,7 +1813,10 @@ __global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x
             for (int q = 0; q < VE; q++) acc = gn_plus<T>(v[k].e[q], acc);       // vectors past the group hold zeros
         }
     }
-    const float mean = row_sum<BT>(acc) / (float)glen;
+    // joined and divided in f32 the mean would be off by some ulps, which all outputs of the group share: f32 [8,320,4097] of
+    // mean 100 and deviation 1 was 5.6e-6 from 64 bits, is now 2.2e-6 (the launches for larger groups: 2.5e-6)
+    __shared__ double red[2][BT / WAVE];
+    const float mean = (float)(gn_block_sum<BT>(acc, red[0]) * inv_n);
     // the group stays in registers as it was loaded: the widened values of one pass must not be kept for the next, but with few
     // blocks of few vectors, which run alone on their CU and where keeping what fits saves instructions (32 groups of 93 KiB f16
     // 6.0 us, 6.8 when every pass widens again)
@@ -1834,7 +1839,7 @@ __global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x
             for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
         }
     }
-    const float rstd = gn_rstd(gn_block_sum<BT>(m2), (float)glen, eps);
+    const float rstd = gn_rstd(gn_block_sum<BT>(m2, red[1]), (float)glen, eps);
     if (!KEEP) forget();
     const uint32_t lo = (uint32_t)(((uint64_t)nvec * slice) / slices), hi = (uint32_t)(((uint64_t)nvec * (slice + 1)) / slices);
 #pragma unroll
@@ -1901,7 +1906,7 @@ int launch_gn_reg(rt_device* dev, const void* x, const void* scale, const void* 
     // puts the slices of a group on one XCD (all of them when bg is a multiple of 8)
     const uint32_t blocks = bg * slices, per_xcd = (slices > 1 && blocks % 8 == 0) ? blocks / 8 : 0;
     hipLaunchKernelGGL((gn_reg_kernel<T, NV, BT, WPE, SPAN>), dim3(blocks), dim3(BT), 0, dev->stream, (const T*)x, (const T*)scale, (const T*)bias,
-                       (T*)y, glen, cpg, groups, make_fastdiv(L), eps, slices, per_xcd);
+                       (T*)y, glen, 1.0 / (double)glen, cpg, groups, make_fastdiv(L), eps, slices, per_xcd);
     RT_CHECK_LAUNCH("gn_reg_kernel");
     return RT_OK;
 }

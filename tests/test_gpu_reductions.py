@@ -814,6 +814,25 @@ def test_group_norm_at_the_edges_of_the_block_shapes(dev, oracle, glen, B, dtype
             assert bad == 0, (C, L, bad, mx)
 
 
+@pytest.mark.parametrize("B,C,L,G", [(8, 320, 4097, 32),       # 256 ragged groups of 160 KiB, one block each
+                                     (8, 320, 4096, 32),       # the same on vector boundaries
+                                     (16, 512, 4096, 32),      # 512 groups of 256 KiB, 16 vectors a thread
+                                     (1, 512, 3000, 32),       # 32 groups, eight blocks each
+                                     (130, 8, 513, 4)])        # 520 ragged groups of 4 KiB, 256 threads each
+@pytest.mark.parametrize("m", [10.0, 100.0, -1000.0])
+def test_group_norm_of_inputs_far_from_zero(dev, B, C, L, G, m):
+    """f32 groups of mean m and deviation 1, against 64 bits.  The kernel holds the mean in f32, so all outputs of a group share an
+    error of up to half an ulp of m, over the group's deviation; the up to 64 values that a thread adds in f32 may cost half as much
+    again (restated on the host: 0.44 of it at most).  The subtraction is exact, 1 / deviation and the product round: an ulp of y, |y| < 8."""
+    rng = np.random.default_rng(325)
+    x = (rng.standard_normal((B, C, L)) + m).astype(np.float32)
+    groups = x.reshape(B * G, -1).astype(np.float64)
+    want = ((groups - groups.mean(1, keepdims=True)) / np.sqrt(groups.var(1, keepdims=True) + 1e-5)).reshape(x.shape)
+    got = dev.group_norm(dev.upload(x), G, None, None, 1e-5).to_numpy()
+    bound = 1.5 * (np.spacing(np.float32(abs(m))) / 2) / groups.std(1).min() + np.spacing(np.float32(4.0))
+    assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+
+
 def test_group_norm_many_groups_too_large_for_lds(dev, oracle):
     """288 groups of 160 KB in f32 (more pairs than CUs): one block per group with the
     group in registers, two rounds of blocks; against the oracle"""
