@@ -1750,17 +1750,12 @@ template <int BT> __device__ __forceinline__ double gn_block_sum(float v, double
     return wave_step_sum<1>(t);
 }
 
-// 1 / sqrt(m2 / n + eps) to about half an ulp in f32 arithmetic: what the quotient and the sum lost to rounding (n is exact: a group
-// in registers has fewer than 2^24 elements) and what the reciprocal root is off by go into one correction.  The launches for larger
-// groups compute this in double; with the double sum above, every group held in registers is at least as close to 64 bits as they are
-// (f32 [8,320,4097] 5.1e-8, 7.0e-8 without the two, 5.7e-8 by the launches; they cost 0.1 us of a small launch and 0.5 of the [16,512,3000]).  Where the correction means nothing (a variance of 0, inf or NaN) it is left out.
-__device__ __forceinline__ float gn_rstd(double m2d, float n, float eps) {
-    const float m2 = (float)m2d, q = m2 / n, v = q + eps, r = 1.0f / __builtin_sqrtf(v);
-    const float part = v - q;
-    const float lost = ((q - (v - part)) + (eps - part)) + (__builtin_fmaf(-q, n, m2) + (float)(m2d - (double)m2)) / n;
-    const float p = v * r;
-    const float e = (__builtin_fmaf(-p, r, 1.0f) - __builtin_fmaf(v, r, -p) * r) - lost * r * r;
-    return __builtin_fabsf(e) < 0.5f ? __builtin_fmaf(0.5f * r, e, r) : r;
+// 1 / sqrt(v) in double, as the launches for larger groups compute it: the total of the squares of a group, its quotient and a variance
+// below f32's normal range stay representable (f32 [8,320,4097] of deviation 1.2e17 has a total of 5.8e38, which is inf in f32).  The
+// instruction's estimate is good to about 2^-23, one step makes that 2^-45; where the step means nothing (v of 0 or inf) it is left out.
+__device__ __forceinline__ float gn_rstd(double v) {
+    const double r = __builtin_amdgcn_rsq(v), e = __builtin_fma(-v * r, r, 1.0);
+    return (float)(__builtin_fabs(e) < 0.5 ? __builtin_fma(0.5 * r, e, r) : r);
 }
 
 // GroupNorm in one launch: the group in the registers of one block (thread t of BT holds vectors t, t + BT, ...; NV of them), so
@@ -1839,7 +1834,7 @@ __global__ void __launch_bounds__(BT, WPE) gn_reg_kernel(const T* __restrict__ x
             for (int q = 0; q < VE; q++) m2 = gn_dev2<T>(v[k].e[q], mean, m2);
         }
     }
-    const float rstd = gn_rstd(gn_block_sum<BT>(m2, red[1]), (float)glen, eps);
+    const float rstd = gn_rstd(gn_block_sum<BT>(m2, red[1]) * inv_n + (double)eps);
     if (!KEEP) forget();
     const uint32_t lo = (uint32_t)(((uint64_t)nvec * slice) / slices), hi = (uint32_t)(((uint64_t)nvec * (slice + 1)) / slices);
 #pragma unroll

@@ -823,14 +823,40 @@ def test_group_norm_at_the_edges_of_the_block_shapes(dev, oracle, glen, B, dtype
 def test_group_norm_of_inputs_far_from_zero(dev, B, C, L, G, m):
     """f32 groups of mean m and deviation 1, against 64 bits.  The kernel holds the mean in f32, so all outputs of a group share an
     error of up to half an ulp of m, over the group's deviation; the up to 64 values that a thread adds in f32 may cost half as much
-    again (restated on the host: 0.44 of it at most).  The subtraction is exact, 1 / deviation and the product round: an ulp of y, |y| < 8."""
+    again (restated on the host: 0.44 of it at most).  The subtraction is exact; 1 / deviation and the product round by up to 2^-24 of the output each."""
     rng = np.random.default_rng(325)
     x = (rng.standard_normal((B, C, L)) + m).astype(np.float32)
     groups = x.reshape(B * G, -1).astype(np.float64)
     want = ((groups - groups.mean(1, keepdims=True)) / np.sqrt(groups.var(1, keepdims=True) + 1e-5)).reshape(x.shape)
     got = dev.group_norm(dev.upload(x), G, None, None, 1e-5).to_numpy()
-    bound = 1.5 * (np.spacing(np.float32(abs(m))) / 2) / groups.std(1).min() + np.spacing(np.float32(4.0))
+    bound = 1.5 * (np.spacing(np.float32(abs(m))) / 2) / groups.std(1).min() + 2 * 2.0 ** -24 * np.abs(want).max()
     assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+
+
+@pytest.mark.parametrize("B,C,L,G", [(8, 320, 4097, 32), (8, 320, 4096, 32), (16, 512, 4096, 32), (1, 512, 3000, 32), (130, 8, 513, 4)])
+@pytest.mark.parametrize("deviation", [1.2e17, 1e-20])
+def test_group_norm_of_squares_outside_f32(dev, B, C, L, G, deviation):
+    """f32 groups whose squares have a total beyond f32 while every thread's part of it is inside ([8,320,4097]: 5.8e38), and groups
+    whose variance is subnormal in f32 (1e-40), against 64 bits.  The subtraction, 1 / deviation and the product round by up to 2^-24 of
+    the output each.  A subnormal square is off by up to 0.7e-45, 0.7e-5 of 1e-40, either way: over the 1026 and more of a group
+    that leaves 2e-7 of the variance, times an output below 8 and halved by the root."""
+    x = (np.random.default_rng(326).standard_normal((B, C, L)) * deviation).astype(np.float32)
+    groups = x.reshape(B * G, -1).astype(np.float64)
+    want = ((groups - groups.mean(1, keepdims=True)) / groups.std(1, keepdims=True)).reshape(x.shape)
+    got = dev.group_norm(dev.upload(x), G, None, None, 0.0).to_numpy()
+    bound = 3 * 2.0 ** -24 * np.abs(want).max() + (8e-7 if deviation < 1 else 0)
+    assert np.abs(got - want).max() <= bound, (np.abs(got - want).max(), bound)
+
+
+@pytest.mark.parametrize("B,L", [(1, 5000), (33, 5000)])              # several blocks per group; one
+def test_group_norm_without_a_variance(dev, B, L):
+    """constant groups give 0 with an eps and NaN without (0 * inf), a group with an infinity gives NaN, its neighbours numbers"""
+    x = np.full((B, 8, L), 3.0, np.float32)
+    assert np.all(dev.group_norm(dev.upload(x), 4, None, None, 1e-5).to_numpy() == 0)
+    assert np.all(np.isnan(dev.group_norm(dev.upload(x), 4, None, None, 0.0).to_numpy()))
+    x[0, 2, 7] = np.inf
+    got = dev.group_norm(dev.upload(x), 4, None, None, 1e-5).to_numpy()
+    assert np.all(np.isnan(got[0, 2:4])) and np.all(got[0, :2] == 0) and np.all(got[0, 4:] == 0) and np.all(got[1:] == 0)
 
 
 def test_group_norm_many_groups_too_large_for_lds(dev, oracle):
