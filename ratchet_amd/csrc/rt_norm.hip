@@ -1945,7 +1945,9 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
     // Which path (measured on 256 CUs, us against the launches below or the next kernel that would hold the group):
     //   at most half as many groups as CUs, up to 144 KiB (192 in f32): 1024 threads, cus / groups blocks per group (32 groups of
     //        93 KiB f16 5.8, 6.9 by launches; ragged [2,320,3001] f16 7.9 / 10.7).  Larger ones in 16 bits go to the launches (64 groups
-    //        of 160 KiB f16 13.3 / 9.6)
+    //        of 160 KiB f16 13.3 / 9.6).  In place only one block a group may work (the others would load what it has stored), the launches
+    //        keep the chip: theirs are long groups, up to a quarter as many as CUs (f16, one block / launches: 94 KiB x 32 groups 7.5 / 6.2,
+    //        x 64 8.0 / 7.8, x 80 8.3 / 8.4, 144 KiB x 8 9.1 / 5.7; 50 KiB x 8 5.5 / 5.4, x 64 5.9 / 6.4; f32 120 KiB x 8 6.5 / 5.6)
     //   more groups: one block per group, as many threads as leave two blocks or more to a CU.  Up to 12, 24 and 48 KiB: 256, 512,
     //        512 threads of at most 3, 3, 6 vectors (8 KiB x 512 groups 5.0, 5.5 - 6.1 with wider blocks; 47 KiB x 2048 33.8, 35.7
     //        with 1024 threads); up to 96 KiB: 1024 threads of 4 or 6 (94 KiB x 256 groups 9.9, 11.5 with 512 threads of 12); up to
@@ -1959,7 +1961,8 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
 #define RT_GN_REG(NVC, BTC, WPEC)                                                                                                    \
     return vec ? launch_gn_reg<T, NVC, BTC, WPEC, false>(dev, x, scale, bias, y, bg, glen, cpg, groups, L, eps, slices)          \
                : launch_gn_reg<T, NVC, BTC, WPEC, true>(dev, x, scale, bias, y, bg, glen, cpg, groups, L, eps, slices)
-    if (aligned && 2u * bg <= cus && nvec <= (sizeof(T) == 4 ? 12288u : 9216u)) {
+    const bool spread_in_place = x == y && 4u * bg <= cus && glen > 26624 + 96 * bg;
+    if (aligned && 2u * bg <= cus && nvec <= (sizeof(T) == 4 ? 12288u : 9216u) && !spread_in_place) {
         uint32_t slices = x == y ? 1 : cus / bg;                        // in place, a block must not store what another still loads
         if (slices > 32) slices = 32;
         if (slices > nvec) slices = nvec;

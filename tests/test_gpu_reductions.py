@@ -859,6 +859,19 @@ def test_group_norm_without_a_variance(dev, B, L):
     assert np.all(np.isnan(got[0, 2:4])) and np.all(got[0, :2] == 0) and np.all(got[0, 4:] == 0) and np.all(got[1:] == 0)
 
 
+@pytest.mark.parametrize("bg,glen", [(1, 26720), (1, 26728), (64, 32768), (64, 32776), (65, 32776),     # either side of the line between one block a group and the launches
+                                     (64, 32777), (8, 73728)])                                          # ragged; 144 KiB in f16
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_group_norm_in_place_with_few_groups(dev, oracle, bg, glen, dtype):
+    """a block stores nothing that another block still has to load; tolerances of test_group_norm"""
+    rng = np.random.default_rng(glen)
+    tol = 1e-5 if dtype == np.float32 else 1e-3
+    x, w, b = randn(rng, (1, bg, glen), dtype), randn(rng, bg, dtype), randn(rng, bg, dtype)
+    dx = dev.upload(x)
+    bad, mx = oracle.count_not_close(dev.group_norm(dx, bg, dev.upload(w), dev.upload(b), 1e-5, out=dx).to_numpy(), oracle.group_norm(x, bg, w, b, 1e-5), tol, tol)
+    assert bad == 0, (bad, mx)
+
+
 def test_group_norm_many_groups_too_large_for_lds(dev, oracle):
     """288 groups of 160 KB in f32 (more pairs than CUs): one block per group with the
     group in registers, two rounds of blocks; against the oracle"""
