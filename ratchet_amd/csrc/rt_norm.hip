@@ -1951,8 +1951,14 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
     //   more groups: one block per group, as many threads as leave two blocks or more to a CU.  Up to 12, 24 and 48 KiB: 256, 512,
     //        512 threads of at most 3, 3, 6 vectors (8 KiB x 512 groups 5.0, 5.5 - 6.1 with wider blocks; 47 KiB x 2048 33.8, 35.7
     //        with 1024 threads); up to 96 KiB: 1024 threads of 4 or 6 (94 KiB x 256 groups 9.9, 11.5 with 512 threads of 12); up to
-    //        128 KiB 512 threads of 16, which leave room for a second block where 1024 of 8 spill (125 KiB f32 x 512 21.2 / 26.6); up
-    //        to 192 KiB 1024 threads of 9 or 12, one block to a CU (141 KiB f16 x 512 31.7, 39.4 by launches; 188 KiB f16 x 512 39.5 / 46.8)
+    //        128 KiB 512 threads of 16, which leave room for a second block where 1024 of 8 spill (125 KiB f32 x 512 21.2 / 26.6), but in
+    //        16 bits only where there is a second block: up to one group a CU 1024 threads of 9 convert faster (127 KiB f16 x 129
+    //        10.4 / 15.9, x 256 13.2 / 17.4; f32 x 256 12.6 / 12.3); up to 192 KiB 1024 threads of 9 or 12, one block to a CU
+    //        (141 KiB f16 x 512 31.7, 39.4 by launches; 188 KiB f16 x 512 39.5 / 46.8).  16-bit groups of 12 vectors a thread are bound by
+    //        their conversions, so a last round that is nearly empty costs what a full one does, and the launches take those: fewer than
+    //        9/16 of the CUs in the first round, 5/8 of all rounds later (f16, one block / launches: 190 KiB x 129 17.5 / 14.0, x 160
+    //        18.1 / 16.7, 148 KiB x 129 13.3 / 13.0, x 160 13.0 / 13.2; 148 KiB x 257 28.6 / 21.0, x 300 29.8 / 25.5, x 341 30.3 / 27.7, 190
+    //        KiB x 300 35.1 / 32.4, x 341 35.9 / 37.0; bf16 148 KiB x 144 11.7 / 11.8).  Ragged ones never do (the launches go by element)
     //   f32 groups of 192 to 256 KiB (16 vectors a thread; 20 and 24 spill), at least as many groups as CUs: 250 KiB x 512 43.6, 61.9
     //        by launches; 256 KiB x 128: 16.5 / 16.4.  In 16 bits such groups go to the launches (x 512 64.2, 65.8 with 16 vectors)
     //   everything else: the launches below
@@ -1980,9 +1986,10 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
         if (nvec <= 3072) RT_GN_REG(6, 512, 8);
         if (nvec <= 4096) RT_GN_REG(4, 1024, 8);
         if (nvec <= 6144) RT_GN_REG(6, 1024, 8);
-        if (nvec <= 8192) RT_GN_REG(16, 512, 4);
+        if (nvec <= 8192 && (sizeof(T) == 4 || bg > cus)) RT_GN_REG(16, 512, 4);
         if (nvec <= 9216) RT_GN_REG(9, 1024, 4);
-        if (nvec <= 12288) RT_GN_REG(12, 1024, 4);
+        const uint64_t rounds = ((uint64_t)bg + cus - 1) / cus, enough = rounds == 1 ? cus * 9 / 16 : rounds * cus * 5 / 8;
+        if (nvec <= 12288 && (sizeof(T) == 4 || !vec || bg >= enough)) RT_GN_REG(12, 1024, 4);
         if (sizeof(T) == 4 && nvec <= 16384 && bg >= cus) RT_GN_REG(16, 1024, 4);
     }
 #undef RT_GN_REG

@@ -872,6 +872,16 @@ def test_group_norm_in_place_with_few_groups(dev, oracle, bg, glen, dtype):
     assert bad == 0, (bad, mx)
 
 
+@pytest.mark.parametrize("bg,glen", [(143, 73736), (144, 73736), (319, 98304), (320, 98304), (319, 98301),     # one block a group from 144 and from 320 groups on; ragged always
+                                     (256, 49160), (257, 49160), (256, 65536), (257, 65536)])               # 1024 threads of 9 vectors up to a group a CU, then 512 of 16
+def test_group_norm_16_bit_groups_by_rounds(dev, oracle, bg, glen):
+    """both sides of the lines by the number of groups; the tolerance of test_group_norm"""
+    rng = np.random.default_rng(glen)
+    x, w, b = randn(rng, (1, bg, glen), np.float16), randn(rng, bg, np.float16), randn(rng, bg, np.float16)
+    bad, mx = oracle.count_not_close(dev.group_norm(dev.upload(x), bg, dev.upload(w), dev.upload(b), 1e-5).to_numpy(), oracle.group_norm(x, bg, w, b, 1e-5), 1e-3, 1e-3)
+    assert bad == 0, (bad, mx)
+
+
 def test_group_norm_many_groups_too_large_for_lds(dev, oracle):
     """288 groups of 160 KB in f32 (more pairs than CUs): one block per group with the
     group in registers, two rounds of blocks; against the oracle"""
