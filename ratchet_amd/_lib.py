@@ -114,14 +114,16 @@ def check(status):
         raise RatchetError(status, load().rt_last_error().decode("utf-8", "replace"))
 
 
-@functools.lru_cache(maxsize=4096)
-def _shape4(shape):
+def shape4(shape):
+    """Shape::promote(shape, 4): left-pad with 1s (crates/ratchet-core/src/shape.rs:92-96)."""
+    shape = [int(s) for s in shape]
     if len(shape) > 4:
         raise ValueError("rank > 4 is not supported")
-    return (ctypes.c_uint32 * 4)(*([1] * (4 - len(shape)) + [int(s) for s in shape]))
+    return (ctypes.c_uint32 * 4)(*([1] * (4 - len(shape)) + shape))
 
 
-def shape4(shape):
-    """Shape::promote(shape, 4): left-pad with 1s (crates/ratchet-core/src/shape.rs:92-96).  The array is shared by all calls of a
-    shape and belongs to nobody: the library only reads it (0.1 us a call, 0.7 when it is built each time; a decode step makes eight)."""
-    return _shape4(tuple(shape))
+@functools.lru_cache(maxsize=4096)
+def buffer_shape4(shape):
+    """shape4 of a buffer's own shape or of another tuple of ints.  The array is shared by all calls of a shape and belongs to nobody: the
+    library only reads it (0.1 us a call, 0.7 when it is built each time; a decode step makes eight)."""
+    return shape4(shape)

@@ -11,7 +11,7 @@ import ctypes
 import numpy as np
 
 from . import _lib
-from ._lib import RatchetError, check, shape4  # noqa: F401
+from ._lib import RatchetError, buffer_shape4, check, shape4  # noqa: F401
 
 _NP_TO_DT = {np.dtype(np.float32): _lib.F32, np.dtype(np.float16): _lib.F16, np.dtype(np.int32): _lib.I32,
              np.dtype(np.uint32): _lib.U32}
@@ -225,8 +225,8 @@ class Device:
             return out
         shape = tuple(np.broadcast_shapes(a.shape, b.shape))
         out = out or Buffer(self, shape, a.dt)
-        check(self.lib.rt_binary_bcast(self.handle, op, a.dt, a.ptr, shape4(a.shape), b.ptr, shape4(b.shape), out.ptr,
-                                       shape4(shape)))
+        check(self.lib.rt_binary_bcast(self.handle, op, a.dt, a.ptr, buffer_shape4(a.shape), b.ptr, buffer_shape4(b.shape), out.ptr,
+                                       buffer_shape4(shape)))
         return out
 
     def unary(self, op, x, out=None):
@@ -246,7 +246,7 @@ class Device:
         perm = (ctypes.c_uint32 * 4)(*(list(range(pad)) + [d + pad for d in dims]))   # Permute::promote
         out_shape = [x.shape[d] for d in dims]
         out = out or Buffer(self, out_shape, x.dt)
-        check(self.lib.rt_permute(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, shape4(x.shape), perm))
+        check(self.lib.rt_permute(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, buffer_shape4(x.shape), perm))
         return out
 
     def slice(self, x, ranges, out=None):
@@ -254,13 +254,13 @@ class Device:
         dst = [int(r[1]) - int(r[0]) for r in ranges]
         out = out or Buffer(self, dst, x.dt)
         pad = 4 - len(start)
-        check(self.lib.rt_slice(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, shape4(x.shape),
-                                (ctypes.c_uint32 * 4)(*([0] * pad + start)), shape4(dst)))
+        check(self.lib.rt_slice(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, buffer_shape4(x.shape),
+                                (ctypes.c_uint32 * 4)(*([0] * pad + start)), buffer_shape4(tuple(dst))))
         return out
 
     def broadcast_to(self, x, shape, out=None):
         out = out or Buffer(self, shape, x.dt)
-        check(self.lib.rt_broadcast(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, shape4(x.shape), shape4(shape)))
+        check(self.lib.rt_broadcast(self.handle, _DT_BYTES[x.dt], x.ptr, out.ptr, buffer_shape4(x.shape), buffer_shape4(tuple(map(int, shape)))))
         return out
 
     def concat(self, xs, dim, out=None):
@@ -269,7 +269,7 @@ class Device:
         out_shape[dim] = sum(x.shape[dim] for x in xs)
         out = out or Buffer(self, out_shape, xs[0].dt)
         ptrs = (ctypes.c_void_p * len(xs))(*[x.ptr.value for x in xs])
-        shapes = ((ctypes.c_uint32 * 4) * len(xs))(*[shape4(x.shape) for x in xs])
+        shapes = ((ctypes.c_uint32 * 4) * len(xs))(*[buffer_shape4(x.shape) for x in xs])
         check(self.lib.rt_concat(self.handle, _DT_BYTES[xs[0].dt], len(xs), ptrs, shapes, dim + (4 - rank), out.ptr))
         return out
 
@@ -279,7 +279,7 @@ class Device:
         out_shape = list(cache.shape)
         out_shape[dim] = offset + source.shape[dim]
         out = out or Buffer(self, out_shape, cache.dt)
-        check(self.lib.rt_cache(self.handle, _DT_BYTES[cache.dt], cache.ptr, shape4(cache.shape), source.ptr, shape4(source.shape),
+        check(self.lib.rt_cache(self.handle, _DT_BYTES[cache.dt], cache.ptr, buffer_shape4(cache.shape), source.ptr, buffer_shape4(source.shape),
                                 dim + (4 - rank), offset, out.ptr))
         return out
 
@@ -289,7 +289,7 @@ class Device:
         out_shape = list(src.shape)
         out_shape[dim] = indices.numel
         out = out or Buffer(self, out_shape, src.dt)
-        check(self.lib.rt_index_select(self.handle, _DT_BYTES[src.dt], src.ptr, shape4(src.shape), indices.ptr, indices.numel,
+        check(self.lib.rt_index_select(self.handle, _DT_BYTES[src.dt], src.ptr, buffer_shape4(src.shape), indices.ptr, indices.numel,
                                        dim + (4 - rank), out.ptr))
         return out
 
@@ -300,21 +300,21 @@ class Device:
         out_shape = list(src_shape)
         out_shape[dim] = indices.numel
         out = out or Buffer(self, out_shape, scales.dt)
-        check(self.lib.rt_index_select_q8_0(self.handle, scales.dt, packed.ptr, scales.ptr, shape4(src_shape), indices.ptr, indices.numel,
+        check(self.lib.rt_index_select_q8_0(self.handle, scales.dt, packed.ptr, scales.ptr, buffer_shape4(tuple(map(int, src_shape))), indices.ptr, indices.numel,
                                             dim + (4 - rank), out.ptr))
         return out
 
     def index_write(self, dst, src, write_start):
         """dst is modified in place and returned."""
         pad = 4 - len(dst.shape)
-        check(self.lib.rt_index_write(self.handle, _DT_BYTES[dst.dt], dst.ptr, shape4(dst.shape), src.ptr, src.numel,
+        check(self.lib.rt_index_write(self.handle, _DT_BYTES[dst.dt], dst.ptr, buffer_shape4(dst.shape), src.ptr, src.numel,
                                       (ctypes.c_uint32 * 4)(*([0] * pad + [int(w) for w in write_start]))))
         return dst
 
     def rope(self, x, dim, base, offset, out=None):
         """x [B, H, S, D]; out may be x."""
         out = out or Buffer(self, x.shape, x.dt)
-        check(self.lib.rt_rope(self.handle, x.dt, x.ptr, out.ptr, shape4(x.shape), dim, base, offset))
+        check(self.lib.rt_rope(self.handle, x.dt, x.ptr, out.ptr, buffer_shape4(x.shape), dim, base, offset))
         return out
 
     def softmax(self, x, out=None, mode=_lib.SOFTMAX_REFERENCE):
@@ -326,7 +326,7 @@ class Device:
     def softmax_masked(self, x, mask, out=None, mode=_lib.SOFTMAX_REFERENCE):
         """softmax over the last dim of x + mask (mask broadcast over x's leading dims), in x's own arithmetic."""
         out = out or Buffer(self, x.shape, x.dt)
-        check(self.lib.rt_softmax_masked(self.handle, x.dt, x.ptr, shape4(x.shape), mask.ptr, shape4(mask.shape), out.ptr, mode))
+        check(self.lib.rt_softmax_masked(self.handle, x.dt, x.ptr, buffer_shape4(x.shape), mask.ptr, buffer_shape4(mask.shape), out.ptr, mode))
         return out
 
     def layer_norm(self, x, scale, bias, eps=1e-5, out=None):
@@ -354,8 +354,8 @@ class Device:
     def softmax_via_f32(self, x, mask=None, out=None, mode=_lib.SOFTMAX_REFERENCE):
         """softmax over the last dim of (x + mask) with the mask broadcast over x's leading dims."""
         out = out or Buffer(self, x.shape, x.dt)
-        check(self.lib.rt_softmax_via_f32(self.handle, x.dt, x.ptr, shape4(x.shape), mask.ptr if mask is not None else None,
-                                          shape4(mask.shape) if mask is not None else None, out.ptr, mode))
+        check(self.lib.rt_softmax_via_f32(self.handle, x.dt, x.ptr, buffer_shape4(x.shape), mask.ptr if mask is not None else None,
+                                          buffer_shape4(mask.shape) if mask is not None else None, out.ptr, mode))
         return out
 
     def unary_via_f32(self, op, x, out=None):

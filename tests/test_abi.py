@@ -9,7 +9,9 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
+import torch
 
 from ratchet_amd import _lib
 
@@ -265,3 +267,16 @@ def test_python_binding_fails_loudly_without_library(tmp_path, monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "missing.so"))
     with pytest.raises(ImportError):
         _lib.load()
+
+
+def test_shape4_takes_extents_by_value():
+    """numbers of any kind, the value that each has now; the array is the caller's"""
+    from ratchet_amd.runtime import shape4
+    n = torch.tensor(3)
+    assert list(shape4((n, 5))) == [1, 1, 3, 5]
+    n.fill_(7)
+    assert list(shape4((n, 5))) == [1, 1, 7, 5]
+    assert list(shape4([np.array(2), np.int64(4), "6"])) == [1, 2, 4, 6]
+    first = shape4((8, 9))
+    first[3] = 1
+    assert list(shape4((8, 9))) == [1, 1, 8, 9]
