@@ -57,8 +57,8 @@ typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // exp of a 16-bit pattern, the low or the high half of a word: one lookup in the full 65536-entry table (NaN, inf and the saturated
-// ends included), which lies at the start of LDS: the address is one shift of the selected half (as C the compiler spends two
-// instructions on it)
+// ends included), which lies at the start of LDS (sp_allow_lds checks that): the address is one shift of the selected half (as C the
+// compiler spends two instructions on it)
 __device__ __forceinline__ uint32_t sp_exp_lo(uint32_t p) {
     asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(p) : "v"(1u), "v"(p));
     return *(const __attribute__((address_space(3))) uint16_t*)p;
@@ -67,7 +67,6 @@ __device__ __forceinline__ uint32_t sp_exp_hi(uint32_t p) {
     asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(p) : "v"(1u), "v"(p));
     return *(const __attribute__((address_space(3))) uint16_t*)p;
 }
-__device__ __forceinline__ uint32_t sp_exp_pair(uint32_t p) { return sp_exp_lo(p) | sp_exp_hi(p) << 16; }
 
 // Which 30-row groups a block works on.  Rows come in `reps` periods of P rows (P = all rows when nothing repeats; P = the
 // rows one mask covers when a mask is added, e.g. S rows per head for an [S, T] mask under B * H heads); a period holds
@@ -694,6 +693,16 @@ __global__ void __launch_bounds__(BLOCK) mask_tiles_kernel(const T* __restrict__
     }
 }
 
+// Before an instantiation's first launch on a device: its dynamic LDS, and the check that this starts at address 0, where the lookups
+// expect the table (see sp_exp_lo).  Static LDS of a function that is compiled into the kernel would lie in front of it.
+inline int sp_allow_lds(const void* kernel) {
+    hipFuncAttributes a;
+    RT_HIP(hipFuncGetAttributes(&a, kernel));
+    RT_REQUIRE(a.sharedSizeBytes == 0, RT_ERR_SIZE, "softmax16_stream_kernel: %zu bytes of static LDS lie in front of its table", a.sharedSizeBytes);
+    RT_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));
+    return RT_OK;
+}
+
 // mask == nullptr: plain softmax.  Otherwise the mask has `period` rows of `cols` columns and repeats every `period`
 // rows of x (rows % period == 0).  Returns RT_OK with *done = false when the shape does not fit this kernel.
 template <typename T>
@@ -735,8 +744,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     do {                                                                                                                             \
         const uint64_t bit = 1ull << (TI * 32 + (NS == 0 ? 4 : NS == 1 ? 0 : NS == 2 ? 1 : NS == 4 ? 2 : NS == 6 ? 5 : NS == 3 ? 6 : NS == 5 ? 7 : 3) * 4 + (F ? 2 : 0) + (M ? 1 : 0)); \
         if (!(dev->sp_attr_set & bit)) {               /* the LDS opt-in is per function and per device */                           \
-            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, M>),                          \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
+            if (int rc = sp_allow_lds(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, M>))) return rc;               \
             dev->sp_attr_set |= bit;                                                                                                 \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, M>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES, dev->stream, table,  \
@@ -746,8 +754,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     do {                                                                                                                             \
         const uint32_t bit = 1u << (TI * 8 + (NS / 2 - 1) * 2 + (F ? 1 : 0));                                                        \
         if (!(dev->sp_pair_attr_set & bit)) {                                                                                        \
-            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, 2>),                          \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
+            if (int rc = sp_allow_lds(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, 2>))) return rc;               \
             dev->sp_pair_attr_set |= bit;                                                                                            \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, 2>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES, dev->stream, table,  \
@@ -764,8 +771,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     do {                                                                                                                             \
         const uint32_t bit = 1u << (16 + (NS == 5 ? 0 : NS == 6 ? 4 : 8) + (F ? 2 : 0) + (M ? 1 : 0));                               \
         if (!(dev->sp_pair_attr_set & bit)) {                                                                                        \
-            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, M, false, true>),             \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
+            if (int rc = sp_allow_lds(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, F, M, false, true>))) return rc;  \
             dev->sp_pair_attr_set |= bit;                                                                                            \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, F, M, false, true>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES,         \
@@ -782,8 +788,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
     do {                                                                                                                             \
         const uint64_t bit = 1ull << (M * 16 + TI * 8 + (NS == 8 ? 7 : NS));                                                         \
         if (!(dev->sp_ragged_attr_set & bit)) {                                                                                      \
-            RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, false, M, true>),                \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));                             \
+            if (int rc = sp_allow_lds(reinterpret_cast<const void*>(softmax16_stream_kernel<T, NS, false, M, true>))) return rc;     \
             dev->sp_ragged_attr_set |= bit;                                                                                          \
         }                                                                                                                            \
         hipLaunchKernelGGL((softmax16_stream_kernel<T, NS, false, M, true>), dim3(blocks), dim3(SP_BLOCK), SP_SMEM_BYTES,            \
