@@ -877,23 +877,23 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         };
         sch.R = rows_per_group(pair ? SP_HALF : SP_ROWS);
         // f16 rows of 4097 to 8192 columns: in registers, 15 to a group (the LONG variant), or 30 to a group and parked in y?
-        // In registers x is read and y written once, and the walk is the bound: 1.87 us per 512 columns with its barriers, on
+        // In registers x is read and y written once, and the walk is the bound: 1.45 us per 512 columns with its barriers, on
         // half as many rows at a time and in steps of 1024 columns, of which 5, 6 or 8 are taken.  Parked, a round takes the
-        // longer of its steps and its four passes over memory (3/8 ns per column of a group's rows), and the last one's
-        // quotients follow.  So the registers win where the rows come to memory ([1,8,2048,8192] with a causal mask 200 us
-        // parked / 156 in registers, [1,8,2048,4608] 116 / 101) and where all rows are one round either way ([1,8,100,8192]
-        // 49 / 35), and lose where they take one round more or walk far past the row's end ([4096,4104] 39.5 / 44.7,
-        // [4096,6152] 54 / 67, [5000,6656] 57 / 67, [8000,6152] 87 / 96).  Over 800 sizes with inputs and outputs moving
-        // through 580 MB the pick costs 0.2 % on average against the better one of the two, and 8 % at most.
-        // The bf16 walk takes 5 ns an element; in registers it was slower without a mask and on short periods ([1,8,2048,8192]
-        // 243 parked / 264, rows of 1000-row periods with a mask 432 / 530) and faster with a mask of whole rounds
-        // ([1,8,2048,8192] 344 / 293): bf16 parks in y.
+        // longer of its steps and its four passes over memory (5/16 ns per column of a group's rows), and the last one's
+        // quotients follow.  So the registers win nearly everywhere ([1,8,2048,8192] with a causal mask 209 us parked / 142 in
+        // registers, [1,8,2048,4608] 123 / 88, [1,8,100,8192] 45 / 27, [4096,4104] 37.9 / 35.7, [8000,6152] 85 / 74) and lose where
+        // they take two rounds for one and walk far past the row's end ([3841,6152] 49.8 / 51.8, [1,2,2000,6152] with a mask 56.8 / 61.2).
+        // Over 346 sizes, 196 of them on either side of a round and with inputs and outputs moving through 600 MB, the pick costs
+        // 0.2 % on average against the better one of the two, and 11 % at most (4616 columns under 3900 rows of mask).
+        // The bf16 walk takes 5 ns an element; in registers it was slower where there are several rounds ([1,8,2048,8192] 199 parked / 244,
+        // [4096,4104] 50 / 67, [1,16,2048,4608] with a mask 247 / 290) and faster in one round and in some with a mask ([1,8,100,8192]
+        // 65 / 53, [1,8,2048,8192] with a mask 269 / 259): bf16 parks in y.
         bool longer = false;
         if (LONG_ROWS && !ragged && nt > SP_MAX_STEPS && nt <= 2 * SP_MAX_STEPS) {
             const uint32_t R = rows_per_group(SP_HALF);
-            const uint64_t in_registers = rounds_of(R) * long_steps * 3740;                                  // ns
-            const uint64_t memory = (uint64_t)sch.R * cols * 3 / 8, walk = (uint64_t)sch.nsteps * 2000;
-            longer = in_registers <= rounds_of(sch.R) * (memory > walk ? memory : walk) + (uint64_t)sch.nsteps * 400;
+            const uint64_t in_registers = rounds_of(R) * long_steps * 2900;                                  // ns
+            const uint64_t memory = (uint64_t)sch.R * cols * 5 / 16, walk = (uint64_t)sch.nsteps * 2300;
+            longer = in_registers <= rounds_of(sch.R) * (memory > walk ? memory : walk) + (uint64_t)sch.nsteps * 600;
             if (longer) sch.R = R;
         }
         const bool long_full = longer && cols == long_steps * 2 * SP_TC;

@@ -62,3 +62,18 @@ def test_ragged_rows_under_a_mask_shared_by_heads(dev, oracle, cols, kind):
     assert _same(dev.softmax_masked(dx, dm).to_numpy(), want, bf)
     dev.softmax_masked(dx, dm, out=dx)
     assert _same(dx.to_numpy(), want, bf)
+
+
+@pytest.mark.parametrize("heads,rows,cols", [(1, 3840, 6152), (1, 3841, 6152), (1, 4500, 6656),      # f16: one round in registers; two, so parked in y
+                                             (2, 1920, 6152), (2, 1930, 6152), (1, 3900, 4104)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_rows_of_4097_to_8192_columns_around_a_round(dev, oracle, heads, rows, cols, masked):
+    """both sides of the choice between registers and parking in y; also in place"""
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((1, heads, rows, cols), np.float32).astype(np.float16)
+    m = np.triu(np.full((rows, cols), -np.inf, np.float16), k=1 + cols - rows)
+    want = oracle.softmax(oracle.binary("add", x, np.ascontiguousarray(np.broadcast_to(m, x.shape))) if masked else x)
+    dx = dev.upload(x)
+    for out in (None, dx):
+        got = dev.softmax_masked(dx, dev.upload(m), out=out) if masked else dev.softmax(dx, out=out)
+        assert _same(got.to_numpy(), want, False)
