@@ -6,6 +6,9 @@
 #include "rt_arith.h"
 #include "rt_internal.h"
 #include "rt_pace.h"
+#define RT_FN __device__ __forceinline__
+#include "rt_softmax_div.h"
+#undef RT_FN
 
 namespace {
 
@@ -97,7 +100,8 @@ __device__ __forceinline__ void sp_item(const SpSched& s, uint32_t b, uint32_t G
     fd_divmod(b + it * G, s.gp_div, rep, pg);
 }
 
-// What differs between the two 16-bit types: the walker's running sum and how a packed pair is divided by the row sum.
+// What differs between the two 16-bit types: the walker's running sum and how a packed pair is divided by the row sum
+// (short_quotients, for sums in [Div::MIN, Div::MAX]; all pairs are compared with the division on the CPU).
 template <typename T> struct SpType;
 template <> struct SpType<half_t> {
     typedef half_t Run;
@@ -115,16 +119,10 @@ template <> struct SpType<half_t> {
     static __device__ __forceinline__ v4u add_vec(const v4u& a, const v4u& b) {    // eight f16 sums, rounded as the separate add does
         return __builtin_bit_cast(v4u, __builtin_bit_cast(h16x8, a) + __builtin_bit_cast(h16x8, b));
     }
-    // e / s for both halves of a word, s in [SHORT_MIN, SHORT_MAX]: e * rinv + e * rlow, where rinv + rlow is 1 / s to 48 bits, so
-    // the f32 quotient is off by one rounding.  Two 11-bit significands never divide to the middle between two f16 values and stay
-    // 2^-23 away from it, so f16 of that quotient is f16 of e / s (all pairs compared on the CPU; subnormal results too: their
-    // middles are exact f32 values).
-    static constexpr bool SHORT_TWO = true;
-    static constexpr float SHORT_MIN = 6.103515625e-05f, SHORT_MAX = 65504.0f;
+    typedef ShortDivF16 Div;
     static __device__ __forceinline__ uint32_t short_quotients(uint32_t e, float rinv, float rlow) {
         const h16x2 v = __builtin_bit_cast(h16x2, e);
-        float q0 = __builtin_fmaf((float)v[0], rinv, __builtin_fmaf((float)v[0], rlow, 0.0f));
-        float q1 = __builtin_fmaf((float)v[1], rinv, __builtin_fmaf((float)v[1], rlow, 0.0f));
+        float q0 = Div::quotient((float)v[0], rinv, rlow), q1 = Div::quotient((float)v[1], rinv, rlow);
         // keep the f32 quotient and its conversion apart: fused into v_fma_mixlo_f16 the pair rounds
         // subnormal f16 results differently from fma-then-convert
         asm volatile("" : "+v"(q0), "+v"(q1));
@@ -177,13 +175,9 @@ template <> struct SpType<bf16_t> {
         return r;
     }
     static constexpr uint32_t NEG_INF_PAIR = 0xff80ff80u;
-    // e / s for both halves of a word, s in [SHORT_MIN, SHORT_MAX]: e * (1 / s) is within 2^-23 of the quotient, and the quotient
-    // of two 8-bit significands is no closer than 2^-17 to the middle between two bf16 values (and never on it), or, where the
-    // result is subnormal, an exact f32 value when it is on the middle (all pairs compared on the CPU)
-    static constexpr bool SHORT_TWO = false;
-    static constexpr float SHORT_MIN = 0x1p-100f, SHORT_MAX = 0x1p100f;
-    static __device__ __forceinline__ uint32_t short_quotients(uint32_t e, float rinv, float) {
-        return cvt_pk(u2f(e << 16) * rinv, u2f(e & 0xffff0000u) * rinv);
+    typedef ShortDivBf16 Div;
+    static __device__ __forceinline__ uint32_t short_quotients(uint32_t e, float rinv, float rlow) {
+        return cvt_pk(Div::quotient(u2f(e << 16), rinv, rlow), Div::quotient(u2f(e & 0xffff0000u), rinv, rlow));
     }
     static constexpr bool CHUNK_ASM = true;                                       // the walker adds sixteen values per asm statement (add_chunk)
 };
@@ -440,10 +434,10 @@ __global__ void __launch_bounds__(SP_BLOCK) softmax16_stream_kernel(const uint16
             const uint32_t sb = __builtin_amdgcn_readfirstlane((uint32_t)sums[par][LONG ? rr : rr + h * SP_HALF]);
             const float s = ST::widen_bits(sb);
             s_prev[h] = s;
-            fast_prev[h] = s >= ST::SHORT_MIN && s <= ST::SHORT_MAX;
+            fast_prev[h] = s >= ST::Div::MIN && s <= ST::Div::MAX;
             const float rinv = fast_prev[h] ? 1.0f / s : 0.0f;
             rinv_prev[h] = u2f(__builtin_amdgcn_readfirstlane(f2u(rinv)));
-            if (ST::SHORT_TWO) rlow_prev[h] = u2f(__builtin_amdgcn_readfirstlane(f2u(__builtin_fmaf(-s, rinv, 1.0f) * rinv)));
+            if (ST::Div::TWO) rlow_prev[h] = u2f(__builtin_amdgcn_readfirstlane(f2u(ST::Div::low(s, rinv))));
         }
     };
     // exp of the vector that arrived, in place (zeros past the row end: adding +0 is a no-op; rows past the tensor's end

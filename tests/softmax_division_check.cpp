@@ -1,13 +1,16 @@
-// Host check of the streaming softmax's short divisions (SpType<T>::short_quotients in ratchet_amd/csrc/rt_softmax_stream.h):
-// for every exp value e >= 0 and every `stride`-th row sum s inside the range where the kernel takes them, the short form
-// must round to the bits of the correctly rounded f32 quotient rounded to the 16-bit type, which is what the reference's
-// half types compute.  Build: g++ -O2 -ffp-contract=off -mfma.   Usage: softmax_division_check STRIDE
+// Host check of the streaming softmax's short divisions (ratchet_amd/csrc/rt_softmax_div.h, the kernel's own text): for every exp
+// value e >= 0 and every `stride`-th row sum s inside the range where the kernel takes them, the short form must round to the
+// bits of the correctly rounded f32 quotient rounded to the 16-bit type, which is what the reference's half types compute.
+// Build: g++ -O2 -std=c++17 -ffp-contract=off -mfma -I ratchet_amd/csrc.   Usage: softmax_division_check STRIDE
 // prints "f16 <n> bf16 <n> checked <m>" (n: pairs that differ), exit code 0 iff both are 0.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+
+#define RT_FN inline
+#include "rt_softmax_div.h"
 
 static float u2f(uint32_t u) { float f; memcpy(&f, &u, 4); return f; }
 static uint32_t f2u(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
@@ -28,22 +31,22 @@ static uint16_t to_f16(float f) {                             // 0 <= f, nearest
 int main(int argc, char** argv) {
     const unsigned stride = argc > 1 ? (unsigned)strtoul(argv[1], nullptr, 10) : 1;
     unsigned long long bad16 = 0, badbf = 0, checked = 0;
-    for (uint32_t sb = 0x0400; sb < 0x7c00; sb += stride) {   // 2^-14 .. 65504
-        const float s = from_f16((uint16_t)sb), rinv = 1.0f / s, rlow = fmaf(-s, rinv, 1.0f) * rinv;
+    for (uint32_t sb = 1; sb < 0x7c00; sb += stride) {
+        const float s = from_f16((uint16_t)sb), rinv = 1.0f / s, rlow = ShortDivF16::low(s, rinv);
+        if (s < ShortDivF16::MIN || s > ShortDivF16::MAX) continue;
         for (uint32_t eb = 0; eb < 0x7c00; eb++) {
             const float e = from_f16((uint16_t)eb);
-            bad16 += to_f16(fmaf(e, rinv, fmaf(e, rlow, 0.0f))) != to_f16(e / s);
+            bad16 += to_f16(ShortDivF16::quotient(e, rinv, rlow)) != to_f16(e / s);
             checked++;
         }
     }
-    for (uint32_t sb = 0x0080; sb < 0x7f80; sb += stride) {
-        const float s = u2f(sb << 16);
-        if (s < 0x1p-100f || s > 0x1p100f) continue;
-        const float rinv = 1.0f / s;
+    for (uint32_t sb = 1; sb < 0x7f80; sb += stride) {
+        const float s = u2f(sb << 16), rinv = 1.0f / s, rlow = ShortDivBf16::low(s, rinv);
+        if (s < ShortDivBf16::MIN || s > ShortDivBf16::MAX) continue;
         for (uint32_t eb = 0; eb < 0x7f80; eb++) {
             const float e = u2f(eb << 16), q = e / s;
             if (std::isinf(q)) break;                         // a sum is never below its terms
-            badbf += to_bf16(e * rinv) != to_bf16(q);
+            badbf += to_bf16(ShortDivBf16::quotient(e, rinv, rlow)) != to_bf16(q);
             checked++;
         }
     }
