@@ -1,5 +1,5 @@
 // LayerNorm, RMSNorm (one wave64 per row, row held in registers, 16-byte loads, butterfly reductions) and GroupNorm
-// (split statistics + apply, two launches).
+// (groups of up to 192 or 256 KiB in the registers of a block, one launch; larger ones in slices, statistics + apply, two launches).
 //
 // Arithmetic contract for LayerNorm / RMSNorm = crates/ratchet-core/src/cpu/norm.rs:91-147,185-213, in the element type T
 // with one rounding per operation:
@@ -16,7 +16,7 @@
 //   as f32 and one lane per (row, sum) walks its row left to right with v_add_f32.  The walk is latency bound
 //   (one dependent add per element), so many small row groups run side by side.
 // GroupNorm follows torch.nn.functional.group_norm, the ground truth of the reference's own test
-// (ops/norm/groupnorm.rs:24-31): statistics in f32 (Chan-combined partial mean/M2), f32 arithmetic, one final rounding.
+// (ops/norm/groupnorm.rs:24-31): sums in f32 inside a thread (a slice), joined in double, f32 arithmetic, one final rounding.
 #include <type_traits>
 
 #include "rt_arith.h"
@@ -895,7 +895,8 @@ __global__ void __launch_bounds__(64 + RB * 32) norm_flow16_kernel(const T* x, c
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// GroupNorm.  x is [B, C, L] contiguous, so group (b, g) is one contiguous run of glen = (C/G)*L elements.
+// GroupNorm in slices (gn_reg_kernel below takes what fits a block).  x is [B, C, L] contiguous, so group (b, g) is one contiguous run of
+// glen = (C/G)*L elements.
 // stats kernel: grid (B*G, splits); block s of a group reduces elements [s*chunk, min((s+1)*chunk, glen)) to
 //               (mean, M2, count) with a two-pass local variance (second pass re-reads the slice from cache).
 // apply kernel: same grid; every block combines the group's partials (Chan et al.), then normalises its slice:
@@ -1763,8 +1764,8 @@ __device__ __forceinline__ float gn_rstd(double v) {
 // path (mean, then the variance about that mean, f32 arithmetic).  What bounds it is how much of a CU's loads, reductions and
 // stores run at the same time: WPE is the number of waves per SIMD that the registers leave room for, and with the sizes that
 // launch_gn takes two blocks or more share a CU, one storing while another loads ([16,512,3000] f16, 512 groups of 94 KiB: 22.6 us with the
-// group in LDS, one block to a CU, 20.3 with 1024 threads of 6 vectors, 20.4 with 512 of 12; [128,256,3000] f16 97 -> 61 us = 6.4 TB/s;
-// [64,256,1500] f32 35.3 -> 29.3 us).
+// group in LDS, one block to a CU, 20.3 with 1024 threads of 6 vectors, 20.4 with 512 of 12; [128,256,3000] f16 97 -> 63 us = 6.2 TB/s;
+// [64,256,1500] f32 35.3 -> 30.0 us).
 // SPAN: groups that do not start or end on a vector boundary, over the aligned vectors that cover them.  The elements of the
 // neighbouring groups in the first and the last of those stay out of the sums and are not written (such vectors are stored element
 // by element); an aligned vector that holds one byte of the tensor lies in a mapped page.  [16,320,3001] f16 55 -> 15 us against
@@ -1990,7 +1991,9 @@ int launch_gn(rt_device* dev, const void* x, const void* scale, const void* bias
         if (nvec <= 9216) RT_GN_REG(9, 1024, 4);
         const uint64_t rounds = ((uint64_t)bg + cus - 1) / cus, enough = rounds == 1 ? cus * 9 / 16 : rounds * cus * 5 / 8;
         if (nvec <= 12288 && (sizeof(T) == 4 || !vec || bg >= enough)) RT_GN_REG(12, 1024, 4);
-        if (sizeof(T) == 4 && nvec <= 16384 && bg >= cus) RT_GN_REG(16, 1024, 4);
+        if constexpr (sizeof(T) == 4) {
+            if (nvec <= 16384 && bg >= cus) RT_GN_REG(16, 1024, 4);
+        }
     }
 #undef RT_GN_REG
     if (!fixed_scratch && need > dev->gn_scratch_bytes) {

@@ -320,7 +320,10 @@ template <typename T> int launch_lane16(rt_device* dev, const void* x, void* y, 
     return RT_OK;
 }
 
-constexpr uint32_t RAGGED_STREAM_MIN_COLS = 192;   // shorter ragged rows: the two-pass tile walker is faster than the streaming variant
+// shorter ragged rows take the two-pass tile walker.  The line dates from a streaming variant of two launches; against the one there is now
+// it lies too high (us, walker / streaming: f16 [4096,33] 5.8 / 7.8, [4096,129] 8.0 / 8.0, [30000,129] 21.3 / 16.3, [30000,190] 25 / 16; bf16
+// [4096,65] 8.8 / 9.3, [4096,97] 10.5 / 9.4; under a mask, which the walker adds in a launch of its own, f16 [4096,33] 10.4 / 8.2)
+constexpr uint32_t RAGGED_STREAM_MIN_COLS = 192;
 
 // ------------------------------------------------------------------------------------------------------------------
 // The attention caller pattern (ratchet-models/src/phi3/attn.rs:148-153, phi2/attn.rs:143-150, whisper/mha.rs:115-124):
@@ -921,8 +924,8 @@ extern "C" int rt_softmax(rt_device* dev, int dt, const void* x, void* y, uint64
             // 16-bit types, rows that are whole aligned vectors: one pass; up to 128 columns (and enough rows to fill the chip) a lane per row, up to 4096
             // columns (f16: 8192, where that is the faster way) streamed with the row held in registers, longer ones parked in y (also small problems: the per-block table load costs about 5 us, the two-pass walker
             // more); everything else takes the two-pass tile walker
-            // (rows that are not whole vectors stream over their covering vectors, with a second small launch for the
-            // shared ones: measured faster than the tile walker from about 200 columns, 12.7 against 34.5 us on [4096, 1001])
+            // (rows that are not whole vectors stream from their first element on, the last vector over the one before it: [4096, 1001]
+            // 10.8 us, 34.5 by the tile walker)
             if (rt_aligned(x, 16) && rt_aligned(y, 16) && (cols % 8 == 0 || cols >= RAGGED_STREAM_MIN_COLS)) {
                 if (cols % 8 == 0 && cols <= LANE_MAX_COLS && rows >= 32768) return dt == RT_F16 ? launch_lane16<half_t>(dev, x, y, rows, cols) : launch_lane16<bf16_t>(dev, x, y, rows, cols);
                 bool done = false;

@@ -1,5 +1,6 @@
-// The streaming 16-bit softmax (f16 / bf16 reference arithmetic in one pass over HBM) and its launcher.  Included by one translation unit per element type (rt_softmax_stream_f16.hip,
-// rt_softmax_stream_bf16.hip): the kernel has some sixty instantiations per type, and the two compile side by side.
+// The streaming 16-bit softmax (f16 / bf16 reference arithmetic in one pass over HBM) and its launcher.  Included by one
+// translation unit per element type (rt_softmax_stream_f16.hip, rt_softmax_stream_bf16.hip): the kernel has some sixty
+// instantiations per type, and the two compile side by side.
 #ifndef RT_SOFTMAX_STREAM_H
 #define RT_SOFTMAX_STREAM_H
 
@@ -715,7 +716,7 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         if (period * row_bytes > 0x7fffffffull) return RT_OK;
         chunk_rows = (0x7fffffffull / (period * row_bytes)) * period;
     } else if (ragged) {
-        // every chunk must start on a 16-byte boundary (8 rows do)
+        // chunks of whole groups (any row may start one: the accesses are at element alignment)
         const uint64_t max_rows = 0x7fffffe0ull / row_bytes;
         chunk_rows = rows <= max_rows ? rows : max_rows / 120 * 120;
         if (chunk_rows == 0) return RT_OK;

@@ -814,6 +814,22 @@ def test_group_norm_at_the_edges_of_the_block_shapes(dev, oracle, glen, B, dtype
             assert bad == 0, (C, L, bad, mx)
 
 
+@pytest.mark.parametrize("glen", [6144, 6152, 12296, 24584, 32776, 49160, 65544, 73736, 98312, 1, 5, 2049, 24571, 49149, 73723])
+@pytest.mark.parametrize("B", [1, 13])
+def test_group_norm_bf16_at_the_edges_of_the_block_shapes(dev, oracle, glen, B):
+    """the groups of the test above in bf16, of mean 2, against the f32 result of the same values: half a step of bf16, which is up to
+    2^-8 of the value, and the f32 tolerance"""
+    rng = np.random.default_rng(glen)
+    for C, L in ((10, glen), (20, glen // 2)) if glen % 2 == 0 else ((10, glen),):
+        raw = [oracle.cast(a, np.uint16, dst_bf16=True) for a in (randn(rng, (B, C, L), np.float32) + np.float32(2), randn(rng, C, np.float32), randn(rng, C, np.float32))]
+        wide = [oracle.cast(a, np.float32, src_bf16=True) for a in raw]
+        want = oracle.group_norm(wide[0], 10, wide[1], wide[2], 1e-5)
+        dx, dw, db = [dev.upload(a, bf16=True) for a in raw]
+        for got in (dev.group_norm(dx, 10, dw, db, 1e-5), dev.group_norm(dx, 10, dw, db, 1e-5, out=dx)):
+            off = np.abs(oracle.cast(got.to_numpy(), np.float32, src_bf16=True) - want)
+            assert np.all(off <= 2.0 ** -8 * np.abs(want) + 1e-5 * (1 + np.abs(want))), (C, L, off.max())
+
+
 @pytest.mark.parametrize("B,C,L,G", [(8, 320, 4097, 32),       # 256 ragged groups of 160 KiB, one block each
                                      (8, 320, 4096, 32),       # the same on vector boundaries
                                      (16, 512, 4096, 32),      # 512 groups of 256 KiB, 16 vectors a thread
