@@ -295,7 +295,8 @@ template <typename T> int launch_rope_pair(rt_device* dev, const void* x, void* 
     if (chunks > max_chunks) chunks = max_chunks;
     if (chunks > 65535) chunks = 65535;
     if (chunks < 1) chunks = 1;
-    a.bh_chunk = (uint32_t)((a.nbh + chunks - 1) / chunks);
+    // whole trips: of 11 rows in trips of eight, five eighths of the second would idle (f16 [32,4008,64] in place 9.7 -> 8.5 us)
+    a.bh_chunk = (uint32_t)(((a.nbh + chunks - 1) / chunks + per_trip - 1) / per_trip * per_trip);
     chunks = (a.nbh + a.bh_chunk - 1) / a.bh_chunk;
     const dim3 grid((unsigned)blocks_x, (unsigned)chunks);
 #define RT_RP(UC, IP) hipLaunchKernelGGL((rope_pair_kernel<T, UC, IP>), grid, dim3(BLOCK), 0, dev->stream, (const T*)x, (T*)y, a)
@@ -377,10 +378,18 @@ extern "C" int rt_rope(rt_device* dev, int dt, const void* x, void* y, const uin
     a.nbh = shape[0] * shape[1];
     const uint32_t ve = 16u / (uint32_t)eb;
     if ((dim / 2) % ve == 0 && shape[3] % ve == 0 && rt_aligned(x, 16) && rt_aligned(y, 16)) {
-        // in place, on rows of whole 256-byte units and up to 32 MiB, the slot kernel needs no barrier between a trip's loads and
-        // stores and is the faster one (f16 [1,32,1024,128] 5.2 us against 5.7, f32 [4,8,2048,64] 5.5 / 7.3; beyond, f32 [2,32,2048,128]
-        // 22.6 / 22.1, f16 [4,32,4096,128] 46.7 / 43.7); it also takes heads and rotary widths too wide for a block
-        const bool slots = x == y && ((uint64_t)shape[3] * eb) % 256 == 0 && n * eb <= 32ull << 20;
+        // On rows of whole 256-byte units the slot kernel's pieces are whole lines.  In place it needs no barrier between a trip's loads and
+        // stores and leaves no thread idle for the columns that stay where they are: it is the faster one up to 32 MiB (f16 [1,32,1024,128]
+        // 5.2 us against 5.7, f32 [4,8,2048,64] 5.5 / 7.3) and, where the rotary halves are whole 64-byte pieces, at any size with rotary
+        // widths of up to a third of the row, or half where that is 128 bytes (f16 [128,2048,256] width 64 16.6 / 23.7, [128,1000,256] 128
+        // 14.1 / 15.7, [32,4008,384] 128 15.8 / 21.2, f32 [32,4008,512] 64 15.7 / 26.9); beyond, the other one is (f32 [2,32,2048,128]
+        // 22.6 / 22.1, f16 [4,32,4096,128] 46.7 / 43.7, [128,2048,256] width 96 35.3 / 24.9, f32 256 96 46.9 / 40.6).  Out of place it saves a
+        // launch of up to 2 MiB the barrier behind the sines, where all columns rotate (f32 [1,300,64] 3.7 / 4.3, f16 [8,512,128] 4.1 / 4.3,
+        // f32 [8,512,256] 5.0 / 4.6; width 64 of [8,512,128] 4.35 / 4.28).  It also takes heads and rotary widths too wide for a block
+        const uint64_t bytes = n * eb;
+        const uint32_t half_bytes = dim / 2 * (uint32_t)eb;
+        const bool few_move = half_bytes % 64 == 0 && (3ull * dim <= shape[3] || (2ull * dim <= shape[3] && half_bytes <= 128));
+        const bool slots = (uint64_t)shape[3] * eb % 256 == 0 && (x == y ? bytes <= 32ull << 20 || few_move : dim == shape[3] && bytes <= 2ull << 20);
         if (!slots && dim / 2 <= (uint32_t)BLOCK && shape[3] / ve <= (uint32_t)BLOCK) {
             switch (dt) {
                 case RT_F32: return launch_rope_pair<float>(dev, x, y, shape, dim, offset, logf(base));
