@@ -88,7 +88,7 @@ def test_rope_trips_and_in_place_by_size(dev, oracle, shape, dim, kind):
 
 @pytest.mark.parametrize("shape,dim", [((4, 33, 1100, 256), 64), ((3, 33, 1100, 256), 96), ((4, 33, 700, 256), 128), ((2, 33, 1100, 384), 128),   # in place beyond 32 MiB by how much of a row moves
                                        ((1, 1, 300, 64), 64), ((1, 8, 513, 128), 128), ((1, 8, 512, 256), 256),                          # out of place around 2 MiB
-                                       ((1, 11, 4008, 64), 64)])                                                                        # rows of a chunk that are not whole trips
+                                       ((1, 11, 4008, 64), 64), ((1, 16, 2003, 80), 80)])                                                                        # rows of a chunk that are not whole trips
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 def test_rope_by_rotary_width_and_size(dev, oracle, shape, dim, kind):
     """both sides of the lines between the two vector kernels, out of place and in place, against the oracle bit for bit"""
