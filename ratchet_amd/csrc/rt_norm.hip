@@ -1636,8 +1636,10 @@ int launch_norm16_flow(rt_device* dev, const void* x, const void* scale, const v
     const uint64_t groups = (rows + R - 1) / R;
     RT_REQUIRE(groups <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");
     // the walker and a loader wave for every two of the R <= RB rows: waves without a row would issue every instruction of the
-    // others ([16384,3072], 64 rows a CU in rounds of 22: LayerNorm bf16 55.1 -> 48.1 us, f16 45.3 -> 43.0, RMSNorm bf16 43.7 -> 40.8)
-    const uint32_t threads = 64 + (R + 1) / 2 * 64;
+    // others ([16384,3072], 64 rows a CU in rounds of 22: LayerNorm bf16 55.1 -> 48.1 us, f16 45.3 -> 43.0, RMSNorm bf16 43.7 -> 40.8).
+    // Blocks of 8 rows launch all four: they stage the weights together, where one wave, for one or two rows, takes a trip for every 512
+    // columns (LayerNorm f16 [1,4096] 16.7 us, 15.7 with four, [64,1001] 6.85 / 6.65)
+    const uint32_t threads = 64 + (RB == 8 ? 4 : (R + 1) / 2) * 64;
     const uint32_t nt = (cols + 255) / 256;
     const size_t affine_bytes = (size_t)nt * 512 * (KIND == NORM_LAYER ? 2 : 1);
     const uint32_t steps = nf_steps(nt);
