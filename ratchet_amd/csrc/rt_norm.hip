@@ -683,7 +683,7 @@ __device__ __forceinline__ void np_add_f32x16(float& run, const v4u& a, const v4
 #undef NP_ADD
 }
 // The same walk for rows of 8 to NF_MAX_COLS columns as a stream: persistent blocks, one to a CU, that take groups of up to
-// RB rows (8, 16 or 30) in turn.  The loader waves, one for every two rows, keep a group's rows in registers (NT vectors a thread) from the
+// RB rows (8, 16 or 30) in turn.  The loader waves, one for every two rows (four in blocks of 8), keep a group's rows in registers (NT vectors a thread) from the
 // load to the store, and in step t of a group, while wave 0 walks tile t, they normalise and store tile t of the group
 // before and load the tile PF steps ahead, across the groups: x is read once, and reads, walk and writes go on side by
 // side instead of in phases that all blocks of the chip pass at the same time.
