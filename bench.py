@@ -177,7 +177,7 @@ def build_workload(dev, seed):
     d_rms3, d_silu3, d_swiglu3 = dev.empty(x3.shape, F16), dev.empty(gate3.shape, F16), dev.empty(gate3.shape, F16)
     ops.append(Op(3, "rms_norm", "f16", "4096x3072", 2 * x3.nbytes + g3.nbytes, lambda i, o: dev.rms_norm(i[0], i[1], 1e-5, out=o), [d_x3, d_g3], d_rms3,
                   dict(kind="rows", out=d_rms3, x=x3, rows=4096, tol=1e-3, fn=lambda o, xs: o.rms_norm(xs, g3, 1e-5, intended=True)),
-                  "rms16_par_kernel", rotating=[0]))
+                  "norm16_row_kernel", rotating=[0]))
     ops.append(Op(3, "silu(gate)", "f16", "[1,4096,8192]", 2 * gate3.nbytes, lambda i, o: dev.unary("silu", i[0], out=o), [d_gate3], d_silu3,
                   dict(kind="rows", out=d_silu3, x=gate3, rows=4096, tol=1e-3, fn=lambda o, xs: o.unary("silu", xs)), "unary_lut_kernel"))
     ops.append(Op(3, "mul silu(gate)*up", "f16", "[1,4096,8192]x2", 3 * gate3.nbytes, lambda i, o: dev.binary("mul", i[0], i[1], out=o),

@@ -42,7 +42,6 @@ struct rt_device {
     uint64_t sp_ragged_attr_set;   // the same for the ragged-row variants
     uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads (bits 0..15) and for those of f16 rows of 4097 to 8192 columns
     unsigned ry_attr_set;          // the same for the one-wave-per-row softmax (rt_softmax_replay.hip)
-    uint16_t rp_resident[2][9];    // wave-per-row RMSNorm: blocks of an instantiation ([f16, bf16][vectors per lane]) that one CU holds; 0 = not asked yet
     // one word per 512-column tile of the mask of a masked streaming softmax (allocated with the device): the
     // tile's value twice when all its elements are equal, 0xffffffff when the tile has to be loaded; the first RT_SM_TILES_HEAD
     // words always hold 0xffffffff
@@ -126,6 +125,11 @@ int rt_softmax_stream_bf16(rt_device* dev, const void* x, const void* mask, uint
 
 // The f16 reference softmax for a few long rows, one wave per row (rt_softmax_replay.hip); arguments as above
 int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
+
+// The 16-bit LayerNorm / RMSNorm with a wave per row (rt_norm_row.hip): whole vectors, 16-byte aligned operands, at most NR_MAX_COLS columns
+constexpr uint32_t NR_MAX_COLS = 5120;                       // 10 vectors a lane
+int rt_norm16_row(rt_device* dev, bool bf16, int kind, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols,
+                  float eps);
 
 // ---------------------------------------------------------------------------------------------------------
 // u32 division by a launch-time constant: q = (n * m) >> (32 + s), exact for all n < 2^32 (round-up method)

@@ -14,13 +14,15 @@
 //   so a different f32 summation order can flip that rounding and move a whole row by an ulp of r, more than 1e-3
 //   allows.  These kernels therefore replay the reference's order exactly: tiles of x and T(x*x) are staged through LDS
 //   as f32 and one lane per (row, sum) walks its row left to right with v_add_f32.  The walk is latency bound
-//   (one dependent add per element), so many small row groups run side by side.
+//   (one dependent add per element), so many small row groups run side by side.  Where it is faster a wave per row finds what
+//   the ordered sum rounds to without walking it (rt_norm_row.hip).
 // GroupNorm follows torch.nn.functional.group_norm, the ground truth of the reference's own test
 // (ops/norm/groupnorm.rs:24-31): sums in f32 inside a thread (a slice), joined in double, f32 arithmetic, one final rounding.
 #include <type_traits>
 
 #include "rt_arith.h"
 #include "rt_internal.h"
+#include "rt_norm.h"
 
 namespace {
 
@@ -28,45 +30,12 @@ constexpr int WAVE = 64;
 constexpr int BLOCK = 256;
 constexpr int WAVES = BLOCK / WAVE;
 
-enum { NORM_LAYER = 0, NORM_RMS = 1 };
-
 // Partial statistics for rt_group_norm_static, the entry point that allocates nothing: a fixed array in the code object,
 // one copy per GPU.  In host code the array's name is only a stand-in; rt_norm_device_init asks the runtime where the
 // current device's copy lies and every launch is given that pointer.
 constexpr size_t GN_STATIC_SCRATCH_BYTES = 256 * 1024;
 static __device__ __align__(256) unsigned char gn_static_scratch[GN_STATIC_SCRATCH_BYTES];
 constexpr int NORM_WIDE_BLOCK = 1024;                   // threads per row for f32 rows that do not fit 256 threads' registers
-
-// per-row statistics in T arithmetic, given f32 sums
-template <typename T> struct RowStats {
-    T mu, r;
-};
-template <typename T, int KIND> __device__ __forceinline__ RowStats<T> finish_stats(float sum_x, float sum_sq, uint32_t cols, float eps) {
-    typedef Ar<T> A;
-    RowStats<T> st;
-    const T n = A::conv((float)cols);                       // T::from(step as f32)
-    const T x2 = A::div(A::conv(sum_sq), n);
-    T var;
-    if (KIND == NORM_LAYER) {
-        st.mu = A::div(A::conv(sum_x), n);
-        var = A::sub(x2, A::mul(st.mu, st.mu));
-    } else {
-        st.mu = A::conv(0.0f);
-        var = x2;
-    }
-    const T t = A::add(var, A::conv(eps));
-    st.r = A::div(A::conv(1.0f), ar_sqrt<T>(t));
-    return st;
-}
-
-template <typename T, int KIND> __device__ __forceinline__ T norm_one(T x, const RowStats<T>& st, T scale, T bias, bool has_bias) {
-    typedef Ar<T> A;
-    T v = (KIND == NORM_LAYER) ? A::sub(x, st.mu) : x;
-    v = A::mul(v, st.r);
-    v = A::mul(v, scale);
-    if (KIND == NORM_LAYER && has_bias) v = A::add(v, bias);
-    return v;
-}
 
 // x and y 16-byte aligned, at most LANES * NV vectors per row.  Rows of whole vectors (scale and bias 16-byte aligned as
 // well), or SPAN: rows of any length over the aligned vectors that cover them.  A row then starts `shift` elements into
@@ -414,7 +383,6 @@ __global__ void __launch_bounds__(BLOCK) norm_seq16_kernel(const T* __restrict__
 constexpr int NP_BLOCK = 320;
 constexpr uint32_t NP_KEEP_MAX_COLS = 4096;
 constexpr size_t NP_KEEP_BYTES_PER_TILE = 256 * 16 + 2 * 32 * 16;   // the block's x vectors, one scale and one bias vector per column group
-typedef _Float16 np_h8 __attribute__((ext_vector_type(8)));
 // run += the 32 f16 values packed in four vectors, left to right: each add is 1.0 * widen(f16) + run in one instruction
 // with one rounding, which is the f32 sum of the widened values.  One asm statement for the whole run of adds: between
 // separate statements the compiler, which cannot see into them, puts wait states that cost more than the adds.
@@ -638,39 +606,6 @@ __global__ void __launch_bounds__(NP_BLOCK) norm_pipe16_kernel(const T* __restri
     }
 }
 
-// f rounded to bf16 and widened again, in one instruction: converted into the high half of a word whose low half is bf16(0) = 0
-__device__ __forceinline__ float np_round_bf16(float f) {
-    uint32_t r;
-    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(f));
-    return u2f(r);
-}
-// norm_one, with a bias, on the eight elements of a vector.  bf16 goes in f32 form from step to step, two instructions each (through
-// Ar<bf16_t> the roundings and widenings take four), and is packed once at the end.
-template <typename T, int KIND> __device__ __forceinline__ v4u norm_vec16(const v4u& x, const RowStats<T>& st, const v4u& scale, const v4u& bias) {
-    v4u out;
-    if constexpr (std::is_same<T, bf16_t>::value) {
-        const float mu = Ar<T>::widen(st.mu), rs = Ar<T>::widen(st.r);
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            float v[2] = {u2f(x[w] << 16), u2f(x[w] & 0xffff0000u)};
-            const float s[2] = {u2f(scale[w] << 16), u2f(scale[w] & 0xffff0000u)}, b[2] = {u2f(bias[w] << 16), u2f(bias[w] & 0xffff0000u)};
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                if (KIND == NORM_LAYER) v[h] = np_round_bf16(v[h] - mu);
-                v[h] = np_round_bf16(v[h] * rs) * s[h];
-                if (KIND == NORM_LAYER) v[h] = np_round_bf16(v[h]) + b[h];
-            }
-            asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(out[w]) : "v"(v[0]), "v"(v[1]));
-        }
-    } else {
-        np_h8 v = __builtin_bit_cast(np_h8, x);
-        if (KIND == NORM_LAYER) v = v - st.mu;
-        v = v * st.r * __builtin_bit_cast(np_h8, scale);
-        if (KIND == NORM_LAYER) v = v + __builtin_bit_cast(np_h8, bias);
-        out = __builtin_bit_cast(v4u, v);
-    }
-    return out;
-}
 // run += the sixteen f32 values of four vectors, left to right (as one asm statement: with ordinary adds the compiler reads
 // a whole tile ahead, into 256 registers)
 __device__ __forceinline__ void np_add_f32x16(float& run, const v4u& a, const v4u& b, const v4u& c, const v4u& d) {
@@ -1287,269 +1222,6 @@ __global__ void __launch_bounds__(BLOCK) norm16_lane_kernel(const T* x, const T*
     for (uint32_t i = threadIdx.x; i < nvec; i += BLOCK) st_stream(yb + i, stage[(i / NV) * (NV + 1) + i % NV]);
 }
 
-// ------------------------------------------------------------------------------------------------------------------
-// RMSNorm in the 16-bit types, one wave per row, with the reference's row sum replayed exactly but not sequentially.
-//
-// The reference adds T(x*x) left to right in f32 (cpu/norm.rs:72-89, half's Sum): s <- fl(s + a_j), a_j >= 0.  While s
-// stays inside one binade, [2^e, 2^(e+1)), s is 2^e + k * ulp with an integer k, and what one add does to k depends on s
-// only through the parity of k (round to nearest even: the parity decides ties).  A run of adds that stays inside the
-// binade is therefore a function k -> k + c[k & 1] of two constants, and such functions compose.  Both constants come
-// out of the floating-point adder itself: the run is added up twice, from 2^e and from 2^e + ulp, and c[p] is the
-// distance the p-th sum has moved, read off the bit patterns.
-//
-// Lane i of the wave owns the contiguous run of 8 * V elements i * 8V .. (the row is turned through LDS so that it does).
-//   1. approximate sums of the runs and their prefix over the lanes say in which binade each run starts and ends;
-//   2. a lane whose run starts and ends in one binade, with a margin for what the approximation can be off by, is
-//      `clean`: its two sums give its pair (c[0], c[1]);
-//   3. a segmented scan composes the pairs of neighbouring clean lanes;
-//   4. the lanes that are not clean (the first, those in which the sum crosses a power of two: about seven per row,
-//      and any lane the margins do not clear) are taken in order: the composed function of the clean stretch before
-//      such a lane is applied to the running value t, then every lane adds its own run to t left to right and the
-//      result of the lane in question is kept.
-// Nothing rests on the approximation: before a pair is applied, t must lie in the binade the pair was made for, and
-// the result must still lie in it; if either fails the row is done again with every lane treated as not clean, which
-// is the plain left-to-right sum, 64 runs one after the other.  bf16 takes the same path with widened operands.
-// ------------------------------------------------------------------------------------------------------------------
-constexpr int RP_BLOCK = 256;                                // four rows per block; the waves never meet
-template <typename T> struct RpChain;
-template <> struct RpChain<half_t> {
-    // a <- fl(a + h) and b <- fl(b + h) for the eight halves of a vector, left to right: 1.0 * widen(h) + sum in one
-    // instruction with one rounding
-#define RP_MIX2(N)                                                              \
-    "v_fma_mix_f32 %0, %" #N ", %6, %0 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %1, %" #N ", %6, %1 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %0, %" #N ", %6, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"       \
-    "v_fma_mix_f32 %1, %" #N ", %6, %1 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"
-    static __device__ __forceinline__ void add2(float& a, float& b, const v4u& v) {
-        const float one = 1.0f;
-        asm(RP_MIX2(2) RP_MIX2(3) RP_MIX2(4) RP_MIX2(5) : "+v"(a), "+v"(b) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(one));
-    }
-#undef RP_MIX2
-#define RP_MIX1(N)                                                              \
-    "v_fma_mix_f32 %0, %" #N ", %5, %0 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %0, %" #N ", %5, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"
-    static __device__ __forceinline__ void add1(float& a, const v4u& v) {
-        const float one = 1.0f;
-        asm(RP_MIX1(1) RP_MIX1(2) RP_MIX1(3) RP_MIX1(4) : "+v"(a) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(one));
-    }
-#undef RP_MIX1
-    // the sum of the eight halves added to acc, in any order and with any rounding: only the binade is taken from it
-    // (v_dot2_f32_f16 with a pair of ones; written as instructions: through the builtin this compiler fed all four the
-    // vector's first word)
-    static __device__ __forceinline__ float rough(const v4u& v, float acc) {
-        const uint32_t ones = 0x3c003c00u;
-        asm("v_dot2_f32_f16 %0, %1, %5, %0\n"
-            "v_dot2_f32_f16 %0, %2, %5, %0\n"
-            "v_dot2_f32_f16 %0, %3, %5, %0\n"
-            "v_dot2_f32_f16 %0, %4, %5, %0\n"
-            : "+v"(acc)
-            : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(ones));
-        return acc;
-    }
-    static __device__ __forceinline__ v4u square(const v4u& x) {                 // T(x*x): eight f16 products, each rounded once
-        const np_h8 h = __builtin_bit_cast(np_h8, x);
-        return __builtin_bit_cast(v4u, h * h);
-    }
-};
-template <> struct RpChain<bf16_t> {
-    static __device__ __forceinline__ void add2(float& a, float& b, const v4u& v) {
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const float lo = u2f(v[w] << 16), hi = u2f(v[w] & 0xffff0000u);
-            a += lo; b += lo; a += hi; b += hi;
-        }
-    }
-    static __device__ __forceinline__ void add1(float& a, const v4u& v) {
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            a += u2f(v[w] << 16);
-            a += u2f(v[w] & 0xffff0000u);
-        }
-    }
-    static __device__ __forceinline__ float rough(const v4u& v, float acc) {
-#pragma unroll
-        for (int w = 0; w < 4; w++) acc += u2f(v[w] << 16) + u2f(v[w] & 0xffff0000u);
-        return acc;
-    }
-    static __device__ __forceinline__ v4u square(const v4u& x) {
-        Vec16<bf16_t> in, out;
-        in.u = x;
-#pragma unroll
-        for (int q = 0; q < 8; q++) out.e[q] = Ar<bf16_t>::mul(in.e[q], in.e[q]);
-        return out.u;
-    }
-};
-
-template <typename T, int V>
-__global__ void __launch_bounds__(RP_BLOCK) rms16_par_kernel(const T* __restrict__ x, const T* __restrict__ scale, T* __restrict__ y, uint64_t rows,
-                                                             uint32_t cols, float eps) {
-    typedef RpChain<T> C;
-    extern __shared__ __attribute__((aligned(16))) v4u rp_lds[];             // [4 waves][V * 64] vectors of squares
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint64_t first = (uint64_t)blockIdx.x * (RP_BLOCK / 64) + wave, stride = (uint64_t)gridDim.x * (RP_BLOCK / 64);
-    if (first >= rows) return;                                               // a whole wave; the block never synchronises
-    v4u* mine = rp_lds + wave * (V * 64);
-    const uint32_t nvec = cols / 8;
-    // the row as it lies in memory: vector j * 64 + lane (zeros past its end: +0 terms change no sum).  A wave takes rows
-    // first, first + stride, ...; the loads of the next one are in flight while it works on this one (past the last
-    // row they fetch the last row once more, so that no branch stands between the loads and what waits for them)
-    auto fetch = [&](uint64_t r, v4u (&dst)[V]) {
-        const v4u* src = reinterpret_cast<const v4u*>(x + r * cols);
-#pragma unroll
-        for (int j = 0; j < V; j++) {
-            const uint32_t i = j * 64 + lane;
-            dst[j] = v4u{0, 0, 0, 0};
-            if (i < nvec) dst[j] = ld_stream(src + i);
-        }
-    };
-    v4u ahead[V];
-    fetch(first, ahead);
-    for (uint64_t row = first; row < rows; row += stride) {
-    v4u xr[V];
-#pragma unroll
-    for (int j = 0; j < V; j++) xr[j] = ahead[j];
-    fetch(row + stride < rows ? row + stride : rows - 1, ahead);
-    v4u* yrow = reinterpret_cast<v4u*>(y + row * cols);
-#pragma unroll
-    for (int j = 0; j < V; j++) mine[j * 64 + lane] = C::square(xr[j]);
-    // turned: lane i holds the run of vectors i * V .. i * V + V - 1.  The wave wrote them itself and LDS keeps a wave's
-    // order, but other lanes wrote what this lane reads: the fence keeps the compiler from moving a read above a write
-    // that, seen from one lane alone, goes to another address.
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    v4u run[V];
-#pragma unroll
-    for (int v = 0; v < V; v++) run[v] = mine[lane * V + v];
-
-    // 1. approximate sum of the run, inclusive prefix over the lanes
-    float rough = 0.0f;
-#pragma unroll
-    for (int v = 0; v < V; v++) rough = C::rough(run[v], rough);
-    float upto = rough;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const float t = __shfl_up(upto, o, 64);
-        if (lane >= (uint32_t)o) upto += t;
-    }
-    float before = __shfl_up(upto, 1, 64);
-    if (lane == 0) before = 0.0f;
-    // 2. clean: the run starts and ends in the binade of `before`, even if both figures are off by 2^-10 of themselves
-    const uint32_t e = (f2u(before) >> 23) & 0xffu;
-    const uint32_t base = e << 23;                                           // bit pattern of 2^e
-    bool clean = lane != 0 && e >= 1 && e < 254 && ((f2u(before * (1.0f - 0x1p-10f)) >> 23) & 0xffu) == e &&
-                 ((f2u(upto * (1.0f + 0x1p-10f)) >> 23) & 0xffu) == e;
-    float s0 = u2f(base), s1 = u2f(base + 1);
-#pragma unroll
-    for (int v = 0; v < V; v++) C::add2(s0, s1, run[v]);
-    uint32_t c0 = f2u(s0) - base, c1 = f2u(s1) - (base + 1);
-    clean = clean && c0 < (1u << 23) && c1 + 1 < (1u << 23);                 // both sums stayed in the binade
-    // the pairs of a stretch of clean lanes are composed as counts of one and the same ulp: a clean lane behind a clean
-    // lane of another binade (which the margins make all but impossible) starts over as a lane that is not clean
-    {
-        const uint32_t pbase = __shfl_up(base, 1, 64);
-        const uint32_t pclean = __shfl_up((uint32_t)clean, 1, 64);
-        if (lane != 0 && pclean && pbase != base) clean = false;
-    }
-    if (!clean) c0 = c1 = 0;
-
-    // 3. segmented scan: (c0, c1) of lane i becomes the composition of the clean lanes from the start of its stretch up to
-    // i; a lane that is not clean, and the lane behind one, start a stretch.  left then right: p -> l[p] + r[(p + l[p]) & 1]
-    const uint64_t dirty_mask = __builtin_amdgcn_ballot_w64(!clean);
-    uint32_t head = (uint32_t)((dirty_mask >> lane) & 1u) | (lane ? (uint32_t)((dirty_mask >> (lane - 1)) & 1u) : 1u);
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t l0 = __shfl_up(c0, o, 64), l1 = __shfl_up(c1, o, 64), lh = __shfl_up(head, o, 64);
-        if (lane >= (uint32_t)o && !head) {
-            const uint32_t n0 = l0 + ((l0 & 1u) ? c1 : c0);
-            const uint32_t n1 = l1 + (((l1 + 1u) & 1u) ? c1 : c0);
-            c0 = n0;
-            c1 = n1;
-            head = lh;
-        }
-    }
-
-    // 4. the lanes that are not clean, in order, with the clean stretches between them
-    uint32_t tb = 0;                                                         // bit pattern of the running sum, the same in every lane
-    uint64_t todo = dirty_mask;
-    bool redo = false;
-    for (;;) {
-        int prev = -1;
-        bool failed = false;
-        // applies the composed pair of lane `last` (the end of a clean stretch) to the running sum
-        auto stretch = [&](int last) {
-            const uint32_t f0 = __builtin_amdgcn_readlane(c0, last), f1 = __builtin_amdgcn_readlane(c1, last);
-            const uint32_t eb = __builtin_amdgcn_readlane(base, last);
-            const uint32_t k = tb - eb;                                      // t = 2^e + k ulp, if t lies in that binade
-            const uint32_t k2 = k + ((k & 1u) ? f1 : f0);
-            if ((tb & 0x7f800000u) != eb || k2 >= (1u << 23)) failed = true;
-            tb = eb + k2;
-        };
-        while (todo) {
-            const int d = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            if (!redo && d - 1 > prev) stretch(d - 1);
-            float t = u2f(tb);
-#pragma unroll
-            for (int v = 0; v < V; v++) C::add1(t, run[v]);
-            tb = __builtin_amdgcn_readlane(f2u(t), d);
-            prev = d;
-        }
-        if (!redo && prev < 63) stretch(63);
-        if (!failed || redo) break;
-        redo = true;                                                         // the plain sum: every lane's run, one after the other
-        todo = ~0ull;
-        tb = 0;
-    }
-
-    const RowStats<T> st = finish_stats<T, NORM_RMS>(0.0f, u2f(tb), cols, eps);
-#pragma unroll
-    for (int j = 0; j < V; j++) {
-        const uint32_t i = j * 64 + lane;
-        if (i < nvec) {
-            Vec16<T> in, sc, out;
-            in.u = xr[j];
-            sc.u = reinterpret_cast<const v4u*>(scale)[i];
-#pragma unroll
-            for (int q = 0; q < 8; q++) out.e[q] = norm_one<T, NORM_RMS>(in.e[q], st, sc.e[q], sc.e[q], false);
-            st_stream(yrow + i, out.u);
-        }
-    }
-    // the next row's squares go to the same LDS buffer: every lane has read its run by now (the run is in registers)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-}
-
-template <typename T>
-int launch_rms16_par(rt_device* dev, const void* x, const void* scale, void* y, uint64_t rows, uint32_t cols, float eps) {
-    // as many blocks as the chip holds at one time (what the runtime says for the instantiation's registers and LDS,
-    // asked once per device), each wave taking every grid-th row
-    const uint32_t v = (cols + 511) / 512;
-    constexpr int TI = std::is_same<T, half_t>::value ? 0 : 1;
-    uint64_t blocks = (rows + RP_BLOCK / 64 - 1) / (RP_BLOCK / 64);
-#define RT_RP(VC)                                                                                                                    \
-    case VC:                                                                                                                         \
-        if (!dev->rp_resident[TI][VC]) {                                                                                             \
-            int per_cu = 0;                                                                                                          \
-            RT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, rms16_par_kernel<T, VC>, RP_BLOCK,                          \
-                                                                (size_t)(RP_BLOCK / 64) * VC * 64 * 16));                            \
-            dev->rp_resident[TI][VC] = (uint16_t)(per_cu < 1 ? 1 : per_cu);                                                          \
-        }                                                                                                                            \
-        if (blocks > (uint64_t)dev->rp_resident[TI][VC] * dev->num_cus) blocks = (uint64_t)dev->rp_resident[TI][VC] * dev->num_cus;  \
-        hipLaunchKernelGGL((rms16_par_kernel<T, VC>), dim3((unsigned)blocks), dim3(RP_BLOCK), (size_t)(RP_BLOCK / 64) * VC * 64 * 16, \
-                           dev->stream, (const T*)x, (const T*)scale, (T*)y, rows, cols, eps);                                       \
-        break
-    switch (v) {
-        RT_RP(1); RT_RP(2); RT_RP(3); RT_RP(4); RT_RP(5); RT_RP(6); RT_RP(7); RT_RP(8);
-        default: return rt_fail(RT_ERR_ARG, "norm: internal: %u columns in the wave-per-row RMSNorm", cols);
-    }
-#undef RT_RP
-    RT_CHECK_LAUNCH("rms16_par_kernel");
-    return RT_OK;
-}
-
 template <typename T, int KIND>
 int launch_norm16_lane(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
     const uint64_t blocks = (rows + BLOCK - 1) / BLOCK;
@@ -1596,34 +1268,31 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
     if (!bf16) return rows >= (cols > 40 ? 60 : 120) * cus && cols >= 12;
     return (cols >= 40 && rows >= 120 * cus) || (cols >= 24 && rows > 256 * cus);
 }
-// Rows of whole aligned vectors: against norm_pipe16_kernel, whose blocks of 8 rows share the CUs and overlap one another,
+// Rows of whole aligned vectors: where a wave per row (rt_norm_row.hip) takes them, timed like the above; us, the best of the others / that one.
+// It adds in any order where the ordered sum's rounding is sure without the order, which in bf16 it nearly always is: bf16 gains from
+// 264 columns up (RMSNorm [256,5120] 21.4 / 10.5, [2048,2560] 14.9 / 8.4, [16384,3072] 40.6 / 35.5, [65536,384] 31.8 / 22.3; LayerNorm [2048,2560]
+// 14.6 / 10.8, [8192,3072] 32 / 24, [65536,2560] 144 / 118), but for many short rows of LayerNorm, which come to its vector instructions
+// ([32768,512] 20.2 / 22.0, [65536,768] 50.7 / 56.5).  In f16 one row in ten has its squares, and of 2560 columns one in fifty its values
+// added in order, 1 to 4 us a wave.  RMSNorm still gains ([256,2560] 10.2 / 6.1, [4096,3072] 14.3 / 12.9, [32768,1280] 35.7 / 29.8), except where
+// the walk takes its rows in one or two rounds ([8192,1280] 9.3 / 10.9, [10240,1536] 12.7 / 14.1, [6144,4096] 21.8 / 22.8).  LayerNorm, with both sums
+// to be sure of, gains in small numbers, where the walk's latency is the launch ([256,2560] 11.9 / 8.5, [1024,2560] 12.2 / 10.9, but [2048,2560]
+// 12.3 / 12.9 and [1024,3072] 13.8 / 13.2, [1024,4096] 16.0 / 17.7), and in large ones of 1280 to 2560 columns ([32768,1280] 38.7 / 33.5, [65536,2560] 125 / 119).
+inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
+    if (cols <= 256 || cols > NR_MAX_COLS || rows > 0x7fffffffull) return false;
+    if (bf16) return !layer || cols > 1024 || rows <= (cols > 512 ? 128 : 48) * cus;
+    if (!layer) return rows <= 16 * cus || (rows > 28 * cus && cols >= 3072) || rows > 48 * cus;
+    if (rows <= 4 * cus) return cols <= 2560 || (rows <= cus && cols <= 4608);
+    return rows > 60 * cus && cols >= 1280 && cols <= 2560;
+}
+// Where norm_flow16_kernel takes the rest of them, against norm_pipe16_kernel, whose blocks of 8 rows share the CUs and overlap one another,
 // while rows fit the chip in a few rounds, and which needs no empty steps.  Many rows come to memory, which that one
-// reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51, RMSNorm bf16 [12288,3072] 47 / 34).  Up to 40
-// rows a CU, f16 and RMSNorm gain on rows of more than 3072 columns that fill the steps (RMSNorm f16 [7000,4096] 27.8 / 23.5,
-// against [5000,3328] 17.6 / 18.9), RMSNorm in bf16 more widely ([2048,4104] 25.6 / 20).  bf16 LayerNorm, whose walker
-// needs the f32 tiles of both sums, gains in a single round of 8 rows a block ([2048,2560] 16.3 / 14.6, not three tiles in
-// four steps or five in eight: [2048,1280] 9.7 / 10.2) and once its blocks of 8 rows no longer keep their rows in LDS
-// ([7000,2560] 35 / 25.6; [5000,2560] 21.3 / 25.8), except for short rows and for 9000 to 10000 rows in steps a quarter empty
-// ([9000,1280] 22.7 / 26.1, [9000,1792] 29.4 / 27.9).
+// reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51).  Up to 40 rows a CU, f16 gains on rows of more than 3072 columns
+// that fill the steps (RMSNorm [7000,4096] 27.8 / 23.5, against [5000,3328] 17.6 / 18.9).
 inline bool nf_takes_aligned(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
-    const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);
-    if (bf16 && layer) {
-        if (rows <= 8 * cus) return cols > 768 && nt != 5;
-        if (rows <= 16 * cus) return cols > 3328;
-        if (rows <= 24 * cus || cols <= 128) return false;
-        if (cols <= 256) return rows > 48 * cus;
-        if (rows <= 32 * cus || rows > 42 * cus) return true;
-        return nt * 5 >= steps * 4;
-    }
-    // (bf16: not the row counts around 64 a CU, three rounds of 22 rows here and whole rounds there, in steps a quarter empty:
-    // RMSNorm [16384,1280] 23.8 / 25.9)
-    if (rows > 40 * cus) return cols > 512 && !(bf16 && nt * 5 < steps * 4 && rows > 60 * cus && rows <= 66 * cus);
+    if (bf16) return layer && cols > 128 && rows > 48 * cus;
+    if (rows > 40 * cus) return cols > 512;
     if (cols <= 3072) return false;
-    if (bf16) {
-        if (rows <= 16 * cus) return true;
-        if (rows <= 24 * cus) return cols > 3584;
-        return rows <= 32 * cus || nt == steps;
-    }
+    const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);
     if (nt == steps) return layer || rows > 8 * cus;
     return layer && rows >= 64 && rows <= 16 * cus && cols > 3328;
 }
@@ -1662,15 +1331,9 @@ template <typename T, int KIND>
 int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
     const bool vec_ok = (cols % 8 == 0) && rt_aligned(x, 16) && rt_aligned(y, 16) && rt_aligned(scale, 16) && (!bias || rt_aligned(bias, 16));
     if (vec_ok && cols <= 128 && rows >= 16384) return launch_norm16_lane<T, KIND>(dev, x, scale, bias, y, rows, cols, eps);
-    // RMSNorm rows of 256 to 4096 columns, as many of them as the walk below takes in one round (8 rows a block, two
-    // blocks a CU): the row sum replayed by a whole wave per row.  That kernel issues about twice the instructions of
-    // the walk and a row takes a wave about 2.5 us, so it pays where the walk's latency is what the launch costs
-    // ([4096,3072] f16: 12.5 against 14.2 us, [2048,2560] 8.8 against 10.6, [1024,4096] 9.2 against 14.5) and loses
-    // where rows come in several rounds ([8192,3072] 25.5 against 22.1 us, [65536,512] 43 against 25).
-    if (vec_ok && KIND == NORM_RMS && cols >= 256 && cols <= 4096 && rows <= 16ull * (uint64_t)dev->num_cus)
-        return launch_rms16_par<T>(dev, x, scale, y, rows, cols, eps);
     const uint64_t cus = (uint64_t)dev->num_cus;
     constexpr bool BF16 = std::is_same<T, bf16_t>::value, LAYER = KIND == NORM_LAYER;
+    if (vec_ok && nr_takes(BF16, LAYER, rows, cols, cus)) return rt_norm16_row(dev, BF16, KIND, x, scale, bias, y, rows, cols, eps);
     if (cols >= 8 && cols <= NF_MAX_COLS &&
         (vec_ok ? nf_takes_aligned(BF16, LAYER, rows, cols, cus) : nf_takes_ragged(BF16, LAYER, rows, cols, cus))) {
         // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; fewer where that takes no more

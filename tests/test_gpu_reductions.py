@@ -703,6 +703,51 @@ def test_rms_norm_16_bit_row_sums_replayed_in_parallel(dev, oracle, cols, kind):
     assert bad_rows.size == 0, (kind, cols, bad_rows[:10].tolist())
 
 
+@pytest.mark.parametrize("cols", [264, 512, 520, 1032, 2560, 4608, 5120])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_sums_in_any_order_where_the_rounding_is_sure(dev, oracle, cols, kind):
+    """norm16_row_kernel adds a row in any order unless the rounding of the ordered f32 sum could hang on it: rows on either side
+    of that.  Sums of x put next to the middle between two values of the type, constant rows (every partial sum of the squares on
+    the middle sooner or later), sums that cancel, terms far below the sum's last bit, infinities of one and of both signs, NaN,
+    zeros of both signs; into another buffer and in place, with and without a bias."""
+    rng = np.random.default_rng(317 + cols)
+    bf = kind == "bf16"
+    conv = _conv16(oracle, kind)
+    widen = (lambda a: (np.asarray(a).view(np.uint16).astype(np.uint32) << 16).view(np.float32)) if bf else (lambda a: np.asarray(a).astype(np.float32))
+    rows = [rng.standard_normal(cols) for _ in range(24)] + [rng.standard_normal(cols) * 0.1 + 3.0 for _ in range(4)]
+    for _ in range(24):                                                                               # one term takes the sum to a middle
+        r = widen(conv(rng.standard_normal(cols).astype(np.float32))).astype(np.float64)
+        r[cols // 2] = 0.0
+        total = r.sum()
+        step = 2.0 ** (np.floor(np.log2(abs(total))) - (7 if bf else 10))
+        r[cols // 2] = (np.floor(total / step) + 0.5) * step - total
+        rows.append(r)
+    rows += [np.full(cols, v) for v in (1.0, 1.5, -0.75, 3.0, 2.0 ** -13)]
+    rows += [np.where(np.arange(cols) % 2 == 0, 1.0, -1.0) * rng.standard_normal() + 1e-3 * rng.standard_normal(cols) for _ in range(4)]
+    rows += [np.concatenate([rng.standard_normal(cols // 2) * 1e-4, rng.standard_normal(cols - cols // 2)]) * s for s in (1.0, 30.0)]
+    rows += [rng.standard_normal(cols) * 10.0 ** rng.integers(-6, 3, cols) for _ in range(4)]
+    rows += [rng.standard_normal(cols) * s for s in ((1e-4, 100.0) if not bf else (1e-39, 1e-20, 1e18, 2e38))]
+    rows += [np.zeros(cols), -np.zeros(cols), rng.standard_normal(cols) * (rng.random(cols) < 0.02)]
+    for at in ((3,), (3, cols - 5), (0, cols // 2, cols - 1)):
+        r = rng.standard_normal(cols)
+        r[list(at)] = [np.inf, -np.inf, np.nan][: len(at)] if len(at) < 3 else [np.inf, np.inf, np.nan]
+        rows.append(r)
+    with np.errstate(over="ignore"):
+        x = conv(np.stack(rows).astype(np.float32))
+    w, b = conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols))
+    top = 0x7f80 if bf else 0x7c00
+    dw, db = dev.upload(w, bf16=bf), dev.upload(b, bf16=bf)
+    for name, want, run in (("layer", oracle.layer_norm(x, w, b, 1e-5, bf16=bf, intended=True), lambda d, o: dev.layer_norm(d, dw, db, 1e-5, out=o)),
+                            ("layer, no bias", oracle.layer_norm(x, w, None, 1e-5, bf16=bf, intended=True), lambda d, o: dev.layer_norm(d, dw, None, 1e-5, out=o)),
+                            ("rms", oracle.rms_norm(x, w, 1e-5, bf16=bf, intended=True), lambda d, o: dev.rms_norm(d, dw, 1e-5, out=o))):
+        for in_place in (False, True):
+            dx = dev.upload(x, bf16=bf)
+            out = run(dx, dx if in_place else dev.upload(np.zeros_like(x), bf16=bf))
+            g, t = np.asarray(out.to_numpy()).view(np.uint16), np.asarray(want).view(np.uint16)
+            same = (g == t) | (((g & 0x7fff) > top) & ((t & 0x7fff) > top))
+            assert same.all(), (name, in_place, cols, kind, np.flatnonzero(~same.all(axis=1))[:10].tolist())
+
+
 @pytest.mark.parametrize("rows,cols,kind", [(20000, 8, "f16"), (16384 + 3, 64, "f16"), (17000, 128, "f16"), (30000, 24, "bf16"), (16500, 120, "bf16")])
 def test_norms_16_bit_many_narrow_rows(dev, oracle, rows, cols, kind):
     """tens of thousands of rows of at most 128 columns take a kernel with one lane per row; same bits as the walkers"""
