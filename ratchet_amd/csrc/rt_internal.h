@@ -41,6 +41,7 @@ struct rt_device {
     uint64_t sp_attr_set;   // streaming softmax instantiations whose dynamic-LDS limit has been raised on this device
     uint64_t sp_ragged_attr_set;   // the same for the ragged-row variants
     uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads (bits 0..15) and for those of f16 rows of 4097 to 8192 columns
+    uint64_t sr_attr_set;          // the same for the wave-per-rows softmax (rt_softmax_row.hip), two bits an instantiation of ten in f16 and sixteen in bf16
     unsigned ry_attr_set;          // the same for the one-wave-per-row softmax (rt_softmax_replay.hip)
     // one word per 512-column tile of the mask of a masked streaming softmax (allocated with the device): the
     // tile's value twice when all its elements are equal, 0xffffffff when the tile has to be loaded; the first RT_SM_TILES_HEAD
@@ -123,6 +124,8 @@ int rt_unary_table(rt_device* dev, int type_index, int op, const uint16_t** out)
 int rt_softmax_stream_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
 int rt_softmax_stream_bf16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
 
+// The 16-bit reference softmax with two or four rows to a wave (rt_softmax_row.hip); arguments as above.  RT_OK with *done = false where it is not the faster way
+int rt_softmax_row(rt_device* dev, bool bf16, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
 // The f16 reference softmax for a few long rows, one wave per row (rt_softmax_replay.hip); arguments as above
 int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
 

@@ -253,6 +253,8 @@ __global__ void __launch_bounds__(RY_BLOCK) softmax16_replay_kernel(const uint16
 // after the other: [32, 2048] 13.3 -> 9.4 us, [32, 4096] 22.6 -> 12.0 us, [32, 8192] 48.6 -> 20 us, [256, 2048]
 // 13.5 -> 10.4 us, [256, 4096] 22.9 -> 14.3 us; rows of 1024 columns lose (8.8 -> 10 us: the ordered pass costs 4 us
 // whatever the row length), and from four rows per CU the streaming kernel's overlap wins.
+// Over 2048 columns softmax16_row_kernel comes first and leaves it up to 64 rows of 3073 to 4096 columns and masks whose rows are not shared by an
+// even number of the others.
 // Returns RT_OK with *done = false when the shape does not fit.
 int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done) {
     *done = false;

@@ -77,3 +77,44 @@ def test_rows_of_4097_to_8192_columns_around_a_round(dev, oracle, heads, rows, c
     for out in (None, dx):
         got = dev.softmax_masked(dx, dev.upload(m), out=out) if masked else dev.softmax(dx, out=out)
         assert _same(got.to_numpy(), want, False)
+
+
+def _hard_rows(rng, cols, bf):
+    """rows whose sums run through subnormals, ties and many powers of two, stop growing, pass infinity, meet NaN or are all masked"""
+    rows = [rng.standard_normal(cols) * s + m for s, m in ((1, 0), (2, 0), (4, -3), (0.3, 5), (1, -14), (1, -16), (0.01, 0), (8, -8), (1, 6))]
+    rows += [np.full(cols, v) for v in (0.0, -1.0, 3.0, -7.0, -9.7, 8.0, 12.0, -np.inf)]
+    rows += [rng.standard_normal(cols) * s + m for s, m in (((1, -85), (2, -90), (1, 85), (3, 80)) if bf else ((3, 4),))]
+    rows += [np.sort(rng.standard_normal(cols) * 3), -np.sort(rng.standard_normal(cols) * 3), np.linspace(-17, 5, cols)]
+    for k in (1, 8, 31, 33, cols // 2, cols - 1):
+        rows += [np.where(np.arange(cols) < k, rng.standard_normal(cols), -np.inf), np.where(np.arange(cols) < k, -np.inf, rng.standard_normal(cols))]
+    for at, v in ((0, 11.2), (cols - 1, np.inf), (5, np.inf), (cols // 2, np.nan), (cols - 1, np.nan)):
+        rows.append(np.where(np.arange(cols) == at, v, rng.standard_normal(cols)))
+    rows.append(np.where(np.arange(cols) % max(cols - 1, 1) == 0, np.where(np.arange(cols) == 0, np.inf, np.nan), 1.0))
+    return np.stack(rows)
+
+
+@pytest.mark.parametrize("kind,heads,rows,cols", [
+    ("f16", 2, 33, 2056), ("f16", 2, 33, 3072), ("f16", 2, 40, 3080), ("f16", 4, 40, 4096), ("f16", 2, 33, 4104), ("f16", 2, 33, 5128), ("f16", 6, 35, 6144),
+    ("f16", 2, 33, 7176), ("f16", 2, 33, 8184), ("f16", 2, 33, 8192),
+    ("f16", 4, 3850, 257), ("f16", 4, 3850, 511), ("f16", 4, 3850, 513), ("f16", 4, 3841, 1001), ("f16", 4, 3850, 1537), ("f16", 4, 3850, 2047),
+    ("bf16", 4, 33, 1032), ("bf16", 4, 33, 1536), ("bf16", 4, 33, 2048), ("bf16", 2, 33, 2057), ("bf16", 2, 33, 2056), ("bf16", 2, 33, 4095), ("bf16", 2, 33, 4096),
+    ("bf16", 2, 33, 4104), ("bf16", 2, 33, 7168), ("bf16", 2, 33, 8192), ("bf16", 4, 10241, 264), ("bf16", 4, 10241, 520), ("bf16", 4, 3850, 1023)])
+def test_several_rows_to_a_wave(dev, oracle, kind, heads, rows, cols):
+    """softmax16_row_kernel at the edges of its chunks, of both its lane counts and of rows a wave; plain (an odd number of rows
+    among them), under a mask and in place"""
+    bf = kind == "bf16"
+    rng = np.random.default_rng(cols)
+    hard = _hard_rows(rng, cols, bf)
+    n = heads * rows
+    x = hard[rng.integers(0, len(hard), n)] if n > 2 * len(hard) else np.concatenate([hard, rng.standard_normal((max(n - len(hard), 0), cols))])[:n]
+    x = _to(oracle, x, bf).reshape(1, heads, rows, cols)
+    m = np.where(rng.random((rows, cols)) < 0.1, -np.inf, 0.5 * rng.standard_normal((rows, cols)))
+    m[0] = -np.inf
+    m = _to(oracle, m, bf)
+    dx, dm = dev.upload(x, bf16=bf), dev.upload(m, bf16=bf)
+    want = oracle.softmax(oracle.binary("add", x, np.ascontiguousarray(np.broadcast_to(m, x.shape)), bf16=bf), bf16=bf)
+    assert _same(dev.softmax_masked(dx, dm).to_numpy(), want, bf)
+    odd = np.ascontiguousarray(x.reshape(1, n, cols)[:, : n - 1])
+    assert _same(dev.softmax(dev.upload(odd, bf16=bf)).to_numpy(), oracle.softmax(odd, bf16=bf), bf)
+    dev.softmax(dx, out=dx)
+    assert _same(dx.to_numpy(), oracle.softmax(x, bf16=bf), bf)
