@@ -921,7 +921,7 @@ extern "C" int rt_softmax(rt_device* dev, int dt, const void* x, void* y, uint64
     switch (dt) {
         case RT_F32: return launch_f32_style<float, 0>(dev, x, y, rows, cols);
         default: {
-            // 16-bit types, rows that are whole aligned vectors: one pass; up to 128 columns (and enough rows to fill the chip) a lane per row, up to 4096
+            // 16-bit types, rows that are whole aligned vectors: one pass; several rows to a wave where that is the fastest (sr_takes); up to 128 columns (and enough rows to fill the chip) a lane per row, up to 4096
             // columns (f16: 8192, where that is the faster way) streamed with the row held in registers, longer ones parked in y (also small problems: the per-block table load costs about 5 us, the two-pass walker
             // more); everything else takes the two-pass tile walker
             // (rows that are not whole vectors stream from their first element on, the last vector over the one before it: [4096, 1001]

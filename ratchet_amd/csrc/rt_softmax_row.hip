@@ -199,7 +199,7 @@ __device__ __forceinline__ void sr_transpose(v4u (&v)[4], uint32_t lane) {
 // store, and its waves never meet: no walker, no barriers.  A chunk is 32 L columns of each row, four vectors a lane.  The loads of the next
 // rows go out between the stores of these, into the registers that those free.  The exp table lies in LDS as in softmax16_stream_kernel.
 // What bounds it: a quarter of the time is the sums and their waits (without them, and wrong, [8,2048,8192] f16 takes 100 us of 114, with a mask 114 of 125), the
-// rest memory, which 16 free-running waves a CU use less evenly than the streaming kernel's paced steps do (5.4 against 6.2 TB/s on f16 [32,4096,4096]; held to a
+// rest memory, which 16 free-running waves a CU use less evenly than the streaming kernel's paced steps do (5.1 against 6.2 TB/s on f16 [32,4096,4096]; held to a
 // pace these waves only get slower).  Several rows at a time because a row needs a pass for each chunk and for each power of two that its
 // sum passes, most of which fall together: with one row to a wave [8,2048,8192] bf16 took 159 us without a mask and 177 with one, now 122 and 139.
 // bf16 pays five instructions an element and pass, f16 one.
