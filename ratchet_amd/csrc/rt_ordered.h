@@ -17,9 +17,11 @@
 #ifndef RT_ORDERED_H
 #define RT_ORDERED_H
 
-#include "rt_arith.h"
-#include "rt_internal.h"
+#include <cmath>
+#include <cstdint>
 
+// (v4u, u2f, f2u and wave_max come from the includer, rt_arith.h on the GPU: the text is compiled for the host as well, where
+// tests/ordered_sums_check.cpp compares the 64 lanes' sums with the plain ones)
 namespace {
 
 // inclusive prefix sum over the 64 lanes, by DPP moves inside rows of 16 and from row to row
@@ -70,70 +72,6 @@ __device__ __forceinline__ double lane_value(double v, uint32_t lane) {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
     return __builtin_bit_cast(double, (uint64_t)lane_value((uint32_t)(u >> 32), lane) << 32 | lane_value((uint32_t)u, lane));
 }
-
-// The f32 chain of 16-bit terms.  MANT: mantissa bits of the running sum's type, INF: its infinity's bit pattern.  pair(a, b) starts two sums at two bit
-// patterns, run() adds a vector's eight terms to both, lo() and hi() are the sums' bit patterns; one() adds to a single sum.
-template <typename T> struct ChainF32;
-template <> struct ChainF32<half_t> {
-    static constexpr int MANT = 23;
-    static constexpr uint32_t INF = 0x7f800000u;
-    struct Pair {
-        float a, b;
-    };
-    static __device__ __forceinline__ Pair pair(uint32_t a, uint32_t b) { return Pair{u2f(a), u2f(b)}; }
-    static __device__ __forceinline__ uint32_t lo(const Pair& p) { return f2u(p.a); }
-    static __device__ __forceinline__ uint32_t hi(const Pair& p) { return f2u(p.b); }
-    // 1.0 * widen(h) + sum, one instruction with one rounding
-#define RT_MIX2(N)                                                              \
-    "v_fma_mix_f32 %0, %" #N ", %6, %0 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %1, %" #N ", %6, %1 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %0, %" #N ", %6, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"       \
-    "v_fma_mix_f32 %1, %" #N ", %6, %1 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"
-    static __device__ __forceinline__ void run(Pair& p, const v4u& v) {
-        const float one = 1.0f;
-        asm(RT_MIX2(2) RT_MIX2(3) RT_MIX2(4) RT_MIX2(5) : "+v"(p.a), "+v"(p.b) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(one));
-    }
-#undef RT_MIX2
-#define RT_MIX1(N)                                                              \
-    "v_fma_mix_f32 %0, %" #N ", %5, %0 op_sel_hi:[1,0,0]\n"                      \
-    "v_fma_mix_f32 %0, %" #N ", %5, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n"
-    static __device__ __forceinline__ uint32_t one(uint32_t s, const v4u& v) {
-        float a = u2f(s);
-        const float one = 1.0f;
-        asm(RT_MIX1(1) RT_MIX1(2) RT_MIX1(3) RT_MIX1(4) : "+v"(a) : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(one));
-        return f2u(a);
-    }
-#undef RT_MIX1
-};
-template <> struct ChainF32<bf16_t> {
-    static constexpr int MANT = 23;
-    static constexpr uint32_t INF = 0x7f800000u;
-    struct Pair {
-        float a, b;
-    };
-    static __device__ __forceinline__ Pair pair(uint32_t a, uint32_t b) { return Pair{u2f(a), u2f(b)}; }
-    static __device__ __forceinline__ uint32_t lo(const Pair& p) { return f2u(p.a); }
-    static __device__ __forceinline__ uint32_t hi(const Pair& p) { return f2u(p.b); }
-    static __device__ __forceinline__ void run(Pair& p, const v4u& v) {
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            const float l = u2f(v[w] << 16), h = u2f(v[w] & 0xffff0000u);
-            p.a += l;
-            p.b += l;
-            p.a += h;
-            p.b += h;
-        }
-    }
-    static __device__ __forceinline__ uint32_t one(uint32_t s, const v4u& v) {
-        float a = u2f(s);
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-            a += u2f(v[w] << 16);
-            a += u2f(v[w] & 0xffff0000u);
-        }
-        return f2u(a);
-    }
-};
 
 // s, the same in all lanes: the bit pattern of a running sum of terms >= 0 (or NaN).  Returns that of the sum after the 64 runs of NV
 // vectors, lane 0's first.  At the start of a row, where the sum doubles every few lanes, SERIAL lanes are added one by one.
@@ -195,6 +133,116 @@ __device__ __forceinline__ uint32_t ordered_add(uint32_t s, const v4u (&v)[NV], 
     for (int k = 0; k < NV; k++) t = C::one(t, v[k]);
     const uint64_t other = __builtin_amdgcn_ballot_w64(lane >= from && t != s);
     return other ? lane_value(t, __builtin_ctzll(other)) : s;
+}
+
+// the ulp of the binade of m (m finite, at least 2^-103; zero below that)
+__device__ __forceinline__ float nr_ulp(float m) {
+    const uint32_t e = f2u(m) >> 23;
+    return e > 23 ? u2f((e - 23) << 23) : 0.0f;
+}
+// what f, a value of a 16-bit type, is off the nearest multiple of u = magic * 2^-23 / 1.5, a power of two or zero: zero, or NaN for inf and
+// NaN, if it is none.  (Up to 2^22 u the sum has the ulp u; values beyond 2^11 u have no bit below u.)
+__device__ __forceinline__ float nr_off(float f, float magic) {
+    return f - ((f + magic) - magic);
+}
+
+// Both ordered sums take a step of 512 columns, 64 vectors, one a lane.
+//
+// x's: up to a lane the sum runs exactly, and is q (in double), as long as the lanes before it are `easy`: their terms and their q are
+// multiples of the ulp of the binade that their partial sums stay in, and so are their own sums, added up from zero, which can
+// reach twice as far as the running sum does (from -0.9 to 0.9 of the binade, say) and must not round on the way.  The first lane that is
+// not easy adds its eight terms to the exact sum for real, and the lanes behind it start from there.
+// N::widen(x, f): a vector's eight values as floats.
+template <class N>
+__device__ __forceinline__ float norm_ordered_sum(float s, const v4u& x, uint32_t lane) {
+    float f[8], part = 0.0f, low = 0.0f, high = 0.0f;        // a lane's sum, the ends of its partial sums
+    N::widen(x, f);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        part += f[k];
+        low = fminf(low, part);
+        high = fmaxf(high, part);
+    }
+    const float guess = s + lane_before(lanes_scan(part)), near = fmaxf(guess + high, -(guess + low));       // (nothing rests on the guess)
+    const float ulp = nr_ulp(near), coarse = nr_ulp(u2f(__builtin_amdgcn_readfirstlane(f2u(wave_max(near)))));
+    float rest = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) rest += fabsf(nr_off(f[k], ulp * 0x1.8p23f));
+    // (terms far below the coarsest ulp would not be exact in the doubles either: such lanes add for real.  A sum of 2^24 ulp may have been
+    // rounded to that, one of less has not been)
+    const float exact = ulp * 0x1p24f;
+    const bool plain = (ulp > 0.0f) & (ulp >= coarse * 0x1p-20f) & (coarse < 0x1p100f) & (rest == 0.0f) & (high < exact) & (low > -exact);
+    const double mine = plain ? (double)part : 0.0, upto = lanes_scan(mine), before = upto - mine;
+    const double limit = (double)ulp * 0x1p24, magic = (double)ulp * 0x1.8p52;       // sums up to the limit in steps of ulp are f32 values
+    const double above = limit - (double)high, below = -limit - (double)low;
+    const double grid = (double)coarse * 0x1.8p30;           // multiples of coarse * 2^-22
+    double off = (double)s;                                  // the running sum less `before`, or, odd, what a double cannot hold:
+    bool odd = !((off + grid) - grid == off);                // then the next lane adds to s itself
+    for (uint32_t from = 0; from < 64;) {
+        const double q = off + before;
+        const bool easy = plain & ((q + magic) - magic == q) & (q <= above) & (q >= below);
+        const uint64_t hard = (odd ? ~0ull : __builtin_amdgcn_ballot_w64(!easy)) & (~0ull << from);
+        if (hard == 0) return (float)(off + lane_value(upto, 63));
+        const uint32_t l = __builtin_ctzll(hard);
+        float t = (odd & (lane == from)) ? s : (float)q;
+#pragma unroll
+        for (int k = 0; k < 8; k++) t += f[k];
+        const uint64_t even = __builtin_amdgcn_ballot_w64(((double)t + grid) - grid == (double)t);
+        s = u2f(lane_value(f2u(t), l));
+        off = lane_value((double)t - upto, l);
+        odd = !((even >> l) & 1);
+        from = l + 1;
+    }
+    return s;
+}
+
+// T(x*x)'s (v: the squares, s: the sum's bit pattern).  From approximate sums in front of the lanes every lane takes the binade it adds in; a lane
+// is clean if its run starts and ends there, with a margin for what the approximation can be off by.  Pairs of distances as in
+// ordered_add; the parity in front of a lane is followed for both parities that its stretch of clean lanes can start with, and the
+// distances are summed under both.  Then the lanes that are not clean (about eight of a row, where the sum passes a power of two)
+// are taken in order: the stretch in front of one is a single addition, its own run is added for real.  What the approximation claims is checked
+// on the exact sum, and a step on which it fails goes through ordered_add.
+template <class C>
+__device__ __forceinline__ uint32_t norm_ordered_squares(uint32_t s, const v4u& v, uint32_t lane) {
+    const uint32_t start = s;
+    const float run = u2f(C::one(0, v)), upto = lanes_scan(run), carry = u2f(s);
+    const uint32_t e = f2u((carry + upto) * (1.0f + 0x1p-10f)) >> 23;
+    const bool clean = (e - 2 < 252) & (f2u((carry + (upto - run)) * (1.0f - 0x1p-10f)) >> 23 == e);
+    const uint32_t base = e << 23;
+    typename C::Pair p = C::pair(base, base + 1);
+    C::run(p, v);
+    const uint32_t d0 = clean ? C::lo(p) - base : 0, d1 = clean ? C::hi(p) - (base + 1) : 0;
+    const uint64_t dirty = __builtin_amdgcn_ballot_w64(!clean);
+    const uint64_t odd = __builtin_amdgcn_ballot_w64(d0 & 1u), tie = __builtin_amdgcn_ballot_w64(d0 != d1);
+    const uint32_t flip = __builtin_amdgcn_mbcnt_hi((uint32_t)(odd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)odd, 0));
+    const uint64_t flips = __builtin_amdgcn_ballot_w64(flip & 1u);
+    const uint64_t set = tie | dirty, gen0 = set & flips, gen1 = gen0 ^ dirty;
+    const uint64_t prop0 = gen0 | ~set, prop1 = gen1 | ~set;
+    const uint32_t u0 = lanes_scan(__builtin_amdgcn_inverse_ballot_w64(((prop0 + gen0) ^ prop0 ^ gen0) ^ flips) ? d1 : d0);
+    const uint32_t u1 = lanes_scan(__builtin_amdgcn_inverse_ballot_w64(((prop1 + gen1 + 1) ^ prop1 ^ gen1) ^ flips) ? d1 : d0);
+    bool failed = false;
+    uint64_t todo = dirty;
+    uint32_t from = 0, c0 = 0, c1 = 0;
+    for (;;) {
+        const uint32_t at = todo ? __builtin_ctzll(todo) : 64, last = at < 64 ? at : 63;             // (a dirty lane's own distance is zero)
+        const uint32_t n0 = lane_value(u0, last), n1 = lane_value(u1, last), eb = lane_value(base, at ? at - 1 : 0);
+        if (at > from) {
+            failed |= (s ^ eb) >> 23 != 0;
+            s += s & 1u ? n1 - c1 : n0 - c0;
+            failed |= (s ^ eb) >> 23 != 0;
+        }
+        if (at == 64) break;
+        s = lane_value(C::one(s, v), at);
+        c0 = n0;
+        c1 = n1;
+        from = at + 1;
+        todo &= todo - 1;
+    }
+    if (failed) {
+        const v4u one[1] = {v};
+        s = ordered_add<C, 1, 3>(start, one, lane);
+    }
+    return s;
 }
 
 }  // namespace

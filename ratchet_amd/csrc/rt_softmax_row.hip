@@ -2,8 +2,8 @@
 // (rt_ordered.h; arithmetic and table: rt_softmax_stream.h).
 #include <cmath>
 
-#include "rt_ordered.h"
 #include "rt_softmax_stream.h"
+#include "rt_ordered.h"
 
 namespace {
 

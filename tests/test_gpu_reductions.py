@@ -748,6 +748,47 @@ def test_norms_16_bit_sums_in_any_order_where_the_rounding_is_sure(dev, oracle, 
             assert same.all(), (name, in_place, cols, kind, np.flatnonzero(~same.all(axis=1))[:10].tolist())
 
 
+@pytest.mark.parametrize("cols", [264, 512, 1032, 2560, 5120])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_layer_norm_16_bit_sums_that_cancel(dev, oracle, cols, kind):
+    """Rows whose sum comes back to about zero after large excursions: values and their negatives shuffled (of one size, of many, cubed), rows
+    with their mean taken off, runs of eight that swing between signs, and a run whose own sum has more bits than f32 holds where the running sum does
+    not.  No bound settles what such a sum rounds to: the wave-per-row kernel has to add it in order.  Compared over the whole
+    launch, which is few enough rows for that kernel, and over half of the rows with zeros in them, whose outputs show the mean."""
+    rng = np.random.default_rng(331 + cols)
+    bf = kind == "bf16"
+    conv = _conv16(oracle, kind)
+    rows = []
+
+    def both(v):
+        rows.append(rng.permutation(np.concatenate([v, -v])))
+
+    for k in range(60):
+        half = rng.standard_normal(cols // 2)
+        both(half)
+        both(half * 2.0 ** -rng.integers(0, 18 if bf else 10, cols // 2))
+        both(half ** 3)
+        full = rng.standard_normal(cols) * (1.0 if k % 2 else 1.0 + rng.standard_normal(cols) ** 2)
+        rows.append(full - full.mean())
+        swing = np.where(np.arange(cols) // 8 % 2, 1.0, -1.0) * 20.0 * (1 + 0.3 * rng.standard_normal(cols)) * np.where(rng.random(cols) < 0.25, 2.0 ** -rng.integers(0, 24, cols), 1.0)
+        rows.append(swing)
+    lead = {"f16": [(0, -127.0), (8, 100.0), (9, 50.0), (10, 2.0 ** -17), (16, 2.0 ** -7)],
+            "bf16": [(k, -3063808.0) for k in range(5)] + [(8, 1.0)] + [(k, 3506176.0) for k in range(9, 16)] + [(16, -9240576.0), (17, 16384.0)]}[kind]
+    for sign in (1.0, -1.0):
+        r = np.zeros(cols)
+        for at, v in lead:
+            r[at] = sign * v
+        rows.append(r)
+        r = np.zeros(cols)                                                                          # a run of 2^24 + 1 of its last bits
+        r[[0, 8, 9, 10, 16]] = np.array([-5.0, 4.0, 4.0, 2.0 ** -21, 2.0 ** -7]) * sign
+        rows.append(r)
+    x = np.stack(rows).astype(np.float32)
+    x[::2][rng.random((x[::2].shape)) < 0.02] = 0.0
+    x = conv(x)
+    assert len(x) <= 1024
+    _norms_16_bit(dev, oracle, x, conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), bf, 0, 0)
+
+
 @pytest.mark.parametrize("rows,cols,kind", [(20000, 8, "f16"), (16384 + 3, 64, "f16"), (17000, 128, "f16"), (30000, 24, "bf16"), (16500, 120, "bf16")])
 def test_norms_16_bit_many_narrow_rows(dev, oracle, rows, cols, kind):
     """tens of thousands of rows of at most 128 columns take a kernel with one lane per row; same bits as the walkers"""
