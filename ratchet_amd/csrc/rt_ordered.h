@@ -172,6 +172,9 @@ __device__ __forceinline__ float norm_ordered_sum(float s, const v4u& x, uint32_
     // rounded to that, one of less has not been)
     const float exact = ulp * 0x1p24f;
     const bool plain = (ulp > 0.0f) & (ulp >= coarse * 0x1p-20f) & (coarse < 0x1p100f) & (rest == 0.0f) & (high < exact) & (low > -exact);
+    // no terms but zeros: nothing to add, whatever the sum is (past the row's end, where a sum that has cancelled is below every ulp above, each such
+    // lane took a turn of its own)
+    const bool none = ((x[0] | x[1] | x[2] | x[3]) & 0x7fff7fffu) == 0;
     const double mine = plain ? (double)part : 0.0, upto = lanes_scan(mine), before = upto - mine;
     const double limit = (double)ulp * 0x1p24, magic = (double)ulp * 0x1.8p52;       // sums up to the limit in steps of ulp are f32 values
     const double above = limit - (double)high, below = -limit - (double)low;
@@ -180,7 +183,7 @@ __device__ __forceinline__ float norm_ordered_sum(float s, const v4u& x, uint32_
     bool odd = !((off + grid) - grid == off);                // then the next lane adds to s itself
     for (uint32_t from = 0; from < 64;) {
         const double q = off + before;
-        const bool easy = plain & ((q + magic) - magic == q) & (q <= above) & (q >= below);
+        const bool easy = none | (plain & ((q + magic) - magic == q) & (q <= above) & (q >= below));
         const uint64_t hard = (odd ? ~0ull : __builtin_amdgcn_ballot_w64(!easy)) & (~0ull << from);
         if (hard == 0) return (float)(off + lane_value(upto, 63));
         const uint32_t l = __builtin_ctzll(hard);

@@ -4,7 +4,8 @@
 // swing between signs inside and between the lanes, by up to 2^24 of their last bits; tiny and huge ones; inf and NaN; the rows of
 // `found`.  Sums go on over the steps of a row, from the plain sum of the steps before.
 // Build: g++ -O2 -std=c++17 -ffp-contract=off -I ratchet_amd/csrc.   Usage: ordered_sums_check ROWS
-// prints "sum_f16 <n> sum_bf16 <n> squares_f16 <n> squares_bf16 <n> checked <m>" (n: steps whose sums differ), exit code 0 iff all n are 0.
+// prints "sum_f16 <n> sum_bf16 <n> squares_f16 <n> squares_bf16 <n> turns <k> checked <m>" (n: steps whose sums differ; k: the most exchanges between
+// lanes in a step of short rows that cancel, whose upper lanes have no terms), exit code 0 iff all n are 0 and k is at most MOST_TURNS.
 #include <ucontext.h>
 
 #include <algorithm>
@@ -236,6 +237,19 @@ int main(int argc, char** argv) {
         if (n % 9 == 7 || n % 9 == 8) for (float& f : r) f *= n % 9 == 7 ? 0x1p-50f : 0x1p46f;        // (squares at the ends of bf16)
         bad[3] += differ<true, true>(r);
     }
-    printf("sum_f16 %llu sum_bf16 %llu squares_f16 %llu squares_bf16 %llu checked %llu\n", bad[0], bad[1], bad[2], bad[3], checked);
-    return bad[0] || bad[1] || bad[2] || bad[3];
+    // 40 exchanges for the scans and votes of a step and five for each lane that adds for real: a few, not all that have no terms
+    const unsigned MOST_TURNS = 40 + 5 * 12;
+    unsigned turns = 0;
+    for (int n = 0; n < 40; n++) {
+        std::vector<float> r(512, 0.0f);
+        const int cols = 8 * (2 + below(40));
+        for (int i = 0; i < cols; i += 2) r[i + 1] = -(r[i] = normal(rng));
+        std::shuffle(r.begin(), r.begin() + cols, rng);
+        bad[0] += differ<false, false>(r);
+        turns = std::max(turns, turn[0]);
+        bad[1] += differ<true, false>(r);
+        turns = std::max(turns, turn[0]);
+    }
+    printf("sum_f16 %llu sum_bf16 %llu squares_f16 %llu squares_bf16 %llu turns %u checked %llu\n", bad[0], bad[1], bad[2], bad[3], turns, checked);
+    return bad[0] || bad[1] || bad[2] || bad[3] || turns > MOST_TURNS;
 }
