@@ -1278,7 +1278,7 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
 // to be sure of, gains in small numbers, where the walk's latency is the launch ([256,2560] 11.9 / 8.5, [1024,2560] 12.2 / 10.9, but [2048,2560]
 // 12.3 / 12.9 and [1024,3072] 13.8 / 13.2, [1024,4096] 16.0 / 17.7), and in large ones of 1280 to 2560 columns ([32768,1280] 38.7 / 33.5, [65536,2560] 125 / 119).
 inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
-    if (cols <= 256 || cols > NR_MAX_COLS || rows > 0x7fffffffull) return false;
+    if (cols <= 256 || cols > NR_MAX_COLS || rows > NR_MAX_ROWS) return false;
     if (bf16) return !layer || cols > 1024 || rows <= (cols > 512 ? 128 : 48) * cus;
     if (!layer) return rows <= 16 * cus || (rows > 28 * cus && cols >= 3072) || rows > 48 * cus;
     if (rows <= 4 * cus) return cols <= 2560 || (rows <= cus && cols <= 4608);
@@ -1289,7 +1289,7 @@ inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64
 // reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51).  Up to 40 rows a CU, f16 gains on rows of more than 3072 columns
 // that fill the steps (RMSNorm [7000,4096] 27.8 / 23.5, against [5000,3328] 17.6 / 18.9).
 inline bool nf_takes_aligned(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
-    if (bf16) return layer && cols > 128 && rows > 48 * cus;
+    if (bf16) return layer ? cols > 128 && rows > 48 * cus : cols > 512 && rows > 40 * cus;      // (RMSNorm: rows beyond NR_MAX_ROWS)
     if (rows > 40 * cus) return cols > 512;
     if (cols <= 3072) return false;
     const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);

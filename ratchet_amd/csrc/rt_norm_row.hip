@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(NR_BLOCK) norm16_row_kernel(const T* x, const 
 
 template <typename T, int KIND>
 int launch_norm16_row(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
-    RT_REQUIRE(rows <= 0x7fffffffull, RT_ERR_SIZE, "norm: too many rows");
+    RT_REQUIRE(rows <= NR_MAX_ROWS, RT_ERR_SIZE, "norm: too many rows");
 #define RT_NR(VC)                                                                                                                    \
     case VC:                                                                                                                         \
         hipLaunchKernelGGL((norm16_row_kernel<T, VC, KIND>), dim3((unsigned)rows), dim3(NR_BLOCK), 0, dev->stream, (const T*)x,      \

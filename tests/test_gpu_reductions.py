@@ -789,6 +789,31 @@ def test_layer_norm_16_bit_sums_that_cancel(dev, oracle, cols, kind):
     _norms_16_bit(dev, oracle, x, conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), bf, 0, 0)
 
 
+@pytest.mark.parametrize("norm,kind,rows,cols", [("rms", "bf16", 1 << 26, 520), ("rms", "f16", 1 << 26, 264), ("layer", "bf16", 1 << 26, 264), ("rms", "bf16", (1 << 26) - 1, 264)])
+def test_norms_16_bit_more_rows_than_a_launch_has_waves(dev, oracle, norm, kind, rows, cols):
+    """A launch has fewer than 2^32 threads along x: from 2^26 rows on there are none left for a wave to each row, and a kernel with
+    several rows to a block takes them.  In place, 35 and 70 GB; the rows at both ends and in the middle are looked at."""
+    rng = np.random.default_rng(332)
+    bf, conv = kind == "bf16", _conv16(oracle, kind)
+    part = conv(rng.standard_normal((128, cols)) + 0.1)
+    w, b = conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols))
+    dw, db = dev.upload(w, bf16=bf), dev.upload(b, bf16=bf)
+    x = dev.empty((rows, cols), dw.dt)
+    starts = (0, rows // 2 + 3, rows - 128)
+    for at in starts:
+        x.view(at * cols, (128, cols)).upload(part)
+    if norm == "rms":
+        dev.rms_norm(x, dw, 1e-5, out=x)
+        want = oracle.rms_norm(part, w, 1e-5, bf16=bf, intended=True)
+    else:
+        dev.layer_norm(x, dw, db, 1e-5, out=x)
+        want = oracle.layer_norm(part, w, b, 1e-5, bf16=bf, intended=True)
+    for at in starts:
+        assert same_bits(x.view(at * cols, (128, cols)).to_numpy().view(np.uint16), np.asarray(want).view(np.uint16)), at
+    del x
+    dev.pool_trim()
+
+
 @pytest.mark.parametrize("rows,cols,kind", [(20000, 8, "f16"), (16384 + 3, 64, "f16"), (17000, 128, "f16"), (30000, 24, "bf16"), (16500, 120, "bf16")])
 def test_norms_16_bit_many_narrow_rows(dev, oracle, rows, cols, kind):
     """tens of thousands of rows of at most 128 columns take a kernel with one lane per row; same bits as the walkers"""
