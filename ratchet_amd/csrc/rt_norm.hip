@@ -1268,31 +1268,54 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
     if (!bf16) return rows >= (cols > 40 ? 60 : 120) * cus && cols >= 12;
     return (cols >= 40 && rows >= 120 * cus) || (cols >= 24 && rows > 256 * cus);
 }
-// Rows of whole aligned vectors: where a wave per row (rt_norm_row.hip) takes them, timed like the above; us, the best of the others / that one.
-// It adds in any order where the ordered sum's rounding is sure without the order, which in bf16 it nearly always is: bf16 gains from
-// 264 columns up (RMSNorm [256,5120] 21.4 / 10.5, [2048,2560] 14.9 / 8.4, [16384,3072] 40.6 / 35.5, [65536,384] 31.8 / 22.3; LayerNorm [2048,2560]
-// 14.6 / 10.8, [8192,3072] 32 / 24, [65536,2560] 144 / 118), but for many short rows of LayerNorm, which come to its vector instructions
-// ([32768,512] 20.2 / 22.0, [65536,768] 50.7 / 56.5).  In f16 one row in ten has its squares, and of 2560 columns one in fifty its values
-// added in order, 1 to 4 us a wave.  RMSNorm still gains ([256,2560] 10.2 / 6.1, [4096,3072] 14.3 / 12.9, [32768,1280] 35.7 / 29.8), except where
-// the walk takes its rows in one or two rounds ([8192,1280] 9.3 / 10.9, [10240,1536] 12.7 / 14.1, [6144,4096] 21.8 / 22.8).  LayerNorm, with both sums
-// to be sure of, gains in small numbers, where the walk's latency is the launch ([256,2560] 11.9 / 8.5, [1024,2560] 12.2 / 10.9, but [2048,2560]
-// 12.3 / 12.9 and [1024,3072] 13.8 / 13.2, [1024,4096] 16.0 / 17.7), and in large ones of 1280 to 2560 columns ([32768,1280] 38.7 / 33.5, [65536,2560] 125 / 119).
+// Rows of whole aligned vectors: where a wave per row (rt_norm_row.hip) takes them, timed like the above but on 4 kinds of rows; us, the best of the
+// others / that one, for rows of N(0, 1), and where it matters for rows with their mean taken off (c) and the same with four columns 40 times as large (o).
+// It adds in any order where the ordered sum's rounding is sure without the order.  For the squares that hangs little on the rows.
+//   RMSNorm bf16, nearly always sure: from 264 columns up ([256,5120] 22.0 / 10.8, [2048,2560] 9.5 / 8.6, [16384,3072] 40.7 / 37.2, [65536,384] 31.8 / 22.3).
+//   RMSNorm f16, one row in ten open, 1 to 4 us a wave: up to 16 rows a CU (against a kernel that is gone: [4096,264] 7.8 / 5.7, [4096,1280] 9.1 / 7.9, [1024,5120] 18.6 / 11.3; of 3072 to
+//     4096 columns and 32 to 128 rows no gain, 6.9 / 6.9, and rows whose squares are subnormal 6.6 / 7.2); then where the walk takes its rows in many
+//     rounds ([16384,320] 9.6 / 8.0, [16384,1280] 21.3 / 18.0, [16384,2560] 34.3 / 32.6; [14000,1792] 19.9 / 20.9; [16384,264] 9.5 / 10.1), from 3072 columns
+//     where its steps are not full ([10240,3840] 35.5 / 32.8, [16384,4608] 58.5 / 57.1; [12288,3072] 28.7 / 30.7, [7200,4096] 24.6 / 26.9).
+// The sum of x is small against its terms, and of rows with no mean it is nearly all rounding: f16 rows of that kind stay open all of them, bf16 ones one
+// in six, 4 us a wave for 2560 columns.
+//   LayerNorm f16: nowhere (N(0, 1) [32768,1280] 38.7 / 34.2, but c 38.6 / 68; [1024,2560] 12.2 / 12.2, c 12.2 / 15.5; [16,2560] 11.6 / 7.8, c 11.6 / 12.1).
+//   LayerNorm bf16: in small numbers, where the walk's latency is the launch ([1024,2560] 14.6 / 9.4, c 14.7 / 13.0; [1024,264] 6.2 / 4.8, c 6.1 / 5.3;
+//     [1024,5120] 22.9 / 16.0, c 23.0 / 24.0; [2048,1024] 8.1 / 6.9, c 8.2 / 8.9), and in large ones where a quarter of the walk's steps is empty
+//     ([8192,1280] 20.1 / 14.6, c 20.2 / 18.2, o 20.2 / 19.1; [6144,1280] 13.0 / 12.4, c 12.9 / 16.5; [10240,2560] 33.2 / 25.5, c 33.2 / 31.1, o 33.3 / 33.7;
+//     [30000,2560] c 70.7 / 67.2, o 70.6 / 75.3; [8192,1792] 22.4 / 17.8, c 22.3 / 22.4, o 22.4 / 23.9; [8192,3072] 32.5 / 25.6, c 32.5 / 32.2, o 32.6 / 35.0).
+//     (Rows of values and their negatives, whose sum is zero but for the roundings on the way, are open all of them and lose there: [8192,1280] 20.2 / 23.9.)
 inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
     if (cols <= 256 || cols > NR_MAX_COLS || rows > NR_MAX_ROWS) return false;
-    if (bf16) return !layer || cols > 1024 || rows <= (cols > 512 ? 128 : 48) * cus;
-    if (!layer) return rows <= 16 * cus || (rows > 28 * cus && cols >= 3072) || rows > 48 * cus;
-    if (rows <= 4 * cus) return cols <= 2560 || (rows <= cus && cols <= 4608);
-    return rows > 60 * cus && cols >= 1280 && cols <= 2560;
+    if (!layer) {
+        if (bf16 || rows <= 16 * cus) return true;
+        const uint32_t nt = (cols + 255) / 256;
+        if (cols >= 3072) return rows > 28 * cus && nt != nf_steps(nt);
+        return cols >= 320 && rows > (cols <= 1536 ? 48 : 60) * cus;
+    }
+    if (!bf16) return false;
+    if (rows <= (cols <= 4096 ? 4 : 3) * cus) return true;
+    if (cols > 1024 && cols <= 1536) return rows > 28 * cus;
+    return cols > 2048 && cols <= 2560 && rows > 30 * cus && rows <= 64 * cus;
 }
 // Where norm_flow16_kernel takes the rest of them, against norm_pipe16_kernel, whose blocks of 8 rows share the CUs and overlap one another,
 // while rows fit the chip in a few rounds, and which needs no empty steps.  Many rows come to memory, which that one
 // reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51).  Up to 40 rows a CU, f16 gains on rows of more than 3072 columns
-// that fill the steps (RMSNorm [7000,4096] 27.8 / 23.5, against [5000,3328] 17.6 / 18.9).
+// that fill the steps (RMSNorm [7000,4096] 27.8 / 23.5, against [5000,3328] 17.6 / 18.9).  bf16 LayerNorm, whose walker
+// needs the f32 tiles of both sums, gains in a single round of 8 rows a block ([2048,2560] 16.3 / 14.6, not three tiles in
+// four steps or five in eight: [2048,1280] 9.7 / 10.2) and once its blocks of 8 rows no longer keep their rows in LDS
+// ([7000,2560] 35 / 25.6; [5000,2560] 21.3 / 25.8), except for short rows and for 9000 to 10000 rows in steps a quarter empty ([9000,1792] 29.4 / 27.9).
 inline bool nf_takes_aligned(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
-    if (bf16) return layer ? cols > 128 && rows > 48 * cus : cols > 512 && rows > 40 * cus;      // (RMSNorm: rows beyond NR_MAX_ROWS)
-    if (rows > 40 * cus) return cols > 512;
-    if (cols <= 3072) return false;
     const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);
+    if (bf16 && layer) {
+        if (rows <= 8 * cus) return cols > 768 && nt != 5;
+        if (rows <= 16 * cus) return cols > 3328;
+        if (rows <= 24 * cus || cols <= 128) return false;
+        if (cols <= 256) return rows > 48 * cus;
+        if (rows <= 32 * cus || rows > 42 * cus) return true;
+        return nt * 5 >= steps * 4;
+    }
+    if (rows > 40 * cus) return cols > 512;                  // (RMSNorm in bf16: rows beyond NR_MAX_ROWS)
+    if (bf16 || cols <= 3072) return false;
     if (nt == steps) return layer || rows > 8 * cus;
     return layer && rows >= 64 && rows <= 16 * cus && cols > 3328;
 }
@@ -1333,7 +1356,8 @@ int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* 
     if (vec_ok && cols <= 128 && rows >= 16384) return launch_norm16_lane<T, KIND>(dev, x, scale, bias, y, rows, cols, eps);
     const uint64_t cus = (uint64_t)dev->num_cus;
     constexpr bool BF16 = std::is_same<T, bf16_t>::value, LAYER = KIND == NORM_LAYER;
-    if (vec_ok && nr_takes(BF16, LAYER, rows, cols, cus)) return rt_norm16_row(dev, BF16, KIND, x, scale, bias, y, rows, cols, eps);
+    if (vec_ok && nr_takes(BF16, LAYER, rows, cols, cus))
+        return LAYER ? rt_layer_norm_bf16_row(dev, x, scale, bias, y, rows, cols, eps) : rt_rms_norm16_row(dev, BF16, x, scale, y, rows, cols, eps);
     if (cols >= 8 && cols <= NF_MAX_COLS &&
         (vec_ok ? nf_takes_aligned(BF16, LAYER, rows, cols, cus) : nf_takes_ragged(BF16, LAYER, rows, cols, cus))) {
         // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; fewer where that takes no more

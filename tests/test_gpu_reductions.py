@@ -664,6 +664,22 @@ def test_norms_16_bit_both_sides_of_the_kernel_choice(dev, oracle, rows, cols, o
     _norms_16_bit(dev, oracle, x, conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), kind == "bf16", off, off)
 
 
+@pytest.mark.parametrize("rows,cols", [(300, 256), (300, 264), (1024, 1280), (1025, 1280), (1024, 4096), (1025, 4096), (768, 4104), (769, 4104),      # a few rows
+                                       (7168, 1024), (7168, 1032), (7169, 1032), (7169, 1536), (7169, 1544), (7681, 2048), (7680, 2056), (7681, 2056), (7681, 2560),
+                                       (16384, 2568), (16385, 2056),                                                                        # LayerNorm of many
+                                       (4096, 1280), (4097, 1280), (7168, 3840), (7169, 3840), (7169, 3072), (7169, 3080), (12288, 320), (12289, 320), (12289, 312),
+                                       (12289, 1536), (15360, 1544), (15361, 1544), (300, 5120), (300, 5128)])                              # RMSNorm
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_norms_16_bit_both_sides_of_a_wave_per_row(dev, oracle, rows, cols, kind):
+    """the same bits on either side of the lines at which norm16_row_kernel takes over (on 256 CUs); a third of the rows with their mean
+    taken off, whose sums are not sure without their order"""
+    rng = np.random.default_rng(333)
+    conv = _conv16(oracle, kind)
+    x = rng.standard_normal((rows, cols), np.float32) * np.float32(1.5) + np.float32(0.25)
+    x[::3] -= x[::3].mean(axis=1, keepdims=True)
+    _norms_16_bit(dev, oracle, conv(x), conv(1 + 0.02 * rng.standard_normal(cols)), conv(0.02 * rng.standard_normal(cols)), kind == "bf16", 0, 0)
+
+
 @pytest.mark.parametrize("cols", [256, 512, 1000, 1536, 2560, 3072, 4096])
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_rms_norm_16_bit_row_sums_replayed_in_parallel(dev, oracle, cols, kind):
@@ -753,8 +769,8 @@ def test_norms_16_bit_sums_in_any_order_where_the_rounding_is_sure(dev, oracle, 
 def test_layer_norm_16_bit_sums_that_cancel(dev, oracle, cols, kind):
     """Rows whose sum comes back to about zero after large excursions: values and their negatives shuffled (of one size, of many, cubed), rows
     with their mean taken off, runs of eight that swing between signs, and a run whose own sum has more bits than f32 holds where the running sum does
-    not.  No bound settles what such a sum rounds to: the wave-per-row kernel has to add it in order.  Compared over the whole
-    launch, which is few enough rows for that kernel, and over half of the rows with zeros in them, whose outputs show the mean."""
+    not.  No bound settles what such a sum rounds to: the wave-per-row kernel, which takes the bf16 ones, has to add it in order.  Every other
+    row has zeros in it, whose outputs show the mean."""
     rng = np.random.default_rng(331 + cols)
     bf = kind == "bf16"
     conv = _conv16(oracle, kind)
