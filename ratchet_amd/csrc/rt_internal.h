@@ -41,7 +41,7 @@ struct rt_device {
     uint64_t sp_attr_set;   // streaming softmax instantiations whose dynamic-LDS limit has been raised on this device
     uint64_t sp_ragged_attr_set;   // the same for the ragged-row variants
     uint32_t sp_pair_attr_set;     // the same for the variants that take one mask row for two heads (bits 0..15) and for those of f16 rows of 4097 to 8192 columns
-    uint64_t sr_attr_set;          // the same for the wave-per-rows softmax (rt_softmax_row.hip), two bits an instantiation of ten in f16 and sixteen in bf16
+    uint64_t sr_attr_set;          // the same for the wave-per-rows softmax (rt_softmax_row.hip), two bits an instantiation of nine in f16 and thirteen in bf16
     unsigned ry_attr_set;          // the same for the one-wave-per-row softmax (rt_softmax_replay.hip)
     // one word per 512-column tile of the mask of a masked streaming softmax (allocated with the device): the
     // tile's value twice when all its elements are equal, 0xffffffff when the tile has to be loaded; the first RT_SM_TILES_HEAD

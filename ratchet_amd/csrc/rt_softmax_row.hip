@@ -359,32 +359,57 @@ __global__ void __launch_bounds__(64 * sr_waves(V)) softmax16_row_kernel(const u
     }
 }
 
-// Which calls come here, against the streaming kernel (rt_softmax_stream.h); us, that one / this one, [heads, queries, keys].  That one walks rows 30 (f16
-// rows over 4096 columns: 15) to a block, a round costs its walk whatever it holds, and the bf16 walk is three times the f16 one.  This one
-// costs by the row, but reads and writes HBM less evenly than that one with its paced steps.
-//   f16, over 4096 columns: [8,2048,8192] with a mask 131 / 125, [8,512,8192] 54 / 34, [8,700,6000] 47 / 35, [32,256,5120] 50 / 37.
-//   f16, 2049 to 4096 columns: up to 32 rows a CU ([8,1024,3072] 31 / 26, [32,256,4096] 41 / 34; [8,2048,3000] 51 / 53, [32,4096,4096] 374 / 445).
-//      Against softmax16_replay_kernel, which has at most two rows to a CU: [8,64,6000] 29 / 16, [32,1,5120] 17 / 12, [32,16,4096] 18 / 13.6, [32,1,3000] 11.9 / 10.9, but
-//      [32,1,4096] 11.7 / 12.2, [32,1,3584] 11.9 / 12.5.
-//   bf16, over 1024 columns: all with a mask ([32,4096,4096] 549 / 472, [8,2048,8192] 263 / 139, [32,256,4096] 66 / 46, [32,128,2048] 22 / 20); without one
-//      from 32 rows a CU or over 2048 columns ([32,4096,4096] 481 / 450, [32,1536,1536] 85 / 82; [8,600,1601] 21 / 23).
-//   bf16, up to 1024 columns, with a mask: 160 rows a CU ([32,2048,512] 57 / 37, [32,1500,640] 78 / 49; [32,1024,1024] 43 / 44, [32,512,512] 18 / 20).
-//   rows that are not whole vectors, up to 2048 columns: where that kernel's last round would be nearly empty ([32,1001,1001] f16 39 / 33, bf16 59 / 45,
-//      [32,1201,1201] f16 53 / 46, [16,2001,2001] f16 72 / 68; with fuller rounds [32,1601,1601] f16 85 / 90, [32,901,901] bf16 39 / 43).
-template <typename T> bool sr_takes(bool mask, uint64_t rows, uint32_t cols, uint64_t cus) {
+// Which calls come here, against the streaming kernel (rt_softmax_stream.h); us, that one / this one, [heads, queries, keys], causal mask where one is named, inputs and
+// outputs moving through 600 MB.  That one walks rows 30 (f16 rows over 4096 columns: 15) to a block, a round costs its walk whatever it holds, and the bf16 walk is
+// three times the f16 one.  This one costs by the row, but reads and writes HBM less evenly than that one with its paced steps.
+// What a row costs here depends on how often its sum passes a power of two: the figures are N(0, 2), N(0, 1) over 4096 columns; N(2, 3) costs
+// bf16 up to a tenth more, rows sorted upwards a third ([32,1024,4096] plain 131, 132 and 176 us, there 136).
+//   f16, over 4096 columns: [8,2048,8192] with a mask 134 / 126, [8,512,8192] 53 / 34, [8,700,6000] 45 / 35, [32,256,5120] 51 / 37; not where two rounds or more
+//      of that kernel are nearly full ([32,480,8192] 100 / 111, [32,360,5120] with a mask 60 / 67, [32,240,8192] with a mask 65 / 70; [32,320,8192] 76 / 72).
+//   f16, 2049 to 4096 columns: up to 32 rows a CU ([8,1024,3072] 30 / 26, [32,256,4096] 39 / 30; [32,224,2304] 22.4 / 23.3; [8,2048,3000] 49 / 48, [32,4096,4096] 344 / 407).
+//      Against softmax16_replay_kernel, which has at most two rows to a CU: [8,64,6000] 25 / 16, [32,1,5120] 17.6 / 12.8, [32,16,4096] 17.6 / 13.8, [32,1,3000] 12.5 / 11.2, but
+//      [32,1,4096] 12.6 / 12.7, [32,1,3584] 12.2 / 12.5.
+//   bf16, over 4096 columns: [8,2048,8192] 201 / 124, [32,240,8192] with a mask 113 / 79.
+//   bf16, 513 to 4096 columns: by what both take (sr_pays_bf16), with a mask or from 32 rows a CU or over 2048 columns, rows of whole vectors from 1025.
+//   rows that are not whole vectors, up to 2048 columns: where that kernel's last round would be nearly empty ([32,1001,1001] f16 with a mask 42 / 33, bf16 60 / 46,
+//      [32,1201,1201] f16 55 / 48, [16,2001,2001] f16 62 / 58; with fuller rounds f16 [32,1681,1681] 86 / 92, [32,1500,1500] 64 / 66).
+inline bool sr_pays_bf16(bool mask, uint64_t period, uint64_t rows, uint32_t cols, uint64_t cus) {
+    // The walk bounds the streaming kernel: 3.1 us a step and round (4.0 with a mask, 3.5 where a mask row serves two heads), and 5 us and 1.5 a step to fill and drain it;
+    // a twelfth more where rows are not whole vectors.  Here 4 or 2 rows at a time on each SIMD, by the chunk of 512 or 1024 columns.  Over 650 calls of 1025 to 4096 columns the
+    // pick costs half a per cent more than the better one and is never more than 3 % slower than the streaming kernel, where this one, taken for all, was slower by up to a quarter:
+    // [32,1440,2560] 107 / 133, [32,480,2304] with a mask 51 / 59, [32,192,1536] with a mask 19.4 / 21.8; [32,1536,1536] with a mask 104 / 84, [32,256,4096] 60 / 41.
+    const uint32_t nt = (cols + SP_TC - 1) / SP_TC, steps = nt == 7 ? 8 : nt;
+    SpSched sch;
+    const bool pair = sp_periods(sch, mask, period, rows, nt);
+    const uint64_t rounds = sp_rounds(sch, sp_rows_per_group(sch, mask, pair, pair ? SP_HALF : SP_ROWS, cus), cus);
+    double there = 5.0 + 1.5 * steps + (!mask ? 3.1 : pair ? 3.5 : 4.0) * steps * (double)rounds;
+    if (cols % 8 != 0) there *= 1.08;
+    const bool four = cols <= 2048;
+    const uint32_t chunks = four ? nt : (cols + 1023) / 1024, at_once = four ? 16 : 8;
+    const double row = four ? 0.095 + 0.085 * chunks + (mask && chunks > 2 ? 0.055 : 0.0) : 0.17 + 0.17 * chunks + (mask ? 0.06 * (chunks - 2) : 0.0);
+    const double here = 11.0 + row * (double)((rows + at_once * cus - 1) / (at_once * cus) * at_once);
+    return 1.04 * here < there;
+}
+template <typename T> bool sr_takes(bool mask, uint64_t period, uint64_t rows, uint32_t cols, uint64_t cus) {
     constexpr bool BF16 = std::is_same<T, bf16_t>::value;
-    if (cols <= 256 || cols > 8192) return false;
-    const uint32_t steps = (cols + SP_TC - 1) / SP_TC;
-    if (cols % 8 != 0 && cols <= 2048) {
-        const double rounds = (double)rows / (double)(SP_ROWS * cus);
-        return rounds >= 2.0 && ceil(rounds) >= 1.1 * rounds + 0.33 / steps;
+    if (cols <= 512 || cols > 8192) return false;
+    const bool whole = cols % 8 == 0;
+    if (!whole && cols <= 2048) {
+        const uint32_t steps = (cols + SP_TC - 1) / SP_TC;
+        const double rounds = (double)rows / (double)(SP_ROWS * cus), full = ceil(rounds);
+        if (rounds < 2.0 || full < 1.1 * rounds + 0.33 / steps || (!BF16 && full < 1.16 * rounds)) return false;
+        return !BF16 || sr_pays_bf16(mask, period, rows, cols, cus);
     }
     if (BF16) {
-        if (cols % 8 != 0 && cols > 4096) return false;
-        if (cols <= 1024) return mask && rows > 160 * cus;
-        return mask || cols > 2048 || rows >= 32 * cus;
+        if (cols <= 1024 || (!whole && cols > 4096)) return false;
+        if (!mask && cols <= 2048 && rows < 32 * cus) return false;
+        return cols > 4096 || sr_pays_bf16(mask, period, rows, cols, cus);
     }
-    return cols % 8 == 0 && cols > 2048 && (cols > 4096 || (rows <= 32 * cus && (cols <= 3072 || rows > cus / 4)));
+    if (!whole || cols <= 2048) return false;
+    if (cols <= 4096) return rows <= 32 * cus && (cols <= 3072 || rows > cus / 4);
+    const double rounds = (double)rows / (double)(SP_HALF * cus), full = ceil(rounds);
+    if (cols > 7168 && rounds > 1.6) return full >= 1.1 * rounds && !(mask && rows <= 32 * cus);
+    return rounds <= 2.5 || full >= 1.08 * rounds;
 }
 
 template <typename T, int L, int V, bool RAGGED>
@@ -409,8 +434,8 @@ template <typename T>
 int launch_row16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done) {
     *done = false;
     constexpr bool BF16 = std::is_same<T, bf16_t>::value;
-    if (!sr_takes<T>(mask != nullptr, rows, cols, (uint64_t)dev->num_cus)) return RT_OK;
     if (rows > 0x7fffffffull / (2ull * cols)) return RT_OK;              // 32-bit offsets: larger ones go in chunks there
+    if (!sr_takes<T>(mask != nullptr, mask ? period : rows, rows, cols, (uint64_t)dev->num_cus)) return RT_OK;
     if (mask && rows / period % (cols > 2048 ? 2 : 4) != 0) return RT_OK;        // the rows of a wave share a mask row
     if (dev->debug_softmax_pace) return RT_OK;                           // a pace set by hand is the streaming kernel's
     // the exp table is built on first use, which synchronises: not while a graph is being captured
@@ -426,21 +451,24 @@ int launch_row16(rt_device* dev, const void* x, const void* mask, uint64_t perio
     int rc = RT_OK;
 #define RT_SR(LC, VC, RG, BIT)                                                                                     \
     case VC:                                                                                                       \
-        rc = launch_row16_as<T, LC, VC, RG>(dev, (BIT) + (BF16 ? 10 : 0), table, x, mask, y, g);                   \
+        rc = launch_row16_as<T, LC, VC, RG>(dev, (BIT) + (BF16 ? 9 : 0), table, x, mask, y, g);                    \
         break
+#define RT_SR_NONE default: return rt_fail(RT_ERR_ARG, "softmax: internal: %u columns for several rows to a wave", cols)
     if (cols % 8 != 0 && cols <= 2048) {
-        switch (chunks) { RT_SR(16, 1, true, 0); RT_SR(16, 2, true, 1); RT_SR(16, 3, true, 2); RT_SR(16, 4, true, 3); }
+        switch (chunks) { RT_SR(16, 2, true, 0); RT_SR(16, 3, true, 1); RT_SR(16, 4, true, 2); RT_SR_NONE; }
     } else if (cols > 2048 && cols % 8 == 0) {
         switch (chunks) {
-            RT_SR(32, 3, false, 4); RT_SR(32, 4, false, 5); RT_SR(32, 5, false, 6); RT_SR(32, 6, false, 7); RT_SR(32, 7, false, 8); RT_SR(32, 8, false, 9);
+            RT_SR(32, 3, false, 3); RT_SR(32, 4, false, 4); RT_SR(32, 5, false, 5); RT_SR(32, 6, false, 6); RT_SR(32, 7, false, 7); RT_SR(32, 8, false, 8);
+            RT_SR_NONE;
         }
     } else if constexpr (BF16) {
         if (cols > 2048) {
-            switch (chunks) { RT_SR(32, 3, true, 10); RT_SR(32, 4, true, 11); }
+            switch (chunks) { RT_SR(32, 3, true, 9); RT_SR(32, 4, true, 10); RT_SR_NONE; }
         } else {
-            switch (chunks) { RT_SR(16, 1, false, 12); RT_SR(16, 2, false, 13); RT_SR(16, 3, false, 14); RT_SR(16, 4, false, 15); }
+            switch (chunks) { RT_SR(16, 3, false, 11); RT_SR(16, 4, false, 12); RT_SR_NONE; }
         }
     }
+#undef RT_SR_NONE
 #undef RT_SR
     *done = rc == RT_OK;
     return rc;

@@ -698,6 +698,67 @@ inline int sp_allow_lds(const void* kernel) {
     return RT_OK;
 }
 
+// How n rows of nt steps, under a mask of `period` rows (n of them without one), come in periods and items; true if one mask row serves two heads.
+inline bool sp_periods(SpSched& sch, bool mask, uint64_t period, uint64_t n, uint32_t nt) {
+    // a mask of few rows (a [1, T] padding mask, a short prefill): groups run across its periods
+    sch.PM = (uint32_t)(mask ? period : n);
+    sch.pm_div = make_fastdiv(sch.PM);
+    sch.P = (uint32_t)(mask && period >= 8 * SP_ROWS ? period : n);
+    sch.reps = (uint32_t)(n / sch.P);
+    sch.nsteps = (nt + 1) & ~1u;
+    // one mask row for two heads: rows of an even number of steps under a mask that repeats every P rows
+    const bool pair = mask && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
+    sch.item_reps = pair ? (sch.reps + 1) / 2 : sch.reps;
+    return pair;
+}
+inline uint64_t sp_rounds(const SpSched& sch, uint32_t R, uint64_t cus) {
+    const uint64_t groups = (uint64_t)((sch.P + R - 1) / R) * sch.item_reps;
+    return (groups + cus - 1) / cus;
+}
+// rows per group: every block runs ceil(groups / grid) rounds of 8-or-fewer steps whatever the group holds, so
+// 4370 groups of 30 rows on 256 CUs cost 18 rounds where 17.07 are needed; 27-row groups make 19 full rounds.
+// A step takes the longer of the walk (1.5 us whatever the group holds) and the group's memory time (2 KiB per
+// row at a CU's share of the bandwidth: about 0.09 us per row), so a round costs max(R + 1, 18) in units of a
+// row's memory time; pick the size with the cheapest total, the smallest such size on a tie.  Few rows (a decode
+// step's [B * H, T] scores) spread over the CUs the same way: 32 rows run as 32 one-row groups.
+// With a mask that repeats every P rows, group pg of every period reads the same mask rows.  Item w runs on block
+// w % grid, and blocks go to the eight XCDs in turn, so those groups land on 8 / gcd(GP % 8, 8) different XCDs, each
+// of which pulls the mask rows into its own L2.  Among the sizes within 5 % of the cheapest, the one that keeps a
+// mask group on the fewest XCDs is taken ([1,16,4096,4096] with a causal mask: 27 rows, 152 groups a period, 211 us;
+// the cheapest size by the count alone, 26 rows and 158 groups, 224 us; 114 against 121 us on [1,32,2048,2048]).
+inline uint32_t sp_rows_per_group(const SpSched& sch, bool mask, bool pair, uint32_t rmax, uint64_t cus) {
+    const uint32_t rmul = pair ? 2 : 1;
+    auto cost_of = [&](uint32_t R) -> uint64_t { return sp_rounds(sch, R, cus) * (R * rmul + 1 > 18 ? R * rmul + 1 : 18); };
+    uint64_t best = ~0ull;
+    uint32_t pick = rmax;
+    for (uint32_t R = rmax; R >= 1; R--) {
+        const uint64_t cost = cost_of(R);
+        if (cost <= best) {
+            best = cost;
+            pick = R;
+        }
+    }
+    if (mask && sch.reps > 1 && !pair) {
+        auto xcds_of = [&](uint32_t R) -> uint32_t {
+            const uint32_t g = ((sch.P + R - 1) / R) % 8;
+            return g == 0 ? 1 : (g % 4 == 0) ? 2 : (g % 2 == 0) ? 4 : 8;
+        };
+        uint32_t pick_x = xcds_of(pick);
+        uint64_t pick_cost = best;
+        for (uint32_t R = rmax; R >= 1; R--) {
+            const uint64_t cost = cost_of(R);
+            if (cost * 20 > best * 21) continue;
+            const uint32_t xc = xcds_of(R);
+            if (xc < pick_x || (xc == pick_x && cost < pick_cost)) {
+                pick = R;
+                pick_x = xc;
+                pick_cost = cost;
+            }
+        }
+    }
+    return pick;
+}
+
 // mask == nullptr: plain softmax.  Otherwise the mask has `period` rows of `cols` columns and repeats every `period`
 // rows of x (rows % period == 0).  Returns RT_OK with *done = false when the shape does not fit this kernel.
 template <typename T>
@@ -814,63 +875,10 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         const T* xc = (const T*)x + row0 * cols;
         T* yc = (T*)y + row0 * cols;
         SpSched sch;
-        // a mask of few rows (a [1, T] padding mask, a short prefill): groups run across its periods
-        sch.PM = (uint32_t)(mask ? period : n);
-        sch.pm_div = make_fastdiv(sch.PM);
-        sch.P = (uint32_t)(mask && period >= 8 * SP_ROWS ? period : n);
-        sch.reps = (uint32_t)(n / sch.P);
-        sch.nsteps = (nt + 1) & ~1u;
-        // one mask row for two heads: rows of an even number of steps under a mask that repeats every P rows
-        const bool pair = mask && nt <= SP_MAX_STEPS && (nt % 2 == 0 || nt == 7) && sch.PM == sch.P && sch.reps >= 2;
-        sch.item_reps = pair ? (sch.reps + 1) / 2 : sch.reps;
+        const uint64_t cus = (uint64_t)dev->num_cus;
+        const bool pair = sp_periods(sch, mask != nullptr, period, n, nt);
         const uint32_t rmul = pair ? 2 : 1;
-        // rows per group: every block runs ceil(groups / grid) rounds of 8-or-fewer steps whatever the group holds, so
-        // 4370 groups of 30 rows on 256 CUs cost 18 rounds where 17.07 are needed; 27-row groups make 19 full rounds.
-        // A step takes the longer of the walk (1.5 us whatever the group holds) and the group's memory time (2 KiB per
-        // row at a CU's share of the bandwidth: about 0.09 us per row), so a round costs max(R + 1, 18) in units of a
-        // row's memory time; pick the size with the cheapest total, the smallest such size on a tie.  Few rows (a decode
-        // step's [B * H, T] scores) spread over the CUs the same way: 32 rows run as 32 one-row groups.
-        // With a mask that repeats every P rows, group pg of every period reads the same mask rows.  Item w runs on block
-        // w % grid, and blocks go to the eight XCDs in turn, so those groups land on 8 / gcd(GP % 8, 8) different XCDs, each
-        // of which pulls the mask rows into its own L2.  Among the sizes within 5 % of the cheapest, the one that keeps a
-        // mask group on the fewest XCDs is taken ([1,16,4096,4096] with a causal mask: 27 rows, 152 groups a period, 211 us;
-        // the cheapest size by the count alone, 26 rows and 158 groups, 224 us; 114 against 121 us on [1,32,2048,2048]).
-        auto rounds_of = [&](uint32_t R) -> uint64_t {
-            const uint64_t groups = (uint64_t)((sch.P + R - 1) / R) * sch.item_reps;
-            return (groups + dev->num_cus - 1) / dev->num_cus;
-        };
-        auto rows_per_group = [&](uint32_t rmax) -> uint32_t {
-            auto cost_of = [&](uint32_t R) -> uint64_t { return rounds_of(R) * (R * rmul + 1 > 18 ? R * rmul + 1 : 18); };
-            uint64_t best = ~0ull;
-            uint32_t pick = rmax;
-            for (uint32_t R = rmax; R >= 1; R--) {
-                const uint64_t cost = cost_of(R);
-                if (cost <= best) {
-                    best = cost;
-                    pick = R;
-                }
-            }
-            if (mask && sch.reps > 1 && !pair) {
-                auto xcds_of = [&](uint32_t R) -> uint32_t {
-                    const uint32_t g = ((sch.P + R - 1) / R) % 8;
-                    return g == 0 ? 1 : (g % 4 == 0) ? 2 : (g % 2 == 0) ? 4 : 8;
-                };
-                uint32_t pick_x = xcds_of(pick);
-                uint64_t pick_cost = best;
-                for (uint32_t R = rmax; R >= 1; R--) {
-                    const uint64_t cost = cost_of(R);
-                    if (cost * 20 > best * 21) continue;
-                    const uint32_t xc = xcds_of(R);
-                    if (xc < pick_x || (xc == pick_x && cost < pick_cost)) {
-                        pick = R;
-                        pick_x = xc;
-                        pick_cost = cost;
-                    }
-                }
-            }
-            return pick;
-        };
-        sch.R = rows_per_group(pair ? SP_HALF : SP_ROWS);
+        sch.R = sp_rows_per_group(sch, mask != nullptr, pair, pair ? SP_HALF : SP_ROWS, cus);
         // f16 rows of 4097 to 8192 columns: in registers, 15 to a group (the LONG variant), or 30 to a group and parked in y?
         // In registers x is read and y written once, and the walk is the bound: 1.45 us per 512 columns with its barriers, on
         // half as many rows at a time and in steps of 1024 columns, of which 5, 6 or 8 are taken.  Parked, a round takes the
@@ -885,10 +893,10 @@ int launch_stream16(rt_device* dev, const void* x, const void* mask, uint64_t pe
         // 65 / 53, [1,8,2048,8192] with a mask 269 / 259): bf16 parks in y.
         bool longer = false;
         if (LONG_ROWS && !ragged && nt > SP_MAX_STEPS && nt <= 2 * SP_MAX_STEPS) {
-            const uint32_t R = rows_per_group(SP_HALF);
-            const uint64_t in_registers = rounds_of(R) * long_steps * 2900;                                  // ns
+            const uint32_t R = sp_rows_per_group(sch, mask != nullptr, pair, SP_HALF, cus);
+            const uint64_t in_registers = sp_rounds(sch, R, cus) * long_steps * 2900;                                  // ns
             const uint64_t memory = (uint64_t)sch.R * cols * 5 / 16, walk = (uint64_t)sch.nsteps * 2300;
-            longer = in_registers <= rounds_of(sch.R) * (memory > walk ? memory : walk) + (uint64_t)sch.nsteps * 600;
+            longer = in_registers <= sp_rounds(sch, sch.R, cus) * (memory > walk ? memory : walk) + (uint64_t)sch.nsteps * 600;
             if (longer) sch.R = R;
         }
         const bool long_full = longer && cols == long_steps * 2 * SP_TC;

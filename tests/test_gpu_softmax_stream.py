@@ -118,3 +118,33 @@ def test_several_rows_to_a_wave(dev, oracle, kind, heads, rows, cols):
     assert _same(dev.softmax(dev.upload(odd, bf16=bf)).to_numpy(), oracle.softmax(odd, bf16=bf), bf)
     dev.softmax(dx, out=dx)
     assert _same(dx.to_numpy(), oracle.softmax(x, bf16=bf), bf)
+
+
+def _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, seed):
+    """the oracle's bits without a mask, under one of `rows` rows that the heads share, and both in place; rows of _hard_rows among N(0, 1)"""
+    bf = kind == "bf16"
+    rng = np.random.default_rng(seed)
+    hard = _hard_rows(rng, cols, bf)
+    x = rng.standard_normal((heads * rows, cols), np.float32)
+    at = rng.permutation(heads * rows)[: 4 * len(hard)]
+    x[at] = hard[np.arange(len(at)) % len(hard)]
+    x = _to(oracle, x, bf).reshape(1, heads, rows, cols)
+    m = np.where(rng.random((rows, cols)) < 0.1, -np.inf, 0.5 * rng.standard_normal((rows, cols), np.float32))
+    m = _to(oracle, m, bf)
+    dm = dev.upload(m, bf16=bf)
+    for mask in (None, m):
+        want = oracle.softmax(x if mask is None else oracle.binary("add", x, np.ascontiguousarray(np.broadcast_to(m, x.shape)), bf16=bf), bf16=bf)
+        dx = dev.upload(x, bf16=bf)
+        assert _same((dev.softmax(dx) if mask is None else dev.softmax_masked(dx, dm)).to_numpy(), want, bf), (mask is None, "another buffer")
+        dev.softmax(dx, out=dx) if mask is None else dev.softmax_masked(dx, dm, out=dx)
+        assert _same(dx.to_numpy(), want, bf), (mask is None, "in place")
+
+
+@pytest.mark.parametrize("kind,heads,rows,cols", [
+    ("bf16", 4, 2100, 1024), ("bf16", 4, 2047, 1536), ("bf16", 4, 2048, 1536), ("bf16", 4, 1920, 2048), ("bf16", 4, 1800, 2304), ("bf16", 4, 3840, 2304), ("bf16", 4, 2500, 2304),
+    ("bf16", 4, 4100, 511), ("bf16", 4, 4100, 513), ("bf16", 2, 300, 4095), ("bf16", 2, 300, 4097),
+    ("f16", 4, 4100, 511), ("f16", 4, 4100, 513), ("f16", 4, 5700, 1001), ("f16", 2, 4096, 2056), ("f16", 2, 4097, 2056), ("f16", 2, 3840, 7176), ("f16", 2, 4200, 7176),
+    ("f16", 2, 5760, 4104), ("f16", 2, 4900, 4104), ("f16", 2, 32, 3080), ("f16", 2, 33, 3080)])
+def test_both_sides_of_several_rows_to_a_wave(dev, oracle, kind, heads, rows, cols):
+    """the same bits on either side of the lines at which softmax16_row_kernel takes over (on 256 CUs)"""
+    _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, rows + cols)
