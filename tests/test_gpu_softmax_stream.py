@@ -141,6 +141,15 @@ def _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, seed):
 
 
 @pytest.mark.parametrize("kind,heads,rows,cols", [
+    ("f16", 4, 4101, 1001), ("f16", 4, 4101, 1033), ("f16", 4, 4101, 2047), ("bf16", 4, 5951, 1001), ("bf16", 4, 4301, 1033), ("bf16", 4, 4101, 2047),       # four rows a wave: 16384 in a trip, not whole vectors
+    ("bf16", 4, 4301, 1032), ("bf16", 4, 4101, 2048), ("bf16", 2, 4101, 2057), ("bf16", 2, 4101, 3080),                          # two: 8192
+    ("f16", 2, 3100, 4104), ("f16", 2, 2100, 7176), ("bf16", 2, 3100, 5128), ("bf16", 2, 2100, 8192)])                           # 6144 and 4096
+def test_several_rows_to_a_wave_in_several_trips(dev, oracle, kind, heads, rows, cols):
+    """on 256 CUs more rows than the waves of softmax16_row_kernel hold at one time: they store one set of rows while the next one loads"""
+    _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, rows + cols)
+
+
+@pytest.mark.parametrize("kind,heads,rows,cols", [
     ("bf16", 4, 2100, 1024), ("bf16", 4, 2047, 1536), ("bf16", 4, 2048, 1536), ("bf16", 4, 1920, 2048), ("bf16", 4, 1800, 2304), ("bf16", 4, 3840, 2304), ("bf16", 4, 2500, 2304),
     ("bf16", 4, 4100, 511), ("bf16", 4, 4100, 513), ("bf16", 2, 300, 4095), ("bf16", 2, 300, 4097),
     ("f16", 4, 4100, 511), ("f16", 4, 4100, 513), ("f16", 4, 5700, 1001), ("f16", 2, 4096, 2056), ("f16", 2, 4097, 2056), ("f16", 2, 3840, 7176), ("f16", 2, 4200, 7176),
@@ -148,3 +157,36 @@ def _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, seed):
 def test_both_sides_of_several_rows_to_a_wave(dev, oracle, kind, heads, rows, cols):
     """the same bits on either side of the lines at which softmax16_row_kernel takes over (on 256 CUs)"""
     _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, rows + cols)
+
+
+@pytest.mark.parametrize("rows,cols", [(1030, 8192), (1640, 5120), (1367, 6144), (2051, 4104), (1403, 6008), (181, 5120), (175, 6000)])
+def test_f16_rows_of_4097_to_8192_columns_under_a_mask_of_three_heads(dev, oracle, rows, cols):
+    """softmax16_stream_kernel with fifteen rows a block in registers, which has the masks that an odd number of rows share: masks large enough for the
+    table of tile classes (with uniform and with mixed tiles) and smaller ones, rows that fill the kernel's steps and rows that do not, a single row of
+    mask (under an odd number of rows), one head; also in place"""
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((1, 3, rows, cols), np.float32)
+    x[0, :, ::50] = _hard_rows(rng, cols, False)[rng.integers(0, 20, (3, len(x[0, 0, ::50])))]
+    x = x.astype(np.float16)
+    m = np.where(np.arange(cols)[None, :] > np.arange(rows)[:, None] * (cols // rows), -np.inf, 0.0).astype(np.float16)
+    m[:, 512:1024], m[::7, 2048:2560] = -0.5, (0.3 * rng.standard_normal((len(m[::7]), 512))).astype(np.float16)
+    for heads, mask in ((3, m), (1, m), (3 if rows % 2 else 1, m[rows // 2:rows // 2 + 1])):
+        part = np.ascontiguousarray(x[:, :heads, :rows - (rows + 1) % 2] if len(mask) == 1 else x[:, :heads])
+        want = oracle.softmax(oracle.binary("add", part, np.ascontiguousarray(np.broadcast_to(mask, part.shape))))
+        dx, dm = dev.upload(part), dev.upload(mask)
+        assert _same(dev.softmax_masked(dx, dm).to_numpy(), want, False), (heads, mask.shape)
+        dev.softmax_masked(dx, dm, out=dx)
+        assert _same(dx.to_numpy(), want, False), (heads, mask.shape, "in place")
+
+
+def test_f16_rows_of_8192_columns_beyond_2_gib(dev, oracle):
+    """several rows to a wave have 32-bit offsets: a tensor of 2 GiB and more goes in chunks to the kernel that keeps fifteen rows a block in registers"""
+    rng = np.random.default_rng(5)
+    rows, cols, reps = 131072 + 90, 8192, 130
+    block = rng.standard_normal((1009, cols), np.float32).astype(np.float16)
+    x = np.tile(block, (reps, 1))[:rows]
+    got = dev.softmax(dev.upload(x)).to_numpy()
+    want = oracle.softmax(block)
+    for k in range(0, rows, 1009):
+        n = min(1009, rows - k)
+        assert np.array_equal(got[k:k + n].view(np.uint16), want[:n].view(np.uint16)), k
