@@ -27,12 +27,9 @@ namespace {
 constexpr int NR_STREAM = 2;                                 // the non-temporal hint of a buffer access
 constexpr int NR_BLOCK = 64;
 
-// The f32 chain of 16-bit terms.  MANT: mantissa bits of the running sum's type, INF: its infinity's bit pattern.  pair(a, b) starts two sums at two bit
-// patterns, run() adds a vector's eight terms to both, lo() and hi() are the sums' bit patterns; one() adds to a single sum.
+// The f32 chain of 16-bit terms.  pair(a, b) starts two sums at two bit patterns, run() adds a vector's eight terms to both, lo() and hi() are the sums' bit patterns; one() adds to a single sum.
 template <typename T> struct ChainF32;
 template <> struct ChainF32<half_t> {
-    static constexpr int MANT = 23;
-    static constexpr uint32_t INF = 0x7f800000u;
     struct Pair {
         float a, b;
     };
@@ -62,8 +59,6 @@ template <> struct ChainF32<half_t> {
 #undef RT_MIX1
 };
 template <> struct ChainF32<bf16_t> {
-    static constexpr int MANT = 23;
-    static constexpr uint32_t INF = 0x7f800000u;
     struct Pair {
         float a, b;
     };

@@ -7,13 +7,10 @@
 // itself: the run is added up twice, from 2^e and from 2^e + ulp, and d[p] is the distance the p-th sum has moved, read off the bit
 // patterns.  d[0] == d[1] when no tie occurred (both sums moved alike); otherwise both ended on the same parity, whatever they started from.
 //
-// ordered_add takes one run per lane.  Every lane adds its run up from the binade the sum is in at the moment; the parity at the start
-// of each lane's run follows from the lanes before it by one 64-bit addition on the scalar unit (a lane with a tie sets the
-// parity, the others flip or keep it: generate, kill and propagate of a carry chain); the chosen distances are summed over the
-// lanes.  If the sum leaves the binade in a lane, that lane's run is added for real to the exact sum before it, in the same pass that
-// prepares the lanes behind it for the next binade: a pass for every binade the sum passes through, and one for every run of 64.
-// Nothing is approximated: a result is used only if the sum stayed inside the binade it was made for (the sum never
-// decreases, so every sum in between did too).  inf and NaN lie beyond every binade and are absorbed as the adder absorbs them.
+// One run per lane: every lane adds its run up from the binade that the sum is in there; the parity at the start of each lane's run follows from the
+// lanes before it by one 64-bit addition on the scalar unit (a lane with a tie sets the parity, the others flip or keep it: generate, kill and
+// propagate of a carry chain); the chosen distances are summed over the lanes.  Lanes in which the sum leaves the binade add for real to the exact sum before them.
+// norm_ordered_squares below and sr_group_add (rt_softmax_row.hip) do that, each where its sums need it.
 #ifndef RT_ORDERED_H
 #define RT_ORDERED_H
 
@@ -71,68 +68,6 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) { retu
 __device__ __forceinline__ double lane_value(double v, uint32_t lane) {
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
     return __builtin_bit_cast(double, (uint64_t)lane_value((uint32_t)(u >> 32), lane) << 32 | lane_value((uint32_t)u, lane));
-}
-
-// s, the same in all lanes: the bit pattern of a running sum of terms >= 0 (or NaN).  Returns that of the sum after the 64 runs of NV
-// vectors, lane 0's first.  At the start of a row, where the sum doubles every few lanes, SERIAL lanes are added one by one.
-template <class C, int NV, int SERIAL>
-__device__ __forceinline__ uint32_t ordered_add(uint32_t s, const v4u (&v)[NV], uint32_t lane) {
-    constexpr uint32_t ULPS = 1u << C::MANT;                 // sums in a binade
-    uint32_t from = 0;                                       // lanes below it are in s
-    if (s == 0) {
-        for (; from < SERIAL; from++) {
-            uint32_t t = s;
-#pragma unroll
-            for (int k = 0; k < NV; k++) t = C::one(t, v[k]);
-            s = lane_value(t, from);
-        }
-    }
-    bool real = false;                                       // lane `from` adds to s itself
-    uint32_t e = s >> C::MANT;
-    while (s < C::INF) {
-        // the binade; the subnormals and the first normal one have one ulp and count as one
-        const uint32_t base = e <= 1 ? 0 : e << C::MANT, size = e <= 1 ? 2 * ULPS : ULPS;
-        const bool mine = real && lane == from;
-        typename C::Pair p = C::pair(mine ? s : base, base + 1);
-#pragma unroll
-        for (int k = 0; k < NV; k++) C::run(p, v[k]);
-        uint32_t d0 = C::lo(p) - base, d1 = C::hi(p) - (base + 1);
-        if (real) {
-            s = lane_value(C::lo(p), from);
-            if (++from == 64) return s;
-            real = false;
-            if (s >> C::MANT != e && !(e <= 1 && s >> C::MANT <= 1)) {       // not in the binade that the lanes behind prepared for
-                e = s >> C::MANT;
-                continue;
-            }
-        }
-        if (C::MANT == 23) {                                 // (64 distances have to fit into a word)
-            d0 = d0 < 2 * ULPS ? d0 : 2 * ULPS;
-            d1 = d1 < 2 * ULPS ? d1 : 2 * ULPS;
-        }
-        if (lane < from) d0 = d1 = 0;
-        // the parity in front of each lane: `flips` is that of the distances before it alone, a tie in between sets it anew
-        const uint64_t odd = __builtin_amdgcn_ballot_w64(d0 & 1u), tie = __builtin_amdgcn_ballot_w64(d0 != d1);
-        const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(odd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)odd, 0));
-        const uint64_t flips = __builtin_amdgcn_ballot_w64(below & 1u);
-        const uint64_t gen = tie & flips, prop = gen | ~tie;
-        const uint64_t parity = ((prop + gen + (s & 1u)) ^ prop ^ gen) ^ flips;
-        const uint32_t d = __builtin_amdgcn_inverse_ballot_w64(parity) ? d1 : d0;
-        const uint32_t upto = lanes_scan(d);
-        const uint64_t leaves = __builtin_amdgcn_ballot_w64(upto >= base + size - s);
-        if (leaves == 0) return s + lane_value(upto, 63);
-        const uint32_t at = __builtin_ctzll(leaves);
-        s += lane_value(upto, at) - lane_value(d, at);
-        from = at;
-        real = true;
-        e = e <= 1 ? 2 : e + 1;                              // where the lanes behind that one most likely add
-    }
-    // inf or NaN: the next lane that makes anything else of it makes a NaN, which stays
-    uint32_t t = s;
-#pragma unroll
-    for (int k = 0; k < NV; k++) t = C::one(t, v[k]);
-    const uint64_t other = __builtin_amdgcn_ballot_w64(lane >= from && t != s);
-    return other ? lane_value(t, __builtin_ctzll(other)) : s;
 }
 
 // the ulp of the binade of m (m finite, at least 2^-103; zero below that)
@@ -200,14 +135,14 @@ __device__ __forceinline__ float norm_ordered_sum(float s, const v4u& x, uint32_
 }
 
 // T(x*x)'s (v: the squares, s: the sum's bit pattern).  From approximate sums in front of the lanes every lane takes the binade it adds in; a lane
-// is clean if its run starts and ends there, with a margin for what the approximation can be off by.  Pairs of distances as in
-// ordered_add; the parity in front of a lane is followed for both parities that its stretch of clean lanes can start with, and the
-// distances are summed under both.  Then the lanes that are not clean (about eight of a row, where the sum passes a power of two)
-// are taken in order: the stretch in front of one is a single addition, its own run is added for real.  What the approximation claims is checked
-// on the exact sum, and a step on which it fails goes through ordered_add.
+// is clean if its run starts and ends there, with a margin for what the approximation can be off by: the margin is 2^-10, and the approximate and the ordered
+// sum, each of 512 terms >= 0 on the same exact sum, are off the true one by 2^-15 at most, in a clean lane of the binade that both ends lie in (a term so
+// large that what it hides matters takes its lane out of the binade).  So is the binade right for a stretch of clean lanes, which all have the same.  Pairs of
+// distances as above; the parity in front of a lane is followed for both parities that its stretch of clean lanes can start with, and the
+// distances are summed under both.  Then the lanes that are not clean (about eight of a row, where the sum passes a power of two; all where it is
+// subnormal, near overflow or NaN) are taken in order: the stretch in front of one is a single addition, its own run is added for real.
 template <class C>
 __device__ __forceinline__ uint32_t norm_ordered_squares(uint32_t s, const v4u& v, uint32_t lane) {
-    const uint32_t start = s;
     const float run = u2f(C::one(0, v)), upto = lanes_scan(run), carry = u2f(s);
     const uint32_t e = f2u((carry + upto) * (1.0f + 0x1p-10f)) >> 23;
     const bool clean = (e - 2 < 252) & (f2u((carry + (upto - run)) * (1.0f - 0x1p-10f)) >> 23 == e);
@@ -223,29 +158,19 @@ __device__ __forceinline__ uint32_t norm_ordered_squares(uint32_t s, const v4u& 
     const uint64_t prop0 = gen0 | ~set, prop1 = gen1 | ~set;
     const uint32_t u0 = lanes_scan(__builtin_amdgcn_inverse_ballot_w64(((prop0 + gen0) ^ prop0 ^ gen0) ^ flips) ? d1 : d0);
     const uint32_t u1 = lanes_scan(__builtin_amdgcn_inverse_ballot_w64(((prop1 + gen1 + 1) ^ prop1 ^ gen1) ^ flips) ? d1 : d0);
-    bool failed = false;
     uint64_t todo = dirty;
     uint32_t from = 0, c0 = 0, c1 = 0;
     for (;;) {
         const uint32_t at = todo ? __builtin_ctzll(todo) : 64, last = at < 64 ? at : 63;             // (a dirty lane's own distance is zero)
-        const uint32_t n0 = lane_value(u0, last), n1 = lane_value(u1, last), eb = lane_value(base, at ? at - 1 : 0);
-        if (at > from) {
-            failed |= (s ^ eb) >> 23 != 0;
-            s += s & 1u ? n1 - c1 : n0 - c0;
-            failed |= (s ^ eb) >> 23 != 0;
-        }
-        if (at == 64) break;
+        const uint32_t n0 = lane_value(u0, last), n1 = lane_value(u1, last);
+        if (at > from) s += s & 1u ? n1 - c1 : n0 - c0;
+        if (at == 64) return s;
         s = lane_value(C::one(s, v), at);
         c0 = n0;
         c1 = n1;
         from = at + 1;
         todo &= todo - 1;
     }
-    if (failed) {
-        const v4u one[1] = {v};
-        s = ordered_add<C, 1, 3>(start, one, lane);
-    }
-    return s;
 }
 
 }  // namespace

@@ -7,7 +7,8 @@
 
 namespace {
 
-// The 16-bit chains of exponentials for ordered_add (as ChainF32 there).
+// The 16-bit chains of exponentials.  MANT: mantissa bits of the running sum's type, INF: its infinity's bit pattern.  pair(a, b) starts two sums at two bit
+// patterns, run() adds a vector's eight terms to both, lo() and hi() are the sums' bit patterns; one() adds to a single sum.
 template <typename T> struct Chain16;
 template <> struct Chain16<half_t> {
     static constexpr int MANT = 10;
@@ -74,8 +75,10 @@ template <int L> __device__ __forceinline__ uint32_t sr_scan(uint32_t v) {
 template <int L> constexpr uint64_t SR_LOW = L == 16 ? 0x0001000100010001ull : 0x0000000100000001ull;
 template <int L> constexpr uint64_t SR_HIGH = SR_LOW<L> << (L - 1);
 
-// ordered_add (rt_ordered.h) for the 64 / L rows of a wave at one time: s, the bit pattern of a row's sum, is the same in the L lanes of its
-// group; a lane has 32 terms.  All groups make the same passes, and those that are through idle: the passes that a row needs come
+// The ordered sums (rt_ordered.h) of the 64 / L rows of a wave at one time: s, the bit pattern of a row's sum, is the same in the L lanes of its
+// group; a lane has 32 terms.  A lane in which the sum leaves the binade adds for real in the same pass that prepares the lanes behind it for the next
+// binade.  Nothing is approximated: a distance is used only if the sum stayed inside the binade it was made for (it never decreases, so every sum in
+// between did too).  inf and NaN lie beyond every binade and are absorbed as the adder absorbs them.  All groups make the same passes, and those that are through idle: the passes that a row needs come
 // mostly from the powers of two that its sum passes, which is at about the same columns in all of them.
 template <class C, int L>
 __device__ __forceinline__ uint32_t sr_group_add(uint32_t s, const v4u (&v)[4], uint32_t gl) {

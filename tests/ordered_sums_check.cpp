@@ -130,8 +130,6 @@ template <bool BF> struct Half {
     }
     // the chain of norm_ordered_squares
     struct Pair { float a, b; };
-    static constexpr int MANT = 23;
-    static constexpr uint32_t INF = 0x7f800000u;
     static Pair pair(uint32_t a, uint32_t b) { return Pair{u2f(a), u2f(b)}; }
     static uint32_t lo(const Pair& p) { return f2u(p.a); }
     static uint32_t hi(const Pair& p) { return f2u(p.b); }
