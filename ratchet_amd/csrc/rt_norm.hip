@@ -1274,8 +1274,10 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
 //   RMSNorm bf16, nearly always sure: from 264 columns up ([256,5120] 22.0 / 10.8, [2048,2560] 9.5 / 8.6, [16384,3072] 40.7 / 37.2, [65536,384] 31.8 / 22.3).
 //   RMSNorm f16, one row in ten open, 1 to 4 us a wave: up to 16 rows a CU (against a kernel that is gone: [4096,264] 7.8 / 5.7, [4096,1280] 9.1 / 7.9, [1024,5120] 18.6 / 11.3; of 3072 to
 //     4096 columns and 32 to 128 rows no gain, 6.9 / 6.9, and rows whose squares are subnormal 6.6 / 7.2); then where the walk takes its rows in many
-//     rounds ([16384,320] 9.6 / 8.0, [16384,1280] 21.3 / 18.0, [16384,2560] 34.3 / 32.6; [14000,1792] 19.9 / 20.9; [16384,264] 9.5 / 10.1), from 3072 columns
-//     where its steps are not full ([10240,3840] 35.5 / 32.8, [16384,4608] 58.5 / 57.1; [12288,3072] 28.7 / 30.7, [7200,4096] 24.6 / 26.9).
+//     rounds ([16384,320] 9.6 / 8.0, [16384,1280] 21.3 / 18.0, [16384,2560] 34.3 / 32.1; [14000,1792] 19.9 / 20.9, [14000,1024] 11.8 / 13.0, [14000,640] o 10.4 / 11.3;
+//     [16384,264] 9.5 / 10.1), from 3072 columns where its steps are not full ([10240,3840] 35.5 / 32.8, [16384,4608] 58.5 / 57.1; [12288,3072] 28.9 / 30.1,
+//     [7200,4096] 24.3 / 26.5) or are many ([8192,5120] 37.1 / 35.5, [32768,5120] 123 / 119; [7200,5120] 29.9 / 32.1), and where it shares
+//     lines between rows ([12288,4088] 46.4 / 40.7, [12288,5112] 61.6 / 50.3).
 // The sum of x is small against its terms, and of rows with no mean it is nearly all rounding: f16 rows of that kind stay open all of them, bf16 ones one
 // in six, 4 us a wave for 2560 columns.
 //   LayerNorm f16: nowhere (N(0, 1) [32768,1280] 38.7 / 34.2, but c 38.6 / 68; [1024,2560] 12.2 / 12.2, c 12.2 / 15.5; [16,2560] 11.6 / 7.8, c 11.6 / 12.1).
@@ -1289,8 +1291,9 @@ inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64
     if (!layer) {
         if (bf16 || rows <= 16 * cus) return true;
         const uint32_t nt = (cols + 255) / 256;
-        if (cols >= 3072) return rows > 28 * cus && nt != nf_steps(nt);
-        return cols >= 320 && rows > (cols <= 1536 ? 48 : 60) * cus;
+        const bool lines = cols % 32 == 0;                   // rows start on 64 bytes
+        if (cols >= 3072) return rows > 28 * cus && (!lines || nt != nf_steps(nt) || (cols > 4864 && rows > 30 * cus));
+        return cols >= 320 && rows > (!lines || cols <= 512 ? 48 : 60) * cus;
     }
     if (!bf16) return false;
     if (rows <= (cols <= 4096 ? 4 : 3) * cus) return true;
