@@ -18,7 +18,7 @@
 //      between does too), that is t after the run; otherwise (the first lane, a run in which the sum crosses a power
 //      of two, a lag of more than two binades) every lane adds its own run to t left to right and lane i's result is
 //      kept.  A row on which no pair applies costs the plain walk, 64 runs in sequence.
-// (Composing the pairs of neighbouring lanes with a scan, as the 16-bit RMSNorm does for its f32 sum, does not pay here:
+// (Composing the pairs of neighbouring lanes, as norm_ordered_squares (rt_ordered.h) does for an f32 sum, does not pay here:
 // the f16 sum lags the guess, so the stretches of equal guesses and the stretches the sum really spends in a binade are
 // shifted against each other, and every composite ends in the lane where the sum leaves the binade.)
 // The exp values come from the 65536-entry table of the exact f16 exp, which every block copies into LDS first (128 KiB:
@@ -253,13 +253,14 @@ __global__ void __launch_bounds__(RY_BLOCK) softmax16_replay_kernel(const uint16
 // after the other: [32, 2048] 13.3 -> 9.4 us, [32, 4096] 22.6 -> 12.0 us, [32, 8192] 48.6 -> 20 us, [256, 2048]
 // 13.5 -> 10.4 us, [256, 4096] 22.9 -> 14.3 us; rows of 1024 columns lose (8.8 -> 10 us: the ordered pass costs 4 us
 // whatever the row length), and from four rows per CU the streaming kernel's overlap wins.
-// Over 2048 columns softmax16_row_kernel comes first and leaves it up to 64 rows of 3073 to 4096 columns and masks whose rows are not shared by an
-// even number of the others.
+// Over 2048 columns softmax16_row_kernel comes first and leaves it, on 256 CUs, up to 64 rows of 3073 to 4096 columns and masks whose rows are not
+// shared by an even number of the others; without a mask it takes every call of more than 4096 columns that would fit here.
 // Returns RT_OK with *done = false when the shape does not fit.
 int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done) {
     *done = false;
     constexpr uint32_t MAX_RPB = 2;
     if (cols % 8 != 0 || cols < 2048 || cols > 8192 || rows == 0 || rows > (uint64_t)MAX_RPB * (uint64_t)dev->num_cus) return RT_OK;
+    if (cols > 4096 && !mask) return RT_OK;
     if (!rt_aligned(x, 16) || !rt_aligned(y, 16) || (mask && !rt_aligned(mask, 16))) return RT_OK;
     // the exp table is built on first use, which synchronises: not while a graph is being captured
     if (dev->capturing && !dev->unary_lut[0][RT_EXP]) return RT_OK;
@@ -270,7 +271,7 @@ int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint6
     // as few rows per block as keep the blocks within one per CU: every block copies the table, a row per CU runs alone
     const uint32_t rpb = (uint32_t)((rows + dev->num_cus - 1) / dev->num_cus);
     const dim3 grid((unsigned)((rows + rpb - 1) / rpb)), block(RY_BLOCK);
-#define RT_RY1(VC, M, BIT)                                                                                                        \
+#define RT_RY(VC, M, BIT)                                                                                                         \
     do {                                                                                                                          \
         if (!(dev->ry_attr_set & (1u << (BIT)))) {           /* the LDS opt-in is per function and per device */                  \
             RT_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax16_replay_kernel<VC, M>),                             \
@@ -280,18 +281,13 @@ int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint6
         hipLaunchKernelGGL((softmax16_replay_kernel<VC, M>), grid, block, RY_LUT_BYTES, dev->stream, table, (const half_t*)x,     \
                            (const half_t*)mask, period, (half_t*)y, rows, cols, rpb);                                             \
     } while (0)
-#define RT_RY(VC, BIT)                                                                                                            \
-    do {                                                                                                                          \
-        if (mask) RT_RY1(VC, true, 2 * (BIT) + 1);                                                                                \
-        else RT_RY1(VC, false, 2 * (BIT));                                                                                        \
-    } while (0)
     const uint32_t v = (cols / 8 + 63) / 64;                 // vectors per lane
-    if (v <= 2) RT_RY(2, 0);
-    else if (v <= 4) RT_RY(4, 1);
-    else if (v <= 8) RT_RY(8, 2);
-    else RT_RY(16, 3);
+    if (v <= 4 && mask) RT_RY(4, true, 0);
+    else if (v <= 4) RT_RY(4, false, 1);
+    else if (v <= 8 && mask) RT_RY(8, true, 2);
+    else if (v <= 8) RT_RY(8, false, 3);
+    else RT_RY(16, true, 4);
 #undef RT_RY
-#undef RT_RY1
     RT_CHECK_LAUNCH("softmax16_replay_kernel");
     *done = true;
     return RT_OK;
