@@ -324,8 +324,8 @@ __global__ void __launch_bounds__(64 * sr_waves(V)) softmax16_row_kernel(const u
         for (int k = 0; k < R; k++) {
             sums[k] = ST::widen_bits(__builtin_amdgcn_readlane(s, k * L));
             by[k] = 1.0f;
-            if (std::is_same<T, bf16_t>::value) {            // into it, both sides by the same power of two (a value that underflows has a quotient of 0)
-                by[k] = sums[k] < ST::Div::MIN ? 0x1p64f : sums[k] > ST::Div::MAX ? 0x1p-64f : 1.0f;
+            if constexpr (std::is_same<T, bf16_t>::value) {  // into it
+                by[k] = ST::Div::scale(sums[k]);
                 wide |= by[k] != 1.0f;
                 sums[k] *= by[k];
             }

@@ -1,5 +1,6 @@
-// Host check of the streaming softmax's short divisions (ratchet_amd/csrc/rt_softmax_div.h, the kernel's own text): for every exp
-// value e >= 0 and every `stride`-th row sum s inside the range where the kernel takes them, the short form must round to the
+// Host check of the 16-bit softmax's short divisions (ratchet_amd/csrc/rt_softmax_div.h, the kernels' own text): for every exp
+// value e >= 0 and every `stride`-th row sum s inside the range where the streaming kernel takes them, and for every e <= s and every
+// s > 0 outside of it, where the kernel with several rows to a wave takes them too, the short form must round to the
 // bits of the correctly rounded f32 quotient rounded to the 16-bit type, which is what the reference's half types compute.
 // Build: g++ -O2 -std=c++17 -ffp-contract=off -mfma -I ratchet_amd/csrc.   Usage: softmax_division_check STRIDE
 // prints "f16 <n> bf16 <n> checked <m>" (n: pairs that differ), exit code 0 iff both are 0.
@@ -33,16 +34,24 @@ int main(int argc, char** argv) {
     unsigned long long bad16 = 0, badbf = 0, checked = 0;
     for (uint32_t sb = 1; sb < 0x7c00; sb += stride) {
         const float s = from_f16((uint16_t)sb), rinv = 1.0f / s, rlow = ShortDivF16::low(s, rinv);
-        if (s < ShortDivF16::MIN || s > ShortDivF16::MAX) continue;
-        for (uint32_t eb = 0; eb < 0x7c00; eb++) {
+        const uint32_t last = s < ShortDivF16::MIN ? sb : 0x7bff;             // (a sum is never below its terms)
+        for (uint32_t eb = 0; eb <= last; eb++) {
             const float e = from_f16((uint16_t)eb);
             bad16 += to_f16(ShortDivF16::quotient(e, rinv, rlow)) != to_f16(e / s);
             checked++;
         }
     }
     for (uint32_t sb = 1; sb < 0x7f80; sb += stride) {
-        const float s = u2f(sb << 16), rinv = 1.0f / s, rlow = ShortDivBf16::low(s, rinv);
-        if (s < ShortDivBf16::MIN || s > ShortDivBf16::MAX) continue;
+        const float sum = u2f(sb << 16), by = ShortDivBf16::scale(sum), s = sum * by, rinv = 1.0f / s, rlow = ShortDivBf16::low(s, rinv);
+        if (s < ShortDivBf16::MIN || s > ShortDivBf16::MAX) return 2;
+        if (by != 1.0f) {
+            for (uint32_t eb = 0; eb <= sb; eb++) {
+                const float e = u2f(eb << 16);
+                badbf += to_bf16(ShortDivBf16::quotient(u2f((uint32_t)to_bf16(e * by) << 16), rinv, rlow)) != to_bf16(e / sum);
+                checked++;
+            }
+            continue;
+        }
         for (uint32_t eb = 0; eb < 0x7f80; eb++) {
             const float e = u2f(eb << 16), q = e / s;
             if (std::isinf(q)) break;                         // a sum is never below its terms
