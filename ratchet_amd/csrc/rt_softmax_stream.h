@@ -693,7 +693,7 @@ __global__ void __launch_bounds__(BLOCK) mask_tiles_kernel(const T* __restrict__
 inline int sp_allow_lds(const void* kernel) {
     hipFuncAttributes a;
     RT_HIP(hipFuncGetAttributes(&a, kernel));
-    RT_REQUIRE(a.sharedSizeBytes == 0, RT_ERR_SIZE, "softmax16_stream_kernel: %zu bytes of static LDS lie in front of its table", a.sharedSizeBytes);
+    RT_REQUIRE(a.sharedSizeBytes == 0, RT_ERR_SIZE, "softmax: %zu bytes of static LDS lie in front of the kernel's table", a.sharedSizeBytes);
     RT_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SP_SMEM_BYTES));
     return RT_OK;
 }

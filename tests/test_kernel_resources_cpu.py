@@ -4,6 +4,8 @@ import re
 import struct
 import subprocess
 
+import pytest
+
 from ratchet_amd import _lib, build
 
 READELF = os.path.join(os.path.dirname(os.path.dirname(build.HIPCC)), "llvm", "bin", "llvm-readelf")
@@ -26,8 +28,9 @@ def code_objects():
         at = blob.find(MAGIC, at + 1)
 
 
-def test_the_softmax_table_lies_at_the_start_of_lds(tmp_path):
-    """softmax16_stream_kernel reads its table at LDS address 0 + 2 * bits, where its dynamic LDS starts only as long as nothing
+@pytest.mark.parametrize("softmax, least", [("softmax16_stream_kernel", 100), ("softmax16_row_kernel", 40)])
+def test_the_softmax_table_lies_at_the_start_of_lds(tmp_path, softmax, least):
+    """the kernel reads its table at LDS address 0 + 2 * bits, where its dynamic LDS starts only as long as nothing
     that is compiled into the kernel declares static LDS of its own"""
     seen = 0
     for k, code in enumerate(code_objects()):
@@ -36,7 +39,7 @@ def test_the_softmax_table_lies_at_the_start_of_lds(tmp_path):
         notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
         for kernel in re.split(r"\n\s+- \.(?:agpr_count|args)", notes):
             name = re.search(r"\.name:\s+(\S+)", kernel)
-            if name and "softmax16_stream_kernel" in name.group(1):
+            if name and softmax in name.group(1):
                 seen += 1
                 assert re.search(r"\.group_segment_fixed_size:\s+0\n", kernel), name.group(1)
-    assert seen >= 100, seen
+    assert seen >= least, seen
