@@ -731,7 +731,7 @@ def profile_targets(dev, seed, names, reps):
 
             fn = norm_launch
         elif name.startswith("decode_softmax_"):
-            # a decode step's f16 scores [1,32,1,T], T from the name (2048, 4096, 8192): one wave per row
+            # a decode step's f16 scores [1,32,1,T], T from the name (2048, 4096, 8192): one wave per row, two rows to a wave from 4104 columns on
             T = int(name.rsplit("_", 1)[1])
             dsc = dev.upload(normal(seed, 805, (1, H, 1, T), 2.0, np.float16))
             ysc = dev.empty((1, H, 1, T), F16)

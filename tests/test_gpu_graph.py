@@ -115,7 +115,7 @@ def test_replays_of_ragged_row_softmax_match_eager_execution(dev, oracle):
 
 
 def test_replays_of_a_decode_step_softmax_match_eager_execution(dev, oracle):
-    """[B * H, T] f16 scores of a decode step (one wave per row, the row sum replayed from per-lane pairs), plain and with
+    """[B * H, T] f16 scores of a decode step (two rows to a wave, the row sums replayed from per-lane pairs), plain and with
     a [1, T] mask, and the masked f32 row kernel, captured and replayed"""
     rng = np.random.default_rng(803)
     a = randn(rng, (1, 32, 1, 2304), np.float16, 2.0)

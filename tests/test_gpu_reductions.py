@@ -258,7 +258,7 @@ def test_softmax_bf16_streaming_kernel(dev, oracle, shape):
 @pytest.mark.parametrize("shape,kind", [((1, 70, 8192), "f16"), ((2, 33, 4104), "f16"), ((1, 3, 51200), "f16"), ((1, 100, 6008), "f16"),
                                         ((1, 40, 8192), "bf16"), ((1, 5, 20000), "bf16")])
 def test_softmax_16_bit_long_rows(dev, oracle, shape, kind):
-    """rows of more than 4096 columns (few f16 rows of up to 8192: one wave a row; the others park the exp values in y and read them back once the row sum is known); also in place"""
+    """rows of more than 4096 columns (up to 8192: few rows, two to a wave; longer ones park the exp values in y and read them back once the row sum is known); also in place"""
     rng = np.random.default_rng(306)
     n = shape[-1]
     xf = (rng.standard_normal(shape) * 2).astype(np.float32)
@@ -287,9 +287,9 @@ def test_softmax_16_bit_long_rows(dev, oracle, shape, kind):
 @pytest.mark.parametrize("rows,cols", [(530, 4104), (1100, 5112), (1040, 5120), (1100, 5128), (4000, 6144), (530, 6152), (544, 7680), (1100, 8184), (4100, 8192)])
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, kind):
-    """fifteen rows a block in registers, a thread's two vectors 512 columns apart in one row: the oracle's bits where a row
-    ends in the first and in the second half of a step, with one group a block and several, in place, without a mask, under
-    a mask of two periods large enough for the table of tile classes (uniform and mixed tiles) and under a single mask row"""
+    """the oracle's bits where a row ends in the first and in the second half of a step of 1024 columns, for few rows and many, in place, without a
+    mask, under a mask of two periods (uniform and mixed tiles) and under a single mask row.  Two rows to a wave: an even number of rows shares each mask
+    row (an odd one: test_f16_rows_of_4097_to_8192_columns_under_a_mask_of_three_heads)"""
     rng = np.random.default_rng(317)
     bf = kind == "bf16"
     conv = (lambda a: _bf16(oracle, a)) if bf else (lambda a: np.asarray(a, np.float32).astype(np.float16))
@@ -325,7 +325,7 @@ def test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, ki
 
 @pytest.mark.parametrize("rows,cols", [(4096, 4104), (4700, 8192), (6000, 5000), (6144, 6144), (7000, 6152), (8200, 4104)])
 def test_softmax_f16_rows_of_4097_to_8192_columns_in_several_rounds(dev, oracle, rows, cols):
-    """more rows than one round of fifteen a block: in registers or parked in y, whichever takes less time, the oracle's bits"""
+    """more rows than the streaming kernel takes in one round of fifteen a block, but not whole rounds of it: two rows to a wave in several trips"""
     test_softmax_16_bit_rows_of_4097_to_8192_columns(dev, oracle, rows, cols, "f16")
 
 
@@ -683,9 +683,9 @@ def test_norms_16_bit_both_sides_of_a_wave_per_row(dev, oracle, rows, cols, kind
 @pytest.mark.parametrize("cols", [256, 512, 1000, 1536, 2560, 3072, 4096])
 @pytest.mark.parametrize("kind", ["f16", "bf16"])
 def test_rms_norm_16_bit_row_sums_replayed_in_parallel(dev, oracle, cols, kind):
-    """Rows of 256 to 4096 columns take a kernel that replays the reference's left-to-right f32 sum of T(x*x) with the 64
-    lanes of a wave (pairs of sums per lane, composed across lanes) instead of walking it; the output must not differ in
-    one bit from the walk.  Rows that stress what the kernel decides by: sums that land exactly on powers of two, ranges
+    """Rows of 257 to 5120 columns take norm16_row_kernel, a wave to a row, which replays the reference's left-to-right f32 sum of T(x*x) (pairs of
+    sums per lane, joined across lanes) where its sum in any order does not settle the rounding; narrower rows are walked.  The output must not differ
+    in one bit from the walk.  Rows that stress what the kernel decides by: sums that land exactly on powers of two, ranges
     of 2^30 inside a row, heavy tails, squares that overflow the element type, NaN, rows of zeros, single large terms."""
     rng = np.random.default_rng(316 + cols)
     bf = kind == "bf16"
@@ -1141,7 +1141,8 @@ def test_softmax_masked_rows_that_are_not_whole_vectors(dev, oracle, shape, msha
 @pytest.mark.parametrize("shape,mshape,kind", [((1, 4, 50, 8192), (50, 8192), "f16"), ((2, 2, 33, 4200), (1, 1, 33, 4200), "f16"),
                                                ((1, 8, 128, 512), (128, 512), "bf16"), ((1, 3, 40, 6000), (40, 6000), "bf16")])
 def test_softmax_masked_long_rows_and_bf16(dev, oracle, shape, mshape, kind):
-    """the one-launch masked softmax beyond 4096 columns (values parked in y) and in bf16: the bits of add-then-softmax"""
+    """the one-launch masked softmax beyond 4096 columns (two rows to a wave; where an odd number of rows shares a mask row, bf16 parked in y) and in
+    bf16: the bits of add-then-softmax"""
     rng = np.random.default_rng(322)
     bf = kind == "bf16"
     S, T = mshape[-2], mshape[-1]
@@ -1169,9 +1170,9 @@ def test_softmax_masked_long_rows_and_bf16(dev, oracle, shape, mshape, kind):
 @pytest.mark.parametrize("cols", [1536, 2048, 2056, 2560, 4096, 5000 // 8 * 8, 8192])
 @pytest.mark.parametrize("masked", [False, True])
 def test_softmax_f16_few_long_rows_sums_replayed_in_parallel(dev, oracle, cols, masked):
-    """A few rows of 2048 to 8192 columns in f16 (a decode step's scores) take a kernel that replays the reference's
-    left-to-right f16 sum of the exp values with the 64 lanes of a wave instead of walking it; not one bit may differ from the
-    step-wise model.  Rows that stress what the kernel decides by: sums that stop growing (terms below half an ulp),
+    """A few rows of 2048 to 8192 columns in f16 (a decode step's scores) take kernels that replay the reference's
+    left-to-right f16 sum of the exp values with the 64 (one row to a wave: 2048 columns, up to 64 rows of 3073 to 4096, a mask row over an odd number of
+    rows) or 32 (two) lanes instead of walking it; not one bit may differ from the step-wise model.  Rows that stress what the kernel decides by: sums that stop growing (terms below half an ulp),
     sums that land on powers of two, tiny terms before and after large ones, overflow to inf, NaN, rows of -inf, a causal
     tail, every term in a binade of its own."""
     rng = np.random.default_rng(327 + cols)

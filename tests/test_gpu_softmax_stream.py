@@ -64,8 +64,8 @@ def test_ragged_rows_under_a_mask_shared_by_heads(dev, oracle, cols, kind):
     assert _same(dx.to_numpy(), want, bf)
 
 
-@pytest.mark.parametrize("heads,rows,cols", [(1, 3840, 6152), (1, 3841, 6152), (1, 4500, 6656),      # f16: one round in registers; two, so parked in y
-                                             (2, 1920, 6152), (2, 1930, 6152), (1, 3900, 4104)])
+@pytest.mark.parametrize("heads,rows,cols", [(1, 3840, 6152), (1, 3841, 6152), (1, 4500, 6656),      # under a mask: one round in registers; two, so parked in y
+                                             (2, 1920, 6152), (2, 1930, 6152), (1, 3900, 4104)])                    # two rows to a wave, as without a mask; registers
 @pytest.mark.parametrize("masked", [False, True])
 def test_rows_of_4097_to_8192_columns_around_a_round(dev, oracle, heads, rows, cols, masked):
     """both sides of the choice between registers and parking in y; also in place"""
@@ -153,7 +153,7 @@ def test_several_rows_to_a_wave_in_several_trips(dev, oracle, kind, heads, rows,
     ("bf16", 4, 2100, 1024), ("bf16", 4, 2047, 1536), ("bf16", 4, 2048, 1536), ("bf16", 4, 1920, 2048), ("bf16", 4, 1800, 2304), ("bf16", 4, 3840, 2304), ("bf16", 4, 2500, 2304),
     ("bf16", 4, 4100, 511), ("bf16", 4, 4100, 513), ("bf16", 2, 300, 4095), ("bf16", 2, 300, 4097),
     ("f16", 4, 4100, 511), ("f16", 4, 4100, 513), ("f16", 4, 5700, 1001), ("f16", 2, 4096, 2056), ("f16", 2, 4097, 2056), ("f16", 2, 3840, 7176), ("f16", 2, 4200, 7176),
-    ("f16", 2, 5760, 4104), ("f16", 2, 4900, 4104), ("f16", 2, 32, 3080), ("f16", 2, 33, 3080)])
+    ("f16", 2, 5760, 4104), ("f16", 2, 4900, 4104), ("f16", 2, 5760, 5120), ("f16", 2, 5760, 6008), ("f16", 2, 5760, 6144), ("f16", 2, 32, 3080), ("f16", 2, 33, 3080)])
 def test_both_sides_of_several_rows_to_a_wave(dev, oracle, kind, heads, rows, cols):
     """the same bits on either side of the lines at which softmax16_row_kernel takes over (on 256 CUs)"""
     _plain_masked_in_place(dev, oracle, kind, heads, rows, cols, rows + cols)
