@@ -4,8 +4,9 @@
 // swing between signs inside and between the lanes, by up to 2^24 of their last bits; tiny and huge ones; inf and NaN; the rows of
 // `found`.  Sums go on over the steps of a row, from the plain sum of the steps before.
 // Build: g++ -O2 -std=c++17 -ffp-contract=off -I ratchet_amd/csrc.   Usage: ordered_sums_check ROWS
-// prints "sum_f16 <n> sum_bf16 <n> squares_f16 <n> squares_bf16 <n> turns <k> checked <m>" (n: steps whose sums differ; k: the most exchanges between
-// lanes in a step of short rows that cancel, whose upper lanes have no terms), exit code 0 iff all n are 0 and k is at most MOST_TURNS.
+// prints "sum_f16 <n> sum_bf16 <n> squares_f16 <n> squares_bf16 <n> turns <k> centred <c> checked <m>" (n: steps whose sums differ; k: the most exchanges
+// between lanes in a step of short rows that cancel, whose upper lanes have no terms; c: the mean of them in steps of rows without a mean), exit code 0 iff
+// all n are 0, k is at most MOST_TURNS and c at most MEAN_TURNS.
 #include <ucontext.h>
 
 #include <algorithm>
@@ -248,6 +249,35 @@ int main(int argc, char** argv) {
         bad[1] += differ<true, false>(r);
         turns = std::max(turns, turn[0]);
     }
-    printf("sum_f16 %llu sum_bf16 %llu squares_f16 %llu squares_bf16 %llu turns %u checked %llu\n", bad[0], bad[1], bad[2], bad[3], turns, checked);
-    return bad[0] || bad[1] || bad[2] || bad[3] || turns > MOST_TURNS;
+    // 25 exchanges for the scans and votes of a step; a lane adds for real in fewer than half of the steps (each in which the lane's own sum passes 2^24
+    // of its last bits, where the running one crosses zero, would make it 33 on average)
+    const double MEAN_TURNS = 30;
+    unsigned long long exchanges = 0, steps = 0;
+    for (int n = 0; n < 40; n++) {
+        std::vector<float> r(5 * 512);
+        double mean = 0;
+        for (float& f : r) mean += (f = normal(rng)) / (double)r.size();
+        for (float& f : r) f -= (float)mean;
+        for (bool bf : {false, true}) {
+            float s = 0.0f;
+            for (size_t i = 0; i < r.size(); i += 512, steps++) {
+                uint16_t t[512];
+                float want = s;
+                for (int k = 0; k < 512; k++) {
+                    t[k] = bf ? to_bf16(r[i + k]) : to_f16(r[i + k]);
+                    want += bf ? from_bf16(t[k]) : from_f16(t[k]);
+                }
+                terms = t;
+                s_in = s;
+                run_wave(bf ? lane_work<true, false> : lane_work<false, false>);
+                for (float got : s_out) bad[bf] += f2u(got) != f2u(want);
+                exchanges += turn[0];
+                s = want;
+            }
+        }
+    }
+    const double centred = (double)exchanges / (double)steps;
+    printf("sum_f16 %llu sum_bf16 %llu squares_f16 %llu squares_bf16 %llu turns %u centred %.1f checked %llu\n", bad[0], bad[1], bad[2], bad[3], turns, centred,
+           checked);
+    return bad[0] || bad[1] || bad[2] || bad[3] || turns > MOST_TURNS || centred > MEAN_TURNS;
 }
