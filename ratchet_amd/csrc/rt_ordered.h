@@ -153,7 +153,8 @@ __device__ __forceinline__ float norm_ordered_sum(float s, const v4u& x, uint32_
 // large that what it hides matters takes its lane out of the binade).  So is the binade right for a stretch of clean lanes, which all have the same.  Pairs of
 // distances as above; the parity in front of a lane is followed for both parities that its stretch of clean lanes can start with, and the
 // distances are summed under both.  Then the lanes that are not clean (about eight of a row, where the sum passes a power of two; all where it is
-// subnormal, near overflow or NaN) are taken in order: the stretch in front of one is a single addition, its own run is added for real.
+// subnormal, near overflow or NaN) are taken in order: the stretch in front of one is a single addition, its own run is added for real.  A lane without terms, past
+// the row's end, has no distance whatever the sum is: of a sum within the margin of a power of two each took a turn (f16 RMSNorm [667,2056] 11.6 us, 6.5 so).
 template <class C>
 __device__ __forceinline__ uint32_t norm_ordered_squares(uint32_t s, const v4u& v, uint32_t lane) {
     const float run = u2f(C::one(0, v)), upto = lanes_scan(run), carry = u2f(s);
@@ -163,7 +164,8 @@ __device__ __forceinline__ uint32_t norm_ordered_squares(uint32_t s, const v4u& 
     typename C::Pair p = C::pair(base, base + 1);
     C::run(p, v);
     const uint32_t d0 = clean ? C::lo(p) - base : 0, d1 = clean ? C::hi(p) - (base + 1) : 0;
-    const uint64_t dirty = __builtin_amdgcn_ballot_w64(!clean);
+    // (no terms but zeros: nothing to add, whatever the sum is)
+    const uint64_t dirty = __builtin_amdgcn_ballot_w64(!clean & ((v[0] | v[1] | v[2] | v[3]) != 0));
     const uint64_t odd = __builtin_amdgcn_ballot_w64(d0 & 1u), tie = __builtin_amdgcn_ballot_w64(d0 != d1);
     const uint32_t flip = __builtin_amdgcn_mbcnt_hi((uint32_t)(odd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)odd, 0));
     const uint64_t flips = __builtin_amdgcn_ballot_w64(flip & 1u);

@@ -5,7 +5,7 @@
 // `found`.  Sums go on over the steps of a row, from the plain sum of the steps before.
 // Build: g++ -O2 -std=c++17 -ffp-contract=off -I ratchet_amd/csrc.   Usage: ordered_sums_check ROWS
 // prints "sum_f16 <n> sum_bf16 <n> squares_f16 <n> squares_bf16 <n> turns <k> centred <c> checked <m>" (n: steps whose sums differ; k: the most exchanges
-// between lanes in a step of short rows that cancel, whose upper lanes have no terms; c: the mean of them in steps of rows without a mean), exit code 0 iff
+// between lanes in a step whose upper lanes have no terms, of rows that cancel and of squares next to a power of two; c: the mean of them in steps of rows without a mean), exit code 0 iff
 // all n are 0, k is at most MOST_TURNS and c at most MEAN_TURNS.
 #include <ucontext.h>
 
@@ -247,6 +247,19 @@ int main(int argc, char** argv) {
         bad[0] += differ<false, false>(r);
         turns = std::max(turns, turn[0]);
         bad[1] += differ<true, false>(r);
+        turns = std::max(turns, turn[0]);
+    }
+    // the squares of rows whose sum ends next to a power of two, with few terms in their last step
+    for (int n = 0; n < 40; n++) {
+        std::vector<float> r(1024, 0.0f);
+        double total = 0;
+        const int cols = 512 + 8 * (1 + below(20));
+        for (int i = 0; i < cols; i++) total += (r[i] = normal(rng)) * (double)r[i];
+        const float by = (float)std::sqrt(std::exp2(below(16) - 4) / total);
+        for (int i = 0; i < cols; i++) r[i] *= by;
+        bad[2] += differ<false, true>(r);
+        turns = std::max(turns, turn[0]);
+        bad[3] += differ<true, true>(r);
         turns = std::max(turns, turn[0]);
     }
     // 25 exchanges for the scans and votes of a step; a lane adds for real in fewer than half of the steps (each in which the lane's own sum passes 2^24
