@@ -129,11 +129,11 @@ int rt_softmax_row(rt_device* dev, bool bf16, const void* x, const void* mask, u
 // The f16 reference softmax for a few long rows, one wave per row (rt_softmax_replay.hip); arguments as above
 int rt_softmax_replay_f16(rt_device* dev, const void* x, const void* mask, uint64_t period, void* y, uint64_t rows, uint32_t cols, bool* done);
 
-// The 16-bit RMSNorm and the bf16 LayerNorm with a wave per row (rt_norm_row.hip): whole vectors, 16-byte aligned operands, at most NR_MAX_COLS columns and NR_MAX_ROWS rows
+// The 16-bit LayerNorm / RMSNorm with a wave per row (rt_norm_row.hip): whole vectors, 16-byte aligned operands, at most NR_MAX_COLS columns and NR_MAX_ROWS rows
 constexpr uint32_t NR_MAX_COLS = 5120;                       // 10 vectors a lane
 constexpr uint64_t NR_MAX_ROWS = (1ull << 26) - 1;           // a block of 64 threads to a row, and a launch has at most 2^32 - 1 threads along x
-int rt_rms_norm16_row(rt_device* dev, bool bf16, const void* x, const void* scale, void* y, uint64_t rows, uint32_t cols, float eps);
-int rt_layer_norm_bf16_row(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps);
+int rt_norm16_row(rt_device* dev, bool bf16, int kind, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols,
+                  float eps);
 
 // ---------------------------------------------------------------------------------------------------------
 // u32 division by a launch-time constant: q = (n * m) >> (32 + s), exact for all n < 2^32 (round-up method)

@@ -1278,14 +1278,16 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
 //     [16384,264] 9.5 / 10.1), from 3072 columns where its steps are not full ([10240,3840] 35.5 / 32.8, [16384,4608] 58.5 / 57.1; [12288,3072] 28.9 / 30.1,
 //     [7200,4096] 24.3 / 26.5) or are many ([8192,5120] 37.1 / 35.5, [32768,5120] 123 / 119; [7200,5120] 29.9 / 32.1), and where it shares
 //     lines between rows ([12288,4088] 46.4 / 40.7, [12288,5112] 61.6 / 50.3).
-// The sum of x is small against its terms, and of rows with no mean it is nearly all rounding: f16 rows of that kind stay open all of them, bf16 ones one
-// in six, 4 us a wave for 2560 columns.
-//   LayerNorm f16: nowhere (N(0, 1) [32768,1280] 38.7 / 34.2, but c 38.6 / 68; [1024,2560] 12.2 / 12.2, c 12.2 / 15.5; [16,2560] 11.6 / 7.8, c 11.6 / 12.1).
-//   LayerNorm bf16: in small numbers, where the walk's latency is the launch ([1024,2560] 14.6 / 9.4, c 14.7 / 13.0; [1024,264] 6.2 / 4.8, c 6.1 / 5.3;
-//     [1024,5120] 22.9 / 16.0, c 23.0 / 24.0; [2048,1024] 8.1 / 6.9, c 8.2 / 8.9), and in large ones where a quarter of the walk's steps is empty
-//     ([8192,1280] 20.1 / 14.6, c 20.2 / 18.2, o 20.2 / 19.1; [6144,1280] 13.0 / 12.4, c 12.9 / 16.5; [10240,2560] 33.2 / 25.5, c 33.2 / 31.1, o 33.3 / 33.7;
-//     [30000,2560] c 70.7 / 67.2, o 70.6 / 75.3; [8192,1792] 22.4 / 17.8, c 22.3 / 22.4, o 22.4 / 23.9; [8192,3072] 32.5 / 25.6, c 32.5 / 32.2, o 32.6 / 35.0).
-//     (Rows of values and their negatives, whose sum is zero but for the roundings on the way, are open all of them and lose there: [8192,1280] 20.2 / 23.9.)
+// The sum of x is small against its terms, and of rows with no mean it is nearly all rounding: f16 rows of that kind are added in order all of them, bf16 ones one
+// in six, 3 us a wave for 2560 columns.  A line holds for rows of N(0, 1), c and o alike.  (Rows of values and their negatives, whose sum is zero but for the
+// roundings on the way, are added in order all of them; they lose where the others gain little: bf16 [1536,1280] 9.5 / 10.8, [16384,2560] 47.6 / 59.5.)
+//   LayerNorm f16: up to a row a CU, where the walk's latency is the launch and ordered rows take as long ([256,2560] 11.8 / 8.7, c 11.9 / 11.1; [16,4608] 18.5 / 10.7, c 18.5 / 17.0;
+//     [256,4096] 15.6 / 15.4, c 15.6 / 16.3; [256,640] 5.4 / 4.7, c 5.4 / 6.0; [512,1280] 7.2 / 6.2, c 7.2 / 8.2).
+//   LayerNorm bf16: up to 4 rows a CU ([1024,2560] 14.6 / 8.8, c 14.5 / 11.2; [1024,5120] 22.6 / 15.5, c 22.6 / 20.5), up to 11 of up to 3072 columns
+//     ([2048,2560] 14.8 / 11.6, c 14.9 / 11.9, o 14.8 / 13.7; [2816,1408] 12.2 / 9.9, c 12.3 / 10.2; but [3584,1408] c 12.6 / 12.3, o 12.5 / 13.7, [2048,4096] c 19.4 / 22.3); where three of
+//     the walk's blocks fit a CU, at 16 to 24 rows ([4608,904] 15.6 / 10.4, c 15.6 / 11.7); and in large numbers where a quarter of the walk's steps is
+//     empty ([9000,1408] 25.3 / 19.1, c 25.5 / 21.2, o 25.2 / 21.3; [8192,1280] 20.3 / 18.9, c 20.3 / 20.7, o 20.3 / 23.4; [8192,2560] 31.1 / 22.4, c 30.8 / 26.7, o 30.9 / 28.8;
+//     [20000,2688] 59.3 / 54.7, c 59.4 / 63.3, o 59.4 / 68.5).
 inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
     if (cols <= 256 || cols > NR_MAX_COLS || rows > NR_MAX_ROWS) return false;
     if (!layer) {
@@ -1295,22 +1297,23 @@ inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64
         if (cols >= 3072) return rows > 28 * cus && (!lines || nt != nf_steps(nt) || (cols > 4864 && rows > 30 * cus));
         return cols >= 320 && rows > (!lines || cols <= 512 ? 48 : 60) * cus;
     }
-    if (!bf16) return false;
-    if (rows <= (cols <= 4096 ? 4 : 3) * cus) return true;
-    if (cols > 1024 && cols <= 1536) return rows > 28 * cus;
+    if (!bf16) return rows <= cus / 16 || (cols <= 3584 && rows <= (cols > 384 && cols <= 768 ? cus / 2 : cus));
+    if (rows <= 4 * cus) return true;
+    if (rows <= 11 * cus) return cols <= 3072;
+    if (rows > 16 * cus && rows <= 24 * cus) return cols > 768 && cols <= 1024;
+    if (cols > 1024 && cols <= 1536) return rows > 32 * cus;
     return cols > 2048 && cols <= 2560 && rows > 30 * cus && rows <= 64 * cus;
 }
 // Where norm_flow16_kernel takes the rest of them, against norm_pipe16_kernel, whose blocks of 8 rows share the CUs and overlap one another,
 // while rows fit the chip in a few rounds, and which needs no empty steps.  Many rows come to memory, which that one
 // reads twice (LayerNorm f16 [12288,1024] 16.4 / 12.2, [24000,2560] 62 / 51).  Up to 40 rows a CU, f16 gains on rows of more than 3072 columns
 // that fill the steps (RMSNorm [7000,4096] 27.8 / 23.5, against [5000,3328] 17.6 / 18.9).  bf16 LayerNorm, whose walker
-// needs the f32 tiles of both sums, gains in a single round of 8 rows a block ([2048,2560] 16.3 / 14.6, not three tiles in
-// four steps or five in eight: [2048,1280] 9.7 / 10.2) and once its blocks of 8 rows no longer keep their rows in LDS
-// ([7000,2560] 35 / 25.6; [5000,2560] 21.3 / 25.8), except for short rows and for 9000 to 10000 rows in steps a quarter empty ([9000,1792] 29.4 / 27.9).
+// needs the f32 tiles of both sums, gains in a single round of 8 rows a block (measured at [2048,2560] 16.3 / 14.6, which the wave per row now takes)
+// and once its blocks of 8 rows no longer keep their rows in LDS ([7000,2560] 35 / 25.6; [5000,2560] 21.3 / 25.8), except for short rows and for 9000 to 10000 rows in steps a quarter empty ([9000,1792] 29.4 / 27.9).
 inline bool nf_takes_aligned(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64_t cus) {
     const uint32_t nt = (cols + 255) / 256, steps = nf_steps(nt);
     if (bf16 && layer) {
-        if (rows <= 8 * cus) return cols > 768 && nt != 5;
+        if (rows <= 8 * cus) return cols > 3072;
         if (rows <= 16 * cus) return cols > 3328;
         if (rows <= 24 * cus || cols <= 128) return false;
         if (cols <= 256) return rows > 48 * cus;
@@ -1359,8 +1362,7 @@ int launch_norm16(rt_device* dev, const void* x, const void* scale, const void* 
     if (vec_ok && cols <= 128 && rows >= 16384) return launch_norm16_lane<T, KIND>(dev, x, scale, bias, y, rows, cols, eps);
     const uint64_t cus = (uint64_t)dev->num_cus;
     constexpr bool BF16 = std::is_same<T, bf16_t>::value, LAYER = KIND == NORM_LAYER;
-    if (vec_ok && nr_takes(BF16, LAYER, rows, cols, cus))
-        return LAYER ? rt_layer_norm_bf16_row(dev, x, scale, bias, y, rows, cols, eps) : rt_rms_norm16_row(dev, BF16, x, scale, y, rows, cols, eps);
+    if (vec_ok && nr_takes(BF16, LAYER, rows, cols, cus)) return rt_norm16_row(dev, BF16, KIND, x, scale, bias, y, rows, cols, eps);
     if (cols >= 8 && cols <= NF_MAX_COLS &&
         (vec_ok ? nf_takes_aligned(BF16, LAYER, rows, cols, cus) : nf_takes_ragged(BF16, LAYER, rows, cols, cus))) {
         // rows a block walks at one time: 30 fill its 1024 threads and the walker's lanes; fewer where that takes no more

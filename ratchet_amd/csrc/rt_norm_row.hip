@@ -1,11 +1,11 @@
-// The 16-bit RMSNorm and the bf16 LayerNorm with a wave per row (arithmetic contract: rt_norm.hip).
+// The 16-bit LayerNorm / RMSNorm with a wave per row (arithmetic contract: rt_norm.hip).
 #include "rt_norm.h"
 #include "rt_ordered.h"
 
 namespace {
 
 // ------------------------------------------------------------------------------------------------------------------
-// RMSNorm in the 16-bit types and LayerNorm in bf16, one wave per row, the row in registers: the reference's sums without a walk.
+// LayerNorm / RMSNorm in the 16-bit types, one wave per row, the row in registers: the reference's sums without a walk.
 //
 // The reference adds x and T(x*x) left to right in f32 and rounds each sum to T once (cpu/norm.rs:72-89, half's Sum).  What is needed is
 // therefore not the f32 sum but what it rounds to, and that is the same for almost every sum near it: this kernel adds in any order,
@@ -18,8 +18,8 @@ namespace {
 //        in those where the sum later grows into coarser binades, is at most u/2 + 2u/2 + 4u/2 + ... <= U.  The partial sums are bounded by a prefix
 //        sum over the lanes and the largest partial sum inside a lane's vector.  That bound does not shrink with the sum, and what the sum rounds to
 //        does: N(0, 1) rows of 2560 columns stay open one in a thousand, the same with their mean taken off one in six, rows whose sum is
-//        zero but for the roundings on the way all of them (f16, of whose terms more are not multiples of U: one in fifty, all, all; its LayerNorm walks).
-// Rows that stay open get the ordered sum itself (norm_ordered_squares, norm_ordered_sum), 2.5 and 4 us a wave for 2560 columns.
+//        zero but for the roundings on the way all of them (f16, of whose terms more are not multiples of U: one in fifty, all, all).
+// Rows that stay open get the ordered sum itself (norm_ordered_squares, norm_ordered_sum), 2.5 and 3 us a wave for 2560 columns.
 // What bounds it: memory where there are many rows ([16384,3072] bf16 RMSNorm 40.3 -> 36.9 us, a copy of its bytes 31.5), and in LayerNorm the vector
 // instructions, of which it takes twenty an element (47 -> 41 us); where there are few, launch, loads and the rows that stay open
 // ([256,2560] bf16 RMSNorm 14.3 -> 6.1 us).  A block is one wave: a row that takes longer then keeps no place but its own.
@@ -294,10 +294,11 @@ int launch_norm16_row(rt_device* dev, const void* x, const void* scale, const vo
 
 }  // namespace
 
-int rt_rms_norm16_row(rt_device* dev, bool bf16, const void* x, const void* scale, void* y, uint64_t rows, uint32_t cols, float eps) {
+int rt_norm16_row(rt_device* dev, bool bf16, int kind, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols,
+                  float eps) {
+    if (kind == NORM_LAYER)
+        return bf16 ? launch_norm16_row<bf16_t, NORM_LAYER>(dev, x, scale, bias, y, rows, cols, eps)
+                    : launch_norm16_row<half_t, NORM_LAYER>(dev, x, scale, bias, y, rows, cols, eps);
     return bf16 ? launch_norm16_row<bf16_t, NORM_RMS>(dev, x, scale, nullptr, y, rows, cols, eps)
                 : launch_norm16_row<half_t, NORM_RMS>(dev, x, scale, nullptr, y, rows, cols, eps);
-}
-int rt_layer_norm_bf16_row(rt_device* dev, const void* x, const void* scale, const void* bias, void* y, uint64_t rows, uint32_t cols, float eps) {
-    return launch_norm16_row<bf16_t, NORM_LAYER>(dev, x, scale, bias, y, rows, cols, eps);
 }
