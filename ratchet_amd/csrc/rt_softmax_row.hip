@@ -201,17 +201,18 @@ __device__ __forceinline__ void sr_transpose(v4u (&v)[4], uint32_t lane) {
 // A wave takes 64 / L rows: four of up to 2048 columns (L = 16 lanes to a row), two of up to 8192 (L = 32), held in registers from the load to the
 // store, and its waves never meet: no walker, no barriers.  A chunk is 32 L columns of each row, four vectors a lane.  The loads of the next
 // rows go out between the stores of these, into the registers that those free.  The exp table lies in LDS as in softmax16_stream_kernel.
-// What bounds it: a quarter of the time is the sums and their waits (without them, and wrong, [8,2048,8192] f16 takes 100 us of 114, with a mask 114 of 125), the
-// rest memory, which 16 free-running waves a CU use less evenly than the streaming kernel's paced steps do (5.1 against 6.2 TB/s on f16 [32,4096,4096]; held to a
-// pace these waves only get slower).  Several rows at a time because a row needs a pass for each chunk and for each power of two that its
-// sum passes, most of which fall together: with one row to a wave [8,2048,8192] bf16 took 159 us without a mask and 177 with one, now 122 and 139.
+// What bounds it: a tenth of the time is the sums and their waits (without them, and wrong, [8,2048,8192] f16 takes 100 us of 114, with a mask 114 of 125), the
+// rest memory, which 16 free-running waves a CU use less evenly than the streaming kernel's paced steps do (5.3 against 6.2 TB/s on f16 [32,4096,4096], 407 and 344 us; held
+// to a pace these waves only get slower).  Several rows at a time because a row needs a pass for each chunk and for each power of two that its
+// sum passes, most of which fall together: with one row to a wave [8,2048,8192] bf16 took 159 us without a mask and 177 with one, now 124 and 139.
 // bf16 pays five instructions an element and pass, f16 one.
 // ------------------------------------------------------------------------------------------------------------------
 constexpr uint32_t SR_NONE = 0x80000000u;                    // an offset outside every buffer, and so after adding a column's
 constexpr int sr_waves(int v) { return v <= 4 ? 16 : v <= 6 ? 12 : 8; }
 
-// Row i of the launch: with a mask the `reps` rows that share a mask row come one after the other, so that the groups of a wave and the
-// waves of a block read it at about the same time.
+// Row i of the launch: with a mask the `reps` rows that share a mask row come one after the other, in the groups of a wave and then in neighbouring
+// blocks, which read it at about the same time but on different XCDs: under eight heads two to a wave HBM is asked for it four times ([8,2048,8192] f16: 131 MiB
+// of reads for a mask of 32 MiB, by FETCH_SIZE).
 struct SrRows {
     uint32_t rows, cols, period, waves;                      // waves: of a block, that have rows
     FastDiv reps_div;                                        // reps = rows / period (1 without a mask)
