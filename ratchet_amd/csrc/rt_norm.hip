@@ -1282,7 +1282,8 @@ inline bool nf_takes_ragged(bool bf16, bool layer, uint64_t rows, uint32_t cols,
 // in six, 3 us a wave for 2560 columns.  A line holds for rows of N(0, 1), c and o alike.  (Rows of values and their negatives, whose sum is zero but for the
 // roundings on the way, are added in order all of them; they lose where the others gain little: bf16 [1536,1280] 9.5 / 10.8, [16384,2560] 47.6 / 59.5.)
 //   LayerNorm f16: up to a row a CU, where the walk's latency is the launch and ordered rows take as long ([256,2560] 11.8 / 8.7, c 11.9 / 11.1; [16,4608] 18.5 / 10.7, c 18.5 / 17.0;
-//     [256,4096] 15.6 / 15.4, c 15.6 / 16.3; [256,640] 5.4 / 4.7, c 5.4 / 6.0; [512,1280] 7.2 / 6.2, c 7.2 / 8.2).
+//     [256,4096] 15.6 / 15.4, c 15.6 / 16.3; [256,640] 5.4 / 4.7, c 5.4 / 5.9; [512,1280] 7.2 / 6.0, c 7.2 / 7.8), and up to 4 of one step and less
+//     ([1024,384] 4.7 / 3.8, c 4.7 / 4.4; [1024,512] 4.4 / 4.2, c 4.4 / 4.9).
 //   LayerNorm bf16: up to 4 rows a CU ([1024,2560] 14.6 / 8.8, c 14.5 / 11.2; [1024,5120] 22.6 / 15.5, c 22.6 / 20.5), up to 11 of up to 3072 columns
 //     ([2048,2560] 14.8 / 11.6, c 14.9 / 11.9, o 14.8 / 13.7; [2816,1408] 12.2 / 9.9, c 12.3 / 10.2; but [3584,1408] c 12.6 / 12.3, o 12.5 / 13.7, [2048,4096] c 19.4 / 22.3); where three of
 //     the walk's blocks fit a CU, at 16 to 24 rows ([4608,904] 15.6 / 10.4, c 15.6 / 11.7); and in large numbers where a quarter of the walk's steps is
@@ -1297,7 +1298,10 @@ inline bool nr_takes(bool bf16, bool layer, uint64_t rows, uint32_t cols, uint64
         if (cols >= 3072) return rows > 28 * cus && (!lines || nt != nf_steps(nt) || (cols > 4864 && rows > 30 * cus));
         return cols >= 320 && rows > (!lines || cols <= 512 ? 48 : 60) * cus;
     }
-    if (!bf16) return rows <= cus / 16 || (cols <= 3584 && rows <= (cols > 384 && cols <= 768 ? cus / 2 : cus));
+    if (!bf16) {
+        if (cols <= 448) return rows <= 4 * cus;
+        return rows <= cus / 16 || (cols <= 3584 && rows <= (cols <= 768 ? cus / 2 : cus));
+    }
     if (rows <= 4 * cus) return true;
     if (rows <= 11 * cus) return cols <= 3072;
     if (rows > 16 * cus && rows <= 24 * cus) return cols > 768 && cols <= 1024;
